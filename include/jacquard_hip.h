@@ -241,12 +241,14 @@ usize jq_wait_limit(usize polls);
 /* Synchronisation of value-only scan launches (no counterpart in the
  * reference, whose kernel always takes a grid barrier after each major
  * stage, csrc/kernel_v1_impl.cuh:565-626).  mode 1 (the default): every
- * launch without timing first derives from the script which blocks each
- * (block, major stage) reads, and a block then waits only for those
- * blocks' progress; launches of fewer than 8 cycles and scripts with more
- * than 256 blocks or 120 major stages still use grid barriers.  The
- * derived table is the one allocation these launches make: 4 bytes per
- * state word plus 256 bytes per (block, major stage), taken with
+ * launch without timing exchanges its words through a ring in which every
+ * word carries the number of its snapshot, and a block waits only for the
+ * words it reads.  Launches of fewer than 8 cycles and scripts that do not
+ * fit (a writeout word written twice, a read past the first writeout word
+ * of a word that no partition writes or that is written in the same or a
+ * later major stage) still use grid barriers.  The ring and what its
+ * builders find in the script are the one allocation these launches make:
+ * 68 bytes per state word plus 128 per block, taken with
  * hipMallocAsync on the launch's stream and released with hipFreeAsync
  * after it (if the allocation fails, the launch uses grid barriers, and so
  * does a launch issued while its stream is being captured into a graph).

@@ -290,16 +290,16 @@ __device__ void io_step(const CosimArgs &A) {
 constexpr u32 kCopyBatch = 8;
 __device__ __forceinline__ void copy_words(u32 *dst, const u32 *src, u32 n, u32 t,
                                            bool coherent) {
-  for (u32 base = t; base < n; base += 256 * kCopyBatch) {
+  for (u32 base = t; base < n; base += blockDim.x * kCopyBatch) {
     u32 v[kCopyBatch];
 #pragma unroll
     for (u32 k = 0; k < kCopyBatch; ++k) {
-      const u32 i = base + 256 * k;
+      const u32 i = base + blockDim.x * k;
       v[k] = i < n ? ld_coherent(src + i) : 0u;
     }
 #pragma unroll
     for (u32 k = 0; k < kCopyBatch; ++k) {
-      const u32 i = base + 256 * k;
+      const u32 i = base + blockDim.x * k;
       if (i < n) {
         if (coherent)
           st_coherent(dst + i, v[k]);
@@ -368,16 +368,16 @@ __device__ void between_phase(const CosimArgs &A, u32 t, u32 b, u32 nb, u32 e) {
   const u32 pe = (u32)(((usize)A.sched_offset + e) % A.num_sched);
   const u32 ob = A.op_start[pe], oe = A.op_start[pe + 1];
   const u32 dbits = s_din;
-  for (u32 base = lo + t; base < hi; base += 256 * kCopyBatch) {
+  for (u32 base = lo + t; base < hi; base += blockDim.x * kCopyBatch) {
     u32 v[kCopyBatch];
 #pragma unroll
     for (u32 k = 0; k < kCopyBatch; ++k) {
-      const u32 i = base + 256 * k;
+      const u32 i = base + blockDim.x * k;
       v[k] = i < hi ? ld_coherent(A.states + A.ss + i) : 0u;
     }
 #pragma unroll
     for (u32 k = 0; k < kCopyBatch; ++k) {
-      const u32 i = base + 256 * k;
+      const u32 i = base + blockDim.x * k;
       if (i >= hi) continue;
       u32 w = v[k];
       for (u32 j = ob; j < oe; ++j) {

@@ -1,18 +1,17 @@
-// Plain drop-in interpreter for gfx950 (wave64, 4 waves per workgroup).
+// Plain drop-in interpreter for gfx950 (wave64, 8 waves per workgroup).
 //
 // One workgroup per script block, persistent over all cycles and major
 // stages, a grid barrier after every major stage (the contract of
-// csrc/kernel_v1_impl.cuh:565-626) or, in value-only launches, a wait for
-// just the blocks whose words the next stage reads.  Inside a partition the
-// work is mapped to CDNA4 as follows:
-//   - script sections are streamed with 16-byte per-thread loads (each
-//     section is one fully coalesced 4 KiB request), the next boomerang
-//     stage's permutation words are in flight while the current tree runs,
-//     and a partition's prologue loads are issued before the barrier that
-//     precedes it;
+// csrc/kernel_v1_impl.cuh:565-626) or, in value-only launches, waits on the
+// very words the partition reads.  Inside a partition the work is mapped to
+// CDNA4 as follows:
+//   - script sections are streamed with 16-byte per-thread loads, each
+//     issued as soon as the registers of its predecessor are free: the next
+//     boomerang stage's (or partition's) words are in flight while the
+//     current tree runs, and headers are requested two partitions ahead;
 //   - snapshot words move between workgroups only through agent-coherent
 //     loads and stores, so the grid barrier carries no cache maintenance;
-//   - the 8192-bit shuffle is 32 LDS bit-gathers per thread on all 4 waves;
+//   - the 8192-bit shuffle is 16 LDS bit-gathers per thread on all 8 waves;
 //   - the whole AND tree (hier 0..7 and the in-word tail) runs in wave 0
 //     with permlane / DPP cross-lane moves, so a boomerang stage costs two
 //     workgroup barriers instead of one per tree level;
@@ -36,12 +35,6 @@ namespace jqd {
 __device__ u32 g_barrier[kCohSlots * kCohSlotWords];
 __device__ u32 g_error;
 __device__ u32 g_wait_polls = kDefaultWaitPolls;  // bound of every wait here
-// progress words of the dataflow-synchronised launches: per barrier slot,
-// 256 words one 128-byte line apart (packed into 8 lines, every block's
-// polls and the producers' stores met on the same lines, and the 1M-gate
-// launch ran 20% slower than with grid barriers)
-constexpr u32 kProgStride = 32;
-__device__ u32 g_prog[kCohSlots * 256 * kProgStride];
 
 namespace {
 
@@ -52,6 +45,8 @@ struct Ev {
   u32 type, msg, cycle, r;
   u32 data[4];
 };
+
+using u64 = unsigned long long;
 
 struct ScanArgs {
   u32 num_blocks, num_major_stages;
@@ -68,11 +63,11 @@ struct ScanArgs {
   u32 ev_cap;
   i32 arrival_state_offset;
   u32 *bar;
-  // dataflow synchronisation (value-only launches): the producer table of
-  // build_flow_tables, the flag its builders raise when a script does not
-  // fit it, and the blocks' progress words; dep == null: grid barriers
-  const u32 *dep;
-  const u32 *dep_bad;
+  // dataflow synchronisation (value-only launches, see below): the exchange
+  // ring, what its builders found in the script and the blocks' completed
+  // cycles; ring == null: grid barriers
+  u64 *ring;
+  const u32 *flow;  // kFlow* words
   u32 *prog;
   // profiling
   const u32 *part_index;
@@ -85,20 +80,38 @@ __device__ __forceinline__ uint4 ld4(const u32 *p) {
   return *reinterpret_cast<const uint4 *>(p);
 }
 
-// 32 LDS bit-gathers: word bit 2k (2k+1) <- src bit lo16 (hi16) of perm
-// word k (src/flatten.rs:1027-1034).
-__device__ __forceinline__ u32 gather_bits(const u32 *src, uint4 q0, uint4 q1,
-                                           uint4 q2, uint4 q3) {
+// Threads of a workgroup: two adjacent lanes per word of the 256-word
+// layer, half 0 its bits 0..15 (and the first half of its global-read
+// rounds), half 1 the rest.  A partition is a chain of short steps that one
+// workgroup per CU runs alone, so what counts is the length of the chain:
+// with one thread per word the 32 LDS bit-gathers and the pext loop were
+// twice as long, and each SIMD had a single wave to issue from.  Two
+// threads also halve the registers a thread needs for prefetched words
+// (218 of the 256 that two waves per SIMD leave; one thread per word had
+// spilled).  Measured together with the earlier loads, in launches that keep
+// grid barriers: 4M gates with X and timing, 248 -> 202 us per cycle; one
+// co-simulation edge of a one-block design, 12.1 -> 10.5 us.
+constexpr int kScanThreads = 512;
+
+// Value of the other lane of a thread's pair (DPP quad_perm 1,0,3,2).
+__device__ __forceinline__ u32 from_pair(u32 v) {
+  return __builtin_amdgcn_update_dpp(0u, v, 0xB1, 0xF, 0xF, false);
+}
+
+// The 32 LDS bit-gathers of a word, 16 in each thread of its pair: bit 2k
+// (2k+1) of a half <- src bit lo16 (hi16) of its perm word k
+// (src/flatten.rs:1027-1034).  Both threads return the whole word.
+__device__ __forceinline__ u32 gather_bits(const u32 *src, uint4 qa, uint4 qb) {
   u32 r = 0;
-  const u32 w[16] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w,
-                     q2.x, q2.y, q2.z, q2.w, q3.x, q3.y, q3.z, q3.w};
+  const u32 w[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
 #pragma unroll
-  for (int k = 0; k < 16; ++k) {
+  for (int k = 0; k < 8; ++k) {
     u32 i1 = w[k] & 0xffffu, i2 = w[k] >> 16;
     r |= ((src[i1 >> 5] >> (i1 & 31)) & 1u) << (2 * k);
     r |= ((src[i2 >> 5] >> (i2 & 31)) & 1u) << (2 * k + 1);
   }
-  return r;
+  const u32 o = from_pair(r);
+  return (threadIdx.x & 1) ? (r << 16) | o : (o << 16) | r;
 }
 
 __device__ __forceinline__ u16 arr_step(u16 a, u16 b, u32 ob, u32 dly) {
@@ -124,8 +137,8 @@ __device__ __forceinline__ void push_event(EvHdr *ev, u32 cap, u32 type,
   }
 }
 
-// Header of one partition (src/flatten.rs:198-258) and this thread's
-// writeout hook; `base` is the header's word offset in blocks_data.
+// Header of one partition (src/flatten.rs:198-258) and the writeout hook of
+// this thread's word; `base` is the header's word offset in blocks_data.
 struct PartHdr {
   size_t base;
   u32 num_stages, is_last, num_ios, io_offset, num_srams, sram_offset, rounds,
@@ -133,22 +146,42 @@ struct PartHdr {
   bool is_x;
 };
 
-__device__ __forceinline__ PartHdr load_hdr(const u32 *__restrict__ bd, size_t off) {
-  PartHdr h;
+// The same as it comes from memory.  Nothing here looks at the words, so
+// their loads stay in flight until settle() is called, a partition later.
+struct RawHdr {
+  size_t base;
+  uint4 a, b;
+  uint2 x;
+  u32 hook;
+};
+
+__device__ __forceinline__ RawHdr load_hdr(const u32 *__restrict__ bd, size_t off) {
+  RawHdr r;
   const u32 *s = bd + off;
-  h.base = off;
-  h.num_stages = s[0];
-  h.is_last = s[1];
-  h.num_ios = s[2];
-  h.io_offset = s[3];
-  h.num_srams = s[4];
-  h.sram_offset = s[5];
-  h.rounds = s[6];
-  h.num_dups = s[7];
-  h.is_x = s[8] != 0;
-  h.xoff = s[9];
-  const u32 hook = s[128 + (threadIdx.x >> 1)];
-  h.hook = (threadIdx.x & 1) ? (hook >> 16) : (hook & 0xffffu);
+  r.base = off;
+  r.a = ld4(s);
+  r.b = ld4(s + 4);
+  r.x = *reinterpret_cast<const uint2 *>(s + 8);
+  r.hook = s[128 + (threadIdx.x >> 2)];
+  return r;
+}
+
+__device__ __forceinline__ u32 uniform(u32 v) { return __builtin_amdgcn_readfirstlane(v); }
+
+__device__ __forceinline__ PartHdr settle(const RawHdr &r) {
+  PartHdr h;
+  h.base = r.base;
+  h.num_stages = uniform(r.a.x);
+  h.is_last = uniform(r.a.y);
+  h.num_ios = uniform(r.a.z);
+  h.io_offset = uniform(r.a.w);
+  h.num_srams = uniform(r.b.x);
+  h.sram_offset = uniform(r.b.y);
+  h.rounds = uniform(r.b.z);
+  h.num_dups = uniform(r.b.w);
+  h.is_x = uniform(r.x.x) != 0;
+  h.xoff = uniform(r.x.y);
+  h.hook = (threadIdx.x & 2) ? (r.hook >> 16) : (r.hook & 0xffffu);
   return h;
 }
 
@@ -162,60 +195,201 @@ __device__ __forceinline__ size_t part_words(const PartHdr &h) {
   return 256 + (size_t)512 * h.rounds + (size_t)5120 * (h.num_stages + 2);
 }
 
-// Everything a partition loads before its state gather: the global-read
-// entries (up to kPreRounds rounds), the stage-0 permutation and wave 0's
-// stage-0 tree flags, both writeout permutation sections and the commit's
-// old values.  Script words are read-only and the old values are the
-// partition's own writeouts of the previous cycle, so these loads are
-// issued before the barrier that precedes the partition, and their latency
-// hides behind the barrier wait (or the previous partition of the block).
-constexpr u32 kPreRounds = 16;
+// What a partition holds before its state gather: the global-read entries
+// (up to kPreRounds rounds of each thread's half), the stage-0 permutation
+// and wave 0's stage-0 tree flags.  They are read-only script words, so each
+// is loaded for the next partition as soon as the current one has used its
+// own, and lands while the rest of the current partition and its wait run.
+constexpr u32 kPreRounds = 8;
 struct PartPre {
   uint2 e[kPreRounds];
-  uint4 q0, q1, q2, q3, fA, fB, fC, fD;
-  uint4 sd0, sd1, sd2, sd3, sdf, ck0, ck1, ck2, ck3, ckf;
-  u32 old_v, old_x;
+  uint4 qa, qb, fA, fB, fC, fD;
 };
 
-__device__ __forceinline__ void load_pre(PartPre &P, const u32 *__restrict__ bd,
-                                         const PartHdr &h, const u32 *in) {
-  const int t = threadIdx.x;
-  const int lane = t & 63;
-  const size_t pi = h.base + 256;
-  const uint2 *gr = reinterpret_cast<const uint2 *>(bd + pi);
+// The global-read rounds of this thread: of a word's rounds the first
+// (rounds + 1) / 2 go to half 0, the others to half 1.
+__device__ __forceinline__ u32 first_round(u32 rounds) {
+  return (threadIdx.x & 1) ? (rounds + 1) / 2 : 0;
+}
+__device__ __forceinline__ u32 num_rounds(u32 rounds) {
+  return (threadIdx.x & 1) ? rounds / 2 : (rounds + 1) / 2;
+}
+
+__device__ __forceinline__ void load_entries(PartPre &P, const u32 *__restrict__ bd,
+                                             const PartHdr &h) {
+  const uint2 *gr = reinterpret_cast<const uint2 *>(bd + h.base + 256) +
+                    256 * first_round(h.rounds) + (threadIdx.x >> 1);
+  const u32 n = num_rounds(h.rounds), most = (h.rounds + 1) / 2;
 #pragma unroll
-  for (u32 k = 0; k < kPreRounds; ++k)
-    P.e[k] = (k < h.rounds) ? gr[256 * k + t] : make_uint2(0, 0);
-  const size_t p_st = pi + (size_t)512 * h.rounds;
-  const size_t p_sd = p_st + (size_t)5120 * h.num_stages;
-  const size_t p_ck = p_sd + 5120;
-  P.q0 = ld4(bd + p_st + 4 * t);
-  P.q1 = ld4(bd + p_st + 1024 + 4 * t);
-  P.q2 = ld4(bd + p_st + 2048 + 4 * t);
-  P.q3 = ld4(bd + p_st + 3072 + 4 * t);
-  // wave 0's tree flags of stage 0 (words 0..255 of the flag block)
-  P.fA = P.fB = P.fC = P.fD = make_uint4(0, 0, 0, 0);
-  if (t < 64) {
-    const u32 *fl0 = bd + p_st + 4096;
-    P.fA = ld4(fl0 + 4 * lane);
-    P.fB = ld4(fl0 + 4 * (64 + lane));
-    P.fC = ld4(fl0 + 4 * (128 + lane));
-    P.fD = ld4(fl0 + 4 * (192 + lane));
+  for (u32 k = 0; k < kPreRounds; ++k) {
+    P.e[k] = make_uint2(0, 0);
+    if (k < most) {  // uniform
+      if (k < n) P.e[k] = gr[256 * k];
+    }
   }
-  P.sd0 = ld4(bd + p_sd + 4 * t);
-  P.sd1 = ld4(bd + p_sd + 1024 + 4 * t);
-  P.sd2 = ld4(bd + p_sd + 2048 + 4 * t);
-  P.sd3 = ld4(bd + p_sd + 3072 + 4 * t);
-  P.sdf = ld4(bd + p_sd + 4096 + 4 * t);
-  P.ck0 = ld4(bd + p_ck + 4 * t);
-  P.ck1 = ld4(bd + p_ck + 1024 + 4 * t);
-  P.ck2 = ld4(bd + p_ck + 2048 + 4 * t);
-  P.ck3 = ld4(bd + p_ck + 3072 + 4 * t);
-  P.ckf = ld4(bd + p_ck + 4096 + 4 * t);
-  P.old_v = P.old_x = 0;
-  if ((u32)t < h.num_ios) {
-    P.old_v = ld_coherent(in + h.io_offset + (u32)t);
-    if (h.is_x) P.old_x = ld_coherent(in + h.xoff + h.io_offset + (u32)t);
+}
+
+// The stage section at `st`: this thread's permutation words and, on wave
+// 0, the tree flags (words 0..255 of the flag block).
+__device__ __forceinline__ void load_stage(PartPre &P, const u32 *__restrict__ st) {
+  const int t = threadIdx.x;
+  const u32 *q = st + 2048 * (t & 1) + 4 * (t >> 1);
+  P.qa = ld4(q);
+  P.qb = ld4(q + 1024);
+  if (t < 64) {
+    const u32 *fl = st + 4096;
+    P.fA = ld4(fl + 4 * t);
+    P.fB = ld4(fl + 4 * (64 + t));
+    P.fC = ld4(fl + 4 * (128 + t));
+    P.fD = ld4(fl + 4 * (192 + t));
+  }
+}
+
+// First stage section of a partition.
+__device__ __forceinline__ const u32 *stage0(const u32 *__restrict__ bd, const PartHdr &h) {
+  return bd + h.base + 256 + (size_t)512 * h.rounds;
+}
+
+// ---- dataflow synchronisation of value-only launches
+//
+// Partitions read snapshot words that other blocks wrote in an earlier
+// major stage of the same cycle (`out`, bit 31 of a global-read entry) or
+// in any stage of the previous cycle (`in`); every cycle has its own
+// snapshot and SRAMs belong to one partition, so those reads are the only
+// dependencies between blocks.  Every commit therefore also stores its word
+// with the number of the snapshot it belongs to, as one 8-byte word, in an
+// exchange ring of kRing snapshots, and a gather reads the ring and repeats
+// the loads whose snapshot number is not there yet.  The word is its own
+// flag: a stage costs one store and one load across the chip, where a
+// barrier (or progress words) needs the stores to complete, a flag to
+// follow them, its poll, and only then the load.  Measured with the two
+// threads per word and the script words loaded a partition ahead (below):
+// 1M-gate netlist, 249 blocks, 11 major stages, 90.6 us per cycle with
+// progress words, 63.0 with the ring.
+//
+// Slot s % kRing of the ring is written again kRing snapshots later.  Each
+// block publishes the cycles it has completed and, every kRing / 2 cycles,
+// waits until no block is so far behind that one of the next kRing / 2
+// commits could overwrite a word it has still to read (flow_room).
+//
+// Words below the first writeout word are primary inputs, filled in by the
+// host before the launch; those, and all of snapshot 0, are read from the
+// snapshot buffer.
+constexpr u32 kRing = 8;
+constexpr u32 kFlowMinCycles = 8;
+// what the builders leave in ScanArgs::flow
+constexpr u32 kFlowNegLo = 0;  // ~(first writeout word), 0 when there is none
+constexpr u32 kFlowXoff = 1;   // X mask offset of the X-capable partitions, or 0
+constexpr u32 kFlowBad = 2;    // nonzero: the script does not fit, grid barriers
+constexpr u32 kFlowWords = 64;
+constexpr u32 kProgStride = 32;  // one progress word per 128-byte line
+
+struct Flow {
+  u64 *ring;
+  u32 slot;       // words of one ring slot (the state size)
+  u32 lo, xoff;   // first writeout word; X mask offset of the launch or 0
+  u32 *bar, *aborted;
+};
+
+__device__ __forceinline__ u64 ld_coherent64(const u64 *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void st_coherent64(u64 *p, u64 v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// One failed poll of a wave: sleeps, and ends the wait (true) past the poll
+// limit, aborting the launch, or when the launch has aborted (read every 256
+// polls).  Wave-uniform.
+__device__ __forceinline__ bool flow_gives_up(const Flow &F, u32 &spins) {
+  __builtin_amdgcn_s_sleep(1);
+  ++spins;
+  bool stop = false;
+  if (spins > g_wait_polls) {
+    abort_launch(F.bar, &g_error);
+    stop = true;
+  } else if ((spins & 255u) == 0 && ld_coherent(&F.bar[kAbortWord]) != 0) {
+    stop = true;
+  }
+  if (stop) *F.aborted = 1;
+  return stop;
+}
+
+// The state words of the entries e (cycle c, snapshots in and out) into v
+// and, for X-capable partitions, their X masks into x.
+template <bool X>
+__device__ __forceinline__ void flow_gather(const Flow &F, const uint2 *e, const u32 *in,
+                                            const u32 *out, u32 c, u32 *v, u32 *x) {
+  u32 pend = 0;  // bit k: entry k's value, bit 16 + k: its X mask
+#pragma unroll
+  for (u32 k = 0; k < kPreRounds; ++k) {
+    v[k] = 0;
+    if (X) x[k] = 0;
+    if (e[k].y) {
+      const u32 w = e[k].x & 0x7fffffffu, o = e[k].x >> 31;
+      if (w >= F.lo && (o | c)) {
+        pend |= (X ? 0x10001u : 1u) << k;
+      } else {
+        const u32 *base = o ? out : in;
+        v[k] = base[w];
+        if (X) x[k] = base[F.xoff + w];
+      }
+    }
+  }
+  u32 spins = 0;
+  for (;;) {
+    u64 q[kPreRounds], r[X ? kPreRounds : 1];
+#pragma unroll
+    for (u32 k = 0; k < kPreRounds; ++k) {
+      const u32 w = e[k].x & 0x7fffffffu, s = c + (e[k].x >> 31);
+      const u64 *a = F.ring + ((s & (kRing - 1)) * F.slot + w);
+      if ((pend >> k) & 1u) q[k] = ld_coherent64(a);
+      if (X && ((pend >> (16 + k)) & 1u)) r[k] = ld_coherent64(a + F.xoff);
+    }
+#pragma unroll
+    for (u32 k = 0; k < kPreRounds; ++k) {
+      const u32 s = c + (e[k].x >> 31);
+      if (((pend >> k) & 1u) && (u32)(q[k] >> 32) == s) {
+        v[k] = (u32)q[k];
+        pend &= ~(1u << k);
+      }
+      if (X && ((pend >> (16 + k)) & 1u) && (u32)(r[k] >> 32) == s) {
+        x[k] = (u32)r[k];
+        pend &= ~(0x10000u << k);
+      }
+    }
+    if (!__any(pend)) return;
+    if (flow_gives_up(F, spins)) return;
+  }
+}
+
+// State word w of snapshot in (o = 0) or out (o = 1) of cycle c, for the
+// rounds past kPreRounds; `off` is 0 or the X mask offset.  Every lane of
+// the wave calls it; `need` lanes get their word.
+__device__ __forceinline__ u32 flow_word(const Flow &F, bool need, u32 w, u32 o, u32 off,
+                                         const u32 *in, const u32 *out, u32 c) {
+  if (!need) return 0;
+  if (w < F.lo || !(o | c)) return (o ? out : in)[off + w];
+  const u32 s = c + o;
+  const u64 *a = F.ring + ((s & (kRing - 1)) * F.slot + off + w);
+  u32 spins = 0;
+  for (;;) {
+    const u64 q = ld_coherent64(a);
+    if ((u32)(q >> 32) == s) return (u32)q;
+    if (flow_gives_up(F, spins)) return 0;
+  }
+}
+
+// Before cycle c (a multiple of kRing / 2): the commits of cycles c ..
+// c + kRing / 2 - 1 overwrite snapshots up to c + kRing / 2 - kRing, last
+// read in the cycle of that number, so every block must have completed it.
+// The block that is furthest behind never waits here.
+__device__ __forceinline__ void flow_room(const Flow &F, const u32 *prog, u32 nb, u32 c) {
+  if (threadIdx.x < 64) {
+    u32 spins = 0;
+    for (u32 i = threadIdx.x; __any(i < nb); i += 64)
+      while (__any(i < nb && ld_coherent(&prog[i * kProgStride]) + (kRing / 2 - 1) < c))
+        if (flow_gives_up(F, spins)) return;
   }
 }
 
@@ -263,17 +437,22 @@ __device__ __forceinline__ void tree_level(u32 &cur, u32 &curx, u16 &cura, const
 }
 
 // One partition (src/sim/cpu_reference.rs:25-262 per partition;
-// kernel_v1_impl.cuh:62-558), its prologue loads already in P.
-template <bool TIMING, bool PROFILE>
-__device__ void run_partition(const ScanArgs &A, const u32 *__restrict__ bd,
-                              const PartHdr &h, PartPre &P,
-                              const u32 *__restrict__ in, u32 *__restrict__ out,
+// kernel_v1_impl.cuh:62-558), its prologue loads already in P; `hn` is the
+// block's next partition (num_stages 0: none), whose prologue replaces them.
+template <bool TIMING, bool PROFILE, bool FLOW>
+__device__ __forceinline__ void run_partition(const ScanArgs &A, const u32 *__restrict__ bd,
+                              const PartHdr &h, const PartHdr &hn, PartPre &P,
+                              const Flow &F, const u32 *__restrict__ in,
+                              u32 *__restrict__ out,
                               u32 cycle, u32 part, u32 *st_v, u32 *st_x,
                               u32 *hin_v, u32 *hin_x, u32 *wo_v, u32 *wo_x,
                               u16 *st_arr, u16 *wo_arr) {
-  const int t = threadIdx.x;
-  const int lane = t & 63;
-  const bool w0 = t < 64;
+  const int lane = threadIdx.x & 63;
+  const bool w0 = threadIdx.x < 64;
+  // the thread's word, and its first thread
+  const int t = threadIdx.x >> 1;
+  const bool h0 = (threadIdx.x & 1) == 0;
+  const u32 *pq = bd + 2048 * (threadIdx.x & 1) + 4 * t;  // its permutation words
   long long t_start = 0;
   if (PROFILE) t_start = clock64();
   const u32 num_stages = h.num_stages;
@@ -287,30 +466,60 @@ __device__ void run_partition(const ScanArgs &A, const u32 *__restrict__ bd,
   const u32 xoff = h.xoff;
   const u32 hook = h.hook;
   const u32 *script = bd + h.base;
-  size_t pi = 256;
-  const uint2 *gr = reinterpret_cast<const uint2 *>(script + pi);
+  const uint2 *gr = reinterpret_cast<const uint2 *>(script + 256);
   const uint2 *e = P.e;
-  uint4 q0 = P.q0, q1 = P.q1, q2 = P.q2, q3 = P.q3;
-  uint4 fA = P.fA, fB = P.fB, fC = P.fC, fD = P.fD;
-  const uint4 sd0 = P.sd0, sd1 = P.sd1, sd2 = P.sd2, sd3 = P.sd3, sdf = P.sdf;
-  const uint4 ck0 = P.ck0, ck1 = P.ck1, ck2 = P.ck2, ck3 = P.ck3, ckf = P.ckf;
-  const u32 old_v = P.old_v, old_x = P.old_x;
-  const size_t p_st = pi + (size_t)512 * rounds;
+  const u32 *p_st = stage0(bd, h);                        // this stage's section
+  const u32 *p_sd = p_st + (size_t)5120 * num_stages;     // SRAM/dup section
+  const u32 *p_ck = p_sd + 5120;                          // clock-enable section
+  const u32 nperm = num_srams * 4 + num_dups;
+  uint4 sda, sdb, sdf, cka, ckb, ckf;
+  u32 old_v = 0, old_x = 0;
 
-    // ---- global read (pext-gather), kernel_v1_impl.cuh:87-151: the state
-    // words are gathered now, after the barrier that published them
-    u32 acc_v = 0, acc_x = 0;
+    // ---- global read (pext-gather), kernel_v1_impl.cuh:87-151
+    u32 acc_v = 0, acc_x = 0, bits = 0;
     {
       u32 v[kPreRounds], x[kPreRounds];
+      if (FLOW) {
+        if (is_x)
+          flow_gather<true>(F, e, in, out, cycle, v, x);
+        else
+          flow_gather<false>(F, e, in, out, cycle, v, x);
+      } else {
 #pragma unroll
-      for (u32 k = 0; k < kPreRounds; ++k) {
-        v[k] = 0;
-        x[k] = 0;
-        if (e[k].y) {
-          const u32 *base = (e[k].x >> 31) ? out : in;
-          u32 w = e[k].x & 0x7fffffffu;
-          v[k] = ld_coherent(base + w);
-          if (is_x) x[k] = ld_coherent(base + xoff + w);
+        for (u32 k = 0; k < kPreRounds; ++k) {
+          v[k] = 0;
+          x[k] = 0;
+          if (e[k].y) {
+            const u32 *base = (e[k].x >> 31) ? out : in;
+            u32 w = e[k].x & 0x7fffffffu;
+            v[k] = ld_coherent(base + w);
+            if (is_x) x[k] = ld_coherent(base + xoff + w);
+          }
+        }
+      }
+      // the writeout sections and the old values, used after the stages
+      if (nperm) {
+        sda = ld4(pq + (p_sd - bd));
+        sdb = ld4(pq + (p_sd - bd) + 1024);
+        sdf = ld4(p_sd + 4096 + 4 * t);
+      }
+      cka = ld4(pq + (p_ck - bd));
+      ckb = ld4(pq + (p_ck - bd) + 1024);
+      ckf = ld4(p_ck + 4096 + 4 * t);
+      if (h0 && (u32)t < num_ios) {
+        // under dataflow a word of the snapshot buffer is stored and read
+        // back by the same thread only (and a word without X lane keeps the
+        // mask the host put there)
+        const u32 w = io_offset + (u32)t;
+        if (FLOW) {
+          old_v = in[w];
+          if (is_x)
+            old_x = in[xoff + w];
+          else if (F.xoff)
+            old_x = out[F.xoff + w];
+        } else {
+          old_v = ld_coherent(in + w);
+          if (is_x) old_x = ld_coherent(in + xoff + w);
         }
       }
       // pext, lowest mask bit first into the accumulator (kernel_v1_impl.cuh:
@@ -330,48 +539,58 @@ __device__ void run_partition(const ScanArgs &A, const u32 *__restrict__ bd,
           for (u32 m = e[k].y; m; m &= m - 1)
             acc_v = (acc_v << 1) | ((v[k] >> __builtin_ctz(m)) & 1u);
       }
+#pragma unroll
+      for (u32 k = 0; k < kPreRounds; ++k) bits += __builtin_popcount(e[k].y);
     }
-    for (u32 r = kPreRounds; r < rounds; ++r) {  // rare: very wide reads
-      uint2 er = gr[256 * r + t];
-      if (!er.y) continue;
-      const u32 *base = (er.x >> 31) ? out : in;
+    for (u32 r = kPreRounds; r < num_rounds(rounds); ++r) {  // rare: very wide reads
+      uint2 er = gr[256 * (first_round(rounds) + r) + t];
       u32 w = er.x & 0x7fffffffu;
-      u32 v = ld_coherent(base + w), x = is_x ? ld_coherent(base + xoff + w) : 0u;
+      u32 v = 0, x = 0;
+      if (FLOW) {
+        v = flow_word(F, er.y != 0, w, er.x >> 31, 0, in, out, cycle);
+        if (is_x) x = flow_word(F, er.y != 0, w, er.x >> 31, F.xoff, in, out, cycle);
+      } else if (er.y) {
+        const u32 *base = (er.x >> 31) ? out : in;
+        v = ld_coherent(base + w);
+        if (is_x) x = ld_coherent(base + xoff + w);
+      }
       for (u32 m = er.y; m; m &= m - 1) {
         const u32 p = __builtin_ctz(m);
         acc_v = (acc_v << 1) | ((v >> p) & 1u);
         acc_x = (acc_x << 1) | ((x >> p) & 1u);
       }
+      bits += __builtin_popcount(er.y);
     }
-    pi = p_st;
-    st_v[t] = acc_v;
-    st_x[t] = acc_x;
-    if (TIMING) wo_arr[t] = 0;  // pinned rule: reset per partition
+    // half 1's bits follow half 0's
+    {
+      const u32 nb1 = from_pair(bits);
+      const u32 hi_v = from_pair(acc_v), hi_x = from_pair(acc_x);
+      acc_v = (nb1 < 32 ? acc_v << nb1 : 0u) | hi_v;  // half 0's result is kept
+      acc_x = (nb1 < 32 ? acc_x << nb1 : 0u) | hi_x;
+    }
+    const bool next = hn.num_stages != 0;
+    if (next) load_entries(P, bd, hn);
+    if (h0) {
+      st_v[t] = acc_v;
+      st_x[t] = acc_x;
+      if (TIMING) wo_arr[t] = 0;  // pinned rule: reset per partition
+    }
     __syncthreads();
 
     // ---- boomerang stages
     for (u32 bs = 0; bs < num_stages; ++bs) {
-      u32 hv = gather_bits(st_v, q0, q1, q2, q3);
-      u32 hx = is_x ? gather_bits(st_x, q0, q1, q2, q3) : 0u;
-      pi += 5120;
-      // next stage's permutation and tree flags are loaded now, a stage
-      // ahead of their use; this stage's came with the previous one
-      uint4 nA = fA, nB = fB, nC = fC, nD = fD;
-      if (bs + 1 < num_stages) {
-        q0 = ld4(script + pi + 4 * t);
-        q1 = ld4(script + pi + 1024 + 4 * t);
-        q2 = ld4(script + pi + 2048 + 4 * t);
-        q3 = ld4(script + pi + 3072 + 4 * t);
-        if (w0) {
-          const u32 *fn = script + pi + 4096;
-          nA = ld4(fn + 4 * lane);
-          nB = ld4(fn + 4 * (64 + lane));
-          nC = ld4(fn + 4 * (128 + lane));
-          nD = ld4(fn + 4 * (192 + lane));
-        }
+      const u32 hv = gather_bits(st_v, P.qa, P.qb);
+      const u32 hx = is_x ? gather_bits(st_x, P.qa, P.qb) : 0u;
+      // the next section (the next stage's, or the first of the next
+      // partition) is loaded now, a stage ahead of its use; this one's came
+      // with the previous stage
+      const uint4 fA = P.fA, fB = P.fB, fC = P.fC, fD = P.fD;
+      p_st = bs + 1 < num_stages ? p_st + 5120 : stage0(bd, hn);
+      if (bs + 1 < num_stages || next) load_stage(P, p_st);
+      if (h0) {
+        hin_v[t] = hv;
+        hin_x[t] = hx;
       }
-      hin_v[t] = hv;
-      hin_x[t] = hx;
       __syncthreads();
       if (w0) {
         // hier0: words 128+L, 192+L; hier1: word 64+L
@@ -443,34 +662,28 @@ __device__ void run_partition(const ScanArgs &A, const u32 *__restrict__ bd,
         }
       }
       __syncthreads();
-      if ((hook >> 8) == bs) {
+      if (h0 && (hook >> 8) == bs) {
         wo_v[t] = st_v[hook & 255];
         if (is_x) wo_x[t] = st_x[hook & 255];
         if (TIMING) wo_arr[t] = st_arr[hook & 255];
       }
-      fA = nA;
-      fB = nB;
-      fC = nC;
-      fD = nD;
     }
     __syncthreads();
 
     // ---- SRAM + duplicate permutation, kernel_v1_impl.cuh:365-443
-    const u32 nperm = num_srams * 4 + num_dups;
-    pi += 5120;
     // partitions without SRAMs or duplicate words skip the phase (and
     // its two workgroup barriers); the condition is uniform
     if (nperm) {
       u32 pv = 0, px = 0;
       if ((u32)t < nperm) {
-        pv = (gather_bits(wo_v, sd0, sd1, sd2, sd3) & ~sdf.y) ^ sdf.x;
-        if (is_x) px = gather_bits(wo_x, sd0, sd1, sd2, sd3) & ~sdf.y;
+        pv = (gather_bits(wo_v, sda, sdb) & ~sdf.y) ^ sdf.x;
+        if (is_x) px = gather_bits(wo_x, sda, sdb) & ~sdf.y;
       }
-      const u32 en = __shfl(pv, (lane + 1) & 63);
-      const u32 wdata = __shfl(pv, (lane + 2) & 63);
-      const u32 wdata_x = __shfl(px, (lane + 2) & 63);
+      const u32 en = __shfl(pv, (lane + 2) & 63);
+      const u32 wdata = __shfl(pv, (lane + 4) & 63);
+      const u32 wdata_x = __shfl(px, (lane + 4) & 63);
       __syncthreads();  // every gather of wo_* is done before it is written
-      if ((u32)t < num_srams * 4) {
+      if (h0 && (u32)t < num_srams * 4) {
         if ((t & 3) == 0) {
           u32 s = (u32)t >> 2;
           size_t st = (size_t)sram_offset + (size_t)s * kSramWords;
@@ -491,7 +704,7 @@ __device__ void run_partition(const ScanArgs &A, const u32 *__restrict__ bd,
             wo_x[num_ios - num_srams + s] = rx;
           }
         }
-      } else if ((u32)t < nperm) {
+      } else if (h0 && (u32)t < nperm) {
         u32 d = num_ios - num_srams - num_dups + ((u32)t - num_srams * 4);
         wo_v[d] = pv;
         if (is_x) wo_x[d] = px;
@@ -508,29 +721,42 @@ __device__ void run_partition(const ScanArgs &A, const u32 *__restrict__ bd,
         // only words holding DFFs pay for the 32 LDS reads
         const bool gated = f.y != 0xFFFFFFFFu;
         u32 ck = f.x;
-        if (gated) ck = (gather_bits(wo_v, ck0, ck1, ck2, ck3) & ~f.y) ^ f.x;
-        u32 data = wo_v[t] ^ f.z;
-        u32 w = io_offset + (u32)t;
-        st_coherent(out + w, (old_v & ~ck) | (data & ck));
-        if (is_x) {
-          u32 ckx = 0;
-          if (gated) ckx = gather_bits(wo_x, ck0, ck1, ck2, ck3) & ~f.y;
-          st_coherent(out + xoff + w, (old_x & ~ck & ~ckx) | (wo_x[t] & ck & ~ckx) | ckx);
-        }
-        if (TIMING) {
-          u16 arr = wo_arr[t];
-          if (A.arrival_state_offset != 0)
-            st_coherent(out + (u32)A.arrival_state_offset + w, (u32)arr);
-          if (ck != 0 && A.constraints) {
-            u32 cons = A.constraints[w];
-            if (cons != 0) {
-              u32 setup = cons >> 16, hold = cons & 0xffffu;
-              if (arr > 0 && (u32)arr + setup > A.clock_ps)
-                push_event(A.events, A.ev_cap, 4u, w, cycle,
-                           (int)A.clock_ps - (int)arr - (int)setup, arr, setup);
-              if ((u32)arr < hold)
-                push_event(A.events, A.ev_cap, 5u, w, cycle,
-                           (int)arr - (int)hold, arr, hold);
+        if (gated) ck = (gather_bits(wo_v, cka, ckb) & ~f.y) ^ f.x;
+        u32 ckx = 0;
+        if (is_x && gated) ckx = gather_bits(wo_x, cka, ckb) & ~f.y;
+        if (h0) {
+          u32 data = wo_v[t] ^ f.z;
+          u32 w = io_offset + (u32)t;
+          const u32 nv = (old_v & ~ck) | (data & ck);
+          u32 nx = old_x;
+          if (is_x) nx = (old_x & ~ck & ~ckx) | (wo_x[t] & ck & ~ckx) | ckx;
+          if (FLOW) {
+            const u32 s = cycle + 1;
+            const u64 tag = (u64)s << 32;
+            u64 *a = F.ring + ((s & (kRing - 1)) * F.slot + w);
+            st_coherent64(a, tag | nv);
+            if (F.xoff) st_coherent64(a + F.xoff, tag | nx);
+            out[w] = nv;
+            if (is_x) out[xoff + w] = nx;
+          } else {
+            st_coherent(out + w, nv);
+            if (is_x) st_coherent(out + xoff + w, nx);
+          }
+          if (TIMING) {
+            u16 arr = wo_arr[t];
+            if (A.arrival_state_offset != 0)
+              st_coherent(out + (u32)A.arrival_state_offset + w, (u32)arr);
+            if (ck != 0 && A.constraints) {
+              u32 cons = A.constraints[w];
+              if (cons != 0) {
+                u32 setup = cons >> 16, hold = cons & 0xffffu;
+                if (arr > 0 && (u32)arr + setup > A.clock_ps)
+                  push_event(A.events, A.ev_cap, 4u, w, cycle,
+                             (int)A.clock_ps - (int)arr - (int)setup, arr, setup);
+                if ((u32)arr < hold)
+                  push_event(A.events, A.ev_cap, 5u, w, cycle,
+                             (int)arr - (int)hold, arr, hold);
+              }
             }
           }
         }
@@ -538,50 +764,37 @@ __device__ void run_partition(const ScanArgs &A, const u32 *__restrict__ bd,
     }
     if (PROFILE) {
       __syncthreads();
-      if (t == 0 && cycle < A.sample_cycles && part < A.num_parts)
+      if (threadIdx.x == 0 && cycle < A.sample_cycles && part < A.num_parts)
         A.samples[(size_t)cycle * A.num_parts + part] = (u32)(clock64() - t_start);
     }
     __syncthreads();
 }
 
-// ---- dataflow synchronisation of value-only launches
-//
-// Partitions read snapshot words that other blocks wrote in an earlier
-// major stage of the same cycle (`out`, bit 31 of a global-read entry) or
-// in any stage of the previous cycle (`in`); every cycle has its own
-// snapshot and SRAMs belong to one partition, so those reads are the only
-// dependencies between blocks.  Instead of a grid barrier after every major
-// stage, each block publishes its progress (c * M + m + 1 once it has
-// finished major stage m of cycle c and its stores have completed) and,
-// before a stage, waits only for the blocks it reads from, each up to the
-// stage that wrote the words.  The producer table holds, per (block, major
-// stage), one u32 per lane of wave 0: byte j of lane L is the producer
-// block L + 64 j's offset d (its progress must reach c * M + d), or 0x80
-// when the stage reads nothing of that block.  Results are those of the
-// barrier schedule: every read still sees exactly the writes it saw there.
-constexpr u32 kFlowMaxBlocks = 256;
-constexpr u32 kFlowMaxStages = 120;
-constexpr u32 kFlowNone = 0xFFFFFFFFu;
-constexpr u32 kFlowMinCycles = 8;
+// ---- what a dataflow launch needs to know about its script
 
 struct FlowBuild {
   const usize *blocks_start;
   const u32 *bd;
   u32 nb, M;
   usize state_size;
-  u32 *owner;  // state_size words: (block << 16 | major stage) of the writer
-  u32 *dep;    // nb * M * 64 words
-  u32 *bad;    // nonzero: the launch falls back to grid barriers
+  u32 *owner;  // state_size words: (block << 16 | major stage) + 1 of the writer
+  u32 *flow;   // kFlow* words
 };
 
-__global__ __launch_bounds__(256) void flow_fill_kernel(u32 *p, usize n, u32 v) {
+__global__ __launch_bounds__(256) void flow_zero_kernel(uint4 *p, usize n) {
   for (usize i = (usize)blockIdx.x * 256u + threadIdx.x; i < n; i += (usize)gridDim.x * 256u)
-    p[i] = v;
+    p[i] = make_uint4(0, 0, 0, 0);
+}
+
+// Raises *p to v.  Most workgroups find it there already, so the word is
+// read first: an atomic from each would queue up on its line.
+__device__ __forceinline__ void raise_to(u32 *p, u32 v) {
+  if (ld_coherent(p) < v) atomicMax(p, v);
 }
 
 // Workgroup (m, b) records the writer of every writeout word of block b's
-// partitions in major stage m; a word written twice or out of range makes
-// the table unusable.
+// partitions in major stage m, the first such word and the X mask offset; a
+// word written twice or out of range does not fit.
 __global__ __launch_bounds__(256) void flow_owner_kernel(FlowBuild F) {
   const u32 m = blockIdx.x / F.nb, b = blockIdx.x % F.nb;
   size_t off = F.blocks_start[(size_t)m * F.nb + b];
@@ -589,230 +802,238 @@ __global__ __launch_bounds__(256) void flow_owner_kernel(FlowBuild F) {
     const u32 *s = F.bd + off;
     const u32 ns = s[0], is_last = s[1], nio = s[2], io = s[3], rounds = s[6];
     if (ns == 0) break;
-    if (threadIdx.x < nio) {
-      const usize w = (usize)io + threadIdx.x;
-      if (w >= F.state_size)
-        atomicOr(F.bad, 1u);
-      else if (atomicExch(&F.owner[w], (b << 16) | m) != kFlowNone)
-        atomicOr(F.bad, 2u);
+    const usize top = (usize)io + nio + (s[8] ? s[9] : 0u);
+    if (threadIdx.x == 0) {
+      if (top > F.state_size || nio > 256u) atomicOr(&F.flow[kFlowBad], 1u);
+      if (nio) raise_to(&F.flow[kFlowNegLo], ~io);
+      if (s[8]) raise_to(&F.flow[kFlowXoff], s[9]);
     }
+    if (top <= F.state_size && threadIdx.x < nio &&
+        atomicExch(&F.owner[io + threadIdx.x], ((b << 16) | m) + 1u) != 0u)
+      atomicOr(&F.flow[kFlowBad], 2u);
     if (is_last) break;
     off += 256 + (size_t)512 * rounds + (size_t)5120 * (ns + 2);
   }
 }
 
-// Workgroup (m, b) reduces the global-read entries of block b's partitions
-// in major stage m to the latest progress it needs of every other block.
-__global__ __launch_bounds__(256) void flow_dep_kernel(FlowBuild F) {
-  __shared__ u32 r[kFlowMaxBlocks];
+// Workgroup (m, b) checks the global-read entries of block b's partitions
+// in major stage m: a word at or past the first writeout word must be one
+// that some partition writes, in an earlier stage when it is read from the
+// same cycle; X masks must lie at one offset, past the words themselves.
+__global__ __launch_bounds__(256) void flow_check_kernel(FlowBuild F) {
   const u32 m = blockIdx.x / F.nb, b = blockIdx.x % F.nb;
   const u32 t = threadIdx.x;
-  r[t] = 0;
-  __syncthreads();
+  const u32 lo = ~F.flow[kFlowNegLo], xoff = F.flow[kFlowXoff];
+  u32 bad = 0;
   size_t off = F.blocks_start[(size_t)m * F.nb + b];
   for (;;) {
     const u32 *s = F.bd + off;
-    const u32 ns = s[0], is_last = s[1], rounds = s[6];
+    const u32 ns = s[0], is_last = s[1], nio = s[2], io = s[3], rounds = s[6];
     if (ns == 0) break;
+    if (xoff && ((s[8] && s[9] != xoff) || (usize)io + nio > xoff ||
+                 (usize)xoff + io + nio > F.state_size))
+      bad |= 4u;
     const uint2 *gr = reinterpret_cast<const uint2 *>(s + 256);
     for (u32 k = 0; k < rounds; ++k) {
       const uint2 e = gr[256 * k + t];
       if (!e.y) continue;
       const u32 w = e.x & 0x7fffffffu;
-      const bool from_out = (e.x >> 31) != 0;
-      if (w >= F.state_size) {
-        atomicOr(F.bad, 4u);
-        continue;
+      if ((usize)w + (s[8] ? xoff : 0u) >= F.state_size) {
+        bad |= 8u;
+      } else if (w >= lo) {
+        const u32 o = F.owner[w];
+        if (o == 0 || ((e.x >> 31) && ((o - 1u) & 0xffffu) >= m)) bad |= 16u;
       }
-      const u32 o = F.owner[w];
-      if (o == kFlowNone) continue;  // a primary input: written by the host
-      const u32 q = o >> 16, sq = o & 0xffffu;
-      if (q == b) continue;  // the block's own earlier work
-      if (from_out && sq >= m) {  // not written before this stage
-        atomicOr(F.bad, 8u);
-        continue;
-      }
-      const int d = from_out ? (int)sq + 1 : (int)sq + 1 - (int)F.M;
-      atomicMax(&r[q], (u32)(d + 128));
     }
     if (is_last) break;
     off += 256 + (size_t)512 * rounds + (size_t)5120 * (ns + 2);
   }
-  __syncthreads();
-  if (t < 64) {
-    u32 word = 0;
-#pragma unroll
-    for (u32 j = 0; j < 4; ++j) {
-      const u32 v = r[t + 64 * j];
-      word |= (v ? ((v - 128u) & 0xffu) : 0x80u) << (8 * j);
-    }
-    F.dep[((size_t)b * F.M + m) * 64 + t] = word;
+  if (bad) atomicOr(&F.flow[kFlowBad], bad);
+}
+
+// A block's partitions in execution order: cycle, major stage, then
+// position in the stage's section of blocks_data (kernel_v1_impl.cuh:
+// 565-626).  A stage without partitions is one step with an empty header.
+// `next` is the step after the one that runs; the header of the one after
+// that is in flight, and so is the section start it may need.
+struct Walk {
+  PartHdr cur, next;
+  RawHdr raw;
+  bool have;     // raw is a step of the launch
+  u32 c, m;      // of raw
+  usize after;   // blocks_start of the stage that follows raw's
+};
+
+__device__ __forceinline__ usize section(const ScanArgs &A, u32 m) {
+  const u32 k = m + 1 == A.num_major_stages ? 0 : m + 1;
+  return A.blocks_start[(size_t)k * A.num_blocks + blockIdx.x];
+}
+
+__device__ __forceinline__ usize uniform64(usize v) {
+  return (usize)uniform((u32)(v >> 32)) << 32 | uniform((u32)v);
+}
+
+// Requests the header of the step after h (the one raw held).
+__device__ __forceinline__ void fetch_step(const ScanArgs &A, const u32 *bd, u32 cycles,
+                                           Walk &w, const PartHdr &h) {
+  if (h.num_stages != 0 && h.is_last == 0) {
+    w.raw = load_hdr(bd, h.base + part_words(h));
+    return;
+  }
+  if (++w.m == A.num_major_stages) {
+    w.m = 0;
+    ++w.c;
+  }
+  w.have = w.c < cycles;
+  if (!w.have) return;
+  w.raw = load_hdr(bd, uniform64(w.after));
+  w.after = section(A, w.m);
+}
+
+// The walk at the block's first step (num_major_stages > 0).
+__device__ __forceinline__ void start_walk(const ScanArgs &A, const u32 *bd, u32 cycles, Walk &w,
+                                           PartPre &P) {
+  w.c = w.m = 0;
+  w.have = true;
+  w.raw = load_hdr(bd, A.blocks_start[blockIdx.x]);
+  w.after = section(A, 0);
+  w.cur = settle(w.raw);
+  fetch_step(A, bd, cycles, w, w.cur);
+  if (w.cur.num_stages) {
+    load_entries(P, bd, w.cur);
+    load_stage(P, stage0(bd, w.cur));
   }
 }
 
-// Publishes `done` as block b's progress once every wave has waited for its
-// stores, then wave 0 polls the progress of the producers in `row` until
-// each reaches base + its offset.  The wait is bounded like the grid
-// barrier's (the poll limit, and the launch's abort word in `bar` read every
-// 256 polls); an abort sets the caller's LDS word s_aborted to 1.
-__device__ __forceinline__ void flow_publish_wait(u32 *prog, u32 b, u32 done, u32 row,
-                                                  u32 base, u32 *bar, u32 *err,
-                                                  u32 &s_aborted) {
-  __syncthreads();
-  if (threadIdx.x == 0) st_coherent(&prog[b * kProgStride], done);
-  bool aborted = false;
-  if (threadIdx.x < 64 && row != 0x80808080u) {
-    const u32 lane = threadIdx.x;
-    u32 tg[4];
-    bool need[4];
-#pragma unroll
-    for (u32 j = 0; j < 4; ++j) {
-      const u32 d = (row >> (8 * j)) & 0xffu;
-      need[j] = d != 0x80u;
-      tg[j] = base + (u32)(int)(signed char)d;
-    }
-    const u32 lim = g_wait_polls;
-    u32 spins = 0;
-    for (;;) {
-      u32 p[4];
-#pragma unroll
-      for (u32 j = 0; j < 4; ++j) p[j] = need[j] ? ld_coherent(&prog[(lane + 64 * j) * kProgStride]) : 0u;
-      bool pend = false;
-#pragma unroll
-      for (u32 j = 0; j < 4; ++j)
-        if (need[j]) {
-          if ((int)(p[j] - tg[j]) >= 0)
-            need[j] = false;
-          else
-            pend = true;
-        }
-      if (!__any(pend)) break;
-      __builtin_amdgcn_s_sleep(1);
-      // the outcome is wave-uniform (every lane counts the same polls and
-      // reads the same word); one lane raises the abort
-      if (++spins > lim) {
-        if (lane == 0) abort_launch(bar, err);
-        aborted = true;
-        break;
-      }
-      if ((spins & 255u) == 0 && ld_coherent(&bar[kAbortWord]) != 0) {
-        aborted = true;
-        break;
-      }
-    }
+// Before the step that runs: the header requested during the last one
+// becomes `next`, and the one after it is requested.
+__device__ __forceinline__ void peek_step(const ScanArgs &A, const u32 *bd, u32 cycles, Walk &w) {
+  if (!w.have) {
+    w.next = no_hdr();
+    return;
   }
-  if (threadIdx.x == 0 && aborted) s_aborted = 1;
-  asm volatile("" ::: "memory");
-  __syncthreads();
+  w.next = settle(w.raw);
+  fetch_step(A, bd, cycles, w, w.next);
 }
 
-template <bool TIMING, bool PROFILE>
-__global__ __launch_bounds__(256) void scan_kernel(ScanArgs A) {
-  if (A.timing) {
-    A.clock_ps = A.timing[0];
-    A.constraints = A.timing + 1;
-  }
-  __shared__ u32 st_v[256], st_x[256], hin_v[256], hin_x[256];
-  __shared__ u32 wo_v[256], wo_x[256];
-  __shared__ u16 st_arr[256], wo_arr[256];
-  __shared__ u32 s_aborted;  // set by a wait when the launch has aborted
-  const int t = threadIdx.x;
-  if (t == 0) s_aborted = 0;
-  st_x[t] = 0;
-  hin_x[t] = 0;
-  wo_x[t] = 0;
-  wo_arr[t] = 0;
-  st_arr[t] = 0;
-  u32 gen = read_gen(A.bar);
-  __syncthreads();
+// The LDS arrays of one workgroup.
+#define JQ_SCAN_LDS                                             \
+  __shared__ u32 st_v[256], st_x[256], hin_v[256], hin_x[256]; \
+  __shared__ u32 wo_v[256], wo_x[256];                          \
+  __shared__ u16 st_arr[256], wo_arr[256];                      \
+  __shared__ u32 s_aborted; /* set by a wait when the launch has aborted */
+
+template <bool TIMING, bool PROFILE, bool FLOW>
+__device__ __forceinline__ void scan_loop(const ScanArgs &A, u32 *st_v, u32 *st_x, u32 *hin_v,
+                                          u32 *hin_x, u32 *wo_v, u32 *wo_x, u16 *st_arr,
+                                          u16 *wo_arr, u32 &s_aborted, u32 gen) {
   const u32 b = blockIdx.x;
   const u32 nb = A.num_blocks, M = A.num_major_stages;
   const u32 *bd = A.blocks_data;
-  // the block's partitions in execution order: cycle, major stage, then
-  // position in the stage's section of blocks_data (kernel_v1_impl.cuh:
-  // 565-626); h / P always describe the next partition to run
-  // value-only launches whose producer table was built synchronise by
-  // dataflow; the flag is the same word for every block
-  const bool flow = !TIMING && !PROFILE && A.dep != nullptr && *A.dep_bad == 0;
-  if (flow) {
-    if (t == 0) st_coherent(&A.prog[b * kProgStride], 0u);
-    grid_sync_coherent(A.bar, nb, b, gen, &g_error, &g_wait_polls, s_aborted);
+  if (M == 0) return;
+  Flow F{};
+  if (FLOW) {
+    F.ring = A.ring;
+    F.slot = (u32)A.state_size;
+    F.lo = ~A.flow[kFlowNegLo];
+    F.xoff = A.flow[kFlowXoff];
+    F.bar = A.bar;
+    F.aborted = &s_aborted;
   }
-  PartHdr h = M ? load_hdr(bd, A.blocks_start[b]) : no_hdr();
-  PartPre P;
-  if (h.num_stages) load_pre(P, bd, h, A.states);
+  Walk w{};
+  PartPre P{};
+  start_walk(A, bd, A.num_cycles, w, P);
   for (u32 c = 0; c < A.num_cycles; ++c) {
     // an aborted launch (a bounded wait gave up; the waits that follow end
     // within 256 polls each) leaves at the next cycle
     if (s_aborted) return;
+    if (FLOW && nb > 1 && c != 0 && c % (kRing / 2) == 0) {
+      flow_room(F, A.prog, nb, c);
+      __syncthreads();
+    }
     const u32 *in = A.states + (size_t)c * A.state_size;
     u32 *out = A.states + (size_t)(c + 1) * A.state_size;
     for (u32 m = 0; m < M; ++m) {
       u32 part = PROFILE ? A.part_index[(size_t)m * nb + b] : 0u;
-      const bool wrap = m + 1 == M;
-      const u32 nc = wrap ? c + 1 : c, nm = wrap ? 0u : m + 1;
-      // the next stage's producer row is read a stage ahead of its use
-      u32 row = 0x80808080u;
-      if (flow && t < 64 && nc < A.num_cycles)
-        row = A.dep[((size_t)b * M + nm) * 64 + t];
       for (;;) {
-        const bool last = h.num_stages == 0 || h.is_last != 0;
-        // the successor's header is requested before this partition runs
-        PartHdr hn = no_hdr();
-        if (!last)
-          hn = load_hdr(bd, h.base + part_words(h));
-        else if (nc < A.num_cycles)
-          hn = load_hdr(bd, A.blocks_start[(size_t)nm * nb + b]);
-        if (h.num_stages) {
-          run_partition<TIMING, PROFILE>(A, bd, h, P, in, out, c, part, st_v, st_x,
-                                         hin_v, hin_x, wo_v, wo_x, st_arr, wo_arr);
+        const bool last = w.cur.num_stages == 0 || w.cur.is_last != 0;
+        peek_step(A, bd, A.num_cycles, w);
+        if (w.cur.num_stages) {
+          run_partition<TIMING, PROFILE, FLOW>(A, bd, w.cur, w.next, P, F, in, out, c, part,
+                                               st_v, st_x, hin_v, hin_x, wo_v, wo_x, st_arr,
+                                               wo_arr);
           ++part;
+        } else if (w.next.num_stages) {
+          load_entries(P, bd, w.next);
+          load_stage(P, stage0(bd, w.next));
         }
-        if (last) {
-          // this wave's stores complete before the next stage's prologue
-          // loads are issued, so the barrier need not wait for those loads
-          wait_vmem();
-          if (hn.num_stages) load_pre(P, bd, hn, A.states + (size_t)nc * A.state_size);
-          h = hn;
-          break;
-        }
-        if (hn.num_stages) load_pre(P, bd, hn, in);
-        h = hn;
+        w.cur = w.next;
+        if (last) break;
       }
-      if (flow)
-        flow_publish_wait(A.prog, b, c * M + m + 1, row, nc * M, A.bar, &g_error,
-                          s_aborted);
-      else
-        grid_arrive_wait(A.bar, nb, b, gen, &g_error, &g_wait_polls, s_aborted);
+      if (!FLOW) grid_sync_coherent(A.bar, nb, b, gen, &g_error, &g_wait_polls, s_aborted);
+    }
+    if (FLOW) {
+      // the last partition's closing workgroup barrier is behind every wave:
+      // none of them reads a snapshot of this cycle any more
+      __syncthreads();
+      if (nb > 1 && threadIdx.x == 0) st_coherent(&A.prog[b * kProgStride], c + 1);
     }
   }
 }
+
+template <bool TIMING, bool PROFILE>
+__global__ __launch_bounds__(kScanThreads) void scan_kernel(ScanArgs A) {
+  if (A.timing) {
+    A.clock_ps = A.timing[0];
+    A.constraints = A.timing + 1;
+  }
+  JQ_SCAN_LDS
+  const int t = threadIdx.x;
+  if (t == 0) s_aborted = 0;
+  if (t < 256) {
+    st_x[t] = 0;
+    hin_x[t] = 0;
+    wo_x[t] = 0;
+    wo_arr[t] = 0;
+    st_arr[t] = 0;
+  }
+  const u32 gen = read_gen(A.bar);
+  __syncthreads();
+  // the flag is the same word for every block
+  if (!TIMING && !PROFILE && A.ring != nullptr && A.flow[kFlowBad] == 0)
+    scan_loop<TIMING, PROFILE, !TIMING && !PROFILE>(A, st_v, st_x, hin_v, hin_x, wo_v, wo_x,
+                                                    st_arr, wo_arr, s_aborted, gen);
+  else
+    scan_loop<TIMING, PROFILE, false>(A, st_v, st_x, hin_v, hin_x, wo_v, wo_x, st_arr, wo_arr,
+                                      s_aborted, gen);
+}
+
 // Persistent co-simulation: C.num_edges edges of one cycle each over the
 // two snapshots of C.states (timing events carry cycle 0, as every edge of
 // the reference's co-simulation dispatch does, src/sim/cosim_metal.rs:
 // 591-600), every workgroup doing its share of the
 // between-edges work of jq_cosim.hpp ahead of every cycle (and once after
-// the last).  A cycle
-// walks the partitions as scan_kernel does, except that the first
-// partition of a cycle is loaded after the barrier that follows the
-// preparation, which may change any input word.
-template <bool TIMING>
-__global__ __launch_bounds__(256) void cosim_kernel(ScanArgs A, cosim::CosimArgs C) {
+// the last).  A cycle walks the partitions as scan_kernel does.
+//
+// WAVES is the number of waves per SIMD that the registers must leave room
+// for: 2 is one workgroup per CU, 4 (with spills) two, for launches of more
+// blocks than CUs.
+template <bool TIMING, int WAVES>
+__global__ __launch_bounds__(kScanThreads, WAVES) void cosim_kernel(ScanArgs A, cosim::CosimArgs C) {
   if (A.timing) {
     A.clock_ps = A.timing[0];
     A.constraints = A.timing + 1;
   }
-  __shared__ u32 st_v[256], st_x[256], hin_v[256], hin_x[256];
-  __shared__ u32 wo_v[256], wo_x[256];
-  __shared__ u16 st_arr[256], wo_arr[256];
-  __shared__ u32 s_aborted;  // set by a wait when the launch has aborted
+  JQ_SCAN_LDS
   const int t = threadIdx.x;
   if (t == 0) s_aborted = 0;
-  st_x[t] = 0;
-  hin_x[t] = 0;
-  wo_x[t] = 0;
-  wo_arr[t] = 0;
-  st_arr[t] = 0;
+  if (t < 256) {
+    st_x[t] = 0;
+    hin_x[t] = 0;
+    wo_x[t] = 0;
+    wo_arr[t] = 0;
+    st_arr[t] = 0;
+  }
   u32 gen = read_gen(A.bar);
   __syncthreads();
   const u32 b = blockIdx.x;
@@ -820,44 +1041,35 @@ __global__ __launch_bounds__(256) void cosim_kernel(ScanArgs A, cosim::CosimArgs
   const u32 *bd = A.blocks_data;
   const u32 *in = A.states;
   u32 *out = A.states + A.state_size;
-  // co-simulation snapshots are 2-state: a partition flagged X-capable runs
-  // its value lane only
-  auto hdr2 = [&](size_t off) {
-    PartHdr x = load_hdr(bd, off);
-    x.is_x = false;
-    return x;
-  };
+  const Flow F{};
+  Walk w{};
+  PartPre P{};
+  if (M) start_walk(A, bd, C.num_edges, w, P);
   for (u32 e = 0; e <= C.num_edges; ++e) {
     // an aborted launch (a bounded wait gave up) leaves at the next edge
     if (s_aborted) return;
     cosim::between_phase(C, (u32)t, b, nb, e);
     if (e == C.num_edges) break;
     grid_sync_coherent(A.bar, nb, b, gen, &g_error, &g_wait_polls, s_aborted);
-    PartHdr h = M ? hdr2(A.blocks_start[b]) : no_hdr();
-    PartPre P;
-    if (h.num_stages) load_pre(P, bd, h, in);
     for (u32 m = 0; m < M; ++m) {
-      const bool wrap = m + 1 == M;
       for (;;) {
-        const bool last = h.num_stages == 0 || h.is_last != 0;
-        PartHdr hn = no_hdr();
-        if (!last)
-          hn = hdr2(h.base + part_words(h));
-        else if (!wrap)
-          hn = hdr2(A.blocks_start[(size_t)(m + 1) * nb + b]);
-        if (h.num_stages)
-          run_partition<TIMING, false>(A, bd, h, P, in, out, 0u, 0u, st_v, st_x, hin_v,
-                                       hin_x, wo_v, wo_x, st_arr, wo_arr);
-        if (last) {
-          wait_vmem();
-          if (hn.num_stages) load_pre(P, bd, hn, in);
-          h = hn;
-          break;
+        const bool last = w.cur.num_stages == 0 || w.cur.is_last != 0;
+        peek_step(A, bd, C.num_edges, w);
+        if (w.cur.num_stages) {
+          // co-simulation snapshots are 2-state: a partition flagged
+          // X-capable runs its value lane only
+          w.cur.is_x = false;
+          run_partition<TIMING, false, false>(A, bd, w.cur, w.next, P, F, in, out, 0u, 0u,
+                                              st_v, st_x, hin_v, hin_x, wo_v, wo_x, st_arr,
+                                              wo_arr);
+        } else if (w.next.num_stages) {
+          load_entries(P, bd, w.next);
+          load_stage(P, stage0(bd, w.next));
         }
-        if (hn.num_stages) load_pre(P, bd, hn, in);
-        h = hn;
+        w.cur = w.next;
+        if (last) break;
       }
-      grid_arrive_wait(A.bar, nb, b, gen, &g_error, &g_wait_polls, s_aborted);
+      grid_sync_coherent(A.bar, nb, b, gen, &g_error, &g_wait_polls, s_aborted);
     }
   }
 }
@@ -889,12 +1101,6 @@ int launch_scan(ScanArgs &A, hipStream_t stream) {
   if (hipGetSymbolAddress((void **)&bar_base, HIP_SYMBOL(g_barrier)) != hipSuccess)
     return fail("hipGetSymbolAddress(g_barrier) failed");
   A.bar = bar_base + kCohSlotWords * (__atomic_fetch_add(&g_slot, 1u, __ATOMIC_RELAXED) % kCohSlots);
-  if (A.dep) {
-    u32 *pb = nullptr;
-    if (hipGetSymbolAddress((void **)&pb, HIP_SYMBOL(g_prog)) != hipSuccess)
-      return fail("hipGetSymbolAddress(g_prog) failed");
-    A.prog = pb + (size_t)256 * kProgStride * ((A.bar - bar_base) / kCohSlotWords);
-  }
   void *args[] = {&A};
   const void *kern = reinterpret_cast<const void *>(&scan_kernel<TIMING, PROFILE>);
   // Under stream capture (a hipGraph of the launch) the launch is an
@@ -909,38 +1115,38 @@ int launch_scan(ScanArgs &A, hipStream_t stream) {
     int dev = 0, cus = 0, per = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kern, 256, 0) != hipSuccess)
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kern, kScanThreads, 0) != hipSuccess)
       return fail("occupancy query failed");
     if ((long long)per * cus < (long long)A.num_blocks)
       return fail("scan launch: more blocks than workgroups that can be resident at once");
-    e = hipLaunchKernel(kern, dim3(A.num_blocks), dim3(256), args, 0, stream);
+    e = hipLaunchKernel(kern, dim3(A.num_blocks), dim3(kScanThreads), args, 0, stream);
   } else {
-    e = hipLaunchCooperativeKernel(kern, dim3(A.num_blocks), dim3(256), args, 0, stream);
+    e = hipLaunchCooperativeKernel(kern, dim3(A.num_blocks), dim3(kScanThreads), args, 0, stream);
   }
   if (e != hipSuccess)
     return fail(std::string("scan launch failed: ") + hipGetErrorString(e));
   return 0;
 }
 
-// Builds the producer table of a value-only launch on `stream` ahead of it
-// and returns its stream-ordered allocation (freed after the launch), or
-// null when the launch runs with grid barriers: the mode is off, the
-// script is outside the table's limits, the launch is shorter than
-// kFlowMinCycles (the table's ~30 us build is then comparable to the
-// barriers it saves), the stream is being captured into a graph (no
-// allocation or builder kernels go into the caller's graph), or the
-// allocation failed.  A
-// script that the builders find unusable (a writeout word written twice or
-// out of range, a same-cycle read of a word not written in an earlier
-// stage) raises the flag that the kernel reads, and the launch then uses
-// grid barriers as well.
-void *build_flow_tables(ScanArgs &A, hipStream_t stream) {
-  A.dep = nullptr;
-  A.dep_bad = nullptr;
+// Prepares a value-only launch for dataflow on `stream` ahead of it and
+// returns its stream-ordered allocation (the exchange ring, the builders'
+// words and the progress words, freed after the launch), or null when the
+// launch runs with grid barriers: the mode is off, the script is outside
+// the builders' packing, the launch is shorter than kFlowMinCycles (the
+// builders' time is then comparable to the barriers they save), the stream
+// is being captured into a graph (no allocation or builder kernels go into
+// the caller's graph), or the allocation failed.  A script that the
+// builders find unusable (a writeout word written twice or out of range, a
+// read of a word past the first writeout word that no partition writes, a
+// same-cycle read of a word not written in an earlier stage) raises the
+// flag that the kernel reads, and the launch then uses grid barriers as
+// well.
+void *build_flow(ScanArgs &A, hipStream_t stream) {
+  A.ring = nullptr;
   const u32 nb = A.num_blocks, M = A.num_major_stages;
-  if (!__atomic_load_n(&g_scan_sync, __ATOMIC_RELAXED) || nb > kFlowMaxBlocks || M == 0 ||
-      M > kFlowMaxStages || A.num_cycles < kFlowMinCycles || A.state_size == 0 ||
-      A.state_size > (usize(1) << 28))
+  if (!__atomic_load_n(&g_scan_sync, __ATOMIC_RELAXED) || M == 0 || M > 65534u ||
+      A.num_cycles < kFlowMinCycles || A.state_size == 0 ||
+      A.state_size > (usize(1) << 28) || (usize)nb * M > 0x7fffffffu)
     return nullptr;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &cap) != hipSuccess) {
@@ -948,33 +1154,34 @@ void *build_flow_tables(ScanArgs &A, hipStream_t stream) {
     return nullptr;
   }
   if (cap != hipStreamCaptureStatusNone) return nullptr;
-  const size_t own_words = ((size_t)A.state_size + 63) & ~(size_t)63;
-  const size_t dep_words = (size_t)nb * M * 64;
+  const size_t own = ((size_t)A.state_size + 63) & ~(size_t)63;  // whole 256-byte units
+  const size_t ring = 2 * kRing * own, prog = (size_t)nb * kProgStride;
+  const size_t words = ring + own + kFlowWords + prog;
   void *buf = nullptr;
-  if (hipMallocAsync(&buf, 4 * (own_words + dep_words + 64), stream) != hipSuccess) {
+  if (hipMallocAsync(&buf, 4 * words, stream) != hipSuccess) {
     (void)hipGetLastError();
     return nullptr;
   }
+  u32 *p = static_cast<u32 *>(buf);
   FlowBuild F{};
   F.blocks_start = A.blocks_start;
   F.bd = A.blocks_data;
   F.nb = nb;
   F.M = M;
   F.state_size = A.state_size;
-  F.owner = static_cast<u32 *>(buf);
-  F.dep = F.owner + own_words;
-  F.bad = F.dep + dep_words;
-  const u32 fill_blocks = (u32)std::min<size_t>(1024, (own_words + 255) / 256);
-  flow_fill_kernel<<<fill_blocks, 256, 0, stream>>>(F.owner, A.state_size, kFlowNone);
-  flow_fill_kernel<<<1, 256, 0, stream>>>(F.bad, 1, 0u);
+  F.owner = p + ring;
+  F.flow = F.owner + own;
+  const u32 fill_blocks = (u32)std::min<size_t>(1024, (words / 4 + 255) / 256);
+  flow_zero_kernel<<<fill_blocks, 256, 0, stream>>>(reinterpret_cast<uint4 *>(buf), words / 4);
   flow_owner_kernel<<<nb * M, 256, 0, stream>>>(F);
-  flow_dep_kernel<<<nb * M, 256, 0, stream>>>(F);
+  flow_check_kernel<<<nb * M, 256, 0, stream>>>(F);
   if (hipGetLastError() != hipSuccess) {
     (void)hipFreeAsync(buf, stream);
     return nullptr;
   }
-  A.dep = F.dep;
-  A.dep_bad = F.bad;
+  A.ring = reinterpret_cast<u64 *>(buf);
+  A.flow = F.flow;
+  A.prog = F.flow + kFlowWords;
   return buf;
 }
 
@@ -1011,7 +1218,7 @@ int scan_common(usize num_blocks, usize num_major_stages, const usize *blocks_st
   const bool timing = A.timing != nullptr || arrival_state_offset != 0;
   if (samples) return launch_scan<false, true>(A, stream);
   if (timing) return launch_scan<true, false>(A, stream);
-  void *flow_buf = build_flow_tables(A, stream);
+  void *flow_buf = build_flow(A, stream);
   const int rc = launch_scan<false, false>(A, stream);
   if (flow_buf) (void)hipFreeAsync(flow_buf, stream);
   return rc;
@@ -1091,7 +1298,8 @@ extern "C" int jq_max_resident_blocks(int kind, int *out_blocks) {
     return fail("CU count query failed");
   if (kind == 0) {
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per, reinterpret_cast<const void *>(&scan_kernel<true, false>), 256, 0) !=
+            &per, reinterpret_cast<const void *>(&scan_kernel<true, false>), kScanThreads,
+            0) !=
         hipSuccess)
       return fail("occupancy query failed");
   } else {
@@ -1208,9 +1416,15 @@ extern "C" int jq_cosim_edges(usize num_blocks, usize num_major_stages,
   // 36, counters from 256)
   C.fsbuf = A.bar + 64;
   void *args[] = {&A, &C};
-  const void *k = timing ? reinterpret_cast<const void *>(&cosim_kernel<true>)
-                        : reinterpret_cast<const void *>(&cosim_kernel<false>);
-  hipError_t e = hipLaunchCooperativeKernel(k, dim3(A.num_blocks), dim3(256), args, 0,
+  const void *k = timing ? reinterpret_cast<const void *>(&cosim_kernel<true, 2>)
+                        : reinterpret_cast<const void *>(&cosim_kernel<false, 2>);
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    return fail("CU count query failed");
+  if (!timing && A.num_blocks > (u32)cus)
+    k = reinterpret_cast<const void *>(&cosim_kernel<false, 4>);
+  hipError_t e = hipLaunchCooperativeKernel(k, dim3(A.num_blocks), dim3(kScanThreads), args, 0,
                                             (hipStream_t)stream);
   if (e != hipSuccess) return fail(std::string("cosim launch failed: ") + hipGetErrorString(e));
   return 0;

@@ -442,3 +442,66 @@ def test_global_read_wider_than_prefetched_rounds(xprop):
     oracle.run(s, ref, cycles)  # the original script: same values
     got = sim.run_scan(w, st.copy(), cycles)["states"]
     assert np.array_equal(got, ref)
+
+
+class _WideState:
+    """The script over a snapshot of `extra` more words, with every global
+    read of input word 0 sent to the word after the last writeout instead:
+    a word past the first writeout that no partition writes."""
+
+    def __init__(self, script, extra):
+        self._s, self.extra = script, extra
+        bd = np.array(script.blocks_data, np.uint32)
+        self.moved = 0
+        for off in script.parts[:, 3].tolist():
+            a, R = int(off) + 256, int(bd[int(off) + 6])
+            gr = bd[a:a + 512 * R].reshape(-1, 2)
+            hit = ((gr[:, 0] & 0x7FFFFFFF) == 0) & (gr[:, 1] != 0)
+            gr[hit, 0] = (gr[hit, 0] & 0x80000000) | script.reg_io_state_size
+            self.moved += int(hit.sum())
+        self.blocks_data = bd
+
+    def effective_state_size(self):
+        return self._s.effective_state_size() + self.extra
+
+    def __getattr__(self, name):
+        return getattr(self._s, name)
+
+
+def test_a_script_that_reads_past_the_writeouts_keeps_grid_barriers():
+    """A read past the first writeout word of a word that no partition
+    writes would wait for ever in the exchange ring: the builders see it and
+    the launch keeps grid barriers, with the oracle's snapshots."""
+    nl, comp = design("sync", level_split=4, seed=9, gates=40000, depth=48,
+                      dffs=3000, inputs=64, outputs=32, geometric_p=0.3, srams=3)
+    w = _WideState(comp.flatten(48), 2)
+    assert w.moved > 0
+    cycles = 60
+    rio = w.reg_io_state_size
+    st = np.zeros((cycles + 1, rio + 2), np.uint32)
+    st[:, :rio] = stimulus.build_states(w._s, cycles, seed=20, p=0.3).reshape(cycles + 1, rio)
+    st[:, rio] = st[:, 0]
+    st = st.reshape(-1)
+    ref = st.copy()
+    oracle.run(w, ref, cycles)
+    got = sim.run_scan(w, st.copy(), cycles, validate=False)["states"]
+    assert np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("blocks,xprop", [(3, True), (1, False), (61, True)])
+def test_dataflow_over_many_laps_of_the_ring(blocks, xprop):
+    """300 cycles, 37 laps of the exchange ring, with one block, with fewer
+    blocks than partitions and with more: every snapshot is the oracle's."""
+    from jacquard_amd.script import Compiled
+    nl, _ = design("laps", level_split=3, seed=23, gates=9000, depth=30, dffs=700,
+                   inputs=40, outputs=24, geometric_p=0.3, srams=2)
+    s = Compiled(nl, level_split=3, max_level_nodes=200).flatten(blocks, xprop=xprop)
+    cycles = 300
+    st = stimulus.build_states(s, cycles, seed=4, p=0.2)
+    ref = st.copy()
+    sram = np.zeros(s.sram_storage_size, np.uint32)
+    sram_x = np.full(s.sram_storage_size, 0xFFFFFFFF, np.uint32)
+    oracle.run(s, ref, cycles, sram=sram, sram_x=sram_x if xprop else None)
+    out = sim.run_scan(s, st.copy(), cycles)
+    assert np.array_equal(out["states"], ref)
+    assert np.array_equal(out["sram"][:s.sram_storage_size], sram)
