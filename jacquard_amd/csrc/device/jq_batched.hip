@@ -44,6 +44,7 @@ __device__ u32 gb_error;
 
 namespace {
 
+constexpr u32 kT = 1024;  // threads of a workgroup: 16 waves, 4 per SIMD
 constexpr int kLayerWords = 8192;
 constexpr int kSecWords = 5120;  // 4096 permutation words + 256 x 4 flags
 // LDS: the layer, the writeout area, two script-section buffers and the
@@ -102,7 +103,8 @@ __device__ __forceinline__ u32 mix32(u32 x) {
   return x;
 }
 
-// Row swizzle of the 8192-word LDS arrays.
+// Row swizzle of the 8192-word LDS arrays.  Positions 1024 apart have the
+// same pattern: sw(p + 1024 k) == sw(p) + 1024 k.
 __device__ __forceinline__ u32 sw(u32 p) { return p ^ ((p >> 5) & 31u); }
 
 // u16 permutation entry of bit position p of a 4x1024-word section
@@ -121,40 +123,26 @@ __device__ __forceinline__ u32 fbit(u32 word, u32 p) {
   return 0u - ((word >> (p & 31)) & 1u);
 }
 
-struct Flags {
-  u32 xa, xb, ob;
-};
-
-__device__ __forceinline__ Flags flags_at(const u32 *fl, u32 p) {
-  uint4 f = *reinterpret_cast<const uint4 *>(fl + 4 * (p >> 5));
-  return Flags{fbit(f.x, p), fbit(f.y, p), fbit(f.z, p)};
-}
-
-__device__ __forceinline__ u32 lgate(u32 a, u32 b, Flags f) {
-  return (a ^ f.xa) & ((b ^ f.xb) | f.ob);
-}
-
 // Copy one 5120-word script section from global memory straight into LDS
 // (global_load_lds_dwordx4: no registers, completes asynchronously).  Lane
-// l of wave w moves the 16 bytes at word 4*(t + 256j), t = 64w + l, to the
+// l of wave w moves the 16 bytes at word 4*(t + kT*j), t = 64w + l, to the
 // same word offset in LDS; the LDS base of each instruction is wave-uniform.
 __device__ __forceinline__ void sec_fetch(const u32 *g, u32 *l) {
-  const u32 t = threadIdx.x, w = t >> 6;
-#pragma unroll
-  for (int j = 0; j < 5; ++j)
-    __builtin_amdgcn_global_load_lds(g + 4 * (t + 256 * j), l + 4 * (64 * w + 256 * j),
-                                     16, 0, 0);
+  const u32 t = threadIdx.x, w = uniform(t >> 6);
+  __builtin_amdgcn_global_load_lds(g + 4 * t, l + 256 * w, 16, 0, 0);
+  if (w < 4)
+    __builtin_amdgcn_global_load_lds(g + 4 * (t + kT), l + 256 * w + 4 * kT, 16, 0, 0);
 }
 
 // Copy the n (a multiple of 32) words at g into LDS at l, 16 bytes per
 // lane, with the agent-coherent cache policy of ld_coherent (sc1): the
 // words may have been written by other workgroups of the lane group.
 __device__ __forceinline__ void coherent_fetch(const u32 *g, u32 *l, u32 n) {
-  const u32 t = threadIdx.x, w = t >> 6;
+  const u32 t = threadIdx.x, w = uniform(t >> 6);
 #pragma unroll
-  for (int j = 0; j < 8; ++j)
-    if (4 * (t + 256 * j) < n)
-      __builtin_amdgcn_global_load_lds(g + 4 * (t + 256 * j), l + 4 * (64 * w + 256 * j),
+  for (int j = 0; j < 2; ++j)
+    if (4 * (t + kT * j) < n)
+      __builtin_amdgcn_global_load_lds(g + 4 * (t + kT * j), l + 256 * w + 4 * kT * j,
                                        16, 0, 16);
 }
 
@@ -163,25 +151,62 @@ __device__ __forceinline__ void coherent_fetch(const u32 *g, u32 *l, u32 n) {
 // the workgroup barrier that precedes the first read of a fetched section.
 __device__ __forceinline__ void sec_wait() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
-// Header of one partition (src/flatten.rs:198-258) and this thread's
-// writeout hook.
+// Header of one partition (src/flatten.rs:198-258) and the writeout hook of
+// this thread's row, four threads to a row.  The words stay as they were
+// loaded (nothing waits for them) until the partition starts.
 struct BHdr {
-  u32 S, is_last, num_ios, io, ns, so, R, nd, hook;
+  uint4 a, b;
+  u32 hook;
 };
 
 __device__ __forceinline__ BHdr load_bhdr(const u32 *p) {
   BHdr h;
-  h.S = p[0];
-  h.is_last = p[1];
-  h.num_ios = p[2];
-  h.io = p[3];
-  h.ns = p[4];
-  h.so = p[5];
-  h.R = p[6];
-  h.nd = p[7];
-  const u32 hk = p[128 + (threadIdx.x >> 1)];
-  h.hook = (threadIdx.x & 1) ? (hk >> 16) : (hk & 0xffffu);
+  h.a = *reinterpret_cast<const uint4 *>(p);
+  h.b = *reinterpret_cast<const uint4 *>(p + 4);
+  h.hook = p[128 + (threadIdx.x >> 3)];
   return h;
+}
+
+// Source lane-words of this thread's first-layer positions t + kT * j.
+constexpr int kG = kLayerWords / kT;
+__device__ __forceinline__ void load_sources(u32 (&src)[kG], const u32 *gsrc) {
+#pragma unroll
+  for (int j = 0; j < kG; ++j) src[j] = gsrc[threadIdx.x + kT * j];
+}
+__device__ __forceinline__ void load_words(u32 (&v)[kG], const u32 (&src)[kG], const u32 *in,
+                                           const u32 *out) {
+#pragma unroll
+  for (int j = 0; j < kG; ++j) {
+    const u32 e = src[j];
+    v[j] = e != kNoSource ? ld_coherent(((e >> 31) ? out : in) + (e & 0x7fffffffu)) : 0u;
+  }
+}
+
+// Value of lane L + HW on lane L, for HW a power of two and the lanes where
+// that stays inside the wave (rows of 16 for HW < 16).
+template <int HW>
+__device__ __forceinline__ u32 lane_up(u32 v) {
+  if constexpr (HW == 32) {
+    return __builtin_amdgcn_permlane32_swap(v, v, false, false)[1];
+  } else if constexpr (HW == 16) {
+    return __builtin_amdgcn_permlane16_swap(v, v, false, false)[1];
+  } else {
+    return __builtin_amdgcn_update_dpp(0u, v, 0x100 + HW, 0xF, 0xF, false);
+  }
+}
+
+// bit b of a flag word, b constant, as an all-lanes mask, in a gate
+__device__ __forceinline__ u32 fgate(u32 a, u32 b, u32 fx, u32 fy, u32 fz, int bit) {
+  return (a ^ bmask(fx, bit)) & ((b ^ bmask(fy, bit)) | bmask(fz, bit));
+}
+
+// Level of wave 0's tree whose nodes are words HW .. 2HW - 1: on entry lane
+// i < 2HW holds word 2HW + i, on exit lane i < HW word HW + i.  Word w's
+// flags are bits 9..11 of lane w's flag word.
+template <int HW>
+__device__ __forceinline__ u32 top_level(u32 cur, u32 fw) {
+  return fgate(cur, lane_up<HW>(cur), lane_up<HW>(fw), lane_up<HW>(fw) >> 1,
+               lane_up<HW>(fw) >> 2, 9);
 }
 
 // Runs the partitions of one (major stage, block).  On entry h and src hold
@@ -189,13 +214,21 @@ __device__ __forceinline__ BHdr load_bhdr(const u32 *p) {
 // script is not empty); on return they hold those of the first partition of
 // the block's next major stage (script nscript, table ngsrc), loaded while
 // this stage ran.
+//
+// Four adjacent lanes (quarter q) share the subtree that the script's lane
+// layout gives one of 256 threads (v): quarter q owns its level-1 gates q,
+// q + 4, q + 8, q + 12, hence its level-2 gates q, q + 4 and its level-3
+// gate q, in registers; levels 4 and 5 are two moves inside the four lanes.
 __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__restrict__ script,
                                 const u32 *__restrict__ gsrc,
                                 const u32 *__restrict__ in, u32 *__restrict__ out,
                                 u32 *ram_group, u32 *lds, u32 *prof, BHdr &h,
-                                u32 (&src)[32], const u32 *nscript, const u32 *ngsrc) {
+                                u32 (&src)[kG], const u32 *nscript, const u32 *ngsrc) {
   const u32 t = threadIdx.x;
   const u32 lane = t & 63;
+  const u32 v = t >> 2, q4 = t & 3;
+  const u32 swt = sw(t);             // swizzled positions of this thread
+  const u32 swp = sw(v + 256 * q4);  // of its gates at p0 = v + 256 * q4
   u32 *layer = lds, *WO = lds + kLayerWords;
   u32 *OLD = lds + 2 * kLayerWords + 2 * kSecWords;
   // section buffer k & 1 (pointer arithmetic, not an array: no scratch)
@@ -205,156 +238,146 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
   // the current partition when both are in this major stage (their sources
   // are earlier major stages and the previous snapshot, complete since the
   // barrier before this stage)
-  u32 vnext[32];
+  u32 vnext[kG];
   bool have_next = false;
   for (;; gsrc += kLayerWords) {
-    if (h.S == 0) {  // no partition in this stage: fetch the next stage's first
+    const u32 S = uniform(h.a.x);
+    if (S == 0) {  // no partition in this stage: fetch the next stage's first
       h = load_bhdr(nscript);
-      if (h.S != 0) {
-#pragma unroll
-        for (int j = 0; j < 32; ++j) src[j] = ngsrc[t + 256 * j];
-      }
+      if (uniform(h.a.x) != 0) load_sources(src, ngsrc);
       break;
     }
     const unsigned long long tick0 = prof ? clock64() : 0;
-    const u32 S = h.S, is_last = h.is_last, num_ios = h.num_ios, io = h.io;
-    const u32 ns = h.ns, so = h.so, R = h.R, nd = h.nd, hook = h.hook;
+    const u32 is_last = uniform(h.a.y), num_ios = uniform(h.a.z), io = uniform(h.a.w);
+    const u32 ns = uniform(h.b.x), so = uniform(h.b.y), R = uniform(h.b.z);
+    const u32 nd = uniform(h.b.w);
+    const u32 hook = (t & 4) ? (h.hook >> 16) : (h.hook & 0xffffu);
     // sections: stage 0..S-1, SRAM/dup, clock enable, contiguous
     const u32 *secg = script + pi + 256 + (size_t)512 * R;
     pi += 256 + (size_t)512 * R + (size_t)kSecWords * (S + 2);
-    // the successor's header (the next partition here, or the next stage's
-    // first) is requested now, a partition ahead of its use
-    h = is_last ? load_bhdr(nscript) : load_bhdr(script + pi);
-    const u32 next_s = h.S;
 
     sec_fetch(secg, secb(0));
-    // the commit's old values (this partition's writeouts in the previous
-    // snapshot, which nothing changes during the cycle) go to LDS now and
-    // land while the partition runs
-    coherent_fetch(in + (size_t)io * 32, OLD, num_ios * 32);
-    // ---- global read through the gather table: 32 independent loads of
-    // state words at entries prefetched one partition ahead (or the words
-    // themselves, when the previous partition of this stage loaded them)
+    // ---- global read through the gather table: kG independent loads per
+    // thread of state words at entries prefetched one partition ahead (or
+    // the words themselves, when the previous partition of this stage
+    // loaded them)
     {
-      u32 v[32];
+      u32 w[kG];
       if (have_next) {
 #pragma unroll
-        for (int j = 0; j < 32; ++j) v[j] = vnext[j];
+        for (int j = 0; j < kG; ++j) w[j] = vnext[j];
       } else {
-#pragma unroll
-        for (int j = 0; j < 32; ++j) {
-          u32 e = src[j];
-          v[j] = e != kNoSource ? ld_coherent(((e >> 31) ? out : in) + (e & 0x7fffffffu)) : 0u;
-        }
+        load_words(w, src, in, out);
       }
-      // the successor's entries load while this partition runs (the table
-      // is read-only)
-      if (next_s != 0) {
-        const u32 *nx = is_last ? ngsrc : gsrc + kLayerWords;
+      // the commit's old values (this partition's writeouts in the previous
+      // snapshot, which nothing changes during the cycle) go to LDS now and
+      // land while the partition runs
+      coherent_fetch(in + (size_t)io * 32, OLD, num_ios * 32);
+      // the header of the successor (the next partition here, or the next
+      // stage's first)
+      h = load_bhdr(is_last ? nscript : script + pi);
 #pragma unroll
-        for (int j = 0; j < 32; ++j) src[j] = nx[t + 256 * j];
-      }
-#pragma unroll
-      for (int j = 0; j < 32; ++j) layer[sw(t + 256 * j)] = v[j];
+      for (int j = 0; j < kG; ++j) layer[swt + kT * j] = w[j];
     }
     sec_wait();
     __syncthreads();
+    // the successor's entries load while this partition runs
+    const u32 next_s = uniform(h.a.x);
+    if (next_s != 0) load_sources(src, is_last ? ngsrc : gsrc + kLayerWords);
 
     const u32 nperm = ns * 4 + nd;  // SRAM port and duplicate words
     // ---- boomerang stages, in place on the one layer: every thread first
-    // gathers its 32 level-1 operands into registers, then (after a
+    // gathers its 8 level-1 operands into registers, then (after a
     // barrier) the layer is overwritten with this stage's after-layout
     for (u32 s = 0; s < S; ++s) {
-      const uint4 *S4 = reinterpret_cast<const uint4 *>(secb(s));
-      const uint4 P0 = S4[t], P1 = S4[256 + t], P2 = S4[512 + t], P3 = S4[768 + t];
-      const uint4 F = S4[1024 + t];
+      const u32 *sec = secb(s);
+      // operand m = q4 + 4j of thread v: half q4 & 1 of its word (q4 >> 1) +
+      // 2j.  The 16 v of a wave read 256 consecutive bytes per j pair
+      u32 g[8];
+      {
+        u32 pw[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          pw[j] = sec[1024 * (j >> 1) + 4 * v + (q4 >> 1) + 2 * (j & 1)];
+        const u32 sh = 16 * (q4 & 1);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) g[j] = layer[(pw[j] >> sh) & 0xffffu];
+      }
+      const uint4 F = *reinterpret_cast<const uint4 *>(sec + 4096 + 4 * v);
+      const u32 fw = t < 64 ? sec[4096 + 4 * t + 3] : 0u;
       // the next section goes into the other buffer, last read by the
       // previous stage, which finished before the last barrier; after the
       // last stage that is the SRAM/dup section, or the clock-enable
       // section when the partition has no SRAM or duplicate words
       const u32 nxt = (s + 1 == S && nperm == 0) ? S + 1 : s + 1;
       sec_fetch(secg + (size_t)kSecWords * nxt, secb(s + 1));
-      const u32 pw[16] = {P0.x, P0.y, P0.z, P0.w, P1.x, P1.y, P1.z, P1.w,
-                          P2.x, P2.y, P2.z, P2.w, P3.x, P3.y, P3.z, P3.w};
-      u32 g[32];
-#pragma unroll
-      for (int m = 0; m < 32; ++m) g[m] = layer[(pw[m >> 1] >> (16 * (m & 1))) & 0xffffu];
       __syncthreads();  // all operands read before the layer is rewritten
-      // levels 1..5 of the subtree rooted at position 256 + t; gate g's
-      // flags are bit g of F.x / F.y / F.z
-      u32 L1[16];
-#pragma unroll
-      for (int k = 0; k < 16; ++k) {
-        L1[k] = (g[k] ^ bmask(F.x, k)) & ((g[k + 16] ^ bmask(F.y, k)) | bmask(F.z, k));
-        layer[sw(4096 + t + 256u * k)] = L1[k];
-      }
-      u32 L2[8];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        L2[k] = (L1[k] ^ bmask(F.x, 16 + k)) & ((L1[k + 8] ^ bmask(F.y, 16 + k)) |
-                                                 bmask(F.z, 16 + k));
-        layer[sw(2048 + t + 256u * k)] = L2[k];
-      }
-      u32 L3[4];
+      // levels 1..5 of the subtree rooted at position 256 + v; gate g's
+      // flags are bit g of F.x / F.y / F.z, this quarter's 4-apart gates
+      // bits 0, 4, .. of the shifted words
+      const u32 fx = F.x >> q4, fy = F.y >> q4, fz = F.z >> q4;
+      u32 L1[4];
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        L3[k] = (L2[k] ^ bmask(F.x, 24 + k)) & ((L2[k + 4] ^ bmask(F.y, 24 + k)) |
-                                                 bmask(F.z, 24 + k));
-        layer[sw(1024 + t + 256u * k)] = L3[k];
+        L1[k] = fgate(g[k], g[k + 4], fx, fy, fz, 4 * k);
+        layer[4096 + swp + 1024u * k] = L1[k];
       }
-      u32 L4[2];
+      u32 L2[2];
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
-        L4[k] = (L3[k] ^ bmask(F.x, 28 + k)) & ((L3[k + 2] ^ bmask(F.y, 28 + k)) |
-                                                 bmask(F.z, 28 + k));
-        layer[sw(512 + t + 256u * k)] = L4[k];
+        L2[k] = fgate(L1[k], L1[k + 2], fx, fy, fz, 16 + 4 * k);
+        layer[2048 + swp + 1024u * k] = L2[k];
       }
-      layer[sw(256 + t)] = (L4[0] ^ bmask(F.x, 30)) & ((L4[1] ^ bmask(F.y, 30)) | bmask(F.z, 30));
+      const u32 L3 = fgate(L2[0], L2[1], fx, fy, fz, 24);
+      layer[1024 + swp] = L3;
+      // level 4 on quarters 0 and 1 (with 2 and 3), level 5 on quarter 0
+      const u32 L4 = fgate(L3, __builtin_amdgcn_update_dpp(0u, L3, 0x4E, 0xF, 0xF, false), fx,
+                           fy, fz, 28);
+      const u32 L5 = fgate(L4, __builtin_amdgcn_update_dpp(0u, L4, 0xB1, 0xF, 0xF, false), fx,
+                           fy, fz, 30);
+      if (q4 < 2) layer[512 + (swp ^ 16)] = L4;  // sw(512 + p0), p0 < 512
+      if (q4 == 0) layer[256 + (swp ^ 8)] = L5;  // sw(256 + v), v < 256
       __syncthreads();
       if (t < 64) {
-        // wave 0 lane L: flags of positions 128+L, 192+L, 64+L, L in F.w
-        const u32 fw = F.w;
-        auto wg = [fw](u32 a, u32 b, int i) {
-          return (a ^ bmask(fw, 3 * i)) & ((b ^ bmask(fw, 3 * i + 1)) | bmask(fw, 3 * i + 2));
-        };
+        // wave 0 lane L: flags of positions 128+L, 192+L, 64+L, L in fw.
         // level 6: positions 128+L and 192+L; level 7: 64+L
-        u32 o6a = wg(layer[sw(256 + lane)], layer[sw(384 + lane)], 0);
-        u32 o6b = wg(layer[sw(320 + lane)], layer[sw(448 + lane)], 1);
-        u32 o7 = wg(o6a, o6b, 2);
-        // level 8: lanes 32..63 -> position L from L+32 (lane L-32) and
-        // L+64 (own level-7 word)
-        u32 c = 0;
-        u32 a8 = __shfl(o7, (lane + 32) & 63);
-        if (lane >= 32) c = wg(a8, o7, 3);
-#pragma unroll
-        for (int len = 16; len >= 1; len >>= 1) {
-          u32 a = __shfl(c, (lane + len) & 63);
-          u32 b = __shfl(c, (lane + 2 * len) & 63);
-          if (lane >= (u32)len && lane < 2u * len) c = wg(a, b, 3);
-        }
+        const u32 o6a = fgate(layer[sw(256 + lane)], layer[sw(384 + lane)], fw, fw >> 1,
+                              fw >> 2, 0);
+        const u32 o6b = fgate(layer[sw(320 + lane)], layer[sw(448 + lane)], fw, fw >> 1,
+                              fw >> 2, 3);
+        const u32 o7 = fgate(o6a, o6b, fw, fw >> 1, fw >> 2, 6);
         layer[sw(128 + lane)] = o6a;
         layer[sw(192 + lane)] = o6b;
         layer[sw(64 + lane)] = o7;
-        layer[sw(lane)] = c;  // lane 0 keeps position 0 at zero
+        // levels 8..13 by cross-lane moves; word 0 stays zero
+        u32 cur = top_level<32>(o7, fw);
+        if (lane < 32) layer[sw(32 + lane)] = cur;
+        cur = top_level<16>(cur, fw);
+        if (lane < 16) layer[sw(16 + lane)] = cur;
+        cur = top_level<8>(cur, fw);
+        if (lane < 8) layer[8 + lane] = cur;
+        cur = top_level<4>(cur, fw);
+        if (lane < 4) layer[4 + lane] = cur;
+        cur = top_level<2>(cur, fw);
+        if (lane < 2) layer[2 + lane] = cur;
+        cur = top_level<1>(cur, fw);
+        if (lane == 0) {
+          layer[1] = cur;
+          layer[0] = 0;
+        }
       }
       sec_wait();  // section s+1 is read right after this barrier
       __syncthreads();
       if ((hook >> 8) == s) {
-        const u32 src = 32u * (hook & 255u);
+        const u32 from = 32u * (hook & 255u) + 8 * q4, to = 32 * v + 8 * q4;
 #pragma unroll
-        for (u32 q = 0; q < 32; ++q) WO[sw(32 * t + q)] = layer[sw(src + q)];
+        for (u32 k = 0; k < 8; ++k) WO[sw(to + k)] = layer[sw(from + k)];
       }
     }
     // the next partition of this stage: its first-layer words (its gather
     // entries arrived during this partition)
     have_next = !is_last && next_s != 0;
-    if (have_next) {
-#pragma unroll
-      for (int j = 0; j < 32; ++j) {
-        u32 e = src[j];
-        vnext[j] = e != kNoSource ? ld_coherent(((e >> 31) ? out : in) + (e & 0x7fffffffu)) : 0u;
-      }
-    }
+    if (have_next) load_words(vnext, src, in, out);
     __syncthreads();
 
     // ---- SRAM + duplicate permutation into the layer (free now); a
@@ -367,15 +390,15 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
         const u32 *fl = sec + 4096;
         // the clock-enable section goes into the buffer of the last stage
         sec_fetch(secg + (size_t)kSecWords * (S + 1), secb(S + 1));
-        for (u32 q = t; q < nperm * 32; q += 256) {
+        for (u32 q = t; q < nperm * 32; q += kT) {
           uint4 f = *reinterpret_cast<const uint4 *>(fl + 4 * (q >> 5));
-          u32 v = WO[sw(perm_at(sec, q))];
-          layer[sw(q)] = (v & ~fbit(f.y, q)) ^ fbit(f.x, q);
+          u32 w = WO[sw(perm_at(sec, q))];
+          layer[sw(q)] = (w & ~fbit(f.y, q)) ^ fbit(f.x, q);
         }
       }
       __syncthreads();
       // SRAM ports: thread per (sram, lane)
-      for (u32 base = 0; base < ns * 32; base += 256) {
+      for (u32 base = 0; base < ns * 32; base += kT) {
         u32 id = base + t;
         u32 s = id >> 5, l = id & 31;
         u32 r = 0;
@@ -383,10 +406,12 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
         if (act) {
           const u32 P = 128 * s;
           u32 ra = 0, wa = 0, en = 0, data = 0;
+#pragma unroll 1
           for (int k = 0; k < 13; ++k) {
             ra |= ((layer[sw(P + k)] >> l) & 1u) << k;
             wa |= ((layer[sw(P + 16 + k)] >> l) & 1u) << k;
           }
+#pragma unroll 1
           for (int k = 0; k < 32; ++k) {
             en |= ((layer[sw(P + 32 + k)] >> l) & 1u) << k;
             data |= ((layer[sw(P + 64 + k)] >> l) & 1u) << k;
@@ -398,6 +423,7 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
         }
         // transpose the 32 read words of each SRAM into lane-words
         u32 mine = 0;
+#pragma unroll 1
         for (int k = 0; k < 32; ++k) {
           unsigned long long m = __ballot(act && ((r >> k) & 1u));
           u32 half = (u32)(m >> (32 * ((t >> 5) & 1)));
@@ -405,7 +431,7 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
         }
         if (act) WO[sw(32 * (num_ios - ns + s) + l)] = mine;
       }
-      for (u32 q = t; q < nd * 32; q += 256)
+      for (u32 q = t; q < nd * 32; q += kT)
         WO[sw(32 * (num_ios - ns - nd) + q)] = layer[sw(ns * 128 + q)];
       sec_wait();  // the clock-enable section is read after this barrier
       __syncthreads();
@@ -416,7 +442,7 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
       const u32 *sec = secb(nperm ? S + 1 : S);
       const u32 *fl = sec + 4096;
       u32 *o = out + (size_t)io * 32;
-      for (u32 q = t; q < num_ios * 32; q += 256) {
+      for (u32 q = t; q < num_ios * 32; q += kT) {
         uint4 f = *reinterpret_cast<const uint4 *>(fl + 4 * (q >> 5));
         // a bit whose enable is forced (set0) needs no gather: ck = inv
         u32 ck = fbit(f.x, q);
@@ -434,7 +460,7 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
   }
 }
 
-__global__ __launch_bounds__(256) void batched_kernel(BArgs A) {
+__global__ __launch_bounds__(kT) void batched_kernel(BArgs A) {
   extern __shared__ u32 lds[];
   u32 &s_aborted = lds[kAbortLds];  // set by a group wait when the launch aborts
   if (threadIdx.x == 0) s_aborted = 0;
@@ -447,7 +473,7 @@ __global__ __launch_bounds__(256) void batched_kernel(BArgs A) {
   u32 *ram_group = A.sram + (size_t)g * 32 * A.sram_size;
   u32 *slots = A.slots + 32 * g;
   const u32 t = threadIdx.x, l = t & 31;
-  const u32 par = b * 256 + t, npar = A.W * 256;  // group-wide thread index
+  const u32 par = b * kT + t, npar = A.W * kT;  // group-wide thread index
   // every thread mirrors slot l = t & 31 of its group; a launch resumes
   // the group at its recorded cycle, each slot's lane at the group cycle it
   // started
@@ -463,13 +489,9 @@ __global__ __launch_bounds__(256) void batched_kernel(BArgs A) {
   }
   // header and gather entries of the block's first partition of major
   // stage 0
-  u32 src[32];
+  u32 src[kG];
   BHdr h = load_bhdr(A.bd + A.bs[b]);
-  if (h.S != 0) {
-    const u32 *g0 = A.gsrc + (size_t)A.gidx[b] * kLayerWords;
-#pragma unroll
-    for (int j = 0; j < 32; ++j) src[j] = g0[t + 256 * j];
-  }
+  load_sources(src, A.gsrc + (size_t)A.gidx[b] * kLayerWords);
   __syncthreads();
   u32 c = c0;
   for (;; ++c) {
@@ -487,7 +509,7 @@ __global__ __launch_bounds__(256) void batched_kernel(BArgs A) {
     }
     if (b == 0 && c > 0 && c - 1 < A.obs_cap) {
       u32 *o = A.obs_out + ((size_t)g * A.obs_cap + (c - 1)) * A.n_obs;
-      for (u32 k = t; k < A.n_obs; k += 256) o[k] = ld_coherent(in + A.obs_bits[k]);
+      for (u32 k = t; k < A.n_obs; k += kT) o[k] = ld_coherent(in + A.obs_bits[k]);
     }
     // a launch with a budget stops after that many group cycles, with the
     // observation of its last cycle written (the same decision in every
@@ -532,7 +554,7 @@ __global__ __launch_bounds__(256) void batched_kernel(BArgs A) {
       grid_sync_coherent(bar, A.W, b, gen, &gb_error, &gb_wait_polls, s_aborted);
       if (A.stim) {
         // packed stimulus: the new lanes' input bits of their snapshot 0
-        for (u32 k0 = b * 8; k0 < A.n_in; k0 += A.W * 8) {
+        for (u32 k0 = b * (kT / 32); k0 < A.n_in; k0 += A.W * (kT / 32)) {
           const u32 k = k0 + (t >> 5);
           bool bit = false;
           if (k < A.n_in && fin && my_lane != kNoLane) {
@@ -554,7 +576,7 @@ __global__ __launch_bounds__(256) void batched_kernel(BArgs A) {
       // stimulus of snapshot c+1 from the lanes' packed input words: input
       // bit k of slot l is bit in_bits[k] of the lane's snapshot
       // c - start + 1 (inactive slots read 0)
-      for (u32 k0 = b * 8; k0 < A.n_in; k0 += A.W * 8) {
+      for (u32 k0 = b * (kT / 32); k0 < A.n_in; k0 += A.W * (kT / 32)) {
         const u32 k = k0 + (t >> 5);
         bool bit = false;
         if (k < A.n_in && my_lane != kNoLane) {
@@ -569,7 +591,7 @@ __global__ __launch_bounds__(256) void batched_kernel(BArgs A) {
     }
     // stimulus of snapshot c+1: data bit k toggles for the lane in slot l
     // when hash(seed, lane cycle + 1, k) < thresh
-    for (u32 k0 = b * 8; !A.stim && k0 < A.n_data; k0 += A.W * 8) {
+    for (u32 k0 = b * (kT / 32); !A.stim && k0 < A.n_data; k0 += A.W * (kT / 32)) {
       u32 k = k0 + (t >> 5);
       bool act = k < A.n_data && my_lane != kNoLane;
       u32 bit = 0;
@@ -639,7 +661,7 @@ int batched_blocks_per_cu(int *out) {
   }
   int per = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-          &per, reinterpret_cast<const void *>(&batched_kernel), 256,
+          &per, reinterpret_cast<const void *>(&batched_kernel), kT,
           kLdsWords * 4) != hipSuccess)
     return -1;
   *out = per;
@@ -750,11 +772,11 @@ int batched_impl(usize num_groups, usize blocks_per_group, usize num_major_stage
   hipError_t e;
   if (cap == hipStreamCaptureStatusActive) {
     e = hipLaunchKernel(reinterpret_cast<const void *>(&batched_kernel),
-                        dim3((u32)(num_groups * blocks_per_group)), dim3(256), args,
+                        dim3((u32)(num_groups * blocks_per_group)), dim3(kT), args,
                         kLdsWords * 4, (hipStream_t)stream);
   } else {
     e = hipLaunchCooperativeKernel(reinterpret_cast<const void *>(&batched_kernel),
-                                   dim3((u32)(num_groups * blocks_per_group)), dim3(256),
+                                   dim3((u32)(num_groups * blocks_per_group)), dim3(kT),
                                    args, kLdsWords * 4, (hipStream_t)stream);
   }
   if (e != hipSuccess) {

@@ -40,6 +40,9 @@ __device__ __forceinline__ void st_coherent(u32 *p, u32 v) {
 // Wait until this wave's memory operations have completed.
 __device__ __forceinline__ void wait_vmem() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
+// A value that is the same on every lane of the wave, in a scalar register.
+__device__ __forceinline__ u32 uniform(u32 v) { return __builtin_amdgcn_readfirstlane(v); }
+
 // Grid-wide barrier among `n` co-resident workgroups whose inter-workgroup
 // data moves only through ld_coherent / st_coherent.  Those accesses are
 // coherent at agent scope by themselves, so the barrier needs ordering, not

@@ -166,8 +166,6 @@ __device__ __forceinline__ RawHdr load_hdr(const u32 *__restrict__ bd, size_t of
   return r;
 }
 
-__device__ __forceinline__ u32 uniform(u32 v) { return __builtin_amdgcn_readfirstlane(v); }
-
 __device__ __forceinline__ PartHdr settle(const RawHdr &r) {
   PartHdr h;
   h.base = r.base;
