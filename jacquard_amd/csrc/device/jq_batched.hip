@@ -464,7 +464,11 @@ __global__ __launch_bounds__(kT) void batched_kernel(BArgs A) {
   extern __shared__ u32 lds[];
   u32 &s_aborted = lds[kAbortLds];  // set by a group wait when the launch aborts
   if (threadIdx.x == 0) s_aborted = 0;
-  const u32 g = blockIdx.x / A.W, b = blockIdx.x % A.W;
+  // Workgroups go to the 8 XCDs in turn.  Taken XCD by XCD, a group's
+  // blocks share as few L2 caches as can be.
+  const u32 x = blockIdx.x & 7u, n8 = gridDim.x >> 3, rest = gridDim.x & 7u;
+  const u32 place = x * n8 + (x < rest ? x : rest) + (blockIdx.x >> 3);
+  const u32 g = place / A.W, b = place % A.W;
   u32 *bar = A.bar + kCohSlotWords * g;
   u32 gen = read_gen(bar);
   const size_t snap = (size_t)A.rio * 32;
