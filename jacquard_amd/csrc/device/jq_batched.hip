@@ -134,6 +134,20 @@ __device__ __forceinline__ void sec_fetch(const u32 *g, u32 *l) {
     __builtin_amdgcn_global_load_lds(g + 4 * (t + kT), l + 256 * w + 4 * kT, 16, 0, 0);
 }
 
+// The same for a writeout section (SRAM/dup or clock enable), of which the
+// first `rows` rows are used: 4 words a row in each of its four permutation
+// blocks and its flag block, a wave to a block.  Whole, the clock-enable
+// section was a quarter of the bytes a partition streams, and 20 rows of
+// 256 are usual (4M gates 4 x 64: 17079 us against 16460).
+__device__ __forceinline__ void row_fetch(const u32 *g, u32 *l, u32 rows) {
+  const u32 lane = threadIdx.x & 63, k = uniform(threadIdx.x >> 6);
+  if (k < 5)
+    for (u32 u = 0; u < rows; u += 64)
+      if (u + lane < rows)
+        __builtin_amdgcn_global_load_lds(g + 1024 * k + 4 * (u + lane), l + 1024 * k + 4 * u,
+                                         16, 0, 0);
+}
+
 // Copy the n (a multiple of 32) words at g into LDS at l, 16 bytes per
 // lane, with the agent-coherent cache policy of ld_coherent (sc1): the
 // words may have been written by other workgroups of the lane group.
@@ -173,12 +187,29 @@ __device__ __forceinline__ void load_sources(u32 (&src)[kG], const u32 *gsrc) {
 #pragma unroll
   for (int j = 0; j < kG; ++j) src[j] = gsrc[threadIdx.x + kT * j];
 }
-__device__ __forceinline__ void load_words(u32 (&v)[kG], const u32 (&src)[kG], const u32 *in,
-                                           const u32 *out) {
+// A group's two snapshots as a buffer of lane-words, read with the
+// agent-coherent cache policy of ld_coherent (sc1).  A position without
+// source is an offset past the buffer's end and reads 0 without a branch;
+// with 64-bit addresses every word cost a compare, a branch and four address
+// operations (4M gates 4 x 64: 18087 us against 17083).  Snapshots too large
+// for 32-bit offsets (16M state words) take those.
+struct Snaps {
+  __amdgpu_buffer_rsrc_t rsrc;
+  u32 in, out;  // byte offsets of the snapshots
+};
+constexpr u32 kMaxBufferRio = (1u << 24) - 1;  // two snapshots below 4 GiB
+template <bool WIDE>
+__device__ __forceinline__ void load_words(u32 (&v)[kG], const u32 (&src)[kG], const Snaps &B,
+                                           const u32 *in, const u32 *out) {
 #pragma unroll
   for (int j = 0; j < kG; ++j) {
     const u32 e = src[j];
-    v[j] = e != kNoSource ? ld_coherent(((e >> 31) ? out : in) + (e & 0x7fffffffu)) : 0u;
+    if (WIDE) {
+      v[j] = e != kNoSource ? ld_coherent(((e >> 31) ? out : in) + (e & 0x7fffffffu)) : 0u;
+    } else {
+      const u32 at = e == kNoSource ? kNoSource : 4 * e + ((e >> 31) ? B.out : B.in);
+      v[j] = __builtin_amdgcn_raw_buffer_load_b32(B.rsrc, at, 0, 16);
+    }
   }
 }
 
@@ -219,11 +250,13 @@ __device__ __forceinline__ u32 top_level(u32 cur, u32 fw) {
 // layout gives one of 256 threads (v): quarter q owns its level-1 gates q,
 // q + 4, q + 8, q + 12, hence its level-2 gates q, q + 4 and its level-3
 // gate q, in registers; levels 4 and 5 are two moves inside the four lanes.
+template <bool WIDE>
 __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__restrict__ script,
                                 const u32 *__restrict__ gsrc,
                                 const u32 *__restrict__ in, u32 *__restrict__ out,
                                 u32 *ram_group, u32 *lds, u32 *prof, BHdr &h,
-                                u32 (&src)[kG], const u32 *nscript, const u32 *ngsrc) {
+                                u32 (&src)[kG], const u32 *nscript, const u32 *ngsrc,
+                                const Snaps &B) {
   const u32 t = threadIdx.x;
   const u32 lane = t & 63;
   const u32 v = t >> 2, q4 = t & 3;
@@ -267,7 +300,7 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
 #pragma unroll
         for (int j = 0; j < kG; ++j) w[j] = vnext[j];
       } else {
-        load_words(w, src, in, out);
+        load_words<WIDE>(w, src, B, in, out);
       }
       // the commit's old values (this partition's writeouts in the previous
       // snapshot, which nothing changes during the cycle) go to LDS now and
@@ -309,8 +342,11 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
       // previous stage, which finished before the last barrier; after the
       // last stage that is the SRAM/dup section, or the clock-enable
       // section when the partition has no SRAM or duplicate words
-      const u32 nxt = (s + 1 == S && nperm == 0) ? S + 1 : s + 1;
-      sec_fetch(secg + (size_t)kSecWords * nxt, secb(s + 1));
+      if (s + 1 < S)
+        sec_fetch(secg + (size_t)kSecWords * (s + 1), secb(s + 1));
+      else
+        row_fetch(secg + (size_t)kSecWords * (nperm ? S : S + 1), secb(S),
+                  nperm ? nperm : num_ios);
       __syncthreads();  // all operands read before the layer is rewritten
       // levels 1..5 of the subtree rooted at position 256 + v; gate g's
       // flags are bit g of F.x / F.y / F.z, this quarter's 4-apart gates
@@ -377,7 +413,7 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
     // the next partition of this stage: its first-layer words (its gather
     // entries arrived during this partition)
     have_next = !is_last && next_s != 0;
-    if (have_next) load_words(vnext, src, in, out);
+    if (have_next) load_words<WIDE>(vnext, src, B, in, out);
     __syncthreads();
 
     // ---- SRAM + duplicate permutation into the layer (free now); a
@@ -389,7 +425,7 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
         const u32 *sec = secb(S);
         const u32 *fl = sec + 4096;
         // the clock-enable section goes into the buffer of the last stage
-        sec_fetch(secg + (size_t)kSecWords * (S + 1), secb(S + 1));
+        row_fetch(secg + (size_t)kSecWords * (S + 1), secb(S + 1), num_ios);
         for (u32 q = t; q < nperm * 32; q += kT) {
           uint4 f = *reinterpret_cast<const uint4 *>(fl + 4 * (q >> 5));
           u32 w = WO[sw(perm_at(sec, q))];
@@ -460,6 +496,8 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
   }
 }
 
+// WIDE: snapshots of more than kMaxBufferRio words.
+template <bool WIDE>
 __global__ __launch_bounds__(kT) void batched_kernel(BArgs A) {
   extern __shared__ u32 lds[];
   u32 &s_aborted = lds[kAbortLds];  // set by a group wait when the launch aborts
@@ -474,6 +512,8 @@ __global__ __launch_bounds__(kT) void batched_kernel(BArgs A) {
   const size_t snap = (size_t)A.rio * 32;
   u32 *st0 = A.states + (size_t)g * 2 * snap;
   u32 *st1 = st0 + snap;
+  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      st0, 0, WIDE ? 0 : (int)(8 * (u32)snap), 0x00027000);
   u32 *ram_group = A.sram + (size_t)g * 32 * A.sram_size;
   u32 *slots = A.slots + 32 * g;
   const u32 t = threadIdx.x, l = t & 31;
@@ -504,6 +544,8 @@ __global__ __launch_bounds__(kT) void batched_kernel(BArgs A) {
     if (s_aborted) break;
     u32 *in = (c & 1) ? st1 : st0;
     u32 *out = (c & 1) ? st0 : st1;
+    const u32 half = 4 * (u32)snap;
+    const Snaps B{rsrc, (c & 1) ? half : 0u, (c & 1) ? 0u : half};
     // every group finishes within obs_cap cycles (queue bound); a launch
     // whose lane table breaks that bound stops here with an error instead
     // of looping (the same decision in every block of the group)
@@ -617,9 +659,9 @@ __global__ __launch_bounds__(kT) void batched_kernel(BArgs A) {
       // next major stage of this block (stage 0 of the next cycle after
       // the last)
       const size_t kn = mj + 1 < A.num_major ? k + A.W : (size_t)b;
-      run_block_lanes(A, A.bd + A.bs[k], A.gsrc + (size_t)A.gidx[k] * kLayerWords, in,
+      run_block_lanes<WIDE>(A, A.bd + A.bs[k], A.gsrc + (size_t)A.gidx[k] * kLayerWords, in,
                       out, ram_group, lds, prof, h, src, A.bd + A.bs[kn],
-                      A.gsrc + (size_t)A.gidx[kn] * kLayerWords);
+                      A.gsrc + (size_t)A.gidx[kn] * kLayerWords, B);
       grid_sync_coherent(bar, A.W, b, gen, &gb_error, &gb_wait_polls, s_aborted);
     }
   }
@@ -627,6 +669,11 @@ __global__ __launch_bounds__(kT) void batched_kernel(BArgs A) {
 }
 
 u32 b_slot = 0;
+
+const void *kernel_for(u32 rio) {
+  return rio > kMaxBufferRio ? reinterpret_cast<const void *>(&batched_kernel<true>)
+                             : reinterpret_cast<const void *>(&batched_kernel<false>);
+}
 
 }  // namespace
 
@@ -657,16 +704,15 @@ int batched_error_flag(u32 *out, int clear) {
 int batched_blocks_per_cu(int *out) {
   static bool attr = false;
   if (!attr) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void *>(&batched_kernel),
-                            hipFuncAttributeMaxDynamicSharedMemorySize,
-                            kLdsWords * 4) != hipSuccess)
-      return -1;
+    for (u32 rio : {0u, kMaxBufferRio + 1})
+      if (hipFuncSetAttribute(kernel_for(rio), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              kLdsWords * 4) != hipSuccess)
+        return -1;
     attr = true;
   }
   int per = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-          &per, reinterpret_cast<const void *>(&batched_kernel), kT,
-          kLdsWords * 4) != hipSuccess)
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel_for(0), kT, kLdsWords * 4) !=
+      hipSuccess)
     return -1;
   *out = per;
   return 0;
@@ -775,11 +821,10 @@ int batched_impl(usize num_groups, usize blocks_per_group, usize num_major_stage
   }
   hipError_t e;
   if (cap == hipStreamCaptureStatusActive) {
-    e = hipLaunchKernel(reinterpret_cast<const void *>(&batched_kernel),
-                        dim3((u32)(num_groups * blocks_per_group)), dim3(kT), args,
-                        kLdsWords * 4, (hipStream_t)stream);
+    e = hipLaunchKernel(kernel_for(A.rio), dim3((u32)(num_groups * blocks_per_group)),
+                        dim3(kT), args, kLdsWords * 4, (hipStream_t)stream);
   } else {
-    e = hipLaunchCooperativeKernel(reinterpret_cast<const void *>(&batched_kernel),
+    e = hipLaunchCooperativeKernel(kernel_for(A.rio),
                                    dim3((u32)(num_groups * blocks_per_group)), dim3(kT),
                                    args, kLdsWords * 4, (hipStream_t)stream);
   }

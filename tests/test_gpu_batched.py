@@ -259,3 +259,44 @@ def test_wait_time_out_aborts_the_batched_launch():
         assert L.jq_wait_limit(prev) == 1
     run = BatchedRun(s, seeds, probs, cycles, groups=1)
     _check(s, run, seeds, probs, cycles, range(40))
+
+
+class _Moved:
+    """The script with its writeout words moved up to the end of a state of
+    `rio` words; the words between the inputs and the first writeout are
+    left unused."""
+
+    def __init__(self, script, rio):
+        self._s, self.reg_io_state_size = script, rio
+        up = rio - script.reg_io_state_size
+        bd = np.array(script.blocks_data, np.uint32)
+        lo = min(int(bd[int(off) + 3]) for off in script.parts[:, 3].tolist())
+        for off in script.parts[:, 3].tolist():
+            off = int(off)
+            bd[off + 3] += np.uint32(up)
+            gr = bd[off + 256:off + 256 + 512 * int(bd[off + 6])].reshape(-1, 2)
+            hit = (gr[:, 1] != 0) & ((gr[:, 0] & 0x7FFFFFFF) >= lo)
+            gr[hit, 0] += np.uint32(up)
+        self.blocks_data = bd
+        self.output_map = {k: p + 32 * up if p >= 32 * lo else p
+                           for k, p in script.output_map.items()}
+
+    def __getattr__(self, name):
+        if name == "_batched_program":  # built from this script's own words
+            raise AttributeError(name)
+        return getattr(self._s, name)
+
+
+@pytest.mark.parametrize("rio", [(1 << 24) - 1, 1 << 24])
+def test_batched_snapshots_around_32_bit_offsets(rio):
+    """Two snapshots of 2**24 - 1 state words are the most that 32-bit byte
+    offsets reach; one word more takes 64-bit addresses.  The writeouts lie
+    at the snapshots' ends, and the lanes are the original script's."""
+    nl, comp = design("c1", level_split=6, **CONFIG1)
+    s = comp.flatten(8)
+    w = _Moved(s, rio)
+    seeds, probs, cycles = _lanes(33, 4, 9, 12)
+    want = BatchedRun(s, seeds, probs, cycles, groups=1).run()
+    got = BatchedRun(w, seeds, probs, cycles, groups=1).run(validate=False)
+    for k in range(len(seeds)):
+        assert np.array_equal(got[k], want[k]), k
