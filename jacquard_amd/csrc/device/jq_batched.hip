@@ -8,19 +8,24 @@
 // computes for it (src/sim/cpu_reference.rs:17-289), while the 8192 bit
 // gathers per boomerang stage become 8192 word gathers shared by 32 lanes.
 //
-// Work mapping inside a workgroup (256 threads, 4 x wave64):
+// Work mapping inside a workgroup (1024 threads, 16 x wave64: a workgroup
+// has its CU to itself, and with 4 waves nothing hid the LDS and memory
+// latencies; 4M gates 4 x 64, 40 cycles: 21388 us with 4 waves, 19219 with
+// 16):
 //   - global read: a per-partition gather table (built once per script from
 //     its (idx, mask) rounds) gives the source lane-word of each of the 8192
-//     first-layer positions, so each thread issues 32 independent loads
-//     instead of a chain of dependent pext steps;
-//   - every 5120-word script section (boomerang stage, SRAM/dup, clock
-//     enable) is copied into LDS with coalesced 16-byte loads, one section
-//     ahead of its use (double buffer), so the per-position permutation and
-//     flag reads are LDS reads;
-//   - thread t owns level-1 outputs t + 256k (k < 16), so levels 1..5 of its
-//     subtree stay in registers; wave 0 finishes levels 6..13 with
-//     cross-lane moves: two workgroup barriers per boomerang stage;
-//   - the three 8192-word LDS arrays (two after-layouts, the writeout area)
+//     first-layer positions, so each thread issues 8 independent loads
+//     instead of a chain of dependent pext steps.  About 3100 128-byte
+//     lines a partition at 64 bytes a clock and CU: this gather bounds a
+//     major stage, with the barrier before it;
+//   - every 5120-word boomerang section, and the used rows of the writeout
+//     sections, are copied into LDS one section ahead of their use (double
+//     buffer), so the per-position permutation and flag reads are LDS reads;
+//   - four adjacent lanes share the subtree of outputs t + 256k of one of
+//     256 virtual threads: levels 1..3 in registers, 4 and 5 by moves inside
+//     the four lanes; wave 0 finishes levels 6..13 with cross-lane moves:
+//     two workgroup barriers per boomerang stage;
+//   - the three 8192-word LDS arrays (two layers, the writeout area)
 //     are row-swizzled: word w of 32-word row r lives at w ^ (r & 31), so
 //     accesses where each lane touches the same word of a different row
 //     spread over all banks;
@@ -47,10 +52,10 @@ namespace {
 constexpr u32 kT = 1024;  // threads of a workgroup: 16 waves, 4 per SIMD
 constexpr int kLayerWords = 8192;
 constexpr int kSecWords = 5120;  // 4096 permutation words + 256 x 4 flags
-// LDS: the layer, the writeout area, two script-section buffers and the
-// commit's old writeout words (136 KB of the 160 KB), then 4 words whose
-// first is the launch's abort flag (kept in the dynamic region: a static
-// __shared__ word would move the region's start off its 256-byte boundary)
+// LDS: two layers, the writeout area and two script-section buffers (136 KB
+// of the 160 KB), then 4 words whose first is the launch's abort flag (kept
+// in the dynamic region: a static __shared__ word would move the region's
+// start off its 256-byte boundary)
 constexpr int kLdsWords = 3 * kLayerWords + 2 * kSecWords + 4;
 constexpr int kAbortLds = 3 * kLayerWords + 2 * kSecWords;
 constexpr u32 kNoSource = 0xFFFFFFFFu;
@@ -148,18 +153,6 @@ __device__ __forceinline__ void row_fetch(const u32 *g, u32 *l, u32 rows) {
                                          16, 0, 0);
 }
 
-// Copy the n (a multiple of 32) words at g into LDS at l, 16 bytes per
-// lane, with the agent-coherent cache policy of ld_coherent (sc1): the
-// words may have been written by other workgroups of the lane group.
-__device__ __forceinline__ void coherent_fetch(const u32 *g, u32 *l, u32 n) {
-  const u32 t = threadIdx.x, w = uniform(t >> 6);
-#pragma unroll
-  for (int j = 0; j < 2; ++j)
-    if (4 * (t + kT * j) < n)
-      __builtin_amdgcn_global_load_lds(g + 4 * (t + kT * j), l + 256 * w + 4 * kT * j,
-                                       16, 0, 16);
-}
-
 // Wait until this wave's outstanding global loads (including the LDS
 // copies above) have landed: s_waitcnt vmcnt(0).  Every wave runs it before
 // the workgroup barrier that precedes the first read of a fetched section.
@@ -180,6 +173,9 @@ __device__ __forceinline__ BHdr load_bhdr(const u32 *p) {
   h.hook = p[128 + (threadIdx.x >> 3)];
   return h;
 }
+
+// Writeout rows whose old values are held in registers (more are rare).
+constexpr u32 kOldRows = 64;
 
 // Source lane-words of this thread's first-layer positions t + kT * j.
 constexpr int kG = kLayerWords / kT;
@@ -262,8 +258,9 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
   const u32 v = t >> 2, q4 = t & 3;
   const u32 swt = sw(t);             // swizzled positions of this thread
   const u32 swp = sw(v + 256 * q4);  // of its gates at p0 = v + 256 * q4
-  u32 *layer = lds, *WO = lds + kLayerWords;
-  u32 *OLD = lds + 2 * kLayerWords + 2 * kSecWords;
+  u32 *WO = lds + kLayerWords;
+  // layer k & 1: the first layer is 0, stage s reads layer s and writes s + 1
+  auto layerb = [lds](u32 k) { return lds + ((k & 1u) ? 2 * kLayerWords + 2 * kSecWords : 0); };
   // section buffer k & 1 (pointer arithmetic, not an array: no scratch)
   auto secb = [lds](u32 k) { return lds + 2 * kLayerWords + (k & 1u) * kSecWords; };
   size_t pi = 0;
@@ -294,6 +291,7 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
     // thread of state words at entries prefetched one partition ahead (or
     // the words themselves, when the previous partition of this stage
     // loaded them)
+    u32 old[kOldRows * 32 / kT];
     {
       u32 w[kG];
       if (have_next) {
@@ -302,10 +300,13 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
       } else {
         load_words<WIDE>(w, src, B, in, out);
       }
+      u32 *layer = layerb(0);
       // the commit's old values (this partition's writeouts in the previous
-      // snapshot, which nothing changes during the cycle) go to LDS now and
-      // land while the partition runs
-      coherent_fetch(in + (size_t)io * 32, OLD, num_ios * 32);
+      // snapshot, which nothing changes during the cycle) load now and land
+      // while the partition runs; rows past kOldRows load at the commit
+#pragma unroll
+      for (u32 j = 0; j < kOldRows * 32 / kT; ++j)
+        if (t + kT * j < num_ios * 32) old[j] = ld_coherent(in + (size_t)io * 32 + t + kT * j);
       // the header of the successor (the next partition here, or the next
       // stage's first)
       h = load_bhdr(is_last ? nscript : script + pi);
@@ -319,11 +320,15 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
     if (next_s != 0) load_sources(src, is_last ? ngsrc : gsrc + kLayerWords);
 
     const u32 nperm = ns * 4 + nd;  // SRAM port and duplicate words
-    // ---- boomerang stages, in place on the one layer: every thread first
-    // gathers its 8 level-1 operands into registers, then (after a
-    // barrier) the layer is overwritten with this stage's after-layout
+    // ---- boomerang stages: every thread gathers its 8 level-1 operands
+    // from one layer and writes its gates to the other, so no wave waits for
+    // the others' reads: one wave's gathers (LDS) run beside another's gates
+    // (VALU).  In place, with a barrier between, 4M gates 4 x 64 took
+    // 16010 us
     for (u32 s = 0; s < S; ++s) {
       const u32 *sec = secb(s);
+      const u32 *from_layer = layerb(s);
+      u32 *layer = layerb(s + 1);
       // operand m = q4 + 4j of thread v: half q4 & 1 of its word (q4 >> 1) +
       // 2j.  The 16 v of a wave read 256 consecutive bytes per j pair
       u32 g[8];
@@ -334,7 +339,7 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
           pw[j] = sec[1024 * (j >> 1) + 4 * v + (q4 >> 1) + 2 * (j & 1)];
         const u32 sh = 16 * (q4 & 1);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) g[j] = layer[(pw[j] >> sh) & 0xffffu];
+        for (int j = 0; j < 8; ++j) g[j] = from_layer[(pw[j] >> sh) & 0xffffu];
       }
       const uint4 F = *reinterpret_cast<const uint4 *>(sec + 4096 + 4 * v);
       const u32 fw = t < 64 ? sec[4096 + 4 * t + 3] : 0u;
@@ -347,7 +352,6 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
       else
         row_fetch(secg + (size_t)kSecWords * (nperm ? S : S + 1), secb(S),
                   nperm ? nperm : num_ios);
-      __syncthreads();  // all operands read before the layer is rewritten
       // levels 1..5 of the subtree rooted at position 256 + v; gate g's
       // flags are bit g of F.x / F.y / F.z, this quarter's 4-apart gates
       // bits 0, 4, .. of the shifted words
@@ -416,11 +420,12 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
     if (have_next) load_words<WIDE>(vnext, src, B, in, out);
     __syncthreads();
 
-    // ---- SRAM + duplicate permutation into the layer (free now); a
+    // ---- SRAM + duplicate permutation into a layer (free now); a
     // partition without SRAM or duplicate words skips the phase and its
     // barriers (the condition is uniform), its clock-enable section already
     // in place
     if (nperm) {
+      u32 *layer = layerb(0);
       {
         const u32 *sec = secb(S);
         const u32 *fl = sec + 4096;
@@ -478,14 +483,19 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
       const u32 *sec = secb(nperm ? S + 1 : S);
       const u32 *fl = sec + 4096;
       u32 *o = out + (size_t)io * 32;
-      for (u32 q = t; q < num_ios * 32; q += kT) {
-        uint4 f = *reinterpret_cast<const uint4 *>(fl + 4 * (q >> 5));
+      auto commit = [&](u32 q, u32 was) {
+        const uint4 f = *reinterpret_cast<const uint4 *>(fl + 4 * (q >> 5));
         // a bit whose enable is forced (set0) needs no gather: ck = inv
         u32 ck = fbit(f.x, q);
         if (!((f.y >> (q & 31)) & 1u)) ck ^= WO[sw(perm_at(sec, q))];
-        u32 d = WO[sw(q)] ^ fbit(f.z, q);
-        st_coherent(o + q, (OLD[q] & ~ck) | (d & ck));
-      }
+        const u32 d = WO[sw(q)] ^ fbit(f.z, q);
+        st_coherent(o + q, (was & ~ck) | (d & ck));
+      };
+#pragma unroll
+      for (u32 j = 0; j < kOldRows * 32 / kT; ++j)
+        if (t + kT * j < num_ios * 32) commit(t + kT * j, old[j]);
+      for (u32 q = t + kOldRows * 32; q < num_ios * 32; q += kT)
+        commit(q, ld_coherent(in + (size_t)io * 32 + q));
     }
     __syncthreads();
     if (prof) {
