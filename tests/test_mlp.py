@@ -146,3 +146,41 @@ def test_learned_merge_and_assignment_beat_the_heuristic():
         oracle.run(s0, st, int(cyc[lane]))
         want = B.plain_observations(s0, st, int(cyc[lane]), run.obs_lits)
         assert np.array_equal(out[lane], want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dims", [(1, 1, 1), (32, 64, 64), (17, 33, 5), (24, 16, 49), (16, 48, 64)])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 300])
+def test_gpu_dimensions_off_the_matrix_tiles(dims, n):
+    """Layer widths and batch sizes below, at and past the 16-wide tiles and
+    the 64-sample workgroups: padding adds nothing.  A unit's sum has at most
+    64 products, so FP32 rounding stays below 64 * 2**-24 < 4e-6 of the sum
+    of their magnitudes; the bounds leave room for the layers behind it and
+    for sums that nearly cancel."""
+    import torch
+    from jacquard_amd import _native as N
+    from jacquard_amd.costmodel import MLP
+    i, h1, h2 = dims
+    rng = np.random.default_rng(100 * n + i)
+    x = rng.normal(size=(n, i)).astype(np.float32)
+    t = rng.normal(size=n).astype(np.float32)
+    p = mo.init(i, h1, h2, seed=9).astype(np.float32)
+    p += (0.05 * rng.normal(size=p.size)).astype(np.float32)
+    m = MLP(params=p.copy(), i=i, h1=h1, h2=h2)
+    xd, td = torch.from_numpy(x).cuda(), torch.from_numpy(t).cuda()
+    y = torch.full((n + 8,), 7.0, dtype=torch.float32, device="cuda")
+    m.forward_raw(xd, n, y)
+    p64, x64, t64 = (a.astype(np.float64) for a in (p, x, t))
+    y_ref, _ = mo.forward(p64, x64, i, h1, h2)
+    assert np.allclose(y[:n].cpu().numpy(), y_ref, rtol=1e-4, atol=1e-5)
+    assert (y[n:] == 7.0).all(), "outputs past the batch"
+    ws = torch.zeros(int(N.hip().jq_mlp_workspace_floats(i, h1, h2, n)),
+                     dtype=torch.float32, device="cuda")
+    loss = torch.zeros(1, dtype=torch.float32, device="cuda")
+    m.train_step_raw(xd, td, n, 0.25, ws, loss)
+    g_ref = mo.grad(p64, x64, t64, i, h1, h2)
+    scale = np.abs(g_ref).max()
+    assert np.allclose(m.grads.cpu().numpy(), g_ref, rtol=1e-3, atol=1e-5 * scale)
+    assert np.allclose(m.params.cpu().numpy(), p64 - 0.25 * g_ref, rtol=1e-4,
+                       atol=1e-5 * max(scale, 1))
+    assert np.isclose(loss.item(), mo.loss(p64, x64, t64, i, h1, h2), rtol=1e-4)
