@@ -59,164 +59,171 @@ using f4 = __attribute__((ext_vector_type(4))) float;
 // rows spread over the banks.
 constexpr int kLdIn = kMaxIn + 4, kLdH = kMaxH + 4;
 
-__host__ __device__ inline int tiles(int n) { return (n + 15) / 16; }
-
-// acc[t] += A[16 rows][16 * kt] * B[16 t .. 16 t + 15][16 * kt]^T for the
-// first nt column tiles: both operands have the summed index contiguous.
+// acc[t] += A[16 rows][16 * KT] * B[16 t .. 16 t + 15][16 * KT]^T for NT
+// column tiles: both operands have the summed index contiguous, at slot(k).
 // Lane l holds row l % 16 of A and of each B tile; its group g = l / 16 reads
-// elements 16 s + 4 g .. + 3 with one 16-byte read, and the j-th matrix
-// instruction of a step sums the j-th elements of the four groups.  The
-// result has rows 4 g .. 4 g + 3 of column l % 16 in lane l.
-__device__ __forceinline__ void mul_tiles(f4 (&acc)[4], const float *a, int lda, const float *b,
-                                          int ldb, int nt, int kt) {
+// slots 16 s + 4 g .. + 3 with one 16-byte read, and the j-th matrix
+// instruction of a step sums the j-th of them over the four groups: k = 16 s
+// + 4 j + g.  The matrix instruction adds its four products one after the
+// other, each with one rounding, so every sum is the fmaf chain over
+// k = 0, 1, .. that starts from acc, bit for bit: which units a ReLU cuts
+// off, and every gradient, are what a loop over k gives.  The
+// result has rows 4 g .. 4 g + 3 of column l % 16 in lane l.  The tile
+// counts are those of the largest dimensions: with loops over the batch's own
+// counts every step waited for its reads (a step of 4096 samples 27.3 us
+// against 15.9).
+__host__ __device__ constexpr int slot(int k) {
+  return (k & ~15) | ((k & 3) << 2) | ((k >> 2) & 3);
+}
+template <int NT, int KT>
+__device__ __forceinline__ void mul_tiles(f4 (&acc)[NT], const float *a, int lda, const float *b,
+                                          int ldb) {
   const int l = threadIdx.x & 63, r = l & 15, g = l >> 4;
-  for (int s = 0; s < kt; ++s) {
+#pragma unroll
+  for (int s = 0; s < KT; ++s) {
     const f4 av = *reinterpret_cast<const f4 *>(a + r * lda + 16 * s + 4 * g);
+    f4 bv[NT];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      if (t < nt) {
-        const f4 bv = *reinterpret_cast<const f4 *>(b + (16 * t + r) * ldb + 16 * s + 4 * g);
+    for (int t = 0; t < NT; ++t)
+      bv[t] = *reinterpret_cast<const f4 *>(b + (16 * t + r) * ldb + 16 * s + 4 * g);
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[j], bv[j], acc[t], 0, 0, 0);
-      }
-    }
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[j], bv[t][j], acc[t], 0, 0, 0);
+  }
+}
+
+// The same for one tile of B whose rows past the first `rows` are zero and
+// not stored (a vector, or a few of them).
+template <int KT>
+__device__ __forceinline__ void mul_rows(f4 &acc, const float *a, int lda, const float *b, int ldb,
+                                         int rows) {
+  const int l = threadIdx.x & 63, r = l & 15, g = l >> 4;
+#pragma unroll
+  for (int s = 0; s < KT; ++s) {
+    const f4 av = *reinterpret_cast<const f4 *>(a + r * lda + 16 * s + 4 * g);
+    f4 bv = {};
+    if (r < rows) bv = *reinterpret_cast<const f4 *>(b + r * ldb + 16 * s + 4 * g);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av[j], bv[j], acc, 0, 0, 0);
   }
 }
 
 __device__ __forceinline__ float relu(float a) { return a > 0.f ? a : 0.f; }
 
-// Sum over the 16 lanes of a row of the wave, on every one of them; over
-// the wave's four rows, lane by lane.
-__device__ __forceinline__ float sum16(float v) {
+// The weights and the workgroup's 64 samples into LDS, rows of
+// kLdIn and kLdH floats, zeros around them.  A wave reads a row of weights,
+// its lanes the columns, and its own 16 samples; every load is issued before
+// the first store.  TRANSPOSED: W2 and the samples transposed as well.
+template <bool TRANSPOSED>
+__device__ __forceinline__ void load_tiles(float *W1, float *W2, float *X, const Dims &d,
+                                           const float *p, const float *x, int s0, int n,
+                                           float *W3, float *W2T, float *XT) {
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63, c = l & 31;
+  float a[16], b[16], v[8];
+  const float w3 = l < d.h2 ? p[d.oW3() + l] : 0.f;
 #pragma unroll
-  for (int m = 1; m < 16; m <<= 1) v += __shfl_xor(v, m);
-  return v;
-}
-__device__ __forceinline__ float sum_groups(float v) {
-  v += __shfl_xor(v, 16);
-  return v + __shfl_xor(v, 32);
-}
-
-// Rows 0 .. rows - 1 of the packed matrix m[rows][cols] into dst[64][ld],
-// zeros around it up to 64 x width; a wave reads a row, its lanes the columns.
-template <int WIDTH>
-__device__ __forceinline__ void load_matrix(float *dst, int ld, const float *m, int rows,
-                                            int cols) {
-  const int w = threadIdx.x >> 6, c = threadIdx.x & 63;
-#pragma unroll 8
   for (int k = 0; k < 16; ++k) {
     const int r = 4 * k + w;
-    if (c < WIDTH) dst[r * ld + c] = (r < rows && c < cols) ? m[r * cols + c] : 0.f;
+    a[k] = (r < d.h1 && l < d.in) ? p[d.oW1() + r * d.in + l] : 0.f;
+    b[k] = (r < d.h2 && l < d.h1) ? p[d.oW2() + r * d.h1 + l] : 0.f;
   }
-}
-
-// The workgroup's 64 samples into X[64][kLdIn], zeros around them; every
-// wave loads its own 16.
-__device__ __forceinline__ void load_samples(float *X, const float *x, int s0, int n, int in) {
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63, c = l & 31;
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
     const int r = 16 * w + 2 * k + (l >> 5);
-    X[r * kLdIn + c] = (s0 + r < n && c < in) ? x[(size_t)(s0 + r) * in + c] : 0.f;
+    v[k] = (s0 + r < n && c < d.in) ? x[(size_t)(s0 + r) * d.in + c] : 0.f;
+  }
+  if (w == 0) W3[slot(l)] = w3;
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    const int r = 4 * k + w;
+    if (l < kMaxIn) W1[r * kLdIn + slot(l)] = a[k];
+    W2[r * kLdH + slot(l)] = b[k];
+    if (TRANSPOSED) W2T[l * kLdH + slot(r)] = b[k];
+  }
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const int r = 16 * w + 2 * k + (l >> 5);
+    X[r * kLdIn + slot(c)] = v[k];
+    if (TRANSPOSED) XT[c * kLdH + slot(r)] = v[k];
   }
 }
 
-// First layer of the wave's 16 samples: activations in acc (lane l: samples
-// 4 g .. 4 g + 3 of unit 16 t + l % 16) and in H1[64][kLdH].
-__device__ __forceinline__ void layer1(f4 (&acc)[4], const Dims &d, const float *p,
-                                       const float *X, const float *W1, float *H1) {
+// Rows of the wave's 16 samples <- a tile result per 16 columns.
+__device__ __forceinline__ void store_rows(float *rows, const f4 (&v)[4]) {
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, c = l & 15, g = l >> 4;
-#pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const int k = 16 * t + c;
-    const float b = k < d.h1 ? p[d.ob1() + k] : 0.f;
-    acc[t] = f4{b, b, b, b};
-  }
-  mul_tiles(acc, X + 16 * w * kLdIn, kLdIn, W1, kLdIn, tiles(d.h1), tiles(d.in));
 #pragma unroll
   for (int t = 0; t < 4; ++t)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      acc[t][r] = relu(acc[t][r]);
-      H1[(16 * w + 4 * g + r) * kLdH + 16 * t + c] = acc[t][r];
-    }
-  __builtin_amdgcn_wave_barrier();  // the wave reads only its own rows
+    for (int r = 0; r < 4; ++r)
+      rows[(16 * w + 4 * g + r) * kLdH + 16 * t + slot(c)] = v[t][r];
+  __builtin_amdgcn_wave_barrier();  // a wave reads only its own rows
 }
 
-// Second layer of the wave's 16 samples, laid out as layer1's.
-__device__ __forceinline__ void layer2(f4 (&acc)[4], const Dims &d, const float *p,
-                                       const float *H1, const float *W2) {
-  const int w = threadIdx.x >> 6, c = threadIdx.x & 15;
+// The same transposed: 4 consecutive samples of a unit are strided by 4 slots.
+__device__ __forceinline__ void store_columns(float *cols, const f4 (&v)[4]) {
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63, c = l & 15, g = l >> 4;
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      cols[(16 * t + c) * kLdH + 16 * w + slot(4 * g + r)] = v[t][r];
+}
+
+// Activations of a hidden layer for the wave's 16 samples from their inputs
+// a: lane l holds samples 4 g .. 4 g + 3 of unit 16 t + l % 16.
+template <int KT>
+__device__ __forceinline__ void layer(f4 (&acc)[4], const float *bias, int units, const float *a,
+                                      int lda, const float *W, int ldw) {
+  const int c = threadIdx.x & 15;
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
-    const int j = 16 * t + c;
-    const float b = j < d.h2 ? p[d.ob2() + j] : 0.f;
+    const float b = 16 * t + c < units ? bias[16 * t + c] : 0.f;
     acc[t] = f4{b, b, b, b};
   }
-  mul_tiles(acc, H1 + 16 * w * kLdH, kLdH, W2, kLdH, tiles(d.h2), tiles(d.h1));
+  mul_tiles<4, KT>(acc, a, lda, W, ldw);
 #pragma unroll
   for (int t = 0; t < 4; ++t)
 #pragma unroll
     for (int r = 0; r < 4; ++r) acc[t][r] = relu(acc[t][r]);
 }
 
-// Output of samples 4 g .. 4 g + 3, on every lane of group g.
-__device__ __forceinline__ f4 layer3(const Dims &d, const float *p, const f4 (&h2)[4],
-                                     const float (&w3)[4]) {
-  const float b3 = p[d.ob3()];
-  f4 y;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    float a = 0.f;
-#pragma unroll
-    for (int t = 0; t < 4; ++t) a = fmaf(w3[t], h2[t][r], a);
-    y[r] = b3 + sum16(a);
-  }
-  return y;
-}
-
-__device__ __forceinline__ void load_w3(float (&w3)[4], const Dims &d, const float *p) {
-#pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const int j = 16 * t + (threadIdx.x & 15);
-    w3[t] = j < d.h2 ? p[d.oW3() + j] : 0.f;
-  }
-}
-
 __global__ __launch_bounds__(256) void mlp_forward_kernel(Dims d, const float *p,
                                                           const float *x, int n,
                                                           float *y) {
-  __shared__ __align__(16) float W1[kMaxH * kLdIn], W2[kMaxH * kLdH], X[kSamples * kLdIn],
-      H1[kSamples * kLdH];
+  __shared__ __align__(16) float W1[kMaxH * kLdIn], W2[kMaxH * kLdH], W3[kMaxH],
+      X[kSamples * kLdIn], H[kSamples * kLdH];
   const int s0 = blockIdx.x * kSamples;
-  load_samples(X, x, s0, n, d.in);
-  load_matrix<kMaxIn>(W1, kLdIn, p + d.oW1(), d.h1, d.in);
-  load_matrix<kMaxH>(W2, kLdH, p + d.oW2(), d.h2, d.h1);
-  float w3[4];
-  load_w3(w3, d, p);
+  load_tiles<false>(W1, W2, X, d, p, x, s0, n, W3, nullptr, nullptr);
   __syncthreads();
-  f4 h[4];
-  layer1(h, d, p, X, W1, H1);
-  layer2(h, d, p, H1, W2);
-  const f4 out = layer3(d, p, h, w3);
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, g = l >> 4;
+  f4 h[4];
+  layer<kMaxIn / 16>(h, p + d.ob1(), d.h1, X + 16 * w * kLdIn, kLdIn, W1, kLdIn);
+  store_rows(H, h);
+  layer<kMaxH / 16>(h, p + d.ob2(), d.h2, H + 16 * w * kLdH, kLdH, W2, kLdH);
+  store_rows(H, h);
+  const float b3 = p[d.ob3()];
+  f4 out = {b3, b3, b3, b3};
+  mul_rows<kMaxH / 16>(out, H + 16 * w * kLdH, kLdH, W3, 0, 1);
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int s = s0 + 16 * w + 4 * g + r;
-    if ((l & 15) == r && s < n) y[s] = out[r];
+    if ((l & 15) == 0 && s < n) y[s] = out[r];
   }
 }
 
 // LDS of the gradient kernel, in floats
 constexpr int kW1 = 0, kW2 = kW1 + kMaxH * kLdIn, kW2T = kW2 + kMaxH * kLdH;
 constexpr int kX = kW2T + kMaxH * kLdH, kXT = kX + kSamples * kLdIn;
-constexpr int kHD = kXT + kMaxIn * kLdH;    // H1, then dL/d(pre-activation 2)
-constexpr int kH1T = kHD + kSamples * kLdH, kD2T = kH1T + kMaxH * kLdH;
-constexpr int kD1T = kD2T + kMaxH * kLdH;
-constexpr int kSums = kD1T + kMaxH * kLdH;  // per wave: b1, b2, W3 (64 each), b3, loss
-constexpr int kSumW = 3 * kMaxH + 2;
-constexpr int kGradLds = kSums + 4 * kSumW;
+constexpr int kRows = kXT + kMaxIn * kLdH;  // H1, H2, dL/d(pre-activation 2) in turn
+constexpr int kH1T = kRows + kSamples * kLdH, kH2T = kH1T + kMaxH * kLdH;
+constexpr int kD2T = kH2T + kMaxH * kLdH, kD1T = kD2T + kMaxH * kLdH;
+constexpr int kW3 = kD1T + kMaxH * kLdH;
+// ones, dL/dy and squared error of every sample
+constexpr int kVec = kW3 + kMaxH, kGradLds = kVec + 3 * kLdH;
+static_assert(kGradLds * 4 <= 160 * 1024, "LDS of a CU");
 
 // one workgroup = kSamples samples: forward/backward of every sample, then
 // the workgroup's gradient sums into ws[blockIdx.x][param]
@@ -225,166 +232,125 @@ __global__ __launch_bounds__(256) void mlp_grad_kernel(Dims d, const float *p,
                                                        const float *target, int n,
                                                        float *ws, float *wloss) {
   extern __shared__ __align__(16) float lds[];
-  float *X = lds + kX, *XT = lds + kXT, *HD = lds + kHD, *H1T = lds + kH1T;
-  float *D1T = lds + kD1T, *D2T = lds + kD2T;
+  float *rows = lds + kRows, *vec = lds + kVec;
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, c = l & 15, g = l >> 4;
   const int s0 = blockIdx.x * kSamples;
-  load_samples(X, x, s0, n, d.in);
-  load_matrix<kMaxIn>(lds + kW1, kLdIn, p + d.oW1(), d.h1, d.in);
-  load_matrix<kMaxH>(lds + kW2, kLdH, p + d.oW2(), d.h2, d.h1);
-  float w3[4];
-  load_w3(w3, d, p);
+  const float *mine = rows + 16 * w * kLdH;  // the wave's own rows
+  load_tiles<true>(lds + kW1, lds + kW2, lds + kX, d, p, x, s0, n, lds + kW3, lds + kW2T,
+                   lds + kXT);
   f4 tg;
+  float w3[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int s = s0 + 16 * w + 4 * g + r;
     tg[r] = s < n ? target[s] : 0.f;
+    w3[r] = 16 * r + c < d.h2 ? p[d.oW3() + 16 * r + c] : 0.f;
   }
+  const float b3 = p[d.ob3()];
   __syncthreads();
-  // transposes for the products that sum over units or samples
-  {
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const int r = 16 * w + k;
-      lds[kW2T + l * kLdH + r] = lds[kW2 + r * kLdH + l];
-      if (l < kMaxIn) XT[l * kLdH + r] = X[r * kLdIn + l];
-    }
-  }
   f4 h1[4], h2[4];
-  layer1(h1, d, p, X, lds + kW1, HD);
-#pragma unroll
-  for (int t = 0; t < 4; ++t)
-    *reinterpret_cast<f4 *>(H1T + (16 * t + c) * kLdH + 16 * w + 4 * g) = h1[t];
-  layer2(h2, d, p, HD, lds + kW2);
-  const f4 y = layer3(d, p, h2, w3);
-  f4 dy;
-  float e2 = 0.f, gb3 = 0.f;
+  layer<kMaxIn / 16>(h1, p + d.ob1(), d.h1, lds + kX + 16 * w * kLdIn, kLdIn, lds + kW1, kLdIn);
+  store_rows(rows, h1);
+  store_columns(lds + kH1T, h1);
+  layer<kMaxH / 16>(h2, p + d.ob2(), d.h2, mine, kLdH, lds + kW2, kLdH);
+  store_rows(rows, h2);
+  store_columns(lds + kH2T, h2);
+  f4 y = {b3, b3, b3, b3}, dy;
+  mul_rows<kMaxH / 16>(y, mine, kLdH, lds + kW3, 0, 1);
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
+    const int k = 16 * w + slot(4 * g + r);
     const bool in = s0 + 16 * w + 4 * g + r < n;
-    const float e = y[r] - tg[r];
+    const float e = __shfl(y[r], l & 48) - tg[r];
     dy[r] = in ? 2.f * e / (float)n : 0.f;
-    e2 += in ? e * e : 0.f;
-    gb3 += dy[r];
-  }
-  float *sums = lds + kSums + w * kSumW;
-  // dL/d(pre-activation 2), and the sums over samples that it gives
-#pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    f4 d2;
-    float gw3 = 0.f, gb2 = 0.f;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      d2[r] = h2[t][r] > 0.f ? dy[r] * w3[t] : 0.f;
-      gw3 = fmaf(dy[r], h2[t][r], gw3);
-      gb2 += d2[r];
-      HD[(16 * w + 4 * g + r) * kLdH + 16 * t + c] = d2[r];
-    }
-    *reinterpret_cast<f4 *>(D2T + (16 * t + c) * kLdH + 16 * w + 4 * g) = d2;
-    gw3 = sum_groups(gw3);
-    gb2 = sum_groups(gb2);
-    if (g == 0) {
-      sums[kMaxH + 16 * t + c] = gb2;
-      sums[2 * kMaxH + 16 * t + c] = gw3;
+    if (c == 0) {
+      vec[k] = 1.f;
+      vec[kLdH + k] = dy[r];
+      vec[2 * kLdH + k] = in ? e * e : 0.f;
     }
   }
-  e2 = sum_groups(e2);
-  gb3 = sum_groups(gb3);
-  if (l == 0) {
-    sums[3 * kMaxH] = gb3;
-    sums[3 * kMaxH + 1] = e2;
-  }
-  __syncthreads();  // W2T; the wave's own rows of HD need none
-  {
-    f4 d1[4] = {};
-    mul_tiles(d1, HD + 16 * w * kLdH, kLdH, lds + kW2T, kLdH, tiles(d.h1), tiles(d.h2));
+  f4 d2[4];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      float gb1 = 0.f;
+  for (int t = 0; t < 4; ++t)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        d1[t][r] = h1[t][r] > 0.f ? d1[t][r] : 0.f;
-        gb1 += d1[t][r];
-      }
-      *reinterpret_cast<f4 *>(D1T + (16 * t + c) * kLdH + 16 * w + 4 * g) = d1[t];
-      gb1 = sum_groups(gb1);
-      if (g == 0) sums[16 * t + c] = gb1;
-    }
-  }
+    for (int r = 0; r < 4; ++r) d2[t][r] = h2[t][r] > 0.f ? dy[r] * w3[t] : 0.f;
+  store_rows(rows, d2);
+  store_columns(lds + kD2T, d2);
+  f4 d1[4] = {};
+  mul_tiles<4, kMaxH / 16>(d1, mine, kLdH, lds + kW2T, kLdH);
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) d1[t][r] = h1[t][r] > 0.f ? d1[t][r] : 0.f;
+  store_columns(lds + kD1T, d1);
   __syncthreads();
+  // a wave sums units 16 w .. 16 w + 15 of every weight gradient over the
+  // samples
   float *row = ws + (size_t)blockIdx.x * d.np;
-  // rows 16 w .. 16 w + 15 of both weight gradients, summed over the samples
-  {
-    f4 a[4] = {};
-    mul_tiles(a, D2T + 16 * w * kLdH, kLdH, H1T, kLdH, tiles(d.h1), kSamples / 16);
+  const int u0 = 16 * w + 4 * g;
+  // the bias gradients are sums against ones (column 0), W3's against dL/dy
+  // (column 1); every product is under way before the first store
+  f4 gw2[4] = {}, gw1[kMaxIn / 16] = {}, b1 = {}, b2 = {}, g3 = {};
+  mul_tiles<4, kSamples / 16>(gw2, lds + kD2T + 16 * w * kLdH, kLdH, lds + kH1T, kLdH);
+  mul_tiles<kMaxIn / 16, kSamples / 16>(gw1, lds + kD1T + 16 * w * kLdH, kLdH, lds + kXT, kLdH);
+  mul_rows<kSamples / 16>(b1, lds + kD1T + 16 * w * kLdH, kLdH, vec, kLdH, 1);
+  mul_rows<kSamples / 16>(b2, lds + kD2T + 16 * w * kLdH, kLdH, vec, kLdH, 1);
+  mul_rows<kSamples / 16>(g3, lds + kH2T + 16 * w * kLdH, kLdH, vec, kLdH, 2);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int u = u0 + r;
 #pragma unroll
     for (int t = 0; t < 4; ++t)
+      if (u < d.h2 && 16 * t + c < d.h1) row[d.oW2() + u * d.h1 + 16 * t + c] = gw2[t][r];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int j = 16 * w + 4 * g + r, k = 16 * t + c;
-        if (j < d.h2 && k < d.h1) row[d.oW2() + j * d.h1 + k] = a[t][r];
-      }
+    for (int t = 0; t < kMaxIn / 16; ++t)
+      if (u < d.h1 && 16 * t + c < d.in) row[d.oW1() + u * d.in + 16 * t + c] = gw1[t][r];
+    if (c == 0 && u < d.h1) row[d.ob1() + u] = b1[r];
+    if (c == 0 && u < d.h2) row[d.ob2() + u] = b2[r];
+    if (c == 1 && u < d.h2) row[d.oW3() + u] = g3[r];
   }
-  {
-    f4 a[4] = {};
-    mul_tiles(a, D1T + 16 * w * kLdH, kLdH, XT, kLdH, tiles(d.in), kSamples / 16);
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int k = 16 * w + 4 * g + r, i = 16 * t + c;
-        if (k < d.h1 && i < d.in) row[d.oW1() + k * d.in + i] = a[t][r];
-      }
-  }
-  const int t = threadIdx.x;
-  if (t < kSumW) {
-    float v = 0.f;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) v += lds[kSums + q * kSumW + t];
-    const int u = t & (kMaxH - 1);
-    if (t == kSumW - 1)
-      wloss[blockIdx.x] = v;
-    else if (t == kSumW - 2)
-      row[d.ob3()] = v;
-    else if (t < kMaxH && u < d.h1)
-      row[d.ob1() + u] = v;
-    else if (t >= 2 * kMaxH && u < d.h2)
-      row[d.oW3() + u] = v;
-    else if (t >= kMaxH && t < 2 * kMaxH && u < d.h2)
-      row[d.ob2() + u] = v;
+  // b3's gradient and the loss are the sums of vec's own rows 1 and 2
+  if (w == 0) {
+    f4 v = {};
+    // rows 3 .. 15 of the left operand are not used: row 2 again
+    const float *own = vec + (c < 3 ? 0 : 2 - c) * kLdH;
+    mul_rows<kSamples / 16>(v, own, kLdH, vec, kLdH, 1);
+    if (l == 0) {
+      row[d.ob3()] = v[1];
+      wloss[blockIdx.x] = v[2];
+    }
   }
 }
 
-// Sums the workspace rows, 64 parameters a workgroup: wave q takes rows q,
-// q + 4, .. and the four sums are added in order; then the SGD update.
-// Workgroup 0's wave 0 sums the losses.  One thread a parameter walked the
-// 64 rows of a 4096-sample step one load after another.
-__global__ __launch_bounds__(256) void mlp_update_kernel(Dims d, float *p, float *grads,
-                                                         const float *ws,
-                                                         const float *wloss, int nblk,
-                                                         int n, float lr,
-                                                         float *loss_out) {
-  __shared__ float part[4][64];
-  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int q = blockIdx.x * 64 + l;
-  float g = 0.f;
+// Sums the workspace rows in order, a thread a parameter with 32 rows'
+// loads in flight, and applies the SGD update; the last workgroup sums the
+// losses.
+__global__ __launch_bounds__(64) void mlp_update_kernel(Dims d, float *p, float *grads,
+                                                        const float *ws,
+                                                        const float *wloss, int nblk,
+                                                        int n, float lr,
+                                                        float *loss_out) {
+  constexpr int kFlight = 32;
+  const int q = blockIdx.x * 64 + threadIdx.x;
   if (q < d.np) {
-#pragma unroll 8
-    for (int b = w; b < nblk; b += 4) g += ws[(size_t)b * d.np + q];
-  }
-  part[w][l] = g;
-  __syncthreads();
-  if (w == 0 && q < d.np) {
-    g = ((part[0][l] + part[1][l]) + part[2][l]) + part[3][l];
-    grads[q] = g;
-    p[q] -= lr * g;
-  }
-  if (blockIdx.x == 0 && w == 0 && loss_out) {
-    float s = 0.f;
-    for (int b = l; b < nblk; b += 64) s += wloss[b];
+    const float old = p[q];
+    float g = 0.f;
+    for (int b0 = 0; b0 < nblk; b0 += kFlight) {
+      float v[kFlight];
 #pragma unroll
-    for (int m = 1; m < 64; m <<= 1) s += __shfl_xor(s, m);
-    if (l == 0) *loss_out = s / (float)n;
+      for (int k = 0; k < kFlight; ++k)
+        v[k] = b0 + k < nblk ? ws[(size_t)(b0 + k) * d.np + q] : 0.f;
+#pragma unroll
+      for (int k = 0; k < kFlight; ++k)
+        if (b0 + k < nblk) g += v[k];
+    }
+    grads[q] = g;
+    p[q] = fmaf(-lr, g, old);
+  }
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0 && loss_out) {
+    float s = 0.f;
+    for (int b = 0; b < nblk; ++b) s += wloss[b];
+    *loss_out = s / (float)n;
   }
 }
 
@@ -441,7 +407,7 @@ extern "C" int jq_mlp_train_step(float *params, float *grads, float *workspace,
   float *ws = workspace, *wloss = workspace + (size_t)nblk * d.np;
   hipLaunchKernelGGL(mlp_grad_kernel, dim3(nblk), dim3(256), lds, (hipStream_t)stream,
                      d, params, x, target, n, ws, wloss);
-  hipLaunchKernelGGL(mlp_update_kernel, dim3((d.np + 63) / 64), dim3(256), 0,
+  hipLaunchKernelGGL(mlp_update_kernel, dim3((d.np + 63) / 64 + 1), dim3(64), 0,
                      (hipStream_t)stream, d, params, grads, ws, wloss, nblk, n, lr,
                      loss_out);
   hipError_t e = hipGetLastError();
