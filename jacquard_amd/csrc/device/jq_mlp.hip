@@ -7,14 +7,16 @@
 // fixed order and applies the update.
 //
 // Every matrix product runs on the matrix cores in FP32
-// (v_mfma_f32_16x16x4_f32: FP32 inputs, FP32 accumulation).  A wave owns 16
-// samples from their inputs to their pre-activation gradients, so the forward
-// and backward chain needs no workgroup barrier; then a wave owns 16 rows of
-// each weight gradient.  Dimensions are padded with zeros to multiples of 16
-// in LDS.  A thread per sample (its activations in scratch, weights read one
-// by one) kept one wave of a workgroup busy: a step of 4096 samples took
-// 340 us and takes 27, a forward of 5013 samples 140 and 11.  Error against
-// 64 bits over the step's gradients: 1.3e-7 before, 4.5e-8 now.
+// (v_mfma_f32_16x16x4_f32: FP32 inputs, FP32 accumulation).  A pair of waves
+// owns 16 samples from their inputs to their pre-activation gradients, each
+// wave half of a layer's units; then the pair owns 16 rows of each weight
+// gradient.  Dimensions are padded with zeros to multiples of 16 in LDS.
+// What bounds it is the chain load - layer - layer - ... of one workgroup
+// per 64 samples, whose products are a dependent chain per tile.  A thread
+// per sample (its activations in scratch, weights read one by one) kept one
+// wave of a workgroup busy: a step of 4096 samples took 340 us and takes
+// 20.4 (gradients 16, update 5), a forward of 5013 samples 140 and 6.8, with
+// the same result bit for bit.  One wave to 16 samples: 23.3 and 6.9.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -67,11 +69,10 @@ constexpr int kLdIn = kMaxIn + 4, kLdH = kMaxH + 4;
 // + 4 j + g.  The matrix instruction adds its four products one after the
 // other, each with one rounding, so every sum is the fmaf chain over
 // k = 0, 1, .. that starts from acc, bit for bit: which units a ReLU cuts
-// off, and every gradient, are what a loop over k gives.  The
-// result has rows 4 g .. 4 g + 3 of column l % 16 in lane l.  The tile
-// counts are those of the largest dimensions: with loops over the batch's own
-// counts every step waited for its reads (a step of 4096 samples 27.3 us
-// against 15.9).
+// off, and every gradient, are what a loop over k gives.  The result has rows
+// 4 g .. 4 g + 3 of column l % 16 in lane l.  The tile counts are those of
+// the largest dimensions: with loops over the batch's own counts every step
+// waited for its reads (a step of 4096 samples took 12 us more).
 __host__ __device__ constexpr int slot(int k) {
   return (k & ~15) | ((k & 3) << 2) | ((k >> 2) & 3);
 }
@@ -113,104 +114,118 @@ __device__ __forceinline__ void mul_rows(f4 &acc, const float *a, int lda, const
 
 __device__ __forceinline__ float relu(float a) { return a > 0.f ? a : 0.f; }
 
+// A workgroup has 8 waves, two to 16 samples: half 0 of a pair computes units
+// 0 .. 31 of a layer, half 1 the others.
+constexpr int kMlpT = 512;
+
 // The weights and the workgroup's 64 samples into LDS, rows of
 // kLdIn and kLdH floats, zeros around them.  A wave reads a row of weights,
-// its lanes the columns, and its own 16 samples; every load is issued before
-// the first store.  TRANSPOSED: W2 and the samples transposed as well.
+// its lanes the columns; every load is issued before the first store.
+// TRANSPOSED: W2 and the samples transposed as well.
 template <bool TRANSPOSED>
 __device__ __forceinline__ void load_tiles(float *W1, float *W2, float *X, const Dims &d,
                                            const float *p, const float *x, int s0, int n,
                                            float *W3, float *W2T, float *XT) {
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, c = l & 31;
-  float a[16], b[16], v[8];
+  float a[8], b[8], v[4];
   const float w3 = l < d.h2 ? p[d.oW3() + l] : 0.f;
 #pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    const int r = 4 * k + w;
+  for (int k = 0; k < 8; ++k) {
+    const int r = 8 * k + w;
     a[k] = (r < d.h1 && l < d.in) ? p[d.oW1() + r * d.in + l] : 0.f;
     b[k] = (r < d.h2 && l < d.h1) ? p[d.oW2() + r * d.h1 + l] : 0.f;
   }
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const int r = 16 * w + 2 * k + (l >> 5);
+  for (int k = 0; k < 4; ++k) {
+    const int r = 8 * w + 2 * k + (l >> 5);
     v[k] = (s0 + r < n && c < d.in) ? x[(size_t)(s0 + r) * d.in + c] : 0.f;
   }
   if (w == 0) W3[slot(l)] = w3;
 #pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    const int r = 4 * k + w;
+  for (int k = 0; k < 8; ++k) {
+    const int r = 8 * k + w;
     if (l < kMaxIn) W1[r * kLdIn + slot(l)] = a[k];
     W2[r * kLdH + slot(l)] = b[k];
     if (TRANSPOSED) W2T[l * kLdH + slot(r)] = b[k];
   }
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const int r = 16 * w + 2 * k + (l >> 5);
+  for (int k = 0; k < 4; ++k) {
+    const int r = 8 * w + 2 * k + (l >> 5);
     X[r * kLdIn + slot(c)] = v[k];
     if (TRANSPOSED) XT[c * kLdH + slot(r)] = v[k];
   }
 }
 
-// Rows of the wave's 16 samples <- a tile result per 16 columns.
-__device__ __forceinline__ void store_rows(float *rows, const f4 (&v)[4]) {
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63, c = l & 15, g = l >> 4;
-#pragma unroll
-  for (int t = 0; t < 4; ++t)
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      rows[(16 * w + 4 * g + r) * kLdH + 16 * t + slot(c)] = v[t][r];
-  __builtin_amdgcn_wave_barrier();  // a wave reads only its own rows
+// Place of a wave: its 16 samples, its 32 units; of a lane: column c of its
+// tiles, group g.
+struct Place {
+  int w, u, c, g;
+};
+__device__ __forceinline__ Place place() {
+  const int l = threadIdx.x & 63;
+  return Place{(int)(threadIdx.x >> 6) & 3, 32 * (int)(threadIdx.x >> 8), l & 15, l >> 4};
 }
 
-// The same transposed: 4 consecutive samples of a unit are strided by 4 slots.
-__device__ __forceinline__ void store_columns(float *cols, const f4 (&v)[4]) {
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63, c = l & 15, g = l >> 4;
+// The wave's tiles into rows of samples, and into columns of units: 4
+// consecutive samples of a unit are strided by 4 slots.
+__device__ __forceinline__ void store_rows(float *rows, const Place &q, const f4 (&v)[2]) {
 #pragma unroll
-  for (int t = 0; t < 4; ++t)
+  for (int t = 0; t < 2; ++t)
 #pragma unroll
     for (int r = 0; r < 4; ++r)
-      cols[(16 * t + c) * kLdH + 16 * w + slot(4 * g + r)] = v[t][r];
+      rows[(16 * q.w + 4 * q.g + r) * kLdH + q.u + 16 * t + slot(q.c)] = v[t][r];
+}
+__device__ __forceinline__ void store_columns(float *cols, const Place &q, const f4 (&v)[2]) {
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      cols[(q.u + 16 * t + q.c) * kLdH + 16 * q.w + slot(4 * q.g + r)] = v[t][r];
 }
 
-// Activations of a hidden layer for the wave's 16 samples from their inputs
-// a: lane l holds samples 4 g .. 4 g + 3 of unit 16 t + l % 16.
+// Activations of a hidden layer for the wave's 16 samples and 32 units from
+// the samples' inputs a: a lane holds samples 4 g .. 4 g + 3 of units u + c
+// and u + 16 + c.
 template <int KT>
-__device__ __forceinline__ void layer(f4 (&acc)[4], const float *bias, int units, const float *a,
-                                      int lda, const float *W, int ldw) {
-  const int c = threadIdx.x & 15;
+__device__ __forceinline__ void layer(f4 (&acc)[2], const Place &q, const float *bias, int units,
+                                      const float *a, int lda, const float *W, int ldw) {
 #pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const float b = 16 * t + c < units ? bias[16 * t + c] : 0.f;
+  for (int t = 0; t < 2; ++t) {
+    const int u = q.u + 16 * t + q.c;
+    const float b = u < units ? bias[u] : 0.f;
     acc[t] = f4{b, b, b, b};
   }
-  mul_tiles<4, KT>(acc, a, lda, W, ldw);
+  mul_tiles<2, KT>(acc, a + 16 * q.w * lda, lda, W + q.u * ldw, ldw);
 #pragma unroll
-  for (int t = 0; t < 4; ++t)
+  for (int t = 0; t < 2; ++t)
 #pragma unroll
     for (int r = 0; r < 4; ++r) acc[t][r] = relu(acc[t][r]);
 }
 
-__global__ __launch_bounds__(256) void mlp_forward_kernel(Dims d, const float *p,
-                                                          const float *x, int n,
-                                                          float *y) {
+__global__ __launch_bounds__(kMlpT) void mlp_forward_kernel(Dims d, const float *p,
+                                                            const float *x, int n,
+                                                            float *y) {
   __shared__ __align__(16) float W1[kMaxH * kLdIn], W2[kMaxH * kLdH], W3[kMaxH],
-      X[kSamples * kLdIn], H[kSamples * kLdH];
+      X[kSamples * kLdIn], H1[kSamples * kLdH], H2[kSamples * kLdH];
   const int s0 = blockIdx.x * kSamples;
   load_tiles<false>(W1, W2, X, d, p, x, s0, n, W3, nullptr, nullptr);
   __syncthreads();
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63, g = l >> 4;
-  f4 h[4];
-  layer<kMaxIn / 16>(h, p + d.ob1(), d.h1, X + 16 * w * kLdIn, kLdIn, W1, kLdIn);
-  store_rows(H, h);
-  layer<kMaxH / 16>(h, p + d.ob2(), d.h2, H + 16 * w * kLdH, kLdH, W2, kLdH);
-  store_rows(H, h);
+  const Place q = place();
+  f4 h[2];
+  layer<kMaxIn / 16>(h, q, p + d.ob1(), d.h1, X, kLdIn, W1, kLdIn);
+  store_rows(H1, q, h);
+  __syncthreads();
+  layer<kMaxH / 16>(h, q, p + d.ob2(), d.h2, H1, kLdH, W2, kLdH);
+  store_rows(H2, q, h);
+  __syncthreads();
+  if (q.u) return;
   const float b3 = p[d.ob3()];
   f4 out = {b3, b3, b3, b3};
-  mul_rows<kMaxH / 16>(out, H + 16 * w * kLdH, kLdH, W3, 0, 1);
+  mul_rows<kMaxH / 16>(out, H2 + 16 * q.w * kLdH, kLdH, W3, 0, 1);
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    const int s = s0 + 16 * w + 4 * g + r;
-    if ((l & 15) == 0 && s < n) y[s] = out[r];
+    const int s = s0 + 16 * q.w + 4 * q.g + r;
+    if (q.c == 0 && s < n) y[s] = out[r];
   }
 }
 
@@ -227,99 +242,119 @@ static_assert(kGradLds * 4 <= 160 * 1024, "LDS of a CU");
 
 // one workgroup = kSamples samples: forward/backward of every sample, then
 // the workgroup's gradient sums into ws[blockIdx.x][param]
-__global__ __launch_bounds__(256) void mlp_grad_kernel(Dims d, const float *p,
-                                                       const float *x,
-                                                       const float *target, int n,
-                                                       float *ws, float *wloss) {
+__global__ __launch_bounds__(kMlpT) void mlp_grad_kernel(Dims d, const float *p,
+                                                         const float *x,
+                                                         const float *target, int n,
+                                                         float *ws, float *wloss) {
   extern __shared__ __align__(16) float lds[];
   float *rows = lds + kRows, *vec = lds + kVec;
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63, c = l & 15, g = l >> 4;
+  const Place q = place();
+  const int l = threadIdx.x & 63;
   const int s0 = blockIdx.x * kSamples;
-  const float *mine = rows + 16 * w * kLdH;  // the wave's own rows
   load_tiles<true>(lds + kW1, lds + kW2, lds + kX, d, p, x, s0, n, lds + kW3, lds + kW2T,
                    lds + kXT);
   f4 tg;
-  float w3[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    const int s = s0 + 16 * w + 4 * g + r;
+    const int s = s0 + 16 * q.w + 4 * q.g + r;
     tg[r] = s < n ? target[s] : 0.f;
-    w3[r] = 16 * r + c < d.h2 ? p[d.oW3() + 16 * r + c] : 0.f;
+  }
+  float w3[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int u = q.u + 16 * t + q.c;
+    w3[t] = u < d.h2 ? p[d.oW3() + u] : 0.f;
   }
   const float b3 = p[d.ob3()];
   __syncthreads();
-  f4 h1[4], h2[4];
-  layer<kMaxIn / 16>(h1, p + d.ob1(), d.h1, lds + kX + 16 * w * kLdIn, kLdIn, lds + kW1, kLdIn);
-  store_rows(rows, h1);
-  store_columns(lds + kH1T, h1);
-  layer<kMaxH / 16>(h2, p + d.ob2(), d.h2, mine, kLdH, lds + kW2, kLdH);
-  store_rows(rows, h2);
-  store_columns(lds + kH2T, h2);
+  f4 h1[2], h2[2];
+  layer<kMaxIn / 16>(h1, q, p + d.ob1(), d.h1, lds + kX, kLdIn, lds + kW1, kLdIn);
+  store_rows(rows, q, h1);
+  store_columns(lds + kH1T, q, h1);
+  __syncthreads();
+  layer<kMaxH / 16>(h2, q, p + d.ob2(), d.h2, rows, kLdH, lds + kW2, kLdH);
+  store_columns(lds + kH2T, q, h2);
+  __syncthreads();
+  store_rows(rows, q, h2);
+  __syncthreads();
   f4 y = {b3, b3, b3, b3}, dy;
-  mul_rows<kMaxH / 16>(y, mine, kLdH, lds + kW3, 0, 1);
+  mul_rows<kMaxH / 16>(y, rows + 16 * q.w * kLdH, kLdH, lds + kW3, 0, 1);
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    const int k = 16 * w + slot(4 * g + r);
-    const bool in = s0 + 16 * w + 4 * g + r < n;
+    const int k = 16 * q.w + slot(4 * q.g + r);
+    const bool in = s0 + 16 * q.w + 4 * q.g + r < n;
     const float e = __shfl(y[r], l & 48) - tg[r];
     dy[r] = in ? 2.f * e / (float)n : 0.f;
-    if (c == 0) {
+    if (q.c == 0 && q.u == 0) {
       vec[k] = 1.f;
       vec[kLdH + k] = dy[r];
       vec[2 * kLdH + k] = in ? e * e : 0.f;
     }
   }
-  f4 d2[4];
+  f4 d2[2];
 #pragma unroll
-  for (int t = 0; t < 4; ++t)
+  for (int t = 0; t < 2; ++t)
 #pragma unroll
     for (int r = 0; r < 4; ++r) d2[t][r] = h2[t][r] > 0.f ? dy[r] * w3[t] : 0.f;
-  store_rows(rows, d2);
-  store_columns(lds + kD2T, d2);
-  f4 d1[4] = {};
-  mul_tiles<4, kMaxH / 16>(d1, mine, kLdH, lds + kW2T, kLdH);
+  store_columns(lds + kD2T, q, d2);
+  __syncthreads();
+  store_rows(rows, q, d2);
+  __syncthreads();
+  f4 d1[2] = {};
+  mul_tiles<2, kMaxH / 16>(d1, rows + 16 * q.w * kLdH, kLdH, lds + kW2T + q.u * kLdH, kLdH);
 #pragma unroll
-  for (int t = 0; t < 4; ++t)
+  for (int t = 0; t < 2; ++t)
 #pragma unroll
     for (int r = 0; r < 4; ++r) d1[t][r] = h1[t][r] > 0.f ? d1[t][r] : 0.f;
-  store_columns(lds + kD1T, d1);
+  store_columns(lds + kD1T, q, d1);
   __syncthreads();
-  // a wave sums units 16 w .. 16 w + 15 of every weight gradient over the
-  // samples
+  // a pair of waves sums units 16 w .. 16 w + 15 of every weight gradient over
+  // the samples: half 0 columns 0 .. 31 of W2's and the bias gradients, which
+  // are sums against ones (column 0), half 1 the rest of W2's, W1's and W3's,
+  // against dL/dy (column 1).  Every product is under way before the first
+  // store
   float *row = ws + (size_t)blockIdx.x * d.np;
-  const int u0 = 16 * w + 4 * g;
-  // the bias gradients are sums against ones (column 0), W3's against dL/dy
-  // (column 1); every product is under way before the first store
-  f4 gw2[4] = {}, gw1[kMaxIn / 16] = {}, b1 = {}, b2 = {}, g3 = {};
-  mul_tiles<4, kSamples / 16>(gw2, lds + kD2T + 16 * w * kLdH, kLdH, lds + kH1T, kLdH);
-  mul_tiles<kMaxIn / 16, kSamples / 16>(gw1, lds + kD1T + 16 * w * kLdH, kLdH, lds + kXT, kLdH);
-  mul_rows<kSamples / 16>(b1, lds + kD1T + 16 * w * kLdH, kLdH, vec, kLdH, 1);
-  mul_rows<kSamples / 16>(b2, lds + kD2T + 16 * w * kLdH, kLdH, vec, kLdH, 1);
-  mul_rows<kSamples / 16>(g3, lds + kH2T + 16 * w * kLdH, kLdH, vec, kLdH, 2);
+  const float *D1 = lds + kD1T + 16 * q.w * kLdH, *D2 = lds + kD2T + 16 * q.w * kLdH;
+  const int u0 = 16 * q.w + 4 * q.g;
+  f4 gw2[2] = {};
+  mul_tiles<2, kSamples / 16>(gw2, D2, kLdH, lds + kH1T + q.u * kLdH, kLdH);
+  if (q.u == 0) {
+    f4 b1 = {}, b2 = {}, v = {};
+    mul_rows<kSamples / 16>(b1, D1, kLdH, vec, kLdH, 1);
+    mul_rows<kSamples / 16>(b2, D2, kLdH, vec, kLdH, 1);
+    // b3's gradient and the loss: the sums of vec's own rows 1 and 2 (rows 3
+    // .. 15 of the left operand are not used: row 2 again)
+    if (q.w == 0)
+      mul_rows<kSamples / 16>(v, vec + (q.c < 3 ? 0 : 2 - q.c) * kLdH, kLdH, vec, kLdH, 1);
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int u = u0 + r;
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-      if (u < d.h2 && 16 * t + c < d.h1) row[d.oW2() + u * d.h1 + 16 * t + c] = gw2[t][r];
-#pragma unroll
-    for (int t = 0; t < kMaxIn / 16; ++t)
-      if (u < d.h1 && 16 * t + c < d.in) row[d.oW1() + u * d.in + 16 * t + c] = gw1[t][r];
-    if (c == 0 && u < d.h1) row[d.ob1() + u] = b1[r];
-    if (c == 0 && u < d.h2) row[d.ob2() + u] = b2[r];
-    if (c == 1 && u < d.h2) row[d.oW3() + u] = g3[r];
-  }
-  // b3's gradient and the loss are the sums of vec's own rows 1 and 2
-  if (w == 0) {
-    f4 v = {};
-    // rows 3 .. 15 of the left operand are not used: row 2 again
-    const float *own = vec + (c < 3 ? 0 : 2 - c) * kLdH;
-    mul_rows<kSamples / 16>(v, own, kLdH, vec, kLdH, 1);
-    if (l == 0) {
+    for (int r = 0; r < 4; ++r) {
+      if (q.c == 0 && u0 + r < d.h1) row[d.ob1() + u0 + r] = b1[r];
+      if (q.c == 0 && u0 + r < d.h2) row[d.ob2() + u0 + r] = b2[r];
+    }
+    if (threadIdx.x == 0) {
       row[d.ob3()] = v[1];
       wloss[blockIdx.x] = v[2];
     }
+  } else {
+    f4 gw1[kMaxIn / 16] = {}, g3 = {};
+    mul_tiles<kMaxIn / 16, kSamples / 16>(gw1, D1, kLdH, lds + kXT, kLdH);
+    mul_rows<kSamples / 16>(g3, lds + kH2T + 16 * q.w * kLdH, kLdH, vec, kLdH, 2);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int u = u0 + r;
+#pragma unroll
+      for (int t = 0; t < kMaxIn / 16; ++t)
+        if (u < d.h1 && 16 * t + q.c < d.in) row[d.oW1() + u * d.in + 16 * t + q.c] = gw1[t][r];
+      if (q.c == 1 && u < d.h2) row[d.oW3() + u] = g3[r];
+    }
   }
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int u = u0 + r, k = q.u + 16 * t + q.c;
+      if (u < d.h2 && k < d.h1) row[d.oW2() + u * d.h1 + k] = gw2[t][r];
+    }
 }
 
 // Sums the workspace rows in order, a thread a parameter with 32 rows'
@@ -379,7 +414,7 @@ extern "C" int jq_mlp_forward(const float *params, int in, int h1, int h2,
   set_error("");
   if (n <= 0) return 0;
   Dims d = dims(in, h1, h2);
-  hipLaunchKernelGGL(mlp_forward_kernel, dim3((n - 1) / kSamples + 1), dim3(256), 0,
+  hipLaunchKernelGGL(mlp_forward_kernel, dim3((n - 1) / kSamples + 1), dim3(kMlpT), 0,
                      (hipStream_t)stream, d, params, x, n, y);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : set_error(hipGetErrorString(e));
@@ -405,7 +440,7 @@ extern "C" int jq_mlp_train_step(float *params, float *grads, float *workspace,
     attr = true;
   }
   float *ws = workspace, *wloss = workspace + (size_t)nblk * d.np;
-  hipLaunchKernelGGL(mlp_grad_kernel, dim3(nblk), dim3(256), lds, (hipStream_t)stream,
+  hipLaunchKernelGGL(mlp_grad_kernel, dim3(nblk), dim3(kMlpT), lds, (hipStream_t)stream,
                      d, params, x, target, n, ws, wloss);
   hipLaunchKernelGGL(mlp_update_kernel, dim3((d.np + 63) / 64 + 1), dim3(64), 0,
                      (hipStream_t)stream, d, params, grads, ws, wloss, nblk, n, lr,
