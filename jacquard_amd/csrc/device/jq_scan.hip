@@ -9,6 +9,14 @@
 //     issued as soon as the registers of its predecessor are free: the next
 //     boomerang stage's (or partition's) words are in flight while the
 //     current tree runs, and headers are requested two partitions ahead;
+//   - a partition waits for memory in one place, its state gather; all other
+//     words are waited for once, after the stages (wait_loads), and a block's
+//     steps are one loop.  Waits at the uses, for whatever had been issued
+//     since, and copies between the registers of nested loops before that:
+//     4M gates with X and timing, 202 -> 192 us per cycle; 100K gates with X,
+//     67 -> 63; 2K gates in one block, 23.1 -> 21.6;
+//   - the first stage's bits are taken from the gathered words directly, with
+//     permutations composed ahead of the launch;
 //   - snapshot words move between workgroups only through agent-coherent
 //     loads and stores, so the grid barrier carries no cache maintenance;
 //   - the 8192-bit shuffle is 16 LDS bit-gathers per thread on all 8 waves;
@@ -69,6 +77,9 @@ struct ScanArgs {
   u64 *ring;
   const u32 *flow;  // kFlow* words
   u32 *prog;
+  // composed stage-0 permutations (see below) and, per major stage and
+  // block, the first one's slot or kNoSlot; table == null: none
+  const u32 *table, *slots;  // slots: never null
   // profiling
   const u32 *part_index;
   u32 num_parts;
@@ -80,6 +91,12 @@ __device__ __forceinline__ uint4 ld4(const u32 *p) {
   return *reinterpret_cast<const uint4 *>(p);
 }
 
+// Waits for the wave's loads and stores here, where they have had their time,
+// in place of waits at the uses of what was loaded: the compiler counts the
+// loads in flight on every path to a use, and on a path that issued fewer
+// than another it would wait for younger ones as well.
+__device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }
+
 // Threads of a workgroup: two adjacent lanes per word of the 256-word
 // layer, half 0 its bits 0..15 (and the first half of its global-read
 // rounds), half 1 the rest.  A partition is a chain of short steps that one
@@ -87,7 +104,7 @@ __device__ __forceinline__ uint4 ld4(const u32 *p) {
 // with one thread per word the 32 LDS bit-gathers and the pext loop were
 // twice as long, and each SIMD had a single wave to issue from.  Two
 // threads also halve the registers a thread needs for prefetched words
-// (218 of the 256 that two waves per SIMD leave; one thread per word had
+// (194 of the 256 that two waves per SIMD leave; one thread per word had
 // spilled).  Measured together with the earlier loads, in launches that keep
 // grid barriers: 4M gates with X and timing, 248 -> 202 us per cycle; one
 // co-simulation edge of a one-block design, 12.1 -> 10.5 us.
@@ -98,21 +115,76 @@ __device__ __forceinline__ u32 from_pair(u32 v) {
   return __builtin_amdgcn_update_dpp(0u, v, 0xB1, 0xF, 0xF, false);
 }
 
+// Takes bit b (mod 32) of w in at the top of r.
+__device__ __forceinline__ u32 push_bit(u32 r, u32 w, u32 b) {
+  return __builtin_amdgcn_alignbit(w >> (b & 31), r, 1);
+}
+// A pair's word from the 16 bits each thread has pushed.
+__device__ __forceinline__ u32 join_halves(u32 r) {
+  const u32 o = from_pair(r);
+  return (threadIdx.x & 1) ? __builtin_amdgcn_perm(r, o, 0x07060302u)
+                           : __builtin_amdgcn_perm(o, r, 0x07060302u);
+}
+
 // The 32 LDS bit-gathers of a word, 16 in each thread of its pair: bit 2k
 // (2k+1) of a half <- src bit lo16 (hi16) of its perm word k
-// (src/flatten.rs:1027-1034).  Both threads return the whole word.
-__device__ __forceinline__ u32 gather_bits(const u32 *src, uint4 qa, uint4 qb) {
-  u32 r = 0;
+// (src/flatten.rs:1027-1034).  Both threads return the whole word.  With two
+// waves to a SIMD the time is that of the instructions, four clocks each per
+// wave: shifting every bit in at the top takes one where masking, shifting
+// and combining it took three.  WIDE: `hi` holds two more index bits each.
+template <bool WIDE>
+__device__ __forceinline__ u32 gather_bits_of(const u32 *src, uint4 qa, uint4 qb, u32 hi) {
   const u32 w[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
+  u32 d[16];
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
-    u32 i1 = w[k] & 0xffffu, i2 = w[k] >> 16;
-    r |= ((src[i1 >> 5] >> (i1 & 31)) & 1u) << (2 * k);
-    r |= ((src[i2 >> 5] >> (i2 & 31)) & 1u) << (2 * k + 1);
+    u32 a = (w[k] & 0xffffu) >> 5, b = w[k] >> 21;
+    if (WIDE) {
+      a |= ((hi >> (4 * k)) & 3u) << 11;
+      b |= ((hi >> (4 * k + 2)) & 3u) << 11;
+    }
+    d[2 * k] = src[a];
+    d[2 * k + 1] = src[b];
   }
-  const u32 o = from_pair(r);
-  return (threadIdx.x & 1) ? (r << 16) | o : (o << 16) | r;
+  // all of them in flight before the first is waited for
+  asm volatile("" ::"v"(d[0]), "v"(d[1]), "v"(d[2]), "v"(d[3]), "v"(d[4]), "v"(d[5]), "v"(d[6]),
+               "v"(d[7]), "v"(d[8]), "v"(d[9]), "v"(d[10]), "v"(d[11]), "v"(d[12]), "v"(d[13]),
+               "v"(d[14]), "v"(d[15]));
+  u32 r = 0;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    r = push_bit(r, d[2 * k], w[k]);
+    r = push_bit(r, d[2 * k + 1], w[k] >> 16);
+  }
+  return join_halves(r);
 }
+__device__ __forceinline__ u32 gather_bits(const u32 *src, uint4 qa, uint4 qb) {
+  return gather_bits_of<false>(src, qa, qb, 0);
+}
+
+// ---- composed stage-0 permutations
+//
+// A partition's input words are put together bit by bit (the pext of the
+// global-read entries) and the first boomerang stage then takes them apart
+// again with its permutation.  A launch of kFlowMinCycles cycles or more
+// composes the two once, ahead of it: an index of the composed permutation
+// names a bit of the words as they were read, kept in LDS as they are, entry
+// t of round k at 1 + 256 k + t (word 0 is zero, for bits that no entry
+// fills), and the pext, a loop over up to 32 bits per lane, is gone from
+// every cycle.  Measured with and without: 2K gates in one block, 1000 cycles,
+// 21.6 -> 16.2 ms; 100K gates with X and SRAMs, 63 -> 55 us per cycle; 1M
+// gates, 249 blocks, 61 -> 56 us per cycle; one edge of a one-block
+// co-simulation, 10.4 -> 9.6 us.
+//
+// A slot of the table holds a partition's permutation words in the order of
+// the stage sections (the low 16 bits of every index), then one word per
+// thread with two more bits for each of its 16 indexes, read only when the
+// partition has more than kNarrowRounds rounds.
+constexpr u32 kNoSlot = 0xFFFFFFFFu;
+constexpr u32 kSlotWords = 4096 + kScanThreads;
+constexpr u32 kNarrowRounds = 7;  // 1 + 7 * 256 words: 16-bit indexes
+constexpr u32 kRawRounds = 31;    // 1 + 31 * 256 words: 18-bit indexes
+constexpr u32 kRawWords = 1 + 256 * kRawRounds;
 
 __device__ __forceinline__ u16 arr_step(u16 a, u16 b, u32 ob, u32 dly) {
   u16 base = (ob == 0xFFFFFFFFu) ? a : (a > b ? a : b);
@@ -137,60 +209,49 @@ __device__ __forceinline__ void push_event(EvHdr *ev, u32 cap, u32 type,
   }
 }
 
-// Header of one partition (src/flatten.rs:198-258) and the writeout hook of
-// this thread's word; `base` is the header's word offset in blocks_data.
+// Header of one partition (src/flatten.rs:198-258); `base` is its word offset
+// in blocks_data.
 struct PartHdr {
   size_t base;
+  u32 slot;  // of its composed permutation, or kNoSlot
   u32 num_stages, is_last, num_ios, io_offset, num_srams, sram_offset, rounds,
-      num_dups, xoff, hook;
-  bool is_x;
+      num_dups, is_x, xoff;
 };
 
-// The same as it comes from memory.  Nothing here looks at the words, so
-// their loads stay in flight until settle() is called, a partition later.
-struct RawHdr {
-  size_t base;
-  uint4 a, b;
-  uint2 x;
-  u32 hook;
-};
-
-__device__ __forceinline__ RawHdr load_hdr(const u32 *__restrict__ bd, size_t off) {
-  RawHdr r;
-  const u32 *s = bd + off;
-  r.base = off;
-  r.a = ld4(s);
-  r.b = ld4(s + 4);
-  r.x = *reinterpret_cast<const uint2 *>(s + 8);
-  r.hook = s[128 + (threadIdx.x >> 2)];
-  return r;
-}
-
-__device__ __forceinline__ PartHdr settle(const RawHdr &r) {
-  PartHdr h;
-  h.base = r.base;
-  h.num_stages = uniform(r.a.x);
-  h.is_last = uniform(r.a.y);
-  h.num_ios = uniform(r.a.z);
-  h.io_offset = uniform(r.a.w);
-  h.num_srams = uniform(r.b.x);
-  h.sram_offset = uniform(r.b.y);
-  h.rounds = uniform(r.b.z);
-  h.num_dups = uniform(r.b.w);
-  h.is_x = uniform(r.x.x) != 0;
-  h.xoff = uniform(r.x.y);
-  h.hook = (threadIdx.x & 2) ? (r.hook >> 16) : (r.hook & 0xffffu);
-  return h;
-}
-
-__device__ __forceinline__ PartHdr no_hdr() {
-  PartHdr h{};
-  return h;  // num_stages == 0: nothing to run
-}
+// A step's header words as one load of the wave brings them, word k on lane
+// k, with what the step after it may need on three more lanes.  Nothing here
+// looks at them, so the load stays in flight until settle() is called, a
+// partition later.
+constexpr u32 kHdrWords = 10, kAfterLane = 10, kSlotLane = 12;
 
 // Words of one partition's script section (src/flatten.rs:873-1127).
 __device__ __forceinline__ size_t part_words(const PartHdr &h) {
   return 256 + (size_t)512 * h.rounds + (size_t)5120 * (h.num_stages + 2);
+}
+
+// A partition's section as a buffer: a load past its end (kNoLoad, or any
+// load of the section of an empty header) returns zeros without a memory
+// access.  So every load that only some lanes, or only some partitions, need
+// is the same instruction on every path, and the compiler, which knows the
+// loads in flight by their order, never has to wait for younger ones.
+using Section = __amdgpu_buffer_rsrc_t;
+using Word2 = __attribute__((ext_vector_type(2))) u32;
+using Word4 = __attribute__((ext_vector_type(4))) u32;
+constexpr u32 kNoLoad = 0x80000000u;
+
+__device__ __forceinline__ Section section_of(const u32 *bd, const PartHdr &h) {
+  const u32 bytes = 4 * (256 + 512 * h.rounds + 5120 * (h.num_stages + 2));
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<u32 *>(bd + h.base), 0,
+                                           h.num_stages ? bytes & (kNoLoad - 1) : 0, 0x00027000);
+}
+// Words at word offset `at` (lanes that are not `in`: zeros).
+__device__ __forceinline__ uint2 ld2(Section s, bool in, u32 at) {
+  const Word2 v = __builtin_amdgcn_raw_buffer_load_b64(s, in ? 4 * at : kNoLoad, 0, 0);
+  return make_uint2(v.x, v.y);
+}
+__device__ __forceinline__ uint4 ld4(Section s, bool in, u32 at) {
+  const Word4 v = __builtin_amdgcn_raw_buffer_load_b128(s, in ? 4 * at : kNoLoad, 0, 0);
+  return make_uint4(v.x, v.y, v.z, v.w);
 }
 
 // What a partition holds before its state gather: the global-read entries
@@ -202,6 +263,7 @@ constexpr u32 kPreRounds = 8;
 struct PartPre {
   uint2 e[kPreRounds];
   uint4 qa, qb, fA, fB, fC, fD;
+  u32 hi, hook;  // hook: the writeout hook of this thread's word
 };
 
 // The global-read rounds of this thread: of a word's rounds the first
@@ -213,39 +275,61 @@ __device__ __forceinline__ u32 num_rounds(u32 rounds) {
   return (threadIdx.x & 1) ? rounds / 2 : (rounds + 1) / 2;
 }
 
-__device__ __forceinline__ void load_entries(PartPre &P, const u32 *__restrict__ bd,
-                                             const PartHdr &h) {
-  const uint2 *gr = reinterpret_cast<const uint2 *>(bd + h.base + 256) +
-                    256 * first_round(h.rounds) + (threadIdx.x >> 1);
-  const u32 n = num_rounds(h.rounds), most = (h.rounds + 1) / 2;
+// The entries, by how many rounds there are (gather() takes as many), and the
+// hook.
+__device__ __forceinline__ void load_entries(PartPre &P, Section s, u32 rounds) {
+  const u32 at = 256 + 512 * first_round(rounds) + 2 * (threadIdx.x >> 1);
+  const u32 n = num_rounds(rounds), most = (rounds + 1) / 2;
+  const u32 hook =
+      __builtin_amdgcn_raw_buffer_load_b32(s, 4 * (128 + (threadIdx.x >> 2)), 0, 0);
 #pragma unroll
-  for (u32 k = 0; k < kPreRounds; ++k) {
-    P.e[k] = make_uint2(0, 0);
-    if (k < most) {  // uniform
-      if (k < n) P.e[k] = gr[256 * k];
-    }
+  for (u32 k = 0; k < 2; ++k) P.e[k] = ld2(s, k < n, at + 512 * k);
+  if (most > 2) {
+#pragma unroll
+    for (u32 k = 2; k < 4; ++k) P.e[k] = ld2(s, k < n, at + 512 * k);
   }
+  if (most > 4) {
+#pragma unroll
+    for (u32 k = 4; k < kPreRounds; ++k) P.e[k] = ld2(s, k < n, at + 512 * k);
+  }
+  P.hook = hook;
 }
 
-// The stage section at `st`: this thread's permutation words and, on wave
-// 0, the tree flags (words 0..255 of the flag block).
-__device__ __forceinline__ void load_stage(PartPre &P, const u32 *__restrict__ st) {
-  const int t = threadIdx.x;
-  const u32 *q = st + 2048 * (t & 1) + 4 * (t >> 1);
-  P.qa = ld4(q);
-  P.qb = ld4(q + 1024);
+// This thread's permutation words of a stage, from word `q` of perm, and, on
+// wave 0, the tree flags of the stage section at word `at` of s (words 0..255
+// of the flag block).
+__device__ __forceinline__ void load_stage(PartPre &P, Section perm, u32 q, Section s, u32 at) {
+  const u32 t = threadIdx.x;
+  q += 2048 * (t & 1) + 4 * (t >> 1);
+  P.qa = ld4(perm, true, q);
+  P.qb = ld4(perm, true, q + 1024);
+  const u32 f = at + 4096 + 4 * t;
   if (t < 64) {
-    const u32 *fl = st + 4096;
-    P.fA = ld4(fl + 4 * t);
-    P.fB = ld4(fl + 4 * (64 + t));
-    P.fC = ld4(fl + 4 * (128 + t));
-    P.fD = ld4(fl + 4 * (192 + t));
+    P.fA = ld4(s, true, f);
+    P.fB = ld4(s, true, f + 256);
+    P.fC = ld4(s, true, f + 512);
+    P.fD = ld4(s, true, f + 768);
   }
 }
 
 // First stage section of a partition.
-__device__ __forceinline__ const u32 *stage0(const u32 *__restrict__ bd, const PartHdr &h) {
-  return bd + h.base + 256 + (size_t)512 * h.rounds;
+__device__ __forceinline__ u32 stage0(const PartHdr &h) { return 256 + 512 * h.rounds; }
+
+// The permutation of the first stage of a partition with section s: the
+// composed one where there is one.
+__device__ __forceinline__ Section perm0(const u32 *table, const PartHdr &h, Section s) {
+  return h.slot == kNoSlot ? s
+                           : __builtin_amdgcn_make_buffer_rsrc(
+                                 const_cast<u32 *>(table + (size_t)h.slot * kSlotWords), 0,
+                                 4 * kSlotWords, 0x00027000);
+}
+__device__ __forceinline__ u32 perm0_at(const PartHdr &h) {
+  return h.slot == kNoSlot ? stage0(h) : 0;
+}
+__device__ __forceinline__ u32 load_hi(Section perm, const PartHdr &h) {
+  const bool wide = h.slot != kNoSlot && h.rounds > kNarrowRounds;
+  return __builtin_amdgcn_raw_buffer_load_b32(perm, wide ? 4 * (4096 + threadIdx.x) : kNoLoad, 0,
+                                              0);
 }
 
 // ---- dataflow synchronisation of value-only launches
@@ -271,20 +355,22 @@ __device__ __forceinline__ const u32 *stage0(const u32 *__restrict__ bd, const P
 // commits could overwrite a word it has still to read (flow_room).
 //
 // Words below the first writeout word are primary inputs, filled in by the
-// host before the launch; those, and all of snapshot 0, are read from the
-// snapshot buffer.
+// host before the launch; those are read from the snapshot buffer.  The
+// others of snapshot 0 are copied into the ring ahead of the launch.
 constexpr u32 kRing = 8;
 constexpr u32 kFlowMinCycles = 8;
 // what the builders leave in ScanArgs::flow
 constexpr u32 kFlowNegLo = 0;  // ~(first writeout word), 0 when there is none
 constexpr u32 kFlowXoff = 1;   // X mask offset of the X-capable partitions, or 0
 constexpr u32 kFlowBad = 2;    // nonzero: the script does not fit, grid barriers
+constexpr u32 kTableCursor = 32;  // slots of the table given out
 constexpr u32 kFlowWords = 64;
 constexpr u32 kProgStride = 32;  // one progress word per 128-byte line
 
 struct Flow {
-  u64 *ring;
-  u32 slot;       // words of one ring slot (the state size)
+  Section ring;   // kRing slots
+  u64 *slots;     // the same, for the stores
+  u32 slot;       // words of one slot (the state size)
   u32 lo, xoff;   // first writeout word; X mask offset of the launch or 0
   u32 *bar, *aborted;
 };
@@ -313,39 +399,55 @@ __device__ __forceinline__ bool flow_gives_up(const Flow &F, u32 &spins) {
   return stop;
 }
 
-// The state words of the entries e (cycle c, snapshots in and out) into v
-// and, for X-capable partitions, their X masks into x.
-template <bool X>
+// A word of the ring at byte offset `at` (kNoLoad: zeros).  The coherent
+// load of st_coherent64's words, one access of 8 bytes.
+__device__ __forceinline__ u64 ld_ring(Section ring, u32 at) {
+  const Word2 v = __builtin_amdgcn_raw_buffer_load_b64(ring, at, 0, 16);  // agent scope
+  return (u64)v.y << 32 | v.x;
+}
+
+// The state words of the first N entries e (cycle c, snapshots in and out)
+// into v and, for X-capable partitions, their X masks into x.  `between` runs
+// while the loads are in flight.
+template <u32 N, bool X, class Fn>
 __device__ __forceinline__ void flow_gather(const Flow &F, const uint2 *e, const u32 *in,
-                                            const u32 *out, u32 c, u32 *v, u32 *x) {
-  u32 pend = 0;  // bit k: entry k's value, bit 16 + k: its X mask
+                                            const u32 *out, u32 c, u32 *v, u32 *x,
+                                            const Fn &between) {
+  u32 ri = (c & (kRing - 1)) * 8 * F.slot, ro = ((c + 1) & (kRing - 1)) * 8 * F.slot;
+  asm volatile("" : "+s"(ri), "+s"(ro));  // and no multiplication per entry
+  u32 a[N];
+  u64 q[N], r[X ? N : 1];
+  u32 pend = 0;    // bit k: entry k's value, bit 16 + k: its X mask
+  u32 inputs = 0;  // bit k: entry k is a primary input
 #pragma unroll
-  for (u32 k = 0; k < kPreRounds; ++k) {
+  for (u32 k = 0; k < N; ++k) {
+    const u32 w = e[k].x & 0x7fffffffu;
+    const bool o = (int)e[k].x < 0, need = e[k].y != 0, ring = need && w >= F.lo;
+    a[k] = ((e[k].x << 3) + (o ? ro : ri)) | (ring ? 0 : kNoLoad);
+    pend |= ring ? (X ? 0x10001u : 1u) << k : 0;
+    inputs |= need && !ring ? 1u << k : 0;
+  }
+#pragma unroll
+  for (u32 k = 0; k < N; ++k) {
+    q[k] = ld_ring(F.ring, a[k]);
+    if (X) r[k] = ld_ring(F.ring, a[k] + 8 * F.xoff);
     v[k] = 0;
     if (X) x[k] = 0;
-    if (e[k].y) {
-      const u32 w = e[k].x & 0x7fffffffu, o = e[k].x >> 31;
-      if (w >= F.lo && (o | c)) {
-        pend |= (X ? 0x10001u : 1u) << k;
-      } else {
-        const u32 *base = o ? out : in;
-        v[k] = base[w];
-        if (X) x[k] = base[F.xoff + w];
-      }
-    }
   }
-  u32 spins = 0;
-  for (;;) {
-    u64 q[kPreRounds], r[X ? kPreRounds : 1];
+  if (__any(inputs)) {
 #pragma unroll
-    for (u32 k = 0; k < kPreRounds; ++k) {
-      const u32 w = e[k].x & 0x7fffffffu, s = c + (e[k].x >> 31);
-      const u64 *a = F.ring + ((s & (kRing - 1)) * F.slot + w);
-      if ((pend >> k) & 1u) q[k] = ld_coherent64(a);
-      if (X && ((pend >> (16 + k)) & 1u)) r[k] = ld_coherent64(a + F.xoff);
-    }
+    for (u32 k = 0; k < N; ++k)
+      if ((inputs >> k) & 1u) {
+        const u32 *p = ((int)e[k].x < 0 ? out : in) + (e[k].x & 0x7fffffffu);
+        v[k] = *p;
+        if (X) x[k] = p[F.xoff];
+      }
+    wait_loads();
+  }
+  between();
+  const auto check = [&] {
 #pragma unroll
-    for (u32 k = 0; k < kPreRounds; ++k) {
+    for (u32 k = 0; k < N; ++k) {
       const u32 s = c + (e[k].x >> 31);
       if (((pend >> k) & 1u) && (u32)(q[k] >> 32) == s) {
         v[k] = (u32)q[k];
@@ -356,9 +458,49 @@ __device__ __forceinline__ void flow_gather(const Flow &F, const uint2 *e, const
         pend &= ~(0x10000u << k);
       }
     }
-    if (!__any(pend)) return;
-    if (flow_gives_up(F, spins)) return;
+  };
+  check();
+  for (u32 spins = 0; __any(pend);) {
+    if (flow_gives_up(F, spins)) break;
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (u32 k = 0; k < N; ++k) {
+      if ((pend >> k) & 1u) q[k] = ld_ring(F.ring, a[k]);
+      if (X && ((pend >> (16 + k)) & 1u)) r[k] = ld_ring(F.ring, a[k] + 8 * F.xoff);
+    }
+    wait_loads();
+    check();
   }
+}
+
+// The same where the grid barriers order the snapshots.
+template <u32 N, class Fn>
+__device__ __forceinline__ void snap_gather(const uint2 *e, const u32 *in, const u32 *out,
+                                            bool is_x, u32 xoff, u32 *v, u32 *x,
+                                            const Fn &between) {
+  const u32 *a[N];
+#pragma unroll
+  for (u32 k = 0; k < N; ++k) {
+    a[k] = e[k].y ? ((e[k].x >> 31) ? out : in) + (e[k].x & 0x7fffffffu) : in;
+    v[k] = ld_coherent(a[k]);
+  }
+  if (is_x) {
+#pragma unroll
+    for (u32 k = 0; k < N; ++k) x[k] = ld_coherent(a[k] + (e[k].y ? xoff : 0));
+  }
+  between();
+}
+
+template <u32 N, bool FLOW, class Fn>
+__device__ __forceinline__ void gather(const Flow &F, const uint2 *e, const u32 *in,
+                                       const u32 *out, u32 c, bool is_x, u32 xoff, u32 *v,
+                                       u32 *x, const Fn &between) {
+  if (!FLOW)
+    snap_gather<N>(e, in, out, is_x, xoff, v, x, between);
+  else if (is_x)
+    flow_gather<N, true>(F, e, in, out, c, v, x, between);
+  else
+    flow_gather<N, false>(F, e, in, out, c, v, x, between);
 }
 
 // State word w of snapshot in (o = 0) or out (o = 1) of cycle c, for the
@@ -367,9 +509,9 @@ __device__ __forceinline__ void flow_gather(const Flow &F, const uint2 *e, const
 __device__ __forceinline__ u32 flow_word(const Flow &F, bool need, u32 w, u32 o, u32 off,
                                          const u32 *in, const u32 *out, u32 c) {
   if (!need) return 0;
-  if (w < F.lo || !(o | c)) return (o ? out : in)[off + w];
+  if (w < F.lo) return (o ? out : in)[off + w];
   const u32 s = c + o;
-  const u64 *a = F.ring + ((s & (kRing - 1)) * F.slot + off + w);
+  const u64 *a = F.slots + ((size_t)(s & (kRing - 1)) * F.slot + off + w);
   u32 spins = 0;
   for (;;) {
     const u64 q = ld_coherent64(a);
@@ -434,99 +576,284 @@ __device__ __forceinline__ void tree_level(u32 &cur, u32 &curx, u16 &cura, const
   cura = na;
 }
 
+// ---- the builder of the composed permutations
+
+struct TableBuild {
+  const usize *blocks_start;
+  const u32 *bd;
+  u32 cap;  // slots of the table
+  u32 *slots, *table;
+  u32 *cursor;  // slots given out, zero before
+};
+
+// Workgroup (m, b) composes the permutations of block b's partitions in
+// major stage m.  All of them keep the script's own when one has too many
+// rounds, a permutation index is out of range or the table is full.
+__global__ __launch_bounds__(256) void compose_kernel(TableBuild T) {
+  // the composed index of bit p of input word t, at 256 p + t: lanes are
+  // consecutive words
+  __shared__ u32 src[8192];
+  __shared__ u32 s_slot, s_bad;
+  const u32 t = threadIdx.x;
+  const usize start = T.blocks_start[blockIdx.x];
+  size_t off = start;
+  u32 n = 0;
+  bool fits = true;
+  for (;;) {
+    const u32 *s = T.bd + off;
+    const u32 ns = s[0], is_last = s[1], rounds = s[6];
+    if (ns == 0) break;
+    ++n;
+    fits = fits && rounds <= kRawRounds;
+    if (is_last) break;
+    off += 256 + (size_t)512 * rounds + (size_t)5120 * (ns + 2);
+  }
+  if (t == 0) {
+    s_bad = 0;
+    s_slot = kNoSlot;
+    if (n != 0 && fits && n <= T.cap) {
+      const u32 slot = atomicAdd(T.cursor, n);
+      if (slot <= T.cap - n) s_slot = slot;
+    }
+    T.slots[blockIdx.x] = kNoSlot;
+  }
+  __syncthreads();
+  if (s_slot == kNoSlot) return;
+  u32 *q = T.table + (size_t)s_slot * kSlotWords;
+  off = start;
+  for (u32 i = 0; i < n; ++i, q += kSlotWords) {
+    const u32 *s = T.bd + off;
+    const u32 ns = s[0], rounds = s[6];
+    // bit 0 is the last bit of the last round, and so on upwards
+    const uint2 *gr = reinterpret_cast<const uint2 *>(s + 256);
+    u32 p = 0;
+    for (u32 hi = rounds; hi != 0 && p < 32;) {
+      u32 m[8];
+      const u32 lo = hi > 8 ? hi - 8 : 0;
+#pragma unroll
+      for (u32 k = 0; k < 8; ++k) m[k] = lo + k < hi ? gr[256 * (lo + k) + t].y : 0;
+#pragma unroll
+      for (int k = 7; k >= 0; --k)
+        for (; m[k] != 0 && p < 32; ++p) {
+          const u32 b = 31 - __builtin_clz(m[k]);
+          src[256 * p + t] = (1 + 256 * (lo + k) + t) << 5 | b;
+          m[k] ^= 1u << b;
+        }
+      hi = lo;
+    }
+    for (; p < 32; ++p) src[256 * p + t] = 0;  // raw word 0
+    __syncthreads();
+    const u32 *perm = s + 256 + (size_t)512 * rounds;
+#pragma unroll
+    for (u32 half = 0; half < 2; ++half) {
+      u32 hi = 0;
+#pragma unroll
+      for (u32 k = 0; k < 8; ++k) {
+        const u32 at = 2048 * half + 1024 * (k >> 2) + 4 * t + (k & 3);
+        const u32 w = perm[at];
+        const u32 i1 = w & 0xffffu, i2 = w >> 16;
+        if (i1 >= 8192 || i2 >= 8192) {
+          s_bad = 1;
+        } else {
+          const u32 j1 = src[256 * (i1 & 31) + (i1 >> 5)], j2 = src[256 * (i2 & 31) + (i2 >> 5)];
+          q[at] = (j1 & 0xffffu) | j2 << 16;
+          hi |= (j1 >> 16) << (4 * k) | (j2 >> 16) << (4 * k + 2);
+        }
+      }
+      q[4096 + 2 * t + half] = hi;
+    }
+    __syncthreads();
+    off += 256 + (size_t)512 * rounds + (size_t)5120 * (ns + 2);
+  }
+  if (t == 0 && !s_bad) T.slots[blockIdx.x] = s_slot;
+}
+
+// A block's partitions in execution order: cycle, major stage, then
+// position in the stage's section of blocks_data (kernel_v1_impl.cuh:
+// 565-626).  A stage without partitions is one step with an empty header.
+// `next` is the step after the one that runs; the header of the one after
+// that, `far`, is in flight.
+__device__ __forceinline__ usize uniform64(usize v) {
+  return (usize)uniform((u32)(v >> 32)) << 32 | uniform((u32)v);
+}
+
+struct Walk {
+  PartHdr cur, next;
+  u32 far;        // header words of the step after next (see kHdrWords)
+  size_t far_base;
+  u32 far_slot;
+  bool have;      // far is a step of the launch
+  u32 c, m;       // of far
+};
+
+__device__ __forceinline__ u32 lane_of(u32 v, u32 lane) {
+  return __builtin_amdgcn_readlane(v, lane);
+}
+
+// Requests the header at word `off` of bd, the start of the section after
+// w.m's and that section's first slot.
+__device__ __forceinline__ void load_hdr(const ScanArgs &A, Walk &w, size_t off, u32 slot) {
+  const u32 k = w.m + 1 == A.num_major_stages ? 0 : w.m + 1;
+  const size_t i = (size_t)k * A.num_blocks + blockIdx.x;
+  const u32 lane = threadIdx.x & 63;
+  const u32 *p = A.blocks_data + off + lane;
+  if (lane >= kAfterLane) p = reinterpret_cast<const u32 *>(A.blocks_start + i) + (lane & 1);
+  if (lane == kSlotLane) p = A.slots + i;
+  w.far = lane <= kSlotLane ? *p : 0;
+  w.far_base = off;
+  w.far_slot = slot;
+}
+
+__device__ __forceinline__ PartHdr settle(const Walk &w) {
+  PartHdr h;
+  h.base = w.far_base;
+  h.slot = w.far_slot;
+  // past the launch's last step: nothing to run
+  h.num_stages = w.have ? lane_of(w.far, 0) : 0;
+  h.is_last = lane_of(w.far, 1);
+  h.num_ios = lane_of(w.far, 2);
+  h.io_offset = lane_of(w.far, 3);
+  h.num_srams = lane_of(w.far, 4);
+  h.sram_offset = lane_of(w.far, 5);
+  h.rounds = lane_of(w.far, 6);
+  h.num_dups = lane_of(w.far, 7);
+  h.is_x = lane_of(w.far, 8);
+  h.xoff = lane_of(w.far, 9);
+  return h;
+}
+
+// Requests the header of the step after h (the one far held); past the
+// launch's last step that of h again.
+__device__ __forceinline__ void fetch_step(const ScanArgs &A, u32 cycles, Walk &w,
+                                           const PartHdr &h) {
+  size_t off = h.base + part_words(h);
+  u32 slot = h.slot + (h.slot != kNoSlot);
+  if (h.num_stages == 0 || h.is_last != 0) {
+    if (++w.m == A.num_major_stages) {
+      w.m = 0;
+      ++w.c;
+    }
+    w.have = w.c < cycles;
+    off = w.have ? (size_t)lane_of(w.far, kAfterLane + 1) << 32 | lane_of(w.far, kAfterLane)
+                 : h.base;
+    slot = A.table ? lane_of(w.far, kSlotLane) : kNoSlot;
+  }
+  load_hdr(A, w, off, slot);
+}
+
+// The walk at the block's first step (num_major_stages > 0), whose prologue
+// is loaded.
+__device__ __forceinline__ void start_walk(const ScanArgs &A, u32 cycles, Walk &w, PartPre &P) {
+  w.c = w.m = 0;
+  w.have = true;
+  load_hdr(A, w, uniform64(A.blocks_start[blockIdx.x]),
+           A.table ? uniform(A.slots[blockIdx.x]) : kNoSlot);
+  w.cur = settle(w);
+  const Section s = section_of(A.blocks_data, w.cur), q = perm0(A.table, w.cur, s);
+  load_entries(P, s, w.cur.rounds);
+  load_stage(P, q, perm0_at(w.cur), s, stage0(w.cur));
+  P.hi = load_hi(q, w.cur);
+  fetch_step(A, cycles, w, w.cur);
+  wait_loads();
+}
+
 // One partition (src/sim/cpu_reference.rs:25-262 per partition;
 // kernel_v1_impl.cuh:62-558), its prologue loads already in P; `hn` is the
 // block's next partition (num_stages 0: none), whose prologue replaces them.
 template <bool TIMING, bool PROFILE, bool FLOW>
 __device__ __forceinline__ void run_partition(const ScanArgs &A, const u32 *__restrict__ bd,
-                              const PartHdr &h, const PartHdr &hn, PartPre &P,
+                              Walk &wk, u32 cycles, PartPre &P,
                               const Flow &F, const u32 *__restrict__ in,
                               u32 *__restrict__ out,
                               u32 cycle, u32 part, u32 *st_v, u32 *st_x,
                               u32 *hin_v, u32 *hin_x, u32 *wo_v, u32 *wo_x,
-                              u16 *st_arr, u16 *wo_arr) {
+                              u16 *st_arr, u16 *wo_arr, u32 *raw_v, u32 *raw_x) {
   const int lane = threadIdx.x & 63;
   const bool w0 = threadIdx.x < 64;
   // the thread's word, and its first thread
   const int t = threadIdx.x >> 1;
   const bool h0 = (threadIdx.x & 1) == 0;
-  const u32 *pq = bd + 2048 * (threadIdx.x & 1) + 4 * t;  // its permutation words
+  const u32 pq = 2048 * (threadIdx.x & 1) + 4 * t;  // its permutation words
   long long t_start = 0;
   if (PROFILE) t_start = clock64();
-  const u32 num_stages = h.num_stages;
-  const u32 num_ios = h.num_ios;
+  const PartHdr &h = wk.cur, &hn = wk.next;
+  // a step without a partition runs as one of no words: zeros are permuted
+  // and no output is written, while the next one's words arrive
+  const u32 num_stages = h.num_stages ? h.num_stages : 1;
+  const u32 num_ios = h.num_stages ? h.num_ios : 0;
   const u32 io_offset = h.io_offset;
   const u32 num_srams = h.num_srams;
   const u32 sram_offset = h.sram_offset;
-  const u32 rounds = h.rounds;
+  const u32 rounds = h.num_stages ? h.rounds : 0;
   const u32 num_dups = h.num_dups;
-  const bool is_x = h.is_x;
+  const bool is_x = h.is_x != 0;
   const u32 xoff = h.xoff;
-  const u32 hook = h.hook;
-  const u32 *script = bd + h.base;
-  const uint2 *gr = reinterpret_cast<const uint2 *>(script + 256);
+  const u32 hook = (threadIdx.x & 2) ? P.hook >> 16 : P.hook & 0xffffu;
+  const bool comp = !PROFILE && h.slot != kNoSlot && h.num_stages != 0;
+  const Section S = section_of(bd, h), Sn = section_of(bd, hn);
+  const uint2 *gr = reinterpret_cast<const uint2 *>(bd + h.base + 256);
   const uint2 *e = P.e;
-  const u32 *p_st = stage0(bd, h);                        // this stage's section
-  const u32 *p_sd = p_st + (size_t)5120 * num_stages;     // SRAM/dup section
-  const u32 *p_ck = p_sd + 5120;                          // clock-enable section
-  const u32 nperm = num_srams * 4 + num_dups;
+  u32 st = stage0(h);                        // this stage's section
+  const u32 sd = st + 5120 * h.num_stages;     // SRAM/dup section
+  const u32 ck = sd + 5120;                  // clock-enable section
+  const u32 nperm = h.num_stages ? num_srams * 4 + num_dups : 0;
   uint4 sda, sdb, sdf, cka, ckb, ckf;
-  u32 old_v = 0, old_x = 0;
+  u32 old_v, old_x;
 
     // ---- global read (pext-gather), kernel_v1_impl.cuh:87-151
     u32 acc_v = 0, acc_x = 0, bits = 0;
     {
-      u32 v[kPreRounds], x[kPreRounds];
-      if (FLOW) {
-        if (is_x)
-          flow_gather<true>(F, e, in, out, cycle, v, x);
-        else
-          flow_gather<false>(F, e, in, out, cycle, v, x);
-      } else {
-#pragma unroll
-        for (u32 k = 0; k < kPreRounds; ++k) {
-          v[k] = 0;
-          x[k] = 0;
-          if (e[k].y) {
-            const u32 *base = (e[k].x >> 31) ? out : in;
-            u32 w = e[k].x & 0x7fffffffu;
-            v[k] = ld_coherent(base + w);
-            if (is_x) x[k] = ld_coherent(base + xoff + w);
-          }
-        }
-      }
+      u32 v[kPreRounds] = {}, x[kPreRounds] = {};
+      const u32 most = (rounds + 1) / 2;
+      const auto fetch = [&] { fetch_step(A, cycles, wk, hn); };
+      if (most <= 2)
+        gather<2, FLOW>(F, e, in, out, cycle, is_x, xoff, v, x, fetch);
+      else if (most <= 4)
+        gather<4, FLOW>(F, e, in, out, cycle, is_x, xoff, v, x, fetch);
+      else
+        gather<kPreRounds, FLOW>(F, e, in, out, cycle, is_x, xoff, v, x, fetch);
       // the writeout sections and the old values, used after the stages
-      if (nperm) {
-        sda = ld4(pq + (p_sd - bd));
-        sdb = ld4(pq + (p_sd - bd) + 1024);
-        sdf = ld4(p_sd + 4096 + 4 * t);
+      if ((u32)t < nperm) {
+        sda = ld4(S, true, sd + pq);
+        sdb = ld4(S, true, sd + pq + 1024);
+        sdf = ld4(S, true, sd + 4096 + 4 * t);
       }
-      cka = ld4(pq + (p_ck - bd));
-      ckb = ld4(pq + (p_ck - bd) + 1024);
-      ckf = ld4(p_ck + 4096 + 4 * t);
-      if (h0 && (u32)t < num_ios) {
+      if ((u32)t < num_ios) {
+        cka = ld4(S, true, ck + pq);
+        ckb = ld4(S, true, ck + pq + 1024);
+        ckf = ld4(S, true, ck + 4096 + 4 * t);
         // under dataflow a word of the snapshot buffer is stored and read
         // back by the same thread only (and a word without X lane keeps the
         // mask the host put there)
         const u32 w = io_offset + (u32)t;
         if (FLOW) {
+          const u32 *m = is_x ? in + xoff : F.xoff ? out + F.xoff : in;
           old_v = in[w];
-          if (is_x)
-            old_x = in[xoff + w];
-          else if (F.xoff)
-            old_x = out[F.xoff + w];
+          old_x = m[w];
         } else {
           old_v = ld_coherent(in + w);
-          if (is_x) old_x = ld_coherent(in + xoff + w);
+          old_x = ld_coherent((is_x ? in + xoff : in) + w);
         }
       }
-      // pext, lowest mask bit first into the accumulator (kernel_v1_impl.cuh:
-      // 112-119): one ctz, one bit-field extract and one shift-or per bit;
-      // the X lane's work only in X-capable partitions
-      if (is_x) {
+      if (comp) {
+        const u32 n = num_rounds(rounds);
+        u32 *rv = raw_v + 1 + 256 * first_round(rounds) + t;
+        u32 *rx = raw_x + 1 + 256 * first_round(rounds) + t;
+#pragma unroll
+        for (u32 k = 0; k < kPreRounds; ++k) {
+          if (k >= most) break;
+          if (k < n) {
+            rv[256 * k] = v[k];
+            if (is_x) rx[256 * k] = x[k];
+          }
+        }
+      } else if (is_x) {
+        // pext, lowest mask bit first into the accumulator (kernel_v1_impl.cuh:
+        // 112-119): one ctz, one bit-field extract and one shift-or per bit;
+        // the X lane's work only in X-capable partitions
 #pragma unroll
         for (u32 k = 0; k < kPreRounds; ++k)
-          for (u32 m = e[k].y; m; m &= m - 1) {
+          for (u32 m = k < most ? e[k].y : 0; m; m &= m - 1) {
             const u32 p = __builtin_ctz(m);
             acc_v = (acc_v << 1) | ((v[k] >> p) & 1u);
             acc_x = (acc_x << 1) | ((x[k] >> p) & 1u);
@@ -534,11 +861,12 @@ __device__ __forceinline__ void run_partition(const ScanArgs &A, const u32 *__re
       } else {
 #pragma unroll
         for (u32 k = 0; k < kPreRounds; ++k)
-          for (u32 m = e[k].y; m; m &= m - 1)
+          for (u32 m = k < most ? e[k].y : 0; m; m &= m - 1)
             acc_v = (acc_v << 1) | ((v[k] >> __builtin_ctz(m)) & 1u);
       }
+      if (!comp)
 #pragma unroll
-      for (u32 k = 0; k < kPreRounds; ++k) bits += __builtin_popcount(e[k].y);
+        for (u32 k = 0; k < kPreRounds; ++k) bits += k < most ? __builtin_popcount(e[k].y) : 0;
     }
     for (u32 r = kPreRounds; r < num_rounds(rounds); ++r) {  // rare: very wide reads
       uint2 er = gr[256 * (first_round(rounds) + r) + t];
@@ -552,39 +880,60 @@ __device__ __forceinline__ void run_partition(const ScanArgs &A, const u32 *__re
         v = ld_coherent(base + w);
         if (is_x) x = ld_coherent(base + xoff + w);
       }
-      for (u32 m = er.y; m; m &= m - 1) {
-        const u32 p = __builtin_ctz(m);
-        acc_v = (acc_v << 1) | ((v >> p) & 1u);
-        acc_x = (acc_x << 1) | ((x >> p) & 1u);
+      if (comp) {
+        const u32 i = 1 + 256 * (first_round(rounds) + r) + t;
+        raw_v[i] = v;
+        if (is_x) raw_x[i] = x;
+      } else {
+        for (u32 m = er.y; m; m &= m - 1) {
+          const u32 p = __builtin_ctz(m);
+          acc_v = (acc_v << 1) | ((v >> p) & 1u);
+          acc_x = (acc_x << 1) | ((x >> p) & 1u);
+        }
+        bits += __builtin_popcount(er.y);
       }
-      bits += __builtin_popcount(er.y);
+      wait_loads();
     }
     // half 1's bits follow half 0's
-    {
+    if (!comp) {
       const u32 nb1 = from_pair(bits);
       const u32 hi_v = from_pair(acc_v), hi_x = from_pair(acc_x);
       acc_v = (nb1 < 32 ? acc_v << nb1 : 0u) | hi_v;  // half 0's result is kept
       acc_x = (nb1 < 32 ? acc_x << nb1 : 0u) | hi_x;
     }
-    const bool next = hn.num_stages != 0;
-    if (next) load_entries(P, bd, hn);
+    load_entries(P, Sn, hn.rounds);
     if (h0) {
-      st_v[t] = acc_v;
-      st_x[t] = acc_x;
+      if (!comp) {
+        st_v[t] = acc_v;
+        st_x[t] = acc_x;
+      }
       if (TIMING) wo_arr[t] = 0;  // pinned rule: reset per partition
     }
     __syncthreads();
 
     // ---- boomerang stages
     for (u32 bs = 0; bs < num_stages; ++bs) {
-      const u32 hv = gather_bits(st_v, P.qa, P.qb);
-      const u32 hx = is_x ? gather_bits(st_x, P.qa, P.qb) : 0u;
+      u32 hv, hx = 0;
+      if (bs != 0 || !comp) {
+        hv = gather_bits(st_v, P.qa, P.qb);
+        if (is_x) hx = gather_bits(st_x, P.qa, P.qb);
+      } else if (rounds <= kNarrowRounds) {
+        hv = gather_bits_of<false>(raw_v, P.qa, P.qb, 0);
+        if (is_x) hx = gather_bits_of<false>(raw_x, P.qa, P.qb, 0);
+      } else {
+        hv = gather_bits_of<true>(raw_v, P.qa, P.qb, P.hi);
+        if (is_x) hx = gather_bits_of<true>(raw_x, P.qa, P.qb, P.hi);
+      }
       // the next section (the next stage's, or the first of the next
       // partition) is loaded now, a stage ahead of its use; this one's came
       // with the previous stage
       const uint4 fA = P.fA, fB = P.fB, fC = P.fC, fD = P.fD;
-      p_st = bs + 1 < num_stages ? p_st + 5120 : stage0(bd, hn);
-      if (bs + 1 < num_stages || next) load_stage(P, p_st);
+      st += 5120;
+      const bool more = bs + 1 < num_stages;
+      const Section pn = perm0(A.table, hn, Sn);
+      load_stage(P, more ? S : pn, more ? st : perm0_at(hn), more ? S : Sn,
+                 more ? st : stage0(hn));
+      if (!more) P.hi = load_hi(pn, hn);
       if (h0) {
         hin_v[t] = hv;
         hin_x[t] = hx;
@@ -666,6 +1015,8 @@ __device__ __forceinline__ void run_partition(const ScanArgs &A, const u32 *__re
         if (TIMING) wo_arr[t] = st_arr[hook & 255];
       }
     }
+    // everything requested so far has had the stages to arrive
+    wait_loads();
     __syncthreads();
 
     // ---- SRAM + duplicate permutation, kernel_v1_impl.cuh:365-443
@@ -674,6 +1025,7 @@ __device__ __forceinline__ void run_partition(const ScanArgs &A, const u32 *__re
     if (nperm) {
       u32 pv = 0, px = 0;
       if ((u32)t < nperm) {
+        asm volatile("" : "+v"(sdf.y));  // its inverse is not taken at the load
         pv = (gather_bits(wo_v, sda, sdb) & ~sdf.y) ^ sdf.x;
         if (is_x) px = gather_bits(wo_x, sda, sdb) & ~sdf.y;
       }
@@ -715,23 +1067,23 @@ __device__ __forceinline__ void run_partition(const ScanArgs &A, const u32 *__re
       const uint4 f = ckf;
       if ((u32)t < num_ios) {
         // a word whose clock-enable bits are all forced (set0 all ones,
-        // every combinational writeout) needs no gather: ck = inv, ckx = 0;
+        // every combinational writeout) needs no gather: en = inv, ckx = 0;
         // only words holding DFFs pay for the 32 LDS reads
         const bool gated = f.y != 0xFFFFFFFFu;
-        u32 ck = f.x;
-        if (gated) ck = (gather_bits(wo_v, cka, ckb) & ~f.y) ^ f.x;
+        u32 en = f.x;
+        if (gated) en = (gather_bits(wo_v, cka, ckb) & ~f.y) ^ f.x;
         u32 ckx = 0;
         if (is_x && gated) ckx = gather_bits(wo_x, cka, ckb) & ~f.y;
         if (h0) {
           u32 data = wo_v[t] ^ f.z;
           u32 w = io_offset + (u32)t;
-          const u32 nv = (old_v & ~ck) | (data & ck);
+          const u32 nv = (old_v & ~en) | (data & en);
           u32 nx = old_x;
-          if (is_x) nx = (old_x & ~ck & ~ckx) | (wo_x[t] & ck & ~ckx) | ckx;
+          if (is_x) nx = (old_x & ~en & ~ckx) | (wo_x[t] & en & ~ckx) | ckx;
           if (FLOW) {
             const u32 s = cycle + 1;
             const u64 tag = (u64)s << 32;
-            u64 *a = F.ring + ((s & (kRing - 1)) * F.slot + w);
+            u64 *a = F.slots + ((size_t)(s & (kRing - 1)) * F.slot + w);
             st_coherent64(a, tag | nv);
             if (F.xoff) st_coherent64(a + F.xoff, tag | nx);
             out[w] = nv;
@@ -744,7 +1096,7 @@ __device__ __forceinline__ void run_partition(const ScanArgs &A, const u32 *__re
             u16 arr = wo_arr[t];
             if (A.arrival_state_offset != 0)
               st_coherent(out + (u32)A.arrival_state_offset + w, (u32)arr);
-            if (ck != 0 && A.constraints) {
+            if (en != 0 && A.constraints) {
               u32 cons = A.constraints[w];
               if (cons != 0) {
                 u32 setup = cons >> 16, hold = cons & 0xffffu;
@@ -760,12 +1112,15 @@ __device__ __forceinline__ void run_partition(const ScanArgs &A, const u32 *__re
         }
       }
     }
+    // no barrier: what the next partition writes to LDS ahead of its first one
+    // was last read ahead of this one's last, or is the writing thread's own
     if (PROFILE) {
       __syncthreads();
-      if (threadIdx.x == 0 && cycle < A.sample_cycles && part < A.num_parts)
+      if (threadIdx.x == 0 && h.num_stages && cycle < A.sample_cycles &&
+          part < A.num_parts)
         A.samples[(size_t)cycle * A.num_parts + part] = (u32)(clock64() - t_start);
+      __syncthreads();
     }
-    __syncthreads();
 }
 
 // ---- what a dataflow launch needs to know about its script
@@ -779,9 +1134,17 @@ struct FlowBuild {
   u32 *flow;   // kFlow* words
 };
 
-__global__ __launch_bounds__(256) void flow_zero_kernel(uint4 *p, usize n) {
-  for (usize i = (usize)blockIdx.x * 256u + threadIdx.x; i < n; i += (usize)gridDim.x * 256u)
-    p[i] = make_uint4(0, 0, 0, 0);
+// Zeroes n units of 16 bytes but for the first `words` words of 8 bytes, which
+// are the ring's slot 0: snapshot 0 with its number.
+__global__ __launch_bounds__(256) void flow_zero_kernel(uint4 *p, usize n, const u32 *states,
+                                                        usize words) {
+  const usize first = (usize)blockIdx.x * 256u + threadIdx.x, step = (usize)gridDim.x * 256u;
+  for (usize i = first; i < n; i += step) {
+    uint4 v = make_uint4(0, 0, 0, 0);
+    if (2 * i < words) v.x = states[2 * i];
+    if (2 * i + 1 < words) v.z = states[2 * i + 1];
+    p[i] = v;
+  }
 }
 
 // Raises *p to v.  Most workgroups find it there already, so the word is
@@ -849,90 +1212,28 @@ __global__ __launch_bounds__(256) void flow_check_kernel(FlowBuild F) {
   if (bad) atomicOr(&F.flow[kFlowBad], bad);
 }
 
-// A block's partitions in execution order: cycle, major stage, then
-// position in the stage's section of blocks_data (kernel_v1_impl.cuh:
-// 565-626).  A stage without partitions is one step with an empty header.
-// `next` is the step after the one that runs; the header of the one after
-// that is in flight, and so is the section start it may need.
-struct Walk {
-  PartHdr cur, next;
-  RawHdr raw;
-  bool have;     // raw is a step of the launch
-  u32 c, m;      // of raw
-  usize after;   // blocks_start of the stage that follows raw's
-};
-
-__device__ __forceinline__ usize section(const ScanArgs &A, u32 m) {
-  const u32 k = m + 1 == A.num_major_stages ? 0 : m + 1;
-  return A.blocks_start[(size_t)k * A.num_blocks + blockIdx.x];
-}
-
-__device__ __forceinline__ usize uniform64(usize v) {
-  return (usize)uniform((u32)(v >> 32)) << 32 | uniform((u32)v);
-}
-
-// Requests the header of the step after h (the one raw held).
-__device__ __forceinline__ void fetch_step(const ScanArgs &A, const u32 *bd, u32 cycles,
-                                           Walk &w, const PartHdr &h) {
-  if (h.num_stages != 0 && h.is_last == 0) {
-    w.raw = load_hdr(bd, h.base + part_words(h));
-    return;
-  }
-  if (++w.m == A.num_major_stages) {
-    w.m = 0;
-    ++w.c;
-  }
-  w.have = w.c < cycles;
-  if (!w.have) return;
-  w.raw = load_hdr(bd, uniform64(w.after));
-  w.after = section(A, w.m);
-}
-
-// The walk at the block's first step (num_major_stages > 0).
-__device__ __forceinline__ void start_walk(const ScanArgs &A, const u32 *bd, u32 cycles, Walk &w,
-                                           PartPre &P) {
-  w.c = w.m = 0;
-  w.have = true;
-  w.raw = load_hdr(bd, A.blocks_start[blockIdx.x]);
-  w.after = section(A, 0);
-  w.cur = settle(w.raw);
-  fetch_step(A, bd, cycles, w, w.cur);
-  if (w.cur.num_stages) {
-    load_entries(P, bd, w.cur);
-    load_stage(P, stage0(bd, w.cur));
-  }
-}
-
-// Before the step that runs: the header requested during the last one
-// becomes `next`, and the one after it is requested.
-__device__ __forceinline__ void peek_step(const ScanArgs &A, const u32 *bd, u32 cycles, Walk &w) {
-  if (!w.have) {
-    w.next = no_hdr();
-    return;
-  }
-  w.next = settle(w.raw);
-  fetch_step(A, bd, cycles, w, w.next);
-}
-
 // The LDS arrays of one workgroup.
 #define JQ_SCAN_LDS                                             \
   __shared__ u32 st_v[256], st_x[256], hin_v[256], hin_x[256]; \
   __shared__ u32 wo_v[256], wo_x[256];                          \
   __shared__ u16 st_arr[256], wo_arr[256];                      \
+  __shared__ u32 raw_v[kRawWords], raw_x[kRawWords];            \
   __shared__ u32 s_aborted; /* set by a wait when the launch has aborted */
 
 template <bool TIMING, bool PROFILE, bool FLOW>
 __device__ __forceinline__ void scan_loop(const ScanArgs &A, u32 *st_v, u32 *st_x, u32 *hin_v,
                                           u32 *hin_x, u32 *wo_v, u32 *wo_x, u16 *st_arr,
-                                          u16 *wo_arr, u32 &s_aborted, u32 gen) {
+                                          u16 *wo_arr, u32 *raw_v, u32 *raw_x,
+                                          u32 &s_aborted, u32 gen) {
   const u32 b = blockIdx.x;
   const u32 nb = A.num_blocks, M = A.num_major_stages;
   const u32 *bd = A.blocks_data;
   if (M == 0) return;
   Flow F{};
   if (FLOW) {
-    F.ring = A.ring;
+    F.slots = A.ring;
     F.slot = (u32)A.state_size;
+    F.ring = __builtin_amdgcn_make_buffer_rsrc(A.ring, 0, 8 * kRing * F.slot, 0x00027000);
     F.lo = ~A.flow[kFlowNegLo];
     F.xoff = A.flow[kFlowXoff];
     F.bar = A.bar;
@@ -940,42 +1241,41 @@ __device__ __forceinline__ void scan_loop(const ScanArgs &A, u32 *st_v, u32 *st_
   }
   Walk w{};
   PartPre P{};
-  start_walk(A, bd, A.num_cycles, w, P);
-  for (u32 c = 0; c < A.num_cycles; ++c) {
-    // an aborted launch (a bounded wait gave up; the waits that follow end
-    // within 256 polls each) leaves at the next cycle
-    if (s_aborted) return;
-    if (FLOW && nb > 1 && c != 0 && c % (kRing / 2) == 0) {
-      flow_room(F, A.prog, nb, c);
-      __syncthreads();
-    }
-    const u32 *in = A.states + (size_t)c * A.state_size;
-    u32 *out = A.states + (size_t)(c + 1) * A.state_size;
-    for (u32 m = 0; m < M; ++m) {
-      u32 part = PROFILE ? A.part_index[(size_t)m * nb + b] : 0u;
-      for (;;) {
-        const bool last = w.cur.num_stages == 0 || w.cur.is_last != 0;
-        peek_step(A, bd, A.num_cycles, w);
-        if (w.cur.num_stages) {
-          run_partition<TIMING, PROFILE, FLOW>(A, bd, w.cur, w.next, P, F, in, out, c, part,
-                                               st_v, st_x, hin_v, hin_x, wo_v, wo_x, st_arr,
-                                               wo_arr);
-          ++part;
-        } else if (w.next.num_stages) {
-          load_entries(P, bd, w.next);
-          load_stage(P, stage0(bd, w.next));
-        }
-        w.cur = w.next;
-        if (last) break;
+  start_walk(A, A.num_cycles, w, P);
+  const u32 *in = A.states;
+  u32 *out = A.states + A.state_size;
+  u32 part = PROFILE ? A.part_index[b] : 0u;
+  // one loop over the block's steps, whose registers stay where they are
+  for (u32 c = 0, m = 0;;) {
+    const bool last = w.cur.num_stages == 0 || w.cur.is_last != 0;
+    w.next = settle(w);
+    run_partition<TIMING, PROFILE, FLOW>(A, bd, w, A.num_cycles, P, F, in, out, c, part, st_v,
+                                         st_x, hin_v, hin_x, wo_v, wo_x, st_arr, wo_arr, raw_v,
+                                         raw_x);
+    ++part;
+    w.cur = w.next;
+    if (!last) continue;
+    if (!FLOW) grid_sync_coherent(A.bar, nb, b, gen, &g_error, &g_wait_polls, s_aborted);
+    if (++m == M) {
+      m = 0;
+      ++c;
+      if (FLOW) {
+        // behind this barrier no wave reads a snapshot of the last cycle any
+        // more
+        __syncthreads();
+        if (nb > 1 && threadIdx.x == 0) st_coherent(&A.prog[b * kProgStride], c);
       }
-      if (!FLOW) grid_sync_coherent(A.bar, nb, b, gen, &g_error, &g_wait_polls, s_aborted);
+      // an aborted launch (a bounded wait gave up; the waits that follow end
+      // within 256 polls each) leaves at the next cycle
+      if (c == A.num_cycles || s_aborted) return;
+      if (FLOW && nb > 1 && c % (kRing / 2) == 0) {
+        flow_room(F, A.prog, nb, c);
+        __syncthreads();
+      }
+      in = out;
+      out += A.state_size;
     }
-    if (FLOW) {
-      // the last partition's closing workgroup barrier is behind every wave:
-      // none of them reads a snapshot of this cycle any more
-      __syncthreads();
-      if (nb > 1 && threadIdx.x == 0) st_coherent(&A.prog[b * kProgStride], c + 1);
-    }
+    if (PROFILE) part = A.part_index[(size_t)m * nb + b];
   }
 }
 
@@ -987,7 +1287,7 @@ __global__ __launch_bounds__(kScanThreads) void scan_kernel(ScanArgs A) {
   }
   JQ_SCAN_LDS
   const int t = threadIdx.x;
-  if (t == 0) s_aborted = 0;
+  if (t == 0) s_aborted = raw_v[0] = raw_x[0] = 0;
   if (t < 256) {
     st_x[t] = 0;
     hin_x[t] = 0;
@@ -1000,10 +1300,11 @@ __global__ __launch_bounds__(kScanThreads) void scan_kernel(ScanArgs A) {
   // the flag is the same word for every block
   if (!TIMING && !PROFILE && A.ring != nullptr && A.flow[kFlowBad] == 0)
     scan_loop<TIMING, PROFILE, !TIMING && !PROFILE>(A, st_v, st_x, hin_v, hin_x, wo_v, wo_x,
-                                                    st_arr, wo_arr, s_aborted, gen);
+                                                    st_arr, wo_arr, raw_v, raw_x, s_aborted,
+                                                    gen);
   else
     scan_loop<TIMING, PROFILE, false>(A, st_v, st_x, hin_v, hin_x, wo_v, wo_x, st_arr, wo_arr,
-                                      s_aborted, gen);
+                                      raw_v, raw_x, s_aborted, gen);
 }
 
 // Persistent co-simulation: C.num_edges edges of one cycle each over the
@@ -1024,7 +1325,7 @@ __global__ __launch_bounds__(kScanThreads, WAVES) void cosim_kernel(ScanArgs A, 
   }
   JQ_SCAN_LDS
   const int t = threadIdx.x;
-  if (t == 0) s_aborted = 0;
+  if (t == 0) s_aborted = raw_v[0] = raw_x[0] = 0;
   if (t < 256) {
     st_x[t] = 0;
     hin_x[t] = 0;
@@ -1042,32 +1343,26 @@ __global__ __launch_bounds__(kScanThreads, WAVES) void cosim_kernel(ScanArgs A, 
   const Flow F{};
   Walk w{};
   PartPre P{};
-  if (M) start_walk(A, bd, C.num_edges, w, P);
+  if (M) start_walk(A, C.num_edges, w, P);
   for (u32 e = 0; e <= C.num_edges; ++e) {
     // an aborted launch (a bounded wait gave up) leaves at the next edge
     if (s_aborted) return;
     cosim::between_phase(C, (u32)t, b, nb, e);
     if (e == C.num_edges) break;
     grid_sync_coherent(A.bar, nb, b, gen, &g_error, &g_wait_polls, s_aborted);
-    for (u32 m = 0; m < M; ++m) {
-      for (;;) {
-        const bool last = w.cur.num_stages == 0 || w.cur.is_last != 0;
-        peek_step(A, bd, C.num_edges, w);
-        if (w.cur.num_stages) {
-          // co-simulation snapshots are 2-state: a partition flagged
-          // X-capable runs its value lane only
-          w.cur.is_x = false;
-          run_partition<TIMING, false, false>(A, bd, w.cur, w.next, P, F, in, out, 0u, 0u,
-                                              st_v, st_x, hin_v, hin_x, wo_v, wo_x, st_arr,
-                                              wo_arr);
-        } else if (w.next.num_stages) {
-          load_entries(P, bd, w.next);
-          load_stage(P, stage0(bd, w.next));
-        }
-        w.cur = w.next;
-        if (last) break;
-      }
+    for (u32 m = 0; m < M;) {
+      const bool last = w.cur.num_stages == 0 || w.cur.is_last != 0;
+      w.next = settle(w);
+      // co-simulation snapshots are 2-state: a partition flagged X-capable
+      // runs its value lane only
+      w.cur.is_x = 0;
+      run_partition<TIMING, false, false>(A, bd, w, C.num_edges, P, F, in, out, 0u, 0u, st_v,
+                                          st_x, hin_v, hin_x, wo_v, wo_x, st_arr, wo_arr, raw_v,
+                                          raw_x);
+      w.cur = w.next;
+      if (!last) continue;
       grid_sync_coherent(A.bar, nb, b, gen, &g_error, &g_wait_polls, s_aborted);
+      ++m;
     }
   }
 }
@@ -1126,25 +1421,35 @@ int launch_scan(ScanArgs &A, hipStream_t stream) {
   return 0;
 }
 
-// Prepares a value-only launch for dataflow on `stream` ahead of it and
-// returns its stream-ordered allocation (the exchange ring, the builders'
-// words and the progress words, freed after the launch), or null when the
-// launch runs with grid barriers: the mode is off, the script is outside
-// the builders' packing, the launch is shorter than kFlowMinCycles (the
-// builders' time is then comparable to the barriers they save), the stream
-// is being captured into a graph (no allocation or builder kernels go into
-// the caller's graph), or the allocation failed.  A script that the
-// builders find unusable (a writeout word written twice or out of range, a
-// read of a word past the first writeout word that no partition writes, a
-// same-cycle read of a word not written in an earlier stage) raises the
-// flag that the kernel reads, and the launch then uses grid barriers as
-// well.
-void *build_flow(ScanArgs &A, hipStream_t stream) {
+// Prepares a launch of `cycles` cycles on `stream` ahead of it and returns
+// its stream-ordered allocation, to be freed after the launch, or null when
+// there is nothing prepared: the script is outside the builders' packing, the
+// launch is shorter than kFlowMinCycles (the builders' time is then
+// comparable to what they save), the stream is being captured into a graph
+// (no allocation or builder kernels go into the caller's graph), or the
+// allocation failed.
+//
+// `flow`: the launch may synchronise by dataflow (exchange ring, progress
+// words; value-only, and the mode is on).  A script that the builders find
+// unusable for it (a writeout word written twice or out of range, a read of a
+// word past the first writeout word that no partition writes, a same-cycle
+// read of a word not written in an earlier stage) raises the flag that the
+// kernel reads, and the launch then uses grid barriers.
+//
+// Every prepared launch has the composed permutations, with slots for one
+// partition per block and major stage (what a script as wide as its widest
+// stage holds) or up to eight of a narrower one's, in at most kPrepareBytes
+// altogether: a stream-ordered allocation of 64 MiB takes and returns in 60
+// us, one of 66 MiB takes 370.  Where the memory is not to be had the launch
+// does without them.
+constexpr size_t kPrepareBytes = (size_t)64 << 20;
+
+void *prepare(ScanArgs &A, u32 cycles, bool flow, hipStream_t stream) {
   A.ring = nullptr;
+  A.table = nullptr;
   const u32 nb = A.num_blocks, M = A.num_major_stages;
-  if (!__atomic_load_n(&g_scan_sync, __ATOMIC_RELAXED) || M == 0 || M > 65534u ||
-      A.num_cycles < kFlowMinCycles || A.state_size == 0 ||
-      A.state_size > (usize(1) << 28) || (usize)nb * M > 0x7fffffffu)
+  flow = flow && M <= 65534u && A.state_size <= (usize(1) << 25);
+  if (M == 0 || cycles < kFlowMinCycles || A.state_size == 0 || (usize)nb * M > 0x7fffffffu)
     return nullptr;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &cap) != hipSuccess) {
@@ -1152,34 +1457,66 @@ void *build_flow(ScanArgs &A, hipStream_t stream) {
     return nullptr;
   }
   if (cap != hipStreamCaptureStatusNone) return nullptr;
-  const size_t own = ((size_t)A.state_size + 63) & ~(size_t)63;  // whole 256-byte units
-  const size_t ring = 2 * kRing * own, prog = (size_t)nb * kProgStride;
-  const size_t words = ring + own + kFlowWords + prog;
+  const auto whole = [](size_t words) { return (words + 63) & ~(size_t)63; };  // 256-byte units
+  const size_t sections = (size_t)nb * M;
+  const size_t ring = flow ? 2 * kRing * whole(A.state_size) : 0;
+  const size_t own = flow ? whole(A.state_size) : 0;
+  const size_t prog = flow ? (size_t)nb * kProgStride : 0;
+  // zeroed: the ring, the owners, the builders' words, the progress words
+  const size_t zeroed = ring + own + kFlowWords + whole(prog);
+  const size_t before = zeroed + whole(sections), most = kPrepareBytes / 4;
+  const size_t num_slots =
+      std::min(std::max(sections, std::min<size_t>(8 * sections, 2048)),
+               before < most ? (most - before) / kSlotWords : 0);
   void *buf = nullptr;
-  if (hipMallocAsync(&buf, 4 * words, stream) != hipSuccess) {
+  bool table = num_slots != 0;
+  if (table && hipMallocAsync(&buf, 4 * (before + num_slots * kSlotWords), stream) != hipSuccess) {
+    (void)hipGetLastError();
+    table = false;
+  }
+  if (!table && (!flow || hipMallocAsync(&buf, 4 * zeroed, stream) != hipSuccess)) {
     (void)hipGetLastError();
     return nullptr;
   }
   u32 *p = static_cast<u32 *>(buf);
-  FlowBuild F{};
-  F.blocks_start = A.blocks_start;
-  F.bd = A.blocks_data;
-  F.nb = nb;
-  F.M = M;
-  F.state_size = A.state_size;
-  F.owner = p + ring;
-  F.flow = F.owner + own;
-  const u32 fill_blocks = (u32)std::min<size_t>(1024, (words / 4 + 255) / 256);
-  flow_zero_kernel<<<fill_blocks, 256, 0, stream>>>(reinterpret_cast<uint4 *>(buf), words / 4);
-  flow_owner_kernel<<<nb * M, 256, 0, stream>>>(F);
-  flow_check_kernel<<<nb * M, 256, 0, stream>>>(F);
+  u32 *builders = p + ring + own;
+  const u32 fill_blocks = (u32)std::min<size_t>(1024, (zeroed / 4 + 255) / 256);
+  flow_zero_kernel<<<fill_blocks, 256, 0, stream>>>(reinterpret_cast<uint4 *>(buf), zeroed / 4,
+                                                    A.states, flow ? A.state_size : 0);
+  if (flow) {
+    FlowBuild F{};
+    F.blocks_start = A.blocks_start;
+    F.bd = A.blocks_data;
+    F.nb = nb;
+    F.M = M;
+    F.state_size = A.state_size;
+    F.owner = p + ring;
+    F.flow = builders;
+    flow_owner_kernel<<<sections, 256, 0, stream>>>(F);
+    flow_check_kernel<<<sections, 256, 0, stream>>>(F);
+    A.ring = reinterpret_cast<u64 *>(buf);
+    A.flow = builders;
+    A.prog = builders + kFlowWords;
+  }
+  if (table) {
+    TableBuild T{};
+    T.blocks_start = A.blocks_start;
+    T.bd = A.blocks_data;
+    T.cap = (u32)num_slots;
+    T.cursor = builders + kTableCursor;
+    T.slots = p + zeroed;
+    T.table = T.slots + whole(sections);
+    compose_kernel<<<sections, 256, 0, stream>>>(T);
+    A.slots = T.slots;
+    A.table = T.table;
+  }
   if (hipGetLastError() != hipSuccess) {
     (void)hipFreeAsync(buf, stream);
+    A.ring = nullptr;
+    A.table = nullptr;
+    A.slots = reinterpret_cast<const u32 *>(A.blocks_start);
     return nullptr;
   }
-  A.ring = reinterpret_cast<u64 *>(buf);
-  A.flow = F.flow;
-  A.prog = F.flow + kFlowWords;
   return buf;
 }
 
@@ -1204,6 +1541,7 @@ int scan_common(usize num_blocks, usize num_major_stages, const usize *blocks_st
   A.num_cycles = (u32)num_cycles;
   A.state_size = state_size;
   A.states = states;
+  A.slots = reinterpret_cast<const u32 *>(blocks_start);
   A.events = reinterpret_cast<EvHdr *>(event_buffer);
   A.ev_cap = ev_cap;
   A.arrival_state_offset = arrival_state_offset;
@@ -1215,10 +1553,11 @@ int scan_common(usize num_blocks, usize num_major_stages, const usize *blocks_st
   A.sample_cycles = sample_cycles;
   const bool timing = A.timing != nullptr || arrival_state_offset != 0;
   if (samples) return launch_scan<false, true>(A, stream);
-  if (timing) return launch_scan<true, false>(A, stream);
-  void *flow_buf = build_flow(A, stream);
-  const int rc = launch_scan<false, false>(A, stream);
-  if (flow_buf) (void)hipFreeAsync(flow_buf, stream);
+  const bool flow = !timing && __atomic_load_n(&g_scan_sync, __ATOMIC_RELAXED);
+  void *buf = prepare(A, A.num_cycles, flow, stream);
+  const int rc =
+      timing ? launch_scan<true, false>(A, stream) : launch_scan<false, false>(A, stream);
+  if (buf) (void)hipFreeAsync(buf, stream);
   return rc;
 }
 
@@ -1381,6 +1720,7 @@ extern "C" int jq_cosim_edges(usize num_blocks, usize num_major_stages,
   A.num_cycles = 1;
   A.state_size = state_size;
   A.states = states;
+  A.slots = reinterpret_cast<const u32 *>(blocks_start);
   A.timing = timing_constraints;
   A.events = reinterpret_cast<EvHdr *>(event_buffer);
   A.ev_cap = event_capacity;
@@ -1422,8 +1762,10 @@ extern "C" int jq_cosim_edges(usize num_blocks, usize num_major_stages,
     return fail("CU count query failed");
   if (!timing && A.num_blocks > (u32)cus)
     k = reinterpret_cast<const void *>(&cosim_kernel<false, 4>);
+  void *buf = prepare(A, num_edges, false, (hipStream_t)stream);
   hipError_t e = hipLaunchCooperativeKernel(k, dim3(A.num_blocks), dim3(kScanThreads), args, 0,
                                             (hipStream_t)stream);
+  if (buf) (void)hipFreeAsync(buf, (hipStream_t)stream);
   if (e != hipSuccess) return fail(std::string("cosim launch failed: ") + hipGetErrorString(e));
   return 0;
 }

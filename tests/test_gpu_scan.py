@@ -505,3 +505,83 @@ def test_dataflow_over_many_laps_of_the_ring(blocks, xprop):
     out = sim.run_scan(s, st.copy(), cycles)
     assert np.array_equal(out["states"], ref)
     assert np.array_equal(out["sram"][:s.sram_storage_size], sram)
+
+
+class _SplitRounds:
+    """The script with every global-read mask split into masks of at most
+    `bits` bits, in the order the pext takes them, as more rounds of the same
+    words: what a partition computes stays the same."""
+
+    def __init__(self, script, bits):
+        self._s = script
+        bd = np.asarray(script.blocks_data, np.uint32)
+        starts = np.asarray(script.blocks_start, np.uint64)
+        pieces, new_starts, self.rounds = [], [0], set()
+        for k in range(len(starts) - 1):
+            pos, end = int(starts[k]), int(starts[k + 1])
+            while pos < end:
+                ns, last, R = int(bd[pos]), int(bd[pos + 1]), int(bd[pos + 6])
+                if ns == 0:
+                    pieces.append(bd[pos:end])
+                    break
+                gr = bd[pos + 256:pos + 256 + 512 * R].reshape(R, 256, 2)
+                split = [[] for _ in range(256)]
+                for r in range(R):
+                    for t in range(256):
+                        w, m = int(gr[r, t, 0]), int(gr[r, t, 1])
+                        while m:
+                            part = 0
+                            for _ in range(bits):
+                                part |= m & -m
+                                m &= m - 1
+                            split[t].append((w, part))
+                n = max(len(q) for q in split)
+                self.rounds.add(n)
+                new = np.zeros((n, 256, 2), np.uint32)
+                for t, q in enumerate(split):
+                    new[:len(q), t] = np.array(q, np.uint32).reshape(-1, 2)
+                head = bd[pos:pos + 256].copy()
+                head[6] = n
+                tail = pos + 256 + 512 * R
+                pos = tail + 5120 * (ns + 2)
+                pieces += [head, new.reshape(-1), bd[tail:pos]]
+                if last:
+                    pieces.append(bd[pos:end])
+                    break
+            new_starts.append(sum(len(p) for p in pieces))
+        pieces.append(bd[int(starts[-1]):])
+        self.blocks_data = np.concatenate(pieces)
+        self.blocks_start = np.array(new_starts, np.uint64)
+
+    def __getattr__(self, name):
+        return getattr(self._s, name)
+
+
+@pytest.mark.parametrize("blocks,xprop,bits,rounds", [
+    (24, False, 32, (1, 7)), (24, True, 2, (8, 16)), (24, False, 1, (17, 31)),
+    (1, False, 2, (8, 16)), (1, True, 1, (17, 31))])
+def test_composed_permutations(blocks, xprop, bits, rounds):
+    """Launches long enough to compose the first stage's permutations, over
+    partitions of few rounds, of more than 16-bit indexes reach and of more
+    than are prefetched (test_global_read_wider_than_prefetched_rounds has
+    some that are not composed), with a few partitions to a block and with
+    more in the one block than the table has slots; and a launch too short
+    for a table."""
+    nl, _ = design("laps", level_split=3, seed=23, gates=9000, depth=30, dffs=700,
+                   inputs=40, outputs=24, geometric_p=0.3, srams=2)
+    from jacquard_amd.script import Compiled
+    s = Compiled(nl, level_split=3, max_part_nodes=150).flatten(blocks, xprop=xprop)
+    w = _SplitRounds(s, bits)
+    _say("rounds", sorted(w.rounds), "partitions", s.num_parts, "stages", s.num_major_stages)
+    assert rounds[0] <= max(w.rounds) <= rounds[1]
+    if blocks == 1:
+        assert s.num_parts > 8 * s.num_major_stages
+    for cycles in (7, 20):
+        st = stimulus.build_states(s, cycles, seed=4, p=0.2)
+        ref = st.copy()
+        sram = np.zeros(s.sram_storage_size, np.uint32)
+        sram_x = np.full(s.sram_storage_size, 0xFFFFFFFF, np.uint32)
+        oracle.run(s, ref, cycles, sram=sram, sram_x=sram_x if xprop else None)
+        out = sim.run_scan(w, st.copy(), cycles, validate=False)
+        assert np.array_equal(out["states"], ref)
+        assert np.array_equal(out["sram"][:s.sram_storage_size], sram)
