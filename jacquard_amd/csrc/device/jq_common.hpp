@@ -114,6 +114,9 @@ __device__ __forceinline__ bool wait_gives_up(u32 *bar, u32 spins, u32 lim, u32 
 __device__ __forceinline__ void grid_arrive_wait(u32 *bar, u32 n, u32 member, u32 &gen,
                                                  u32 *err, const u32 *limit, u32 &aborted) {
   __syncthreads();
+  // a lone workgroup has nobody to wait for, and its waves' stores have
+  // completed: no round trip of the counter's atomic
+  if (n == 1) return;
   if (threadIdx.x == 0) {
     u32 *set = bar + 256 + ((gen + 1u) & 1u) * 2048;
     bool last = false;

@@ -93,9 +93,12 @@ struct CosimArgs {
 };
 
 // Bit access inside one snapshot of ss words; positions past its end read
-// as 0.
+// as 0 (from word 0: without a branch the loads of several bits are in flight
+// together, where each took a round trip of its own across the chip).
 __device__ __forceinline__ u32 bit_at(const u32 *s, u32 ss, u32 pos) {
-  return (pos >> 5) < ss ? (ld_coherent(s + (pos >> 5)) >> (pos & 31u)) & 1u : 0u;
+  const u32 w = pos >> 5;
+  const u32 v = ld_coherent(s + (w < ss ? w : 0)) >> (pos & 31u);
+  return w < ss ? v & 1u : 0u;
 }
 
 // A byte completed on the SPI bus (csrc/spiflash_model.cc:40-101; the Metal
@@ -171,12 +174,13 @@ __device__ void flash_eval(FlashState &f, u32 clk, u32 csn, u32 d_out, u32 &mode
 // system clock edge).  The reference evaluates twice, with the previous and
 // then the current data; the second evaluation sees no clock or chip-select
 // edge and changes nothing, so one evaluation is made here.
-__device__ FlashState flash_step(const CosimArgs &A, FlashState f) {
+__device__ FlashState flash_step(const CosimArgs &A, const u32 *pins, FlashState f) {
   const u32 *out = A.states + A.ss;
-  const u32 clk = bit_at(out, A.ss, A.pins[4]);
-  const u32 csn = bit_at(out, A.ss, A.pins[5]);
+  const u32 clk = bit_at(out, A.ss, pins[4]);
+  const u32 csn = bit_at(out, A.ss, pins[5]);
   u32 d_out = 0;
-  for (u32 i = 0; i < 4; ++i) d_out |= bit_at(out, A.ss, A.pins[6 + i]) << i;
+#pragma unroll
+  for (u32 i = 0; i < 4; ++i) d_out |= bit_at(out, A.ss, pins[6 + i]) << i;
   if (f.in_reset) {
     f.d_i = 0x0F;
     f.prev_clk = clk;
@@ -270,8 +274,11 @@ __device__ void io_step(const CosimArgs &A) {
     WbTraceChannel &c = *A.wbc;
     if ((ic && is) || (dc && ds) || flags != c.prev_flags) {
       u32 ia = 0, id = 0, da = 0;
+#pragma unroll 4
       for (u32 i = 0; i < kWbAdrBits; ++i) ia |= bit_at(out, A.ss, P.ibus_adr[i]) << i;
+#pragma unroll 4
       for (u32 i = 0; i < kWbDatBits; ++i) id |= bit_at(out, A.ss, P.ibus_rdata[i]) << i;
+#pragma unroll 4
       for (u32 i = 0; i < kWbAdrBits; ++i) da |= bit_at(out, A.ss, P.dbus_adr[i]) << i;
       if (c.write_head < c.capacity) {
         WbTraceEntry *e = reinterpret_cast<WbTraceEntry *>(&c + 1) + c.write_head;
@@ -284,31 +291,8 @@ __device__ void io_step(const CosimArgs &A) {
   }
 }
 
-// dst[i] = src[i] for i < n over one workgroup, src read agent-coherently
-// (dst written so when `coherent`), with kCopyBatch loads in flight per
-// thread before their stores.
-constexpr u32 kCopyBatch = 8;
-__device__ __forceinline__ void copy_words(u32 *dst, const u32 *src, u32 n, u32 t,
-                                           bool coherent) {
-  for (u32 base = t; base < n; base += blockDim.x * kCopyBatch) {
-    u32 v[kCopyBatch];
-#pragma unroll
-    for (u32 k = 0; k < kCopyBatch; ++k) {
-      const u32 i = base + blockDim.x * k;
-      v[k] = i < n ? ld_coherent(src + i) : 0u;
-    }
-#pragma unroll
-    for (u32 k = 0; k < kCopyBatch; ++k) {
-      const u32 i = base + blockDim.x * k;
-      if (i < n) {
-        if (coherent)
-          st_coherent(dst + i, v[k]);
-        else
-          dst[i] = v[k];
-      }
-    }
-  }
-}
+constexpr u32 kCopyBatch = 8;  // words of each snapshot in flight per thread
+constexpr u32 kNumPins = 11;
 
 // Between cycle e-1 and cycle e (e = 0: before the first cycle; e =
 // num_edges: after the last), in every workgroup b of nb.  The snapshot
@@ -324,17 +308,38 @@ __device__ __forceinline__ void copy_words(u32 *dst, const u32 *src, u32 n, u32 
 // caller's), so no workgroup reads a buffer that is being written.
 // Workgroup 0 also runs the UART decoders and the bus trace.  The caller
 // waits for the stores and meets the grid barrier afterwards.
-__device__ void between_phase(const CosimArgs &A, u32 t, u32 b, u32 nb, u32 e) {
-  const bool flash = A.fs != nullptr && A.pins[10] != 0;
+//
+// An edge of a small design is a chain of round trips across the chip, so
+// everything that this phase reads is requested at once, ahead of the first
+// wait: the thread's words of both snapshots, the flash's state and its pins'
+// words.  `pins` is the workgroup's copy of A.pins in LDS.  One edge of a
+// one-block design with a flash and a trace: 9.8 us with a round trip per pin
+// and an atomic per grid barrier, 7.2 without.
+__device__ __forceinline__ void between_phase(const CosimArgs &A, const u32 *pins, u32 t, u32 b,
+                                              u32 nb, u32 e) {
+  const bool flash = A.fs != nullptr && pins[10] != 0;
   const u32 chunk = (A.ss + nb - 1) / nb;
   const u32 lo = b * chunk < A.ss ? b * chunk : A.ss;
   const u32 hi = lo + chunk < A.ss ? lo + chunk : A.ss;
-  const bool last = e == A.num_edges;
+  const bool last = e == A.num_edges, trace = e > 0 && A.trace;
   auto owns = [&](u32 pos) { return (pos >> 5) >= lo && (pos >> 5) < hi; };
+  // the words of the snapshots from `base` on, of every blockDim.x-th
+  u32 vi[kCopyBatch], vo[kCopyBatch];
+  const auto load = [&](u32 base) {
+#pragma unroll
+    for (u32 k = 0; k < kCopyBatch; ++k) {
+      const u32 i = base + blockDim.x * k;
+      if (i < hi) {
+        vo[k] = ld_coherent(A.states + A.ss + i);
+        if (trace) vi[k] = ld_coherent(A.states + i);
+      }
+    }
+  };
+  load(lo + t);
   bool need_fs = false;
   u32 din = 0;  // the flash's d_i for this edge's input (thread 0)
   if (flash)
-    for (u32 i = 0; i < 4; ++i) need_fs |= owns(A.pins[i]);
+    for (u32 i = 0; i < 4; ++i) need_fs |= owns(pins[i]);
   if (t == 0) {
     if (b == 0 && e > 0) io_step(A);
     if (flash && (b == 0 || need_fs)) {
@@ -343,7 +348,7 @@ __device__ void between_phase(const CosimArgs &A, u32 t, u32 b, u32 nb, u32 e) {
         f = *A.fs;
         if (b == 0) store_fs(A.fsbuf, f);
       } else {
-        f = flash_step(A, load_fs(A.fsbuf + 12 * ((e - 1) & 1)));
+        f = flash_step(A, pins, load_fs(A.fsbuf + 12 * ((e - 1) & 1)));
         if (b == 0) {
           store_fs(A.fsbuf + 12 * (e & 1), f);
           if (last) *A.fs = f;
@@ -352,34 +357,27 @@ __device__ void between_phase(const CosimArgs &A, u32 t, u32 b, u32 nb, u32 e) {
       din = f.d_i;
     }
   }
-  if (e > 0 && A.trace) {
-    u32 *tr = A.trace + (size_t)(e - 1) * 2 * A.ss;
-    copy_words(tr + lo, A.states + lo, hi - lo, t, false);
-    copy_words(tr + A.ss + lo, A.states + A.ss + lo, hi - lo, t, false);
-  }
-  if (last) return;
   __shared__ u32 s_din;
   if (t == 0) s_din = din;
   __syncthreads();
   // state preparation (csrc/kernel_v1.metal:678-710, 896-918): the output
   // snapshot becomes the next input, with the edge's bit operations in order
   // and then the flash's data-in bits applied to each word on its way
-  // (kCopyBatch agent-coherent loads in flight per thread)
   const u32 pe = (u32)(((usize)A.sched_offset + e) % A.num_sched);
-  const u32 ob = A.op_start[pe], oe = A.op_start[pe + 1];
+  const u32 ob = last ? 0 : A.op_start[pe], oe = last ? 0 : A.op_start[pe + 1];
   const u32 dbits = s_din;
-  for (u32 base = lo + t; base < hi; base += blockDim.x * kCopyBatch) {
-    u32 v[kCopyBatch];
-#pragma unroll
-    for (u32 k = 0; k < kCopyBatch; ++k) {
-      const u32 i = base + blockDim.x * k;
-      v[k] = i < hi ? ld_coherent(A.states + A.ss + i) : 0u;
-    }
+  u32 *tr = A.trace + (e > 0 ? (size_t)(e - 1) * 2 * A.ss : 0);
+  for (u32 base = lo + t; base < hi;) {
 #pragma unroll
     for (u32 k = 0; k < kCopyBatch; ++k) {
       const u32 i = base + blockDim.x * k;
       if (i >= hi) continue;
-      u32 w = v[k];
+      u32 w = vo[k];
+      if (trace) {
+        tr[i] = vi[k];
+        tr[A.ss + i] = w;
+      }
+      if (last) continue;
       for (u32 j = ob; j < oe; ++j) {
         const u32 pos = A.ops[2 * j];
         if ((pos >> 5) == i) {
@@ -389,12 +387,14 @@ __device__ void between_phase(const CosimArgs &A, u32 t, u32 b, u32 nb, u32 e) {
       }
       if (flash)
         for (u32 q = 0; q < 4; ++q)
-          if ((A.pins[q] >> 5) == i) {
-            const u32 m = 1u << (A.pins[q] & 31u);
+          if ((pins[q] >> 5) == i) {
+            const u32 m = 1u << (pins[q] & 31u);
             w = (dbits >> q) & 1u ? (w | m) : (w & ~m);
           }
       st_coherent(A.states + i, w);
     }
+    base += blockDim.x * kCopyBatch;
+    if (base < hi) load(base);
   }
 }
 

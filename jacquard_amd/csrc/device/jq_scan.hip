@@ -1333,6 +1333,8 @@ __global__ __launch_bounds__(kScanThreads, WAVES) void cosim_kernel(ScanArgs A, 
     wo_arr[t] = 0;
     st_arr[t] = 0;
   }
+  __shared__ u32 pins[cosim::kNumPins];
+  if (C.fs && (u32)t < cosim::kNumPins) pins[t] = C.pins[t];
   u32 gen = read_gen(A.bar);
   __syncthreads();
   const u32 b = blockIdx.x;
@@ -1347,7 +1349,7 @@ __global__ __launch_bounds__(kScanThreads, WAVES) void cosim_kernel(ScanArgs A, 
   for (u32 e = 0; e <= C.num_edges; ++e) {
     // an aborted launch (a bounded wait gave up) leaves at the next edge
     if (s_aborted) return;
-    cosim::between_phase(C, (u32)t, b, nb, e);
+    cosim::between_phase(C, pins, (u32)t, b, nb, e);
     if (e == C.num_edges) break;
     grid_sync_coherent(A.bar, nb, b, gen, &g_error, &g_wait_polls, s_aborted);
     for (u32 m = 0; m < M;) {
