@@ -238,23 +238,28 @@ int jq_device_error_flag(u32 *out, int clear);
  * shorter bound and for tests of the time-out path. */
 usize jq_wait_limit(usize polls);
 
-/* Synchronisation of value-only scan launches (no counterpart in the
- * reference, whose kernel always takes a grid barrier after each major
- * stage, csrc/kernel_v1_impl.cuh:565-626).  mode 1 (the default): every
- * launch without timing exchanges its words through a ring in which every
- * word carries the number of its snapshot, and a block waits only for the
- * words it reads.  Launches of fewer than 8 cycles and scripts that do not
+/* Synchronisation of scan launches (no counterpart in the reference, whose
+ * kernel always takes a grid barrier after each major stage,
+ * csrc/kernel_v1_impl.cuh:565-626).  mode 1 (the default): every launch but
+ * the profiled one exchanges its words through a ring in which every word
+ * carries the number of its snapshot, and a block waits only for the words
+ * it reads.  Launches of fewer than 8 cycles and scripts that do not
  * fit (a writeout word written twice, a read past the first writeout word
  * of a word that no partition writes or that is written in the same or a
  * later major stage) still use grid barriers.  The ring and what its
- * builders find in the script are the one allocation these launches make:
- * 68 bytes per state word plus 128 per block, taken with
- * hipMallocAsync on the launch's stream and released with hipFreeAsync
- * after it (if the allocation fails, the launch uses grid barriers, and so
- * does a launch issued while its stream is being captured into a graph).
- * mode 0: grid barriers everywhere.  mode < 0
- * only queries.  Returns the previous mode.  Results are identical in both
- * modes; set it only while no scan launch is being issued. */
+ * builders find in the script take 68 bytes per state word plus 128 per
+ * block.  mode 0: grid barriers everywhere.  mode < 0 only queries.
+ * Returns the previous mode.  Results are identical in both modes; set it
+ * only while no scan launch is being issued.
+ *
+ * In either mode a launch of 8 cycles or more, and a co-simulation launch of
+ * 8 edges or more, composes the first-stage permutations of its partitions
+ * ahead of the cycles (18 KB per partition, 64 MiB at most with the ring;
+ * partitions past that use the script's own).  The ring and the permutations
+ * are the one allocation a launch makes, taken with hipMallocAsync on the
+ * launch's stream and released with hipFreeAsync after it.  If it fails, or
+ * while the stream is being captured into a graph, the launch uses grid
+ * barriers and the script's permutations. */
 int jq_scan_sync_mode(int mode);
 
 /* ---- Output change extraction (no counterpart in the reference) ---------

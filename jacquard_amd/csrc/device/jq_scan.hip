@@ -2,8 +2,8 @@
 //
 // One workgroup per script block, persistent over all cycles and major
 // stages, a grid barrier after every major stage (the contract of
-// csrc/kernel_v1_impl.cuh:565-626) or, in value-only launches, waits on the
-// very words the partition reads.  Inside a partition the work is mapped to
+// csrc/kernel_v1_impl.cuh:565-626) or, in launches of a few cycles and more,
+// waits on the very words the partition reads.  Inside a partition the work is mapped to
 // CDNA4 as follows:
 //   - script sections are streamed with 16-byte per-thread loads, each
 //     issued as soon as the registers of its predecessor are free: the next
@@ -71,7 +71,7 @@ struct ScanArgs {
   u32 ev_cap;
   i32 arrival_state_offset;
   u32 *bar;
-  // dataflow synchronisation (value-only launches, see below): the exchange
+  // dataflow synchronisation (see below): the exchange
   // ring, what its builders found in the script and the blocks' completed
   // cycles; ring == null: grid barriers
   u64 *ring;
@@ -332,7 +332,7 @@ __device__ __forceinline__ u32 load_hi(Section perm, const PartHdr &h) {
                                               0);
 }
 
-// ---- dataflow synchronisation of value-only launches
+// ---- dataflow synchronisation
 //
 // Partitions read snapshot words that other blocks wrote in an earlier
 // major stage of the same cycle (`out`, bit 31 of a global-read entry) or
@@ -347,7 +347,16 @@ __device__ __forceinline__ u32 load_hi(Section perm, const PartHdr &h) {
 // follow them, its poll, and only then the load.  Measured with the two
 // threads per word and the script words loaded a partition ahead (below):
 // 1M-gate netlist, 249 blocks, 11 major stages, 90.6 us per cycle with
-// progress words, 63.0 with the ring.
+// progress words, 63.0 with the ring.  Launches with timing checks have the
+// ring as well (arrivals are written to the snapshots and read by no block):
+// 4M gates with X and timing, 188 us per cycle with grid barriers, 183 with
+// the ring.
+//
+// In a launch with X masks a word and its mask lie side by side in the ring,
+// each with the snapshot number, and one 16-byte load brings both: a gather's
+// time is that of its lines, about two clocks each.  The same launch with the
+// masks apart 183 us per cycle, side by side 174; 100K gates with X, 54 and
+// 51.
 //
 // Slot s % kRing of the ring is written again kRing snapshots later.  Each
 // block publishes the cycles it has completed and, every kRing / 2 cycles,
@@ -371,8 +380,12 @@ struct Flow {
   Section ring;   // kRing slots
   u64 *slots;     // the same, for the stores
   u32 slot;       // words of one slot (the state size)
+  u32 shift;      // 3, or 4 with X masks: a word's bytes in the ring
   u32 lo, xoff;   // first writeout word; X mask offset of the launch or 0
   u32 *bar, *aborted;
+  __device__ __forceinline__ u64 *word(u32 snapshot, u32 w) const {
+    return slots + (size_t)(snapshot & (kRing - 1)) * slot + ((size_t)w << (shift - 3));
+  }
 };
 
 __device__ __forceinline__ u64 ld_coherent64(const u64 *p) {
@@ -399,11 +412,15 @@ __device__ __forceinline__ bool flow_gives_up(const Flow &F, u32 &spins) {
   return stop;
 }
 
-// A word of the ring at byte offset `at` (kNoLoad: zeros).  The coherent
-// load of st_coherent64's words, one access of 8 bytes.
-__device__ __forceinline__ u64 ld_ring(Section ring, u32 at) {
-  const Word2 v = __builtin_amdgcn_raw_buffer_load_b64(ring, at, 0, 16);  // agent scope
-  return (u64)v.y << 32 | v.x;
+// The words of the ring at byte offset `at` (kNoLoad: zeros): a state word
+// and its tag or, in launches with X masks, those two and the mask and its
+// tag.  The coherent load of st_coherent64's words, each 8 bytes of one
+// access.
+template <bool X>
+__device__ __forceinline__ Word4 ld_ring(Section ring, u32 at) {
+  if (X) return __builtin_amdgcn_raw_buffer_load_b128(ring, at, 0, 16);  // agent scope
+  const Word2 v = __builtin_amdgcn_raw_buffer_load_b64(ring, at, 0, 16);
+  return Word4{v.x, v.y, 0, 0};
 }
 
 // The state words of the first N entries e (cycle c, snapshots in and out)
@@ -415,22 +432,22 @@ __device__ __forceinline__ void flow_gather(const Flow &F, const uint2 *e, const
                                             const Fn &between) {
   u32 ri = (c & (kRing - 1)) * 8 * F.slot, ro = ((c + 1) & (kRing - 1)) * 8 * F.slot;
   asm volatile("" : "+s"(ri), "+s"(ro));  // and no multiplication per entry
+  const u32 sh = X ? 4 : F.shift;
   u32 a[N];
-  u64 q[N], r[X ? N : 1];
-  u32 pend = 0;    // bit k: entry k's value, bit 16 + k: its X mask
+  Word4 q[N];
+  u32 pend = 0;    // bit k: entry k has not arrived
   u32 inputs = 0;  // bit k: entry k is a primary input
 #pragma unroll
   for (u32 k = 0; k < N; ++k) {
     const u32 w = e[k].x & 0x7fffffffu;
     const bool o = (int)e[k].x < 0, need = e[k].y != 0, ring = need && w >= F.lo;
-    a[k] = ((e[k].x << 3) + (o ? ro : ri)) | (ring ? 0 : kNoLoad);
-    pend |= ring ? (X ? 0x10001u : 1u) << k : 0;
+    a[k] = ((e[k].x << sh) + (o ? ro : ri)) | (ring ? 0 : kNoLoad);
+    pend |= ring ? 1u << k : 0;
     inputs |= need && !ring ? 1u << k : 0;
   }
 #pragma unroll
   for (u32 k = 0; k < N; ++k) {
-    q[k] = ld_ring(F.ring, a[k]);
-    if (X) r[k] = ld_ring(F.ring, a[k] + 8 * F.xoff);
+    q[k] = ld_ring<X>(F.ring, a[k]);
     v[k] = 0;
     if (X) x[k] = 0;
   }
@@ -449,13 +466,10 @@ __device__ __forceinline__ void flow_gather(const Flow &F, const uint2 *e, const
 #pragma unroll
     for (u32 k = 0; k < N; ++k) {
       const u32 s = c + (e[k].x >> 31);
-      if (((pend >> k) & 1u) && (u32)(q[k] >> 32) == s) {
-        v[k] = (u32)q[k];
+      if (((pend >> k) & 1u) && q[k].y == s && (!X || q[k].w == s)) {
+        v[k] = q[k].x;
+        if (X) x[k] = q[k].z;
         pend &= ~(1u << k);
-      }
-      if (X && ((pend >> (16 + k)) & 1u) && (u32)(r[k] >> 32) == s) {
-        x[k] = (u32)r[k];
-        pend &= ~(0x10000u << k);
       }
     }
   };
@@ -464,10 +478,8 @@ __device__ __forceinline__ void flow_gather(const Flow &F, const uint2 *e, const
     if (flow_gives_up(F, spins)) break;
     asm volatile("" ::: "memory");
 #pragma unroll
-    for (u32 k = 0; k < N; ++k) {
-      if ((pend >> k) & 1u) q[k] = ld_ring(F.ring, a[k]);
-      if (X && ((pend >> (16 + k)) & 1u)) r[k] = ld_ring(F.ring, a[k] + 8 * F.xoff);
-    }
+    for (u32 k = 0; k < N; ++k)
+      if ((pend >> k) & 1u) q[k] = ld_ring<X>(F.ring, a[k]);
     wait_loads();
     check();
   }
@@ -503,15 +515,14 @@ __device__ __forceinline__ void gather(const Flow &F, const uint2 *e, const u32 
     flow_gather<N, false>(F, e, in, out, c, v, x, between);
 }
 
-// State word w of snapshot in (o = 0) or out (o = 1) of cycle c, for the
-// rounds past kPreRounds; `off` is 0 or the X mask offset.  Every lane of
-// the wave calls it; `need` lanes get their word.
-__device__ __forceinline__ u32 flow_word(const Flow &F, bool need, u32 w, u32 o, u32 off,
+// State word w (x: its X mask) of snapshot in (o = 0) or out (o = 1) of cycle
+// c, for the rounds past kPreRounds; lanes without `need` get zero.
+__device__ __forceinline__ u32 flow_word(const Flow &F, bool need, u32 w, u32 o, u32 x,
                                          const u32 *in, const u32 *out, u32 c) {
   if (!need) return 0;
-  if (w < F.lo) return (o ? out : in)[off + w];
+  if (w < F.lo) return (o ? out : in)[w + (x ? F.xoff : 0)];
   const u32 s = c + o;
-  const u64 *a = F.slots + ((size_t)(s & (kRing - 1)) * F.slot + off + w);
+  const u64 *a = F.word(s, w) + x;
   u32 spins = 0;
   for (;;) {
     const u64 q = ld_coherent64(a);
@@ -874,7 +885,7 @@ __device__ __forceinline__ void run_partition(const ScanArgs &A, const u32 *__re
       u32 v = 0, x = 0;
       if (FLOW) {
         v = flow_word(F, er.y != 0, w, er.x >> 31, 0, in, out, cycle);
-        if (is_x) x = flow_word(F, er.y != 0, w, er.x >> 31, F.xoff, in, out, cycle);
+        if (is_x) x = flow_word(F, er.y != 0, w, er.x >> 31, 1, in, out, cycle);
       } else if (er.y) {
         const u32 *base = (er.x >> 31) ? out : in;
         v = ld_coherent(base + w);
@@ -1083,9 +1094,9 @@ __device__ __forceinline__ void run_partition(const ScanArgs &A, const u32 *__re
           if (FLOW) {
             const u32 s = cycle + 1;
             const u64 tag = (u64)s << 32;
-            u64 *a = F.slots + ((size_t)(s & (kRing - 1)) * F.slot + w);
+            u64 *a = F.word(s, w);
             st_coherent64(a, tag | nv);
-            if (F.xoff) st_coherent64(a + F.xoff, tag | nx);
+            if (F.xoff) st_coherent64(a + 1, tag | nx);
             out[w] = nv;
             if (is_x) out[xoff + w] = nx;
           } else {
@@ -1130,21 +1141,15 @@ struct FlowBuild {
   const u32 *bd;
   u32 nb, M;
   usize state_size;
+  const u32 *states;
+  u64 *ring;
   u32 *owner;  // state_size words: (block << 16 | major stage) + 1 of the writer
   u32 *flow;   // kFlow* words
 };
 
-// Zeroes n units of 16 bytes but for the first `words` words of 8 bytes, which
-// are the ring's slot 0: snapshot 0 with its number.
-__global__ __launch_bounds__(256) void flow_zero_kernel(uint4 *p, usize n, const u32 *states,
-                                                        usize words) {
-  const usize first = (usize)blockIdx.x * 256u + threadIdx.x, step = (usize)gridDim.x * 256u;
-  for (usize i = first; i < n; i += step) {
-    uint4 v = make_uint4(0, 0, 0, 0);
-    if (2 * i < words) v.x = states[2 * i];
-    if (2 * i + 1 < words) v.z = states[2 * i + 1];
-    p[i] = v;
-  }
+__global__ __launch_bounds__(256) void flow_zero_kernel(uint4 *p, usize n) {
+  for (usize i = (usize)blockIdx.x * 256u + threadIdx.x; i < n; i += (usize)gridDim.x * 256u)
+    p[i] = make_uint4(0, 0, 0, 0);
 }
 
 // Raises *p to v.  Most workgroups find it there already, so the word is
@@ -1177,10 +1182,11 @@ __global__ __launch_bounds__(256) void flow_owner_kernel(FlowBuild F) {
   }
 }
 
-// Workgroup (m, b) checks the global-read entries of block b's partitions
-// in major stage m: a word at or past the first writeout word must be one
+// Workgroup (m, b) puts the words of snapshot 0 that block b's partitions of
+// major stage m write into the ring and checks their global-read entries: a word at or past the first writeout word must be one
 // that some partition writes, in an earlier stage when it is read from the
-// same cycle; X masks must lie at one offset, past the words themselves.
+// same cycle; X masks must lie at one offset, past the words themselves (so
+// that two words of 8 bytes for each of the words fit a slot).
 __global__ __launch_bounds__(256) void flow_check_kernel(FlowBuild F) {
   const u32 m = blockIdx.x / F.nb, b = blockIdx.x % F.nb;
   const u32 t = threadIdx.x;
@@ -1194,6 +1200,16 @@ __global__ __launch_bounds__(256) void flow_check_kernel(FlowBuild F) {
     if (xoff && ((s[8] && s[9] != xoff) || (usize)io + nio > xoff ||
                  (usize)xoff + io + nio > F.state_size))
       bad |= 4u;
+    // snapshot 0 (tag 0) into the ring
+    const usize w = (usize)io + t;
+    if (t < nio && nio <= 256u && w + xoff < F.state_size) {
+      if (!xoff) {
+        F.ring[w] = F.states[w];
+      } else if (2 * w + 1 < F.state_size) {
+        F.ring[2 * w] = F.states[w];
+        F.ring[2 * w + 1] = F.states[xoff + w];
+      }
+    }
     const uint2 *gr = reinterpret_cast<const uint2 *>(s + 256);
     for (u32 k = 0; k < rounds; ++k) {
       const uint2 e = gr[256 * k + t];
@@ -1236,6 +1252,7 @@ __device__ __forceinline__ void scan_loop(const ScanArgs &A, u32 *st_v, u32 *st_
     F.ring = __builtin_amdgcn_make_buffer_rsrc(A.ring, 0, 8 * kRing * F.slot, 0x00027000);
     F.lo = ~A.flow[kFlowNegLo];
     F.xoff = A.flow[kFlowXoff];
+    F.shift = F.xoff ? 4 : 3;
     F.bar = A.bar;
     F.aborted = &s_aborted;
   }
@@ -1298,8 +1315,8 @@ __global__ __launch_bounds__(kScanThreads) void scan_kernel(ScanArgs A) {
   const u32 gen = read_gen(A.bar);
   __syncthreads();
   // the flag is the same word for every block
-  if (!TIMING && !PROFILE && A.ring != nullptr && A.flow[kFlowBad] == 0)
-    scan_loop<TIMING, PROFILE, !TIMING && !PROFILE>(A, st_v, st_x, hin_v, hin_x, wo_v, wo_x,
+  if (!PROFILE && A.ring != nullptr && A.flow[kFlowBad] == 0)
+    scan_loop<TIMING, PROFILE, !PROFILE>(A, st_v, st_x, hin_v, hin_x, wo_v, wo_x,
                                                     st_arr, wo_arr, raw_v, raw_x, s_aborted,
                                                     gen);
   else
@@ -1386,7 +1403,7 @@ int set_error(const char *msg) {
 
 namespace {
 
-// 1: value-only launches synchronise by dataflow; 0: by grid barriers.
+// 1: scan launches synchronise by dataflow; 0: by grid barriers.
 int g_scan_sync = 1;
 
 template <bool TIMING, bool PROFILE>
@@ -1432,7 +1449,7 @@ int launch_scan(ScanArgs &A, hipStream_t stream) {
 // allocation failed.
 //
 // `flow`: the launch may synchronise by dataflow (exchange ring, progress
-// words; value-only, and the mode is on).  A script that the builders find
+// words; the mode is on).  A script that the builders find
 // unusable for it (a writeout word written twice or out of range, a read of a
 // word past the first writeout word that no partition writes, a same-cycle
 // read of a word not written in an earlier stage) raises the flag that the
@@ -1483,8 +1500,7 @@ void *prepare(ScanArgs &A, u32 cycles, bool flow, hipStream_t stream) {
   u32 *p = static_cast<u32 *>(buf);
   u32 *builders = p + ring + own;
   const u32 fill_blocks = (u32)std::min<size_t>(1024, (zeroed / 4 + 255) / 256);
-  flow_zero_kernel<<<fill_blocks, 256, 0, stream>>>(reinterpret_cast<uint4 *>(buf), zeroed / 4,
-                                                    A.states, flow ? A.state_size : 0);
+  flow_zero_kernel<<<fill_blocks, 256, 0, stream>>>(reinterpret_cast<uint4 *>(buf), zeroed / 4);
   if (flow) {
     FlowBuild F{};
     F.blocks_start = A.blocks_start;
@@ -1492,6 +1508,8 @@ void *prepare(ScanArgs &A, u32 cycles, bool flow, hipStream_t stream) {
     F.nb = nb;
     F.M = M;
     F.state_size = A.state_size;
+    F.states = A.states;
+    F.ring = reinterpret_cast<u64 *>(buf);
     F.owner = p + ring;
     F.flow = builders;
     flow_owner_kernel<<<sections, 256, 0, stream>>>(F);
@@ -1555,7 +1573,7 @@ int scan_common(usize num_blocks, usize num_major_stages, const usize *blocks_st
   A.sample_cycles = sample_cycles;
   const bool timing = A.timing != nullptr || arrival_state_offset != 0;
   if (samples) return launch_scan<false, true>(A, stream);
-  const bool flow = !timing && __atomic_load_n(&g_scan_sync, __ATOMIC_RELAXED);
+  const bool flow = __atomic_load_n(&g_scan_sync, __ATOMIC_RELAXED);
   void *buf = prepare(A, A.num_cycles, flow, stream);
   const int rc =
       timing ? launch_scan<true, false>(A, stream) : launch_scan<false, false>(A, stream);

@@ -585,3 +585,33 @@ def test_composed_permutations(blocks, xprop, bits, rounds):
         out = sim.run_scan(w, st.copy(), cycles, validate=False)
         assert np.array_equal(out["states"], ref)
         assert np.array_equal(out["sram"][:s.sram_storage_size], sram)
+
+
+@pytest.mark.parametrize("xprop", [False, True])
+@pytest.mark.parametrize("cycles", [7, 60])
+def test_timing_launches_in_both_sync_modes(xprop, cycles):
+    """Setup/hold launches exchange their words through the ring (short ones
+    and mode 0: grid barriers), masks beside the words under X: snapshots with
+    arrivals, SRAMs and the set of events are the oracle's."""
+    nl, comp = design("xts", level_split=6, seed=9, gates=40000, depth=48,
+                      dffs=3000, inputs=64, outputs=32, geometric_p=0.3, srams=2,
+                      delay=(20, 200))
+    s = comp.flatten(24, xprop=xprop)
+    s.inject_timing()
+    s.enable_timing_arrivals()
+    cons = s.build_timing_constraint_buffer(1500, 50, 20)
+    m = stimulus.dff_initial_xmask(s, 0.1, seed=8)[0] if xprop else None
+    st = stimulus.build_states(s, cycles, seed=16, p=0.3, initial_xmask=m)
+    ref = st.copy()
+    sram = np.zeros(s.sram_storage_size, np.uint32)
+    sram_x = np.full(s.sram_storage_size, 0xFFFFFFFF, np.uint32)
+    ev_ref, n_ref = oracle.run(s, ref, cycles, sram=sram, sram_x=sram_x if xprop else None,
+                               constraints=cons, arrival_state_offset=s.arrival_state_offset,
+                               event_capacity=1 << 20)
+    for mode in (1, 0):
+        with _sync_mode(mode):
+            out = sim.run_scan(s, st.copy(), cycles, constraints=cons, event_capacity=1 << 20)
+        assert np.array_equal(out["states"], ref), mode
+        assert np.array_equal(out["sram"][:s.sram_storage_size], sram), mode
+        assert out["event_count"] == n_ref and n_ref > 0
+        assert np.array_equal(sim.canonical_events(out["events"]), sim.canonical_events(ev_ref))
