@@ -559,32 +559,103 @@ __device__ __forceinline__ u32 from_lane_up(u32 v) {
   }
 }
 
+// Words of the layer arrays: the 256 of the layer, then one that nobody reads
+// for each lane of wave 0.  A lane without a result stores there, so that the
+// tree is one run of instructions: a skipped store is a branch, and a taken
+// branch waits for the instruction cache, which two busy CUs share.  (With a
+// branch at every level for the store and for the X lane: 2K gates in one
+// block 15.7 us per cycle, 14.8 without; 1M gates 54.8 and 53.0; 4M gates with
+// X and timing 174 and 169.)
+constexpr u32 kLayerWords = 256 + 64;
+
 // One hier level of wave 0's tree (kernel_v1_impl.cuh:236-293): on entry
 // lane i holds word 2HW + i (lanes i < 2HW); on exit lane i < HW holds word
 // HW + i, also written to the layer.  Word w's flags are fA on lane w.
-template <int HW, bool TIMING>
+template <int HW, bool TIMING, bool X>
 __device__ __forceinline__ void tree_level(u32 &cur, u32 &curx, u16 &cura, const uint4 &fA,
-                                           bool is_x, int lane, u32 *st_v, u32 *st_x,
-                                           u16 *st_arr) {
+                                           int lane, u32 *st_v, u32 *st_x, u16 *st_arr) {
   const u32 b = from_lane_up<HW>(cur);
   const u32 xa = from_lane_up<HW>(fA.x), xb = from_lane_up<HW>(fA.y);
   const u32 ob = from_lane_up<HW>(fA.z);
+  const u32 at = lane < HW ? HW + lane : 256 + lane;
   const u32 n = gate(cur, b, xa, xb, ob);
-  u32 nx = 0;
-  if (is_x) nx = gate_x(cur, curx, b, from_lane_up<HW>(curx), xa, xb, ob);
-  u16 na = 0;
+  st_v[at] = n;
+  if (X) {
+    curx = gate_x(cur, curx, b, from_lane_up<HW>(curx), xa, xb, ob);
+    st_x[at] = curx;
+  }
   if (TIMING) {
     const u32 dly = from_lane_up<HW>(fA.w);
-    na = arr_step(cura, (u16)from_lane_up<HW>((u32)cura), ob, dly);
-  }
-  if (lane < HW) {
-    st_v[HW + lane] = n;
-    if (is_x) st_x[HW + lane] = nx;
-    if (TIMING) st_arr[HW + lane] = na;
+    cura = arr_step(cura, (u16)from_lane_up<HW>((u32)cura), ob, dly);
+    st_arr[at] = cura;
   }
   cur = n;
-  curx = nx;
-  cura = na;
+}
+
+// The AND tree of a boomerang stage, in wave 0: the shuffled words in hin
+// become the 256 words of the layer.
+template <bool TIMING, bool X>
+__device__ __forceinline__ void run_tree(const uint4 &fA, const uint4 &fB, const uint4 &fC,
+                                         const uint4 &fD, const u32 *hin_v, const u32 *hin_x,
+                                         u32 *st_v, u32 *st_x, u16 *st_arr) {
+  const int lane = threadIdx.x & 63;
+  // hier0: words 128+L, 192+L; hier1: word 64+L
+  const u32 s0 = hin_v[lane], s1 = hin_v[64 + lane];
+  const u32 s2 = hin_v[128 + lane], s3 = hin_v[192 + lane];
+  const u32 o2 = gate(s0, s2, fC.x, fC.y, fC.z);
+  const u32 o3 = gate(s1, s3, fD.x, fD.y, fD.z);
+  u32 cur = gate(o2, o3, fB.x, fB.y, fB.z), curx = 0;
+  st_v[128 + lane] = o2;
+  st_v[192 + lane] = o3;
+  st_v[64 + lane] = cur;
+  if (X) {
+    const u32 x0 = hin_x[lane], x1 = hin_x[64 + lane];
+    const u32 x2 = hin_x[128 + lane], x3 = hin_x[192 + lane];
+    const u32 o2x = gate_x(s0, x0, s2, x2, fC.x, fC.y, fC.z);
+    const u32 o3x = gate_x(s1, x1, s3, x3, fD.x, fD.y, fD.z);
+    curx = gate_x(o2, o2x, o3, o3x, fB.x, fB.y, fB.z);
+    st_x[128 + lane] = o2x;
+    st_x[192 + lane] = o3x;
+    st_x[64 + lane] = curx;
+  }
+  u16 cura = 0;
+  if (TIMING) {
+    const u16 a2 = arr_step(0, 0, fC.z, fC.w), a3 = arr_step(0, 0, fD.z, fD.w);
+    cura = arr_step(a2, a3, fB.z, fB.w);
+    st_arr[128 + lane] = a2;
+    st_arr[192 + lane] = a3;
+    st_arr[64 + lane] = cura;
+  }
+  // hier2..7: the node of word hw + i (hw = 32, 16, ..., 1) is computed on
+  // lane i from lanes i (word 2hw + i) and i + hw (word 3hw + i); values and
+  // the node's flags (word L's on lane L in fA) move up by hw with
+  // v_permlane32_swap, v_permlane16_swap and DPP row shifts, a few cycles
+  // each, instead of LDS permutes
+  tree_level<32, TIMING, X>(cur, curx, cura, fA, lane, st_v, st_x, st_arr);
+  tree_level<16, TIMING, X>(cur, curx, cura, fA, lane, st_v, st_x, st_arr);
+  tree_level<8, TIMING, X>(cur, curx, cura, fA, lane, st_v, st_x, st_arr);
+  tree_level<4, TIMING, X>(cur, curx, cura, fA, lane, st_v, st_x, st_arr);
+  tree_level<2, TIMING, X>(cur, curx, cura, fA, lane, st_v, st_x, st_arr);
+  tree_level<1, TIMING, X>(cur, curx, cura, fA, lane, st_v, st_x, st_arr);
+  // in-word tail hier8..12 on lane 0 from word 1, now on lane 0
+  // (kernel_v1_impl.cuh:294-346)
+  const u32 v1 = cur, v1x = curx, xa = fA.x, xb = fA.y, ob = fA.z;
+  const u32 at = lane == 0 ? 0 : 256 + lane;
+  const u32 r8 = ((v1 << 16) ^ xa) & ((v1 ^ xb) | ob) & 0xffff0000u;
+  const u32 r9 = ((r8 >> 8) ^ xa) & (((r8 >> 16) ^ xb) | ob) & 0xff00u;
+  const u32 r10 = ((r9 >> 4) ^ xa) & (((r9 >> 8) ^ xb) | ob) & 0xf0u;
+  const u32 r11 = ((r10 >> 2) ^ xa) & (((r10 >> 4) ^ xb) | ob) & 0xcu;
+  const u32 r12 = ((r11 >> 1) ^ xa) & (((r11 >> 2) ^ xb) | ob) & 0x2u;
+  st_v[at] = r8 | r9 | r10 | r11 | r12;
+  if (X) {
+    const u32 x8 = gate_x(v1 << 16, v1x << 16, v1, v1x, xa, xb, ob) & 0xffff0000u;
+    const u32 x9 = gate_x(r8 >> 8, x8 >> 8, r8 >> 16, x8 >> 16, xa, xb, ob) & 0xff00u;
+    const u32 x10 = gate_x(r9 >> 4, x9 >> 4, r9 >> 8, x9 >> 8, xa, xb, ob) & 0xf0u;
+    const u32 x11 = gate_x(r10 >> 2, x10 >> 2, r10 >> 4, x10 >> 4, xa, xb, ob) & 0xcu;
+    const u32 x12 = gate_x(r11 >> 1, x11 >> 1, r11 >> 2, x11 >> 2, xa, xb, ob) & 0x2u;
+    st_x[at] = x8 | x9 | x10 | x11 | x12;
+  }
+  if (TIMING) st_arr[at] = 0;
 }
 
 // ---- the builder of the composed permutations
@@ -951,73 +1022,10 @@ __device__ __forceinline__ void run_partition(const ScanArgs &A, const u32 *__re
       }
       __syncthreads();
       if (w0) {
-        // hier0: words 128+L, 192+L; hier1: word 64+L
-        u32 s0 = hin_v[lane], s1 = hin_v[64 + lane];
-        u32 s2 = hin_v[128 + lane], s3 = hin_v[192 + lane];
-        u32 o2 = gate(s0, s2, fC.x, fC.y, fC.z);
-        u32 o3 = gate(s1, s3, fD.x, fD.y, fD.z);
-        u32 o1 = gate(o2, o3, fB.x, fB.y, fB.z);
-        u32 o2x = 0, o3x = 0, o1x = 0;
-        if (is_x) {
-          u32 x0 = hin_x[lane], x1 = hin_x[64 + lane];
-          u32 x2 = hin_x[128 + lane], x3 = hin_x[192 + lane];
-          o2x = gate_x(s0, x0, s2, x2, fC.x, fC.y, fC.z);
-          o3x = gate_x(s1, x1, s3, x3, fD.x, fD.y, fD.z);
-          o1x = gate_x(o2, o2x, o3, o3x, fB.x, fB.y, fB.z);
-        }
-        u16 a2 = 0, a3 = 0, a1 = 0;
-        if (TIMING) {
-          a2 = arr_step(0, 0, fC.z, fC.w);
-          a3 = arr_step(0, 0, fD.z, fD.w);
-          a1 = arr_step(a2, a3, fB.z, fB.w);
-        }
-        st_v[128 + lane] = o2;
-        st_v[192 + lane] = o3;
-        st_v[64 + lane] = o1;
-        if (is_x) {
-          st_x[128 + lane] = o2x;
-          st_x[192 + lane] = o3x;
-          st_x[64 + lane] = o1x;
-        }
-        if (TIMING) {
-          st_arr[128 + lane] = a2;
-          st_arr[192 + lane] = a3;
-          st_arr[64 + lane] = a1;
-        }
-        // hier2..7: the node of word hw + i (hw = 32, 16, ..., 1) is
-        // computed on lane i from lanes i (word 2hw + i) and i + hw (word
-        // 3hw + i); values and the node's flags (word L's on lane L in fA)
-        // move up by hw with v_permlane32_swap, v_permlane16_swap and DPP
-        // row shifts, a few cycles each, instead of LDS permutes
-        u32 cur = o1, curx = o1x;
-        u16 cura = a1;
-        tree_level<32, TIMING>(cur, curx, cura, fA, is_x, lane, st_v, st_x, st_arr);
-        tree_level<16, TIMING>(cur, curx, cura, fA, is_x, lane, st_v, st_x, st_arr);
-        tree_level<8, TIMING>(cur, curx, cura, fA, is_x, lane, st_v, st_x, st_arr);
-        tree_level<4, TIMING>(cur, curx, cura, fA, is_x, lane, st_v, st_x, st_arr);
-        tree_level<2, TIMING>(cur, curx, cura, fA, is_x, lane, st_v, st_x, st_arr);
-        tree_level<1, TIMING>(cur, curx, cura, fA, is_x, lane, st_v, st_x, st_arr);
-        // in-word tail hier8..12 on lane 0 from word 1, now on lane 0
-        // (kernel_v1_impl.cuh:294-346)
-        if (lane == 0) {
-          const u32 v1 = cur, v1x = curx;
-          u32 xa = fA.x, xb = fA.y, ob = fA.z;
-          u32 r8 = ((v1 << 16) ^ xa) & ((v1 ^ xb) | ob) & 0xffff0000u;
-          u32 r9 = ((r8 >> 8) ^ xa) & (((r8 >> 16) ^ xb) | ob) & 0xff00u;
-          u32 r10 = ((r9 >> 4) ^ xa) & (((r9 >> 8) ^ xb) | ob) & 0xf0u;
-          u32 r11 = ((r10 >> 2) ^ xa) & (((r10 >> 4) ^ xb) | ob) & 0xcu;
-          u32 r12 = ((r11 >> 1) ^ xa) & (((r11 >> 2) ^ xb) | ob) & 0x2u;
-          st_v[0] = r8 | r9 | r10 | r11 | r12;
-          if (is_x) {
-            u32 x8 = gate_x(v1 << 16, v1x << 16, v1, v1x, xa, xb, ob) & 0xffff0000u;
-            u32 x9 = gate_x(r8 >> 8, x8 >> 8, r8 >> 16, x8 >> 16, xa, xb, ob) & 0xff00u;
-            u32 x10 = gate_x(r9 >> 4, x9 >> 4, r9 >> 8, x9 >> 8, xa, xb, ob) & 0xf0u;
-            u32 x11 = gate_x(r10 >> 2, x10 >> 2, r10 >> 4, x10 >> 4, xa, xb, ob) & 0xcu;
-            u32 x12 = gate_x(r11 >> 1, x11 >> 1, r11 >> 2, x11 >> 2, xa, xb, ob) & 0x2u;
-            st_x[0] = x8 | x9 | x10 | x11 | x12;
-          }
-          if (TIMING) st_arr[0] = 0;
-        }
+        if (is_x)
+          run_tree<TIMING, true>(fA, fB, fC, fD, hin_v, hin_x, st_v, st_x, st_arr);
+        else
+          run_tree<TIMING, false>(fA, fB, fC, fD, hin_v, hin_x, st_v, st_x, st_arr);
       }
       __syncthreads();
       if (h0 && (hook >> 8) == bs) {
@@ -1230,9 +1238,9 @@ __global__ __launch_bounds__(256) void flow_check_kernel(FlowBuild F) {
 
 // The LDS arrays of one workgroup.
 #define JQ_SCAN_LDS                                             \
-  __shared__ u32 st_v[256], st_x[256], hin_v[256], hin_x[256]; \
-  __shared__ u32 wo_v[256], wo_x[256];                          \
-  __shared__ u16 st_arr[256], wo_arr[256];                      \
+  __shared__ u32 st_v[kLayerWords], st_x[kLayerWords];          \
+  __shared__ u32 hin_v[256], hin_x[256], wo_v[256], wo_x[256];  \
+  __shared__ u16 st_arr[kLayerWords], wo_arr[256];              \
   __shared__ u32 raw_v[kRawWords], raw_x[kRawWords];            \
   __shared__ u32 s_aborted; /* set by a wait when the launch has aborted */
 
