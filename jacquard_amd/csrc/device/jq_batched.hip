@@ -158,6 +158,13 @@ __device__ __forceinline__ void row_fetch(const u32 *g, u32 *l, u32 rows) {
 // the workgroup barrier that precedes the first read of a fetched section.
 __device__ __forceinline__ void sec_wait() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
+// A workgroup barrier for what passes through LDS: the wave's own LDS
+// accesses are complete, its global loads and LDS copies may be in flight
+// (__syncthreads waits for those as well when there are LDS copies).
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 // Header of one partition (src/flatten.rs:198-258) and the writeout hook of
 // this thread's row, four threads to a row.  The words stay as they were
 // loaded (nothing waits for them) until the partition starts.
@@ -179,6 +186,7 @@ constexpr u32 kOldRows = 64;
 
 // Source lane-words of this thread's first-layer positions t + kT * j.
 constexpr int kG = kLayerWords / kT;
+static_assert(kG < 16, "the low four bits of a vmcnt");
 __device__ __forceinline__ void load_sources(u32 (&src)[kG], const u32 *gsrc) {
 #pragma unroll
   for (int j = 0; j < kG; ++j) src[j] = gsrc[threadIdx.x + kT * j];
@@ -319,6 +327,7 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
     const u32 next_s = uniform(h.a.x);
     if (next_s != 0) load_sources(src, is_last ? ngsrc : gsrc + kLayerWords);
 
+    have_next = !is_last && next_s != 0;
     const u32 nperm = ns * 4 + nd;  // SRAM port and duplicate words
     // ---- boomerang stages: every thread gathers its 8 level-1 operands
     // from one layer and writes its gates to the other, so no wave waits for
@@ -352,6 +361,17 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
       else
         row_fetch(secg + (size_t)kSecWords * (nperm ? S : S + 1), secb(S),
                   nperm ? nperm : num_ios);
+      // the next partition of this stage: its first-layer words, beside this
+      // one's gates and tree (its entries arrived during the operand reads,
+      // and nothing looks at them before).  The gather is bound by the CU's
+      // bytes per clock, the stages by LDS and instructions: one after the
+      // other, 4M gates 4 x 64 took 16326 us and 1M gates 8 x 32 12514, beside
+      // each other 15729 and 11835
+      if (s == 0 && have_next) {
+#pragma unroll
+        for (int j = 0; j < kG; ++j) asm volatile("" : "+v"(src[j]));
+        load_words<WIDE>(vnext, src, B, in, out);
+      }
       // levels 1..5 of the subtree rooted at position 256 + v; gate g's
       // flags are bit g of F.x / F.y / F.z, this quarter's 4-apart gates
       // bits 0, 4, .. of the shifted words
@@ -377,7 +397,7 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
                            fy, fz, 30);
       if (q4 < 2) layer[512 + (swp ^ 16)] = L4;  // sw(512 + p0), p0 < 512
       if (q4 == 0) layer[256 + (swp ^ 8)] = L5;  // sw(256 + v), v < 256
-      __syncthreads();
+      lds_barrier();
       if (t < 64) {
         // wave 0 lane L: flags of positions 128+L, 192+L, 64+L, L in fw.
         // level 6: positions 128+L and 192+L; level 7: 64+L
@@ -406,19 +426,20 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
           layer[0] = 0;
         }
       }
-      sec_wait();  // section s+1 is read right after this barrier
-      __syncthreads();
+      // section s+1 is read right after this barrier; the next partition's
+      // words, kG loads requested after it, are not waited for
+      if (s == 0 && have_next)
+        __builtin_amdgcn_s_waitcnt(0x0F70 | kG);
+      else
+        sec_wait();
+      lds_barrier();
       if ((hook >> 8) == s) {
         const u32 from = 32u * (hook & 255u) + 8 * q4, to = 32 * v + 8 * q4;
 #pragma unroll
         for (u32 k = 0; k < 8; ++k) WO[sw(to + k)] = layer[sw(from + k)];
       }
     }
-    // the next partition of this stage: its first-layer words (its gather
-    // entries arrived during this partition)
-    have_next = !is_last && next_s != 0;
-    if (have_next) load_words<WIDE>(vnext, src, B, in, out);
-    __syncthreads();
+    lds_barrier();
 
     // ---- SRAM + duplicate permutation into a layer (free now); a
     // partition without SRAM or duplicate words skips the phase and its
@@ -437,7 +458,7 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
           layer[sw(q)] = (w & ~fbit(f.y, q)) ^ fbit(f.x, q);
         }
       }
-      __syncthreads();
+      lds_barrier();
       // SRAM ports: thread per (sram, lane)
       for (u32 base = 0; base < ns * 32; base += kT) {
         u32 id = base + t;
@@ -475,7 +496,7 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
       for (u32 q = t; q < nd * 32; q += kT)
         WO[sw(32 * (num_ios - ns - nd) + q)] = layer[sw(ns * 128 + q)];
       sec_wait();  // the clock-enable section is read after this barrier
-      __syncthreads();
+      lds_barrier();
     }
 
     // ---- clock-enable permutation + commit (coalesced lane-words)
@@ -497,7 +518,7 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
       for (u32 q = t + kOldRows * 32; q < num_ios * 32; q += kT)
         commit(q, ld_coherent(in + (size_t)io * 32 + q));
     }
-    __syncthreads();
+    lds_barrier();
     if (prof) {
       if (t == 0) *prof = (u32)(clock64() - tick0);
       ++prof;
