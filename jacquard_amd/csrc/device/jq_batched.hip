@@ -427,8 +427,9 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
         }
       }
       // section s+1 is read right after this barrier; the next partition's
-      // words, kG loads requested after it, are not waited for
-      if (s == 0 && have_next)
+      // words, kG loads requested after it, are not waited for (WIDE skips the
+      // loads of positions without a source: it cannot count them)
+      if (!WIDE && s == 0 && have_next)
         __builtin_amdgcn_s_waitcnt(0x0F70 | kG);
       else
         sec_wait();
