@@ -20,7 +20,7 @@ class Netlist:
         if not handle:
             raise RuntimeError("netlist construction failed: " + N.host_error())
         self._h = handle
-        self._arrays = None
+        self._arrays = self._ports = None
 
     def __del__(self):
         h = getattr(self, "_h", None)
@@ -116,7 +116,10 @@ class Netlist:
 
     def ports(self):
         """Input and output port bits in declaration order:
-        (inputs: [(name, pin, posedge_flag_pin_or_0)], outputs: [(name, lit)])."""
+        (inputs: [(name, pin, posedge_flag_pin_or_0)], outputs: [(name, lit)]).
+        Read from the library once, as nothing changes a netlist's ports."""
+        if self._ports is not None:
+            return list(self._ports[0]), list(self._ports[1])
         L = N.host()
         cnt = (ctypes.c_uint64 * 2)()
         L.jqh_aig_port_counts(self._h, cnt)
@@ -129,7 +132,8 @@ class Netlist:
             lit = ctypes.c_uint32()
             name = L.jqh_aig_out_port(self._h, i, ctypes.byref(lit))
             outs.append((name.decode(), lit.value))
-        return ins, outs
+        self._ports = ins, outs
+        return list(ins), list(outs)
 
     def dff_names(self):
         """Instance name of every DFF, in DFF order ("" where the netlist
