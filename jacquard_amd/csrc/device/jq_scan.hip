@@ -80,6 +80,7 @@ struct ScanArgs {
   // composed stage-0 permutations (see below) and, per major stage and
   // block, the first one's slot or kNoSlot; table == null: none
   const u32 *table, *slots;  // slots: never null
+  bool local;  // they index the state in LDS (launches of one block, below)
   // profiling
   const u32 *part_index;
   u32 num_parts;
@@ -331,6 +332,11 @@ __device__ __forceinline__ u32 load_hi(Section perm, const PartHdr &h) {
   return __builtin_amdgcn_raw_buffer_load_b32(perm, wide ? 4 * (4096 + threadIdx.x) : kNoLoad, 0,
                                               0);
 }
+// The same for permutations that index the state in LDS.
+__device__ __forceinline__ u32 load_local_hi(Section perm, const PartHdr &h) {
+  return __builtin_amdgcn_raw_buffer_load_b32(
+      perm, h.slot != kNoSlot ? 4 * (4096 + threadIdx.x) : kNoLoad, 0, 0);
+}
 
 // ---- dataflow synchronisation
 //
@@ -373,8 +379,26 @@ constexpr u32 kFlowNegLo = 0;  // ~(first writeout word), 0 when there is none
 constexpr u32 kFlowXoff = 1;   // X mask offset of the X-capable partitions, or 0
 constexpr u32 kFlowBad = 2;    // nonzero: the script does not fit, grid barriers
 constexpr u32 kTableCursor = 32;  // slots of the table given out
+constexpr u32 kTableMissing = 33; // nonzero: a partition has no slot
 constexpr u32 kFlowWords = 64;
 constexpr u32 kProgStride = 32;  // one progress word per 128-byte line
+
+// ---- the state of a one-block launch in LDS
+//
+// The only block of a launch reads what it wrote itself, so a small design's
+// state stays in LDS: two snapshots of up to kLocalWords words, cycle c's input
+// in half c & 1, and the composed permutations index them directly (word
+// kLocalWords, always zero, for bits that no entry fills; the upper half's bit
+// of an index is that of the output snapshot in an even cycle).  A partition
+// has no gather at all, and nothing goes across the chip but the finished
+// words on their way to the snapshot buffer.  2K gates, 4 major stages: 14.8
+// us per cycle with the ring, 9.2 so.
+//
+// It takes a value-only launch that could use the ring, without X and with a
+// slot for every partition, and has functions of its own (run_local): built
+// into the general ones it cost the others 4% (1M gates).
+constexpr u32 kLocalWords = 4095;
+constexpr u32 kLocalHalf = kLocalWords + 1;
 
 struct Flow {
   Section ring;   // kRing slots
@@ -666,6 +690,8 @@ struct TableBuild {
   u32 cap;  // slots of the table
   u32 *slots, *table;
   u32 *cursor;  // slots given out, zero before
+  u32 *missing;  // raised when a partition gets none
+  bool local;    // indexes into the state in LDS
 };
 
 // Workgroup (m, b) composes the permutations of block b's partitions in
@@ -698,6 +724,7 @@ __global__ __launch_bounds__(256) void compose_kernel(TableBuild T) {
       if (slot <= T.cap - n) s_slot = slot;
     }
     T.slots[blockIdx.x] = kNoSlot;
+    if (n != 0 && s_slot == kNoSlot) *T.missing = 1;
   }
   __syncthreads();
   if (s_slot == kNoSlot) return;
@@ -710,20 +737,30 @@ __global__ __launch_bounds__(256) void compose_kernel(TableBuild T) {
     const uint2 *gr = reinterpret_cast<const uint2 *>(s + 256);
     u32 p = 0;
     for (u32 hi = rounds; hi != 0 && p < 32;) {
-      u32 m[8];
+      u32 m[8], word[8];
       const u32 lo = hi > 8 ? hi - 8 : 0;
 #pragma unroll
-      for (u32 k = 0; k < 8; ++k) m[k] = lo + k < hi ? gr[256 * (lo + k) + t].y : 0;
+      for (u32 k = 0; k < 8; ++k) {
+        const uint2 e = lo + k < hi ? gr[256 * (lo + k) + t] : make_uint2(0, 0);
+        m[k] = e.y;
+        word[k] = 1 + 256 * (lo + k) + t;
+        if (T.local) {
+          const u32 w = e.x & 0x7fffffffu;
+          if (w >= kLocalWords) s_bad = 1;
+          word[k] = (e.x >> 31) * kLocalHalf + (w & (kLocalHalf - 1));
+        }
+      }
 #pragma unroll
       for (int k = 7; k >= 0; --k)
         for (; m[k] != 0 && p < 32; ++p) {
           const u32 b = 31 - __builtin_clz(m[k]);
-          src[256 * p + t] = (1 + 256 * (lo + k) + t) << 5 | b;
+          src[256 * p + t] = word[k] << 5 | b;
           m[k] ^= 1u << b;
         }
       hi = lo;
     }
-    for (; p < 32; ++p) src[256 * p + t] = 0;  // raw word 0
+    // raw word 0 or the zero past a half's words
+    for (; p < 32; ++p) src[256 * p + t] = T.local ? kLocalWords << 5 : 0;
     __syncthreads();
     const u32 *perm = s + 256 + (size_t)512 * rounds;
 #pragma unroll
@@ -748,6 +785,7 @@ __global__ __launch_bounds__(256) void compose_kernel(TableBuild T) {
     off += 256 + (size_t)512 * rounds + (size_t)5120 * (ns + 2);
   }
   if (t == 0 && !s_bad) T.slots[blockIdx.x] = s_slot;
+  if (t == 0 && s_bad) *T.missing = 1;
 }
 
 // A block's partitions in execution order: cycle, major stage, then
@@ -1332,6 +1370,156 @@ __global__ __launch_bounds__(kScanThreads) void scan_kernel(ScanArgs A) {
                                       raw_v, raw_x, s_aborted, gen);
 }
 
+// ---- launches that keep the state in LDS
+
+struct LocalLds {
+  u32 state[2 * kLocalHalf];
+  u32 st[kLayerWords], hin[256], wo[256];
+};
+
+// One partition of cycle `cycle`, as run_partition runs it without X and
+// arrivals: its first stage takes its bits from the state, its writeouts go
+// into the other half and to the snapshot `out`.
+__device__ __forceinline__ void run_local(const ScanArgs &A, LocalLds &L, Walk &wk, PartPre &P,
+                                          u32 *__restrict__ out, u32 cycle) {
+  const u32 *bd = A.blocks_data;
+  const int lane = threadIdx.x & 63;
+  const int t = threadIdx.x >> 1;
+  const bool h0 = (threadIdx.x & 1) == 0;
+  const u32 pq = 2048 * (threadIdx.x & 1) + 4 * t;
+  const PartHdr &h = wk.cur, &hn = wk.next;
+  const u32 num_stages = h.num_stages ? h.num_stages : 1;
+  const u32 num_ios = h.num_stages ? h.num_ios : 0;
+  const u32 num_srams = h.num_srams, num_dups = h.num_dups;
+  const u32 nperm = h.num_stages ? num_srams * 4 + num_dups : 0;
+  const u32 hook = (threadIdx.x & 2) ? P.hook >> 16 : P.hook & 0xffffu;
+  const Section S = section_of(bd, h), Sn = section_of(bd, hn);
+  u32 st = stage0(h);
+  const u32 sd = st + 5120 * h.num_stages, ck = sd + 5120;
+  uint4 sda, sdb, sdf, cka, ckb, ckf;
+  fetch_step(A, A.num_cycles, wk, hn);
+  if ((u32)t < nperm) {
+    sda = ld4(S, true, sd + pq);
+    sdb = ld4(S, true, sd + pq + 1024);
+    sdf = ld4(S, true, sd + 4096 + 4 * t);
+  }
+  if ((u32)t < num_ios) {
+    cka = ld4(S, true, ck + pq);
+    ckb = ld4(S, true, ck + pq + 1024);
+    ckf = ld4(S, true, ck + 4096 + 4 * t);
+  }
+  P.hook = __builtin_amdgcn_raw_buffer_load_b32(Sn, 4 * (128 + (threadIdx.x >> 2)), 0, 0);
+  const u32 flip = (cycle & 1) ? 0xAAAAAAAAu : 0u;
+  __syncthreads();  // the previous partition's writeouts are in the state
+  for (u32 bs = 0; bs < num_stages; ++bs) {
+    const u32 hv = bs == 0 ? gather_bits_of<true>(L.state, P.qa, P.qb, P.hi ^ flip)
+                           : gather_bits(L.st, P.qa, P.qb);
+    const uint4 fA = P.fA, fB = P.fB, fC = P.fC, fD = P.fD;
+    st += 5120;
+    const bool more = bs + 1 < num_stages;
+    const Section pn = perm0(A.table, hn, Sn);
+    load_stage(P, more ? S : pn, more ? st : perm0_at(hn), more ? S : Sn,
+               more ? st : stage0(hn));
+    if (!more) P.hi = load_local_hi(pn, hn);
+    if (h0) L.hin[t] = hv;
+    __syncthreads();
+    if (threadIdx.x < 64)
+      run_tree<false, false>(fA, fB, fC, fD, L.hin, nullptr, L.st, nullptr, nullptr);
+    __syncthreads();
+    if (h0 && (hook >> 8) == bs) L.wo[t] = L.st[hook & 255];
+  }
+  wait_loads();
+  __syncthreads();
+  if (nperm) {
+    u32 pv = 0;
+    if ((u32)t < nperm) pv = (gather_bits(L.wo, sda, sdb) & ~sdf.y) ^ sdf.x;
+    const u32 en = __shfl(pv, (lane + 2) & 63);
+    const u32 wdata = __shfl(pv, (lane + 4) & 63);
+    __syncthreads();
+    if (h0 && (u32)t < num_srams * 4) {
+      if ((t & 3) == 0) {
+        const u32 s = (u32)t >> 2;
+        u32 *ram = A.sram_data + (size_t)h.sram_offset + (size_t)s * kSramWords;
+        const u32 ra = (pv & 0xffffu) & (kSramWords - 1);
+        const u32 wa = (pv >> 16) & (kSramWords - 1);
+        const u32 rv = ram[ra], w0v = ram[wa];
+        ram[wa] = (w0v & ~en) | (wdata & en);
+        L.wo[num_ios - num_srams + s] = rv;
+      }
+    } else if (h0 && (u32)t < nperm) {
+      L.wo[num_ios - num_srams - num_dups + ((u32)t - num_srams * 4)] = pv;
+    }
+    __syncthreads();
+  }
+  if ((u32)t < num_ios) {
+    u32 en = ckf.x;
+    if (ckf.y != 0xFFFFFFFFu) en = (gather_bits(L.wo, cka, ckb) & ~ckf.y) ^ ckf.x;
+    if (h0) {
+      const u32 w = h.io_offset + (u32)t;
+      const u32 old = L.state[(cycle & 1) * kLocalHalf + w];
+      const u32 nv = (old & ~en) | ((L.wo[t] ^ ckf.z) & en);
+      L.state[((cycle + 1) & 1) * kLocalHalf + w] = nv;
+      out[w] = nv;
+    }
+  }
+}
+
+__device__ __forceinline__ void local_loop(const ScanArgs &A, LocalLds &L) {
+  const u32 ss = (u32)A.state_size, M = A.num_major_stages, t = threadIdx.x;
+  const u32 lo = ~A.flow[kFlowNegLo] < ss ? ~A.flow[kFlowNegLo] : ss;
+  // snapshot 0, and the primary inputs (words below lo) of snapshot 1; `inp`
+  // is this thread's input word of the one after
+  for (u32 w = t; w < ss; w += kScanThreads) L.state[w] = A.states[w];
+  for (u32 w = t; w < lo; w += kScanThreads) L.state[kLocalHalf + w] = A.states[ss + w];
+  if (t == 0) L.state[kLocalWords] = L.state[kLocalHalf + kLocalWords] = 0;
+  u32 inp = t < lo && A.num_cycles > 1 ? A.states[2 * (size_t)ss + t] : 0;
+  Walk w{};
+  PartPre P{};
+  start_walk(A, A.num_cycles, w, P);
+  P.hi = load_local_hi(perm0(A.table, w.cur, section_of(A.blocks_data, w.cur)), w.cur);
+  u32 *out = A.states + ss;
+  for (u32 c = 0, m = 0;;) {
+    const bool last = w.cur.num_stages == 0 || w.cur.is_last != 0;
+    w.next = settle(w);
+    run_local(A, L, w, P, out, c);
+    w.cur = w.next;
+    if (!last || ++m != M) continue;
+    m = 0;
+    if (++c == A.num_cycles) return;
+    out += ss;
+    // the inputs beside this cycle's outputs, in the half whose last reads (it
+    // was the last cycle's input) are behind a workgroup barrier
+    u32 *half = L.state + ((c + 1) & 1) * kLocalHalf;
+    if (t < lo) half[t] = inp;
+    for (u32 k = t + kScanThreads; k < lo; k += kScanThreads) half[k] = out[k];
+    if (t < lo && c + 1 < A.num_cycles) inp = out[ss + t];
+  }
+}
+
+// A launch of one block that may keep its state in LDS, and does unless the
+// builders found a reason not to.
+__global__ __launch_bounds__(kScanThreads) void local_kernel(ScanArgs A) {
+  if (A.num_major_stages == 0) return;
+  if (A.flow[kFlowBad] == 0 && A.flow[kFlowXoff] == 0 && A.flow[kTableMissing] == 0) {
+    __shared__ LocalLds L;
+    local_loop(A, L);
+    return;
+  }
+  JQ_SCAN_LDS
+  const int t = threadIdx.x;
+  if (t == 0) s_aborted = raw_v[0] = raw_x[0] = 0;
+  if (t < 256) st_x[t] = hin_x[t] = wo_x[t] = wo_arr[t] = st_arr[t] = 0;
+  const u32 gen = read_gen(A.bar);
+  __syncthreads();
+  A.table = nullptr;  // its permutations are for the state in LDS
+  if (A.flow[kFlowBad] == 0)
+    scan_loop<false, false, true>(A, st_v, st_x, hin_v, hin_x, wo_v, wo_x, st_arr, wo_arr, raw_v,
+                                  raw_x, s_aborted, gen);
+  else
+    scan_loop<false, false, false>(A, st_v, st_x, hin_v, hin_x, wo_v, wo_x, st_arr, wo_arr, raw_v,
+                                   raw_x, s_aborted, gen);
+}
+
 // Persistent co-simulation: C.num_edges edges of one cycle each over the
 // two snapshots of C.states (timing events carry cycle 0, as every edge of
 // the reference's co-simulation dispatch does, src/sim/cosim_metal.rs:
@@ -1423,6 +1611,7 @@ int launch_scan(ScanArgs &A, hipStream_t stream) {
   A.bar = bar_base + kCohSlotWords * (__atomic_fetch_add(&g_slot, 1u, __ATOMIC_RELAXED) % kCohSlots);
   void *args[] = {&A};
   const void *kern = reinterpret_cast<const void *>(&scan_kernel<TIMING, PROFILE>);
+  if (A.local) kern = reinterpret_cast<const void *>(&local_kernel);
   // Under stream capture (a hipGraph of the launch) the launch is an
   // ordinary kernel node: co-residency of the workgroups is checked here
   // from the occupancy query, and the bounded waits turn a shortfall at a
@@ -1463,6 +1652,8 @@ int launch_scan(ScanArgs &A, hipStream_t stream) {
 // read of a word not written in an earlier stage) raises the flag that the
 // kernel reads, and the launch then uses grid barriers.
 //
+// `local`: the launch may keep a small one-block design's state in LDS.
+//
 // Every prepared launch has the composed permutations, with slots for one
 // partition per block and major stage (what a script as wide as its widest
 // stage holds) or up to eight of a narrower one's, in at most kPrepareBytes
@@ -1471,9 +1662,10 @@ int launch_scan(ScanArgs &A, hipStream_t stream) {
 // does without them.
 constexpr size_t kPrepareBytes = (size_t)64 << 20;
 
-void *prepare(ScanArgs &A, u32 cycles, bool flow, hipStream_t stream) {
+void *prepare(ScanArgs &A, u32 cycles, bool flow, bool local, hipStream_t stream) {
   A.ring = nullptr;
   A.table = nullptr;
+  A.local = false;
   const u32 nb = A.num_blocks, M = A.num_major_stages;
   flow = flow && M <= 65534u && A.state_size <= (usize(1) << 25);
   if (M == 0 || cycles < kFlowMinCycles || A.state_size == 0 || (usize)nb * M > 0x7fffffffu)
@@ -1534,6 +1726,8 @@ void *prepare(ScanArgs &A, u32 cycles, bool flow, hipStream_t stream) {
     T.cursor = builders + kTableCursor;
     T.slots = p + zeroed;
     T.table = T.slots + whole(sections);
+    T.missing = builders + kTableMissing;
+    T.local = A.local = local && flow && nb == 1 && A.state_size <= kLocalWords;
     compose_kernel<<<sections, 256, 0, stream>>>(T);
     A.slots = T.slots;
     A.table = T.table;
@@ -1542,6 +1736,7 @@ void *prepare(ScanArgs &A, u32 cycles, bool flow, hipStream_t stream) {
     (void)hipFreeAsync(buf, stream);
     A.ring = nullptr;
     A.table = nullptr;
+    A.local = false;
     A.slots = reinterpret_cast<const u32 *>(A.blocks_start);
     return nullptr;
   }
@@ -1582,7 +1777,7 @@ int scan_common(usize num_blocks, usize num_major_stages, const usize *blocks_st
   const bool timing = A.timing != nullptr || arrival_state_offset != 0;
   if (samples) return launch_scan<false, true>(A, stream);
   const bool flow = __atomic_load_n(&g_scan_sync, __ATOMIC_RELAXED);
-  void *buf = prepare(A, A.num_cycles, flow, stream);
+  void *buf = prepare(A, A.num_cycles, flow, !timing, stream);
   const int rc =
       timing ? launch_scan<true, false>(A, stream) : launch_scan<false, false>(A, stream);
   if (buf) (void)hipFreeAsync(buf, stream);
@@ -1790,7 +1985,7 @@ extern "C" int jq_cosim_edges(usize num_blocks, usize num_major_stages,
     return fail("CU count query failed");
   if (!timing && A.num_blocks > (u32)cus)
     k = reinterpret_cast<const void *>(&cosim_kernel<false, 4>);
-  void *buf = prepare(A, num_edges, false, (hipStream_t)stream);
+  void *buf = prepare(A, num_edges, false, false, (hipStream_t)stream);
   hipError_t e = hipLaunchCooperativeKernel(k, dim3(A.num_blocks), dim3(kScanThreads), args, 0,
                                             (hipStream_t)stream);
   if (buf) (void)hipFreeAsync(buf, (hipStream_t)stream);

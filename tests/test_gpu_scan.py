@@ -615,3 +615,35 @@ def test_timing_launches_in_both_sync_modes(xprop, cycles):
         assert np.array_equal(out["sram"][:s.sram_storage_size], sram), mode
         assert out["event_count"] == n_ref and n_ref > 0
         assert np.array_equal(sim.canonical_events(out["events"]), sim.canonical_events(ev_ref))
+
+
+@pytest.mark.parametrize("kw,cycles", [
+    (dict(seed=3, gates=300, depth=9, dffs=40, inputs=5, outputs=7), 9),
+    (dict(seed=4, gates=6000, depth=20, dffs=900, inputs=40, outputs=24, srams=3), 61),
+    # more than 512 words of primary inputs; no flip-flops
+    (dict(seed=5, gates=30000, depth=12, dffs=300, inputs=17000, outputs=32), 12),
+    (dict(seed=6, gates=2000, depth=14, dffs=0, inputs=70, outputs=50), 8),
+    # more state words than stay in LDS
+    (dict(seed=7, gates=200000, depth=12, dffs=140000, inputs=40, outputs=24), 8)])
+def test_one_block_keeps_its_state_in_lds(kw, cycles):
+    """Launches of one block with a small state, beside one whose state is too
+    large and one with X masks (both in the ring): every snapshot and SRAM word
+    is the oracle's, in both sync modes."""
+    from jacquard_amd.netlist import Netlist
+    from jacquard_amd.script import Compiled
+    nl = Netlist.random(geometric_p=0.3, invert_prob=0.4, **kw)
+    comp = Compiled(nl, level_split=3)
+    for xprop in (False, True):
+        s = comp.flatten(1, xprop=xprop)
+        _say("words", s.effective_state_size(), "partitions", s.num_parts)
+        assert (s.effective_state_size() > 4095) == (kw["dffs"] > 100000) or xprop
+        st = stimulus.build_states(s, cycles, seed=4, p=0.3)
+        ref = st.copy()
+        sram = np.zeros(s.sram_storage_size, np.uint32)
+        sram_x = np.full(s.sram_storage_size, 0xFFFFFFFF, np.uint32)
+        oracle.run(s, ref, cycles, sram=sram, sram_x=sram_x if xprop else None)
+        for mode in (1, 0):
+            with _sync_mode(mode):
+                out = sim.run_scan(s, st.copy(), cycles)
+            assert np.array_equal(out["states"], ref), (xprop, mode)
+            assert np.array_equal(out["sram"][:s.sram_storage_size], sram), (xprop, mode)
