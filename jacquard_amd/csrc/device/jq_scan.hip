@@ -133,7 +133,8 @@ __device__ __forceinline__ u32 join_halves(u32 r) {
 // waves to a SIMD the time is that of the instructions, four clocks each per
 // wave: shifting every bit in at the top takes one where masking, shifting
 // and combining it took three.  WIDE: `hi` holds two more index bits each.
-template <bool WIDE>
+// Word i is src[W * i].
+template <bool WIDE, u32 W>
 __device__ __forceinline__ u32 gather_bits_of(const u32 *src, uint4 qa, uint4 qb, u32 hi) {
   const u32 w[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
   u32 d[16];
@@ -144,8 +145,8 @@ __device__ __forceinline__ u32 gather_bits_of(const u32 *src, uint4 qa, uint4 qb
       a |= ((hi >> (4 * k)) & 3u) << 11;
       b |= ((hi >> (4 * k + 2)) & 3u) << 11;
     }
-    d[2 * k] = src[a];
-    d[2 * k + 1] = src[b];
+    d[2 * k] = src[W * a];
+    d[2 * k + 1] = src[W * b];
   }
   // all of them in flight before the first is waited for
   asm volatile("" ::"v"(d[0]), "v"(d[1]), "v"(d[2]), "v"(d[3]), "v"(d[4]), "v"(d[5]), "v"(d[6]),
@@ -159,8 +160,40 @@ __device__ __forceinline__ u32 gather_bits_of(const u32 *src, uint4 qa, uint4 qb
   }
   return join_halves(r);
 }
+// The same of values and X masks that lie side by side: one 8-byte read for
+// both, where two gathers took twice the reads and addresses (100K gates with
+// X, 49.6 -> 44.0 us per cycle; 4M gates with X and timing, 170 -> 158).
+template <bool WIDE>
+__device__ __forceinline__ uint2 gather_pairs_of(const u32 *src, uint4 qa, uint4 qb, u32 hi) {
+  const u64 *pairs = reinterpret_cast<const u64 *>(src);
+  const u32 w[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
+  u64 d[16];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    u32 a = (w[k] & 0xffffu) >> 5, b = w[k] >> 21;
+    if (WIDE) {
+      a |= ((hi >> (4 * k)) & 3u) << 11;
+      b |= ((hi >> (4 * k + 2)) & 3u) << 11;
+    }
+    d[2 * k] = pairs[a];
+    d[2 * k + 1] = pairs[b];
+  }
+  asm volatile("" ::"v"(d[0]), "v"(d[1]), "v"(d[2]), "v"(d[3]), "v"(d[4]), "v"(d[5]), "v"(d[6]),
+               "v"(d[7]), "v"(d[8]), "v"(d[9]), "v"(d[10]), "v"(d[11]), "v"(d[12]), "v"(d[13]),
+               "v"(d[14]), "v"(d[15]));
+  u32 r = 0, x = 0;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    r = push_bit(r, (u32)d[2 * k], w[k]);
+    x = push_bit(x, (u32)(d[2 * k] >> 32), w[k]);
+    r = push_bit(r, (u32)d[2 * k + 1], w[k] >> 16);
+    x = push_bit(x, (u32)(d[2 * k + 1] >> 32), w[k] >> 16);
+  }
+  return make_uint2(join_halves(r), join_halves(x));
+}
+template <u32 W>
 __device__ __forceinline__ u32 gather_bits(const u32 *src, uint4 qa, uint4 qb) {
-  return gather_bits_of<false>(src, qa, qb, 0);
+  return gather_bits_of<false, W>(src, qa, qb, 0);
 }
 
 // ---- composed stage-0 permutations
@@ -595,18 +628,18 @@ constexpr u32 kLayerWords = 256 + 64;
 // One hier level of wave 0's tree (kernel_v1_impl.cuh:236-293): on entry
 // lane i holds word 2HW + i (lanes i < 2HW); on exit lane i < HW holds word
 // HW + i, also written to the layer.  Word w's flags are fA on lane w.
-template <int HW, bool TIMING, bool X>
+template <int HW, bool TIMING, bool X, u32 W>
 __device__ __forceinline__ void tree_level(u32 &cur, u32 &curx, u16 &cura, const uint4 &fA,
-                                           int lane, u32 *st_v, u32 *st_x, u16 *st_arr) {
+                                           int lane, u32 *st, u16 *st_arr) {
   const u32 b = from_lane_up<HW>(cur);
   const u32 xa = from_lane_up<HW>(fA.x), xb = from_lane_up<HW>(fA.y);
   const u32 ob = from_lane_up<HW>(fA.z);
   const u32 at = lane < HW ? HW + lane : 256 + lane;
   const u32 n = gate(cur, b, xa, xb, ob);
-  st_v[at] = n;
+  st[W * at] = n;
   if (X) {
     curx = gate_x(cur, curx, b, from_lane_up<HW>(curx), xa, xb, ob);
-    st_x[at] = curx;
+    st[W * at + 1] = curx;
   }
   if (TIMING) {
     const u32 dly = from_lane_up<HW>(fA.w);
@@ -618,29 +651,29 @@ __device__ __forceinline__ void tree_level(u32 &cur, u32 &curx, u16 &cura, const
 
 // The AND tree of a boomerang stage, in wave 0: the shuffled words in hin
 // become the 256 words of the layer.
-template <bool TIMING, bool X>
+template <bool TIMING, bool X, u32 W>
 __device__ __forceinline__ void run_tree(const uint4 &fA, const uint4 &fB, const uint4 &fC,
-                                         const uint4 &fD, const u32 *hin_v, const u32 *hin_x,
-                                         u32 *st_v, u32 *st_x, u16 *st_arr) {
+                                         const uint4 &fD, const u32 *hin, u32 *st,
+                                         u16 *st_arr) {
   const int lane = threadIdx.x & 63;
   // hier0: words 128+L, 192+L; hier1: word 64+L
-  const u32 s0 = hin_v[lane], s1 = hin_v[64 + lane];
-  const u32 s2 = hin_v[128 + lane], s3 = hin_v[192 + lane];
+  const u32 s0 = hin[W * lane], s1 = hin[W * (64 + lane)];
+  const u32 s2 = hin[W * (128 + lane)], s3 = hin[W * (192 + lane)];
   const u32 o2 = gate(s0, s2, fC.x, fC.y, fC.z);
   const u32 o3 = gate(s1, s3, fD.x, fD.y, fD.z);
   u32 cur = gate(o2, o3, fB.x, fB.y, fB.z), curx = 0;
-  st_v[128 + lane] = o2;
-  st_v[192 + lane] = o3;
-  st_v[64 + lane] = cur;
+  st[W * (128 + lane)] = o2;
+  st[W * (192 + lane)] = o3;
+  st[W * (64 + lane)] = cur;
   if (X) {
-    const u32 x0 = hin_x[lane], x1 = hin_x[64 + lane];
-    const u32 x2 = hin_x[128 + lane], x3 = hin_x[192 + lane];
+    const u32 x0 = hin[W * lane + 1], x1 = hin[W * (64 + lane) + 1];
+    const u32 x2 = hin[W * (128 + lane) + 1], x3 = hin[W * (192 + lane) + 1];
     const u32 o2x = gate_x(s0, x0, s2, x2, fC.x, fC.y, fC.z);
     const u32 o3x = gate_x(s1, x1, s3, x3, fD.x, fD.y, fD.z);
     curx = gate_x(o2, o2x, o3, o3x, fB.x, fB.y, fB.z);
-    st_x[128 + lane] = o2x;
-    st_x[192 + lane] = o3x;
-    st_x[64 + lane] = curx;
+    st[W * (128 + lane) + 1] = o2x;
+    st[W * (192 + lane) + 1] = o3x;
+    st[W * (64 + lane) + 1] = curx;
   }
   u16 cura = 0;
   if (TIMING) {
@@ -655,12 +688,12 @@ __device__ __forceinline__ void run_tree(const uint4 &fA, const uint4 &fB, const
   // the node's flags (word L's on lane L in fA) move up by hw with
   // v_permlane32_swap, v_permlane16_swap and DPP row shifts, a few cycles
   // each, instead of LDS permutes
-  tree_level<32, TIMING, X>(cur, curx, cura, fA, lane, st_v, st_x, st_arr);
-  tree_level<16, TIMING, X>(cur, curx, cura, fA, lane, st_v, st_x, st_arr);
-  tree_level<8, TIMING, X>(cur, curx, cura, fA, lane, st_v, st_x, st_arr);
-  tree_level<4, TIMING, X>(cur, curx, cura, fA, lane, st_v, st_x, st_arr);
-  tree_level<2, TIMING, X>(cur, curx, cura, fA, lane, st_v, st_x, st_arr);
-  tree_level<1, TIMING, X>(cur, curx, cura, fA, lane, st_v, st_x, st_arr);
+  tree_level<32, TIMING, X, W>(cur, curx, cura, fA, lane, st, st_arr);
+  tree_level<16, TIMING, X, W>(cur, curx, cura, fA, lane, st, st_arr);
+  tree_level<8, TIMING, X, W>(cur, curx, cura, fA, lane, st, st_arr);
+  tree_level<4, TIMING, X, W>(cur, curx, cura, fA, lane, st, st_arr);
+  tree_level<2, TIMING, X, W>(cur, curx, cura, fA, lane, st, st_arr);
+  tree_level<1, TIMING, X, W>(cur, curx, cura, fA, lane, st, st_arr);
   // in-word tail hier8..12 on lane 0 from word 1, now on lane 0
   // (kernel_v1_impl.cuh:294-346)
   const u32 v1 = cur, v1x = curx, xa = fA.x, xb = fA.y, ob = fA.z;
@@ -670,14 +703,14 @@ __device__ __forceinline__ void run_tree(const uint4 &fA, const uint4 &fB, const
   const u32 r10 = ((r9 >> 4) ^ xa) & (((r9 >> 8) ^ xb) | ob) & 0xf0u;
   const u32 r11 = ((r10 >> 2) ^ xa) & (((r10 >> 4) ^ xb) | ob) & 0xcu;
   const u32 r12 = ((r11 >> 1) ^ xa) & (((r11 >> 2) ^ xb) | ob) & 0x2u;
-  st_v[at] = r8 | r9 | r10 | r11 | r12;
+  st[W * at] = r8 | r9 | r10 | r11 | r12;
   if (X) {
     const u32 x8 = gate_x(v1 << 16, v1x << 16, v1, v1x, xa, xb, ob) & 0xffff0000u;
     const u32 x9 = gate_x(r8 >> 8, x8 >> 8, r8 >> 16, x8 >> 16, xa, xb, ob) & 0xff00u;
     const u32 x10 = gate_x(r9 >> 4, x9 >> 4, r9 >> 8, x9 >> 8, xa, xb, ob) & 0xf0u;
     const u32 x11 = gate_x(r10 >> 2, x10 >> 2, r10 >> 4, x10 >> 4, xa, xb, ob) & 0xcu;
     const u32 x12 = gate_x(r11 >> 1, x11 >> 1, r11 >> 2, x11 >> 2, xa, xb, ob) & 0x2u;
-    st_x[at] = x8 | x9 | x10 | x11 | x12;
+    st[W * at + 1] = x8 | x9 | x10 | x11 | x12;
   }
   if (TIMING) st_arr[at] = 0;
 }
@@ -877,17 +910,21 @@ __device__ __forceinline__ void start_walk(const ScanArgs &A, u32 cycles, Walk &
   wait_loads();
 }
 
+// X: the launch may have X-capable partitions; the LDS arrays then hold a
+// word's X mask beside it.
+//
 // One partition (src/sim/cpu_reference.rs:25-262 per partition;
 // kernel_v1_impl.cuh:62-558), its prologue loads already in P; `hn` is the
 // block's next partition (num_stages 0: none), whose prologue replaces them.
-template <bool TIMING, bool PROFILE, bool FLOW>
+template <bool TIMING, bool PROFILE, bool FLOW, bool X>
 __device__ __forceinline__ void run_partition(const ScanArgs &A, const u32 *__restrict__ bd,
                               Walk &wk, u32 cycles, PartPre &P,
                               const Flow &F, const u32 *__restrict__ in,
                               u32 *__restrict__ out,
-                              u32 cycle, u32 part, u32 *st_v, u32 *st_x,
-                              u32 *hin_v, u32 *hin_x, u32 *wo_v, u32 *wo_x,
-                              u16 *st_arr, u16 *wo_arr, u32 *raw_v, u32 *raw_x) {
+                              u32 cycle, u32 part, u32 *st, u32 *hin, u32 *wo,
+                              u16 *st_arr, u16 *wo_arr, u32 *raw) {
+  // word i of an LDS array is at W * i, its X mask beside it
+  constexpr u32 W = X ? 2 : 1;
   const int lane = threadIdx.x & 63;
   const bool w0 = threadIdx.x < 64;
   // the thread's word, and its first thread
@@ -906,15 +943,15 @@ __device__ __forceinline__ void run_partition(const ScanArgs &A, const u32 *__re
   const u32 sram_offset = h.sram_offset;
   const u32 rounds = h.num_stages ? h.rounds : 0;
   const u32 num_dups = h.num_dups;
-  const bool is_x = h.is_x != 0;
+  const bool is_x = X && h.is_x != 0;
   const u32 xoff = h.xoff;
   const u32 hook = (threadIdx.x & 2) ? P.hook >> 16 : P.hook & 0xffffu;
   const bool comp = !PROFILE && h.slot != kNoSlot && h.num_stages != 0;
   const Section S = section_of(bd, h), Sn = section_of(bd, hn);
   const uint2 *gr = reinterpret_cast<const uint2 *>(bd + h.base + 256);
   const uint2 *e = P.e;
-  u32 st = stage0(h);                        // this stage's section
-  const u32 sd = st + 5120 * h.num_stages;     // SRAM/dup section
+  u32 at = stage0(h);                        // this stage's section
+  const u32 sd = at + 5120 * h.num_stages;     // SRAM/dup section
   const u32 ck = sd + 5120;                  // clock-enable section
   const u32 nperm = h.num_stages ? num_srams * 4 + num_dups : 0;
   uint4 sda, sdb, sdf, cka, ckb, ckf;
@@ -957,14 +994,13 @@ __device__ __forceinline__ void run_partition(const ScanArgs &A, const u32 *__re
       }
       if (comp) {
         const u32 n = num_rounds(rounds);
-        u32 *rv = raw_v + 1 + 256 * first_round(rounds) + t;
-        u32 *rx = raw_x + 1 + 256 * first_round(rounds) + t;
+        u32 *rv = raw + W * (1 + 256 * first_round(rounds) + t);
 #pragma unroll
         for (u32 k = 0; k < kPreRounds; ++k) {
           if (k >= most) break;
           if (k < n) {
-            rv[256 * k] = v[k];
-            if (is_x) rx[256 * k] = x[k];
+            rv[W * 256 * k] = v[k];
+            if (is_x) rv[W * 256 * k + 1] = x[k];
           }
         }
       } else if (is_x) {
@@ -1002,8 +1038,8 @@ __device__ __forceinline__ void run_partition(const ScanArgs &A, const u32 *__re
       }
       if (comp) {
         const u32 i = 1 + 256 * (first_round(rounds) + r) + t;
-        raw_v[i] = v;
-        if (is_x) raw_x[i] = x;
+        raw[W * i] = v;
+        if (is_x) raw[W * i + 1] = x;
       } else {
         for (u32 m = er.y; m; m &= m - 1) {
           const u32 p = __builtin_ctz(m);
@@ -1024,8 +1060,8 @@ __device__ __forceinline__ void run_partition(const ScanArgs &A, const u32 *__re
     load_entries(P, Sn, hn.rounds);
     if (h0) {
       if (!comp) {
-        st_v[t] = acc_v;
-        st_x[t] = acc_x;
+        st[W * t] = acc_v;
+        if (X) st[W * t + 1] = acc_x;
       }
       if (TIMING) wo_arr[t] = 0;  // pinned rule: reset per partition
     }
@@ -1034,41 +1070,49 @@ __device__ __forceinline__ void run_partition(const ScanArgs &A, const u32 *__re
     // ---- boomerang stages
     for (u32 bs = 0; bs < num_stages; ++bs) {
       u32 hv, hx = 0;
-      if (bs != 0 || !comp) {
-        hv = gather_bits(st_v, P.qa, P.qb);
-        if (is_x) hx = gather_bits(st_x, P.qa, P.qb);
-      } else if (rounds <= kNarrowRounds) {
-        hv = gather_bits_of<false>(raw_v, P.qa, P.qb, 0);
-        if (is_x) hx = gather_bits_of<false>(raw_x, P.qa, P.qb, 0);
+      const bool raw_bits = bs == 0 && comp, wide = rounds > kNarrowRounds;
+      if (X && is_x) {
+        uint2 q;
+        if (!raw_bits)
+          q = gather_pairs_of<false>(st, P.qa, P.qb, 0);
+        else if (!wide)
+          q = gather_pairs_of<false>(raw, P.qa, P.qb, 0);
+        else
+          q = gather_pairs_of<true>(raw, P.qa, P.qb, P.hi);
+        hv = q.x;
+        hx = q.y;
+      } else if (!raw_bits) {
+        hv = gather_bits<W>(st, P.qa, P.qb);
+      } else if (!wide) {
+        hv = gather_bits<W>(raw, P.qa, P.qb);
       } else {
-        hv = gather_bits_of<true>(raw_v, P.qa, P.qb, P.hi);
-        if (is_x) hx = gather_bits_of<true>(raw_x, P.qa, P.qb, P.hi);
+        hv = gather_bits_of<true, W>(raw, P.qa, P.qb, P.hi);
       }
       // the next section (the next stage's, or the first of the next
       // partition) is loaded now, a stage ahead of its use; this one's came
       // with the previous stage
       const uint4 fA = P.fA, fB = P.fB, fC = P.fC, fD = P.fD;
-      st += 5120;
+      at += 5120;
       const bool more = bs + 1 < num_stages;
       const Section pn = perm0(A.table, hn, Sn);
-      load_stage(P, more ? S : pn, more ? st : perm0_at(hn), more ? S : Sn,
-                 more ? st : stage0(hn));
+      load_stage(P, more ? S : pn, more ? at : perm0_at(hn), more ? S : Sn,
+                 more ? at : stage0(hn));
       if (!more) P.hi = load_hi(pn, hn);
       if (h0) {
-        hin_v[t] = hv;
-        hin_x[t] = hx;
+        hin[W * t] = hv;
+        if (X) hin[W * t + 1] = hx;
       }
       __syncthreads();
       if (w0) {
         if (is_x)
-          run_tree<TIMING, true>(fA, fB, fC, fD, hin_v, hin_x, st_v, st_x, st_arr);
+          run_tree<TIMING, X, W>(fA, fB, fC, fD, hin, st, st_arr);
         else
-          run_tree<TIMING, false>(fA, fB, fC, fD, hin_v, hin_x, st_v, st_x, st_arr);
+          run_tree<TIMING, false, W>(fA, fB, fC, fD, hin, st, st_arr);
       }
       __syncthreads();
       if (h0 && (hook >> 8) == bs) {
-        wo_v[t] = st_v[hook & 255];
-        if (is_x) wo_x[t] = st_x[hook & 255];
+        wo[W * t] = st[W * (hook & 255)];
+        if (is_x) wo[W * t + 1] = st[W * (hook & 255) + 1];
         if (TIMING) wo_arr[t] = st_arr[hook & 255];
       }
     }
@@ -1083,8 +1127,13 @@ __device__ __forceinline__ void run_partition(const ScanArgs &A, const u32 *__re
       u32 pv = 0, px = 0;
       if ((u32)t < nperm) {
         asm volatile("" : "+v"(sdf.y));  // its inverse is not taken at the load
-        pv = (gather_bits(wo_v, sda, sdb) & ~sdf.y) ^ sdf.x;
-        if (is_x) px = gather_bits(wo_x, sda, sdb) & ~sdf.y;
+        if (X && is_x) {
+          const uint2 q = gather_pairs_of<false>(wo, sda, sdb, 0);
+          pv = (q.x & ~sdf.y) ^ sdf.x;
+          px = q.y & ~sdf.y;
+        } else {
+          pv = (gather_bits<W>(wo, sda, sdb) & ~sdf.y) ^ sdf.x;
+        }
       }
       const u32 en = __shfl(pv, (lane + 2) & 63);
       const u32 wdata = __shfl(pv, (lane + 4) & 63);
@@ -1099,7 +1148,7 @@ __device__ __forceinline__ void run_partition(const ScanArgs &A, const u32 *__re
           u32 *ram = A.sram_data + st;
           u32 rv = ram[ra], w0v = ram[wa];
           ram[wa] = (w0v & ~en) | (wdata & en);
-          wo_v[num_ios - num_srams + s] = rv;
+          wo[W * (num_ios - num_srams + s)] = rv;
           if (is_x) {
             u32 rx = 0;
             if (A.sram_xmask) {
@@ -1108,13 +1157,13 @@ __device__ __forceinline__ void run_partition(const ScanArgs &A, const u32 *__re
               u32 w0x = ramx[wa];
               ramx[wa] = (w0x & ~en) | (wdata_x & en);
             }
-            wo_x[num_ios - num_srams + s] = rx;
+            wo[W * (num_ios - num_srams + s) + 1] = rx;
           }
         }
       } else if (h0 && (u32)t < nperm) {
         u32 d = num_ios - num_srams - num_dups + ((u32)t - num_srams * 4);
-        wo_v[d] = pv;
-        if (is_x) wo_x[d] = px;
+        wo[W * d] = pv;
+        if (is_x) wo[W * d + 1] = px;
       }
       __syncthreads();
     }
@@ -1128,15 +1177,20 @@ __device__ __forceinline__ void run_partition(const ScanArgs &A, const u32 *__re
         // only words holding DFFs pay for the 32 LDS reads
         const bool gated = f.y != 0xFFFFFFFFu;
         u32 en = f.x;
-        if (gated) en = (gather_bits(wo_v, cka, ckb) & ~f.y) ^ f.x;
         u32 ckx = 0;
-        if (is_x && gated) ckx = gather_bits(wo_x, cka, ckb) & ~f.y;
+        if (X && is_x && gated) {
+          const uint2 q = gather_pairs_of<false>(wo, cka, ckb, 0);
+          en = (q.x & ~f.y) ^ f.x;
+          ckx = q.y & ~f.y;
+        } else if (gated) {
+          en = (gather_bits<W>(wo, cka, ckb) & ~f.y) ^ f.x;
+        }
         if (h0) {
-          u32 data = wo_v[t] ^ f.z;
+          u32 data = wo[W * t] ^ f.z;
           u32 w = io_offset + (u32)t;
           const u32 nv = (old_v & ~en) | (data & en);
           u32 nx = old_x;
-          if (is_x) nx = (old_x & ~en & ~ckx) | (wo_x[t] & en & ~ckx) | ckx;
+          if (is_x) nx = (old_x & ~en & ~ckx) | (wo[W * t + 1] & en & ~ckx) | ckx;
           if (FLOW) {
             const u32 s = cycle + 1;
             const u64 tag = (u64)s << 32;
@@ -1229,10 +1283,11 @@ __global__ __launch_bounds__(256) void flow_owner_kernel(FlowBuild F) {
 }
 
 // Workgroup (m, b) puts the words of snapshot 0 that block b's partitions of
-// major stage m write into the ring and checks their global-read entries: a word at or past the first writeout word must be one
-// that some partition writes, in an earlier stage when it is read from the
-// same cycle; X masks must lie at one offset, past the words themselves (so
-// that two words of 8 bytes for each of the words fit a slot).
+// major stage m write into the ring and checks their global-read entries: a
+// word at or past the first writeout word must be one that some partition
+// writes, in an earlier stage when it is read from the same cycle; X masks
+// must lie at one offset, past the words themselves (so that two words of 8
+// bytes for each of the words fit a slot).
 __global__ __launch_bounds__(256) void flow_check_kernel(FlowBuild F) {
   const u32 m = blockIdx.x / F.nb, b = blockIdx.x % F.nb;
   const u32 t = threadIdx.x;
@@ -1276,16 +1331,14 @@ __global__ __launch_bounds__(256) void flow_check_kernel(FlowBuild F) {
 
 // The LDS arrays of one workgroup.
 #define JQ_SCAN_LDS                                             \
-  __shared__ u32 st_v[kLayerWords], st_x[kLayerWords];          \
-  __shared__ u32 hin_v[256], hin_x[256], wo_v[256], wo_x[256];  \
+  __shared__ __align__(8) u32 st[2 * kLayerWords], hin[512];    \
+  __shared__ __align__(8) u32 wo[512], raw[2 * kRawWords];      \
   __shared__ u16 st_arr[kLayerWords], wo_arr[256];              \
-  __shared__ u32 raw_v[kRawWords], raw_x[kRawWords];            \
   __shared__ u32 s_aborted; /* set by a wait when the launch has aborted */
 
-template <bool TIMING, bool PROFILE, bool FLOW>
-__device__ __forceinline__ void scan_loop(const ScanArgs &A, u32 *st_v, u32 *st_x, u32 *hin_v,
-                                          u32 *hin_x, u32 *wo_v, u32 *wo_x, u16 *st_arr,
-                                          u16 *wo_arr, u32 *raw_v, u32 *raw_x,
+template <bool TIMING, bool PROFILE, bool FLOW, bool X>
+__device__ __forceinline__ void scan_loop(const ScanArgs &A, u32 *st, u32 *hin, u32 *wo,
+                                          u16 *st_arr, u16 *wo_arr, u32 *raw,
                                           u32 &s_aborted, u32 gen) {
   const u32 b = blockIdx.x;
   const u32 nb = A.num_blocks, M = A.num_major_stages;
@@ -1297,7 +1350,7 @@ __device__ __forceinline__ void scan_loop(const ScanArgs &A, u32 *st_v, u32 *st_
     F.slot = (u32)A.state_size;
     F.ring = __builtin_amdgcn_make_buffer_rsrc(A.ring, 0, 8 * kRing * F.slot, 0x00027000);
     F.lo = ~A.flow[kFlowNegLo];
-    F.xoff = A.flow[kFlowXoff];
+    F.xoff = X ? A.flow[kFlowXoff] : 0;
     F.shift = F.xoff ? 4 : 3;
     F.bar = A.bar;
     F.aborted = &s_aborted;
@@ -1312,9 +1365,8 @@ __device__ __forceinline__ void scan_loop(const ScanArgs &A, u32 *st_v, u32 *st_
   for (u32 c = 0, m = 0;;) {
     const bool last = w.cur.num_stages == 0 || w.cur.is_last != 0;
     w.next = settle(w);
-    run_partition<TIMING, PROFILE, FLOW>(A, bd, w, A.num_cycles, P, F, in, out, c, part, st_v,
-                                         st_x, hin_v, hin_x, wo_v, wo_x, st_arr, wo_arr, raw_v,
-                                         raw_x);
+    run_partition<TIMING, PROFILE, FLOW, X>(A, bd, w, A.num_cycles, P, F, in, out, c, part, st,
+                                            hin, wo, st_arr, wo_arr, raw);
     ++part;
     w.cur = w.next;
     if (!last) continue;
@@ -1350,24 +1402,24 @@ __global__ __launch_bounds__(kScanThreads) void scan_kernel(ScanArgs A) {
   }
   JQ_SCAN_LDS
   const int t = threadIdx.x;
-  if (t == 0) s_aborted = raw_v[0] = raw_x[0] = 0;
-  if (t < 256) {
-    st_x[t] = 0;
-    hin_x[t] = 0;
-    wo_x[t] = 0;
-    wo_arr[t] = 0;
-    st_arr[t] = 0;
-  }
+  if (t == 0) s_aborted = raw[0] = raw[1] = 0;
+  hin[t] = wo[t] = 0;
+  if (t < 256) wo_arr[t] = st_arr[t] = 0;
   const u32 gen = read_gen(A.bar);
   __syncthreads();
   // the flag is the same word for every block
-  if (!PROFILE && A.ring != nullptr && A.flow[kFlowBad] == 0)
-    scan_loop<TIMING, PROFILE, !PROFILE>(A, st_v, st_x, hin_v, hin_x, wo_v, wo_x,
-                                                    st_arr, wo_arr, raw_v, raw_x, s_aborted,
-                                                    gen);
-  else
-    scan_loop<TIMING, PROFILE, false>(A, st_v, st_x, hin_v, hin_x, wo_v, wo_x, st_arr, wo_arr,
-                                      raw_v, raw_x, s_aborted, gen);
+  if (!PROFILE && A.ring != nullptr && A.flow[kFlowBad] == 0) {
+    // without X-capable partitions a loop that does not carry the X lane: its
+    // branches alone cost 4.5% (1M gates 53.0 us per cycle, 50.6 without)
+    if (A.flow[kFlowXoff] == 0)
+      scan_loop<TIMING, PROFILE, !PROFILE, false>(A, st, hin, wo, st_arr, wo_arr, raw, s_aborted,
+                                                  gen);
+    else
+      scan_loop<TIMING, PROFILE, !PROFILE, true>(A, st, hin, wo, st_arr, wo_arr, raw, s_aborted,
+                                                 gen);
+  } else {
+    scan_loop<TIMING, PROFILE, false, true>(A, st, hin, wo, st_arr, wo_arr, raw, s_aborted, gen);
+  }
 }
 
 // ---- launches that keep the state in LDS
@@ -1412,8 +1464,8 @@ __device__ __forceinline__ void run_local(const ScanArgs &A, LocalLds &L, Walk &
   const u32 flip = (cycle & 1) ? 0xAAAAAAAAu : 0u;
   __syncthreads();  // the previous partition's writeouts are in the state
   for (u32 bs = 0; bs < num_stages; ++bs) {
-    const u32 hv = bs == 0 ? gather_bits_of<true>(L.state, P.qa, P.qb, P.hi ^ flip)
-                           : gather_bits(L.st, P.qa, P.qb);
+    const u32 hv = bs == 0 ? gather_bits_of<true, 1>(L.state, P.qa, P.qb, P.hi ^ flip)
+                           : gather_bits<1>(L.st, P.qa, P.qb);
     const uint4 fA = P.fA, fB = P.fB, fC = P.fC, fD = P.fD;
     st += 5120;
     const bool more = bs + 1 < num_stages;
@@ -1424,7 +1476,7 @@ __device__ __forceinline__ void run_local(const ScanArgs &A, LocalLds &L, Walk &
     if (h0) L.hin[t] = hv;
     __syncthreads();
     if (threadIdx.x < 64)
-      run_tree<false, false>(fA, fB, fC, fD, L.hin, nullptr, L.st, nullptr, nullptr);
+      run_tree<false, false, 1>(fA, fB, fC, fD, L.hin, L.st, nullptr);
     __syncthreads();
     if (h0 && (hook >> 8) == bs) L.wo[t] = L.st[hook & 255];
   }
@@ -1432,7 +1484,7 @@ __device__ __forceinline__ void run_local(const ScanArgs &A, LocalLds &L, Walk &
   __syncthreads();
   if (nperm) {
     u32 pv = 0;
-    if ((u32)t < nperm) pv = (gather_bits(L.wo, sda, sdb) & ~sdf.y) ^ sdf.x;
+    if ((u32)t < nperm) pv = (gather_bits<1>(L.wo, sda, sdb) & ~sdf.y) ^ sdf.x;
     const u32 en = __shfl(pv, (lane + 2) & 63);
     const u32 wdata = __shfl(pv, (lane + 4) & 63);
     __syncthreads();
@@ -1453,7 +1505,7 @@ __device__ __forceinline__ void run_local(const ScanArgs &A, LocalLds &L, Walk &
   }
   if ((u32)t < num_ios) {
     u32 en = ckf.x;
-    if (ckf.y != 0xFFFFFFFFu) en = (gather_bits(L.wo, cka, ckb) & ~ckf.y) ^ ckf.x;
+    if (ckf.y != 0xFFFFFFFFu) en = (gather_bits<1>(L.wo, cka, ckb) & ~ckf.y) ^ ckf.x;
     if (h0) {
       const u32 w = h.io_offset + (u32)t;
       const u32 old = L.state[(cycle & 1) * kLocalHalf + w];
@@ -1507,17 +1559,16 @@ __global__ __launch_bounds__(kScanThreads) void local_kernel(ScanArgs A) {
   }
   JQ_SCAN_LDS
   const int t = threadIdx.x;
-  if (t == 0) s_aborted = raw_v[0] = raw_x[0] = 0;
-  if (t < 256) st_x[t] = hin_x[t] = wo_x[t] = wo_arr[t] = st_arr[t] = 0;
+  if (t == 0) s_aborted = raw[0] = raw[1] = 0;
+  hin[t] = wo[t] = 0;
+  if (t < 256) wo_arr[t] = st_arr[t] = 0;
   const u32 gen = read_gen(A.bar);
   __syncthreads();
   A.table = nullptr;  // its permutations are for the state in LDS
   if (A.flow[kFlowBad] == 0)
-    scan_loop<false, false, true>(A, st_v, st_x, hin_v, hin_x, wo_v, wo_x, st_arr, wo_arr, raw_v,
-                                  raw_x, s_aborted, gen);
+    scan_loop<false, false, true, true>(A, st, hin, wo, st_arr, wo_arr, raw, s_aborted, gen);
   else
-    scan_loop<false, false, false>(A, st_v, st_x, hin_v, hin_x, wo_v, wo_x, st_arr, wo_arr, raw_v,
-                                   raw_x, s_aborted, gen);
+    scan_loop<false, false, false, true>(A, st, hin, wo, st_arr, wo_arr, raw, s_aborted, gen);
 }
 
 // Persistent co-simulation: C.num_edges edges of one cycle each over the
@@ -1538,14 +1589,9 @@ __global__ __launch_bounds__(kScanThreads, WAVES) void cosim_kernel(ScanArgs A, 
   }
   JQ_SCAN_LDS
   const int t = threadIdx.x;
-  if (t == 0) s_aborted = raw_v[0] = raw_x[0] = 0;
-  if (t < 256) {
-    st_x[t] = 0;
-    hin_x[t] = 0;
-    wo_x[t] = 0;
-    wo_arr[t] = 0;
-    st_arr[t] = 0;
-  }
+  if (t == 0) s_aborted = raw[0] = raw[1] = 0;
+  hin[t] = wo[t] = 0;
+  if (t < 256) wo_arr[t] = st_arr[t] = 0;
   __shared__ u32 pins[cosim::kNumPins];
   if (C.fs && (u32)t < cosim::kNumPins) pins[t] = C.pins[t];
   u32 gen = read_gen(A.bar);
@@ -1571,9 +1617,8 @@ __global__ __launch_bounds__(kScanThreads, WAVES) void cosim_kernel(ScanArgs A, 
       // co-simulation snapshots are 2-state: a partition flagged X-capable
       // runs its value lane only
       w.cur.is_x = 0;
-      run_partition<TIMING, false, false>(A, bd, w, C.num_edges, P, F, in, out, 0u, 0u, st_v,
-                                          st_x, hin_v, hin_x, wo_v, wo_x, st_arr, wo_arr, raw_v,
-                                          raw_x);
+      run_partition<TIMING, false, false, false>(A, bd, w, C.num_edges, P, F, in, out, 0u, 0u, st,
+                                                 hin, wo, st_arr, wo_arr, raw);
       w.cur = w.next;
       if (!last) continue;
       grid_sync_coherent(A.bar, nb, b, gen, &g_error, &g_wait_polls, s_aborted);
