@@ -1329,11 +1329,12 @@ __global__ __launch_bounds__(256) void flow_check_kernel(FlowBuild F) {
   if (bad) atomicOr(&F.flow[kFlowBad], bad);
 }
 
-// The LDS arrays of one workgroup.
-#define JQ_SCAN_LDS                                             \
-  __shared__ __align__(8) u32 st[2 * kLayerWords], hin[512];    \
-  __shared__ __align__(8) u32 wo[512], raw[2 * kRawWords];      \
-  __shared__ u16 st_arr[kLayerWords], wo_arr[256];              \
+// The LDS arrays of one workgroup, W words apiece (2: X masks beside the
+// values).
+#define JQ_SCAN_LDS(W)                                              \
+  __shared__ __align__(8) u32 st[W * kLayerWords], hin[W * 256];    \
+  __shared__ __align__(8) u32 wo[W * 256], raw[W * kRawWords];      \
+  __shared__ u16 st_arr[kLayerWords], wo_arr[256];                  \
   __shared__ u32 s_aborted; /* set by a wait when the launch has aborted */
 
 template <bool TIMING, bool PROFILE, bool FLOW, bool X>
@@ -1400,7 +1401,7 @@ __global__ __launch_bounds__(kScanThreads) void scan_kernel(ScanArgs A) {
     A.clock_ps = A.timing[0];
     A.constraints = A.timing + 1;
   }
-  JQ_SCAN_LDS
+  JQ_SCAN_LDS(2)
   const int t = threadIdx.x;
   if (t == 0) s_aborted = raw[0] = raw[1] = 0;
   hin[t] = wo[t] = 0;
@@ -1557,7 +1558,7 @@ __global__ __launch_bounds__(kScanThreads) void local_kernel(ScanArgs A) {
     local_loop(A, L);
     return;
   }
-  JQ_SCAN_LDS
+  JQ_SCAN_LDS(2)
   const int t = threadIdx.x;
   if (t == 0) s_aborted = raw[0] = raw[1] = 0;
   hin[t] = wo[t] = 0;
@@ -1587,11 +1588,10 @@ __global__ __launch_bounds__(kScanThreads, WAVES) void cosim_kernel(ScanArgs A, 
     A.clock_ps = A.timing[0];
     A.constraints = A.timing + 1;
   }
-  JQ_SCAN_LDS
+  JQ_SCAN_LDS(1)
   const int t = threadIdx.x;
-  if (t == 0) s_aborted = raw[0] = raw[1] = 0;
-  hin[t] = wo[t] = 0;
-  if (t < 256) wo_arr[t] = st_arr[t] = 0;
+  if (t == 0) s_aborted = raw[0] = 0;
+  if (t < 256) hin[t] = wo[t] = wo_arr[t] = st_arr[t] = 0;
   __shared__ u32 pins[cosim::kNumPins];
   if (C.fs && (u32)t < cosim::kNumPins) pins[t] = C.pins[t];
   u32 gen = read_gen(A.bar);
