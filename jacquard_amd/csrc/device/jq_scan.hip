@@ -1298,9 +1298,8 @@ __global__ __launch_bounds__(256) void flow_check_kernel(FlowBuild F) {
     const u32 *s = F.bd + off;
     const u32 ns = s[0], is_last = s[1], nio = s[2], io = s[3], rounds = s[6];
     if (ns == 0) break;
-    if (xoff && ((s[8] && s[9] != xoff) || (usize)io + nio > xoff ||
-                 (usize)xoff + io + nio > F.state_size))
-      bad |= 4u;
+    if (s[8] && (xoff == 0 || s[9] != xoff)) bad |= 4u;
+    if (xoff && ((usize)io + nio > xoff || (usize)xoff + io + nio > F.state_size)) bad |= 4u;
     // snapshot 0 (tag 0) into the ring
     const usize w = (usize)io + t;
     if (t < nio && nio <= 256u && w + xoff < F.state_size) {

@@ -488,6 +488,36 @@ def test_a_script_that_reads_past_the_writeouts_keeps_grid_barriers():
     assert np.array_equal(got, ref)
 
 
+@pytest.mark.parametrize("blocks", [1, 48])
+def test_x_masks_at_offset_0_keep_grid_barriers(blocks):
+    """X-capable partitions whose masks lie on the words themselves: the
+    launch without the X lane must not take them for partitions without X."""
+    nl, comp = design("sync", level_split=4, seed=9, gates=8000, depth=24,
+                      dffs=800, inputs=64, outputs=32, geometric_p=0.3)
+    s = comp.flatten(blocks, xprop=True)
+    bd = np.array(s.blocks_data, np.uint32)
+    capable = 0
+    for off in s.parts[:, 3].tolist():
+        if bd[int(off) + 8]:
+            bd[int(off) + 9] = 0
+            capable += 1
+    assert capable > 0
+
+    class Script:
+        blocks_data = bd
+
+        def __getattr__(self, name):
+            return getattr(s, name)
+
+    cycles = 40
+    st = stimulus.build_states(s, cycles, seed=21, p=0.3)
+    got = []
+    for mode in (0, 1):
+        with _sync_mode(mode):
+            got.append(sim.run_scan(Script(), st.copy(), cycles, validate=False)["states"])
+    assert np.array_equal(got[0], got[1])
+
+
 @pytest.mark.parametrize("blocks,xprop", [(3, True), (1, False), (61, True)])
 def test_dataflow_over_many_laps_of_the_ring(blocks, xprop):
     """300 cycles, 37 laps of the exchange ring, with one block, with fewer
