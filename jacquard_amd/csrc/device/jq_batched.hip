@@ -564,10 +564,11 @@ __global__ __launch_bounds__(kT) void batched_kernel(BArgs A) {
     }
   }
   // header and gather entries of the block's first partition of major
-  // stage 0
+  // stage 0; a block without one has no row of the table there (past the
+  // script's last partition the table ends)
   u32 src[kG];
   BHdr h = load_bhdr(A.bd + A.bs[b]);
-  load_sources(src, A.gsrc + (size_t)A.gidx[b] * kLayerWords);
+  if (uniform(h.a.x) != 0) load_sources(src, A.gsrc + (size_t)A.gidx[b] * kLayerWords);
   __syncthreads();
   u32 c = c0;
   for (;; ++c) {

@@ -300,3 +300,34 @@ def test_batched_snapshots_around_32_bit_offsets(rio):
     got = BatchedRun(w, seeds, probs, cycles, groups=1).run(validate=False)
     for k in range(len(seeds)):
         assert np.array_equal(got[k], want[k]), k
+
+
+def test_blocks_without_partitions_read_no_row_of_the_gather_table():
+    """The entries of a (stage, block) without partitions name the row after
+    the preceding partition's, and past the last partition there is none: the
+    table lies at the very end of its allocation, whose last row is the last
+    partition's."""
+    import torch
+    from jacquard_amd import sim
+    nl, comp = design("c1", level_split=2, **CONFIG1)
+    s = comp.flatten(16)
+    start = s.part_index()
+    assert (start[1:16] == 1).all()  # blocks 1.. have nothing in stage 0
+    start[1:16] = s.num_parts  # as in a script whose only stage this is
+    seeds, probs, cycles = _lanes(20, 10, 30, 8)
+    run = BatchedRun(s, seeds, probs, cycles, groups=1)
+    run.prepare()
+    table = run.d["gtab"]
+    buf = torch.zeros(1 << 22, dtype=torch.int32, device="cuda")  # 16 MiB
+    buf[-table.numel():] = table
+    run.d["gtab"] = buf[-table.numel():]
+    run.d["gstart"] = sim.to_device(start)
+    run.launch()
+    torch.cuda.synchronize()
+    assert not sim.device_error()
+    got = run.lane_outputs()
+    for lane in range(20):
+        c = int(cycles[lane])
+        st = stimulus.build_states(s, c, seed=int(seeds[lane]), p=float(probs[lane]))
+        oracle.run(s, st, c)
+        assert np.array_equal(got[lane], plain_observations(s, st, c, run.obs_lits)), lane
