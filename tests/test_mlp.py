@@ -184,3 +184,30 @@ def test_gpu_dimensions_off_the_matrix_tiles(dims, n):
     assert np.allclose(m.params.cpu().numpy(), p64 - 0.25 * g_ref, rtol=1e-4,
                        atol=1e-5 * max(scale, 1))
     assert np.isclose(loss.item(), mo.loss(p64, x64, t64, i, h1, h2), rtol=1e-4)
+
+
+@pytest.mark.gpu
+def test_a_partition_takes_as_long_first_in_its_block_as_elsewhere():
+    """Profiled ticks are the partition's own: flattened for several block
+    counts, the partitions that lead their block in one placement and follow
+    another in the next take as long in both.  A first-layer gather is about
+    a quarter of a partition here, so ticks that hold it in one place only
+    would differ by that; 10% leaves room for colder caches behind a
+    barrier."""
+    from helpers import design
+    from jacquard_amd import costmodel as CM
+    nl, comp = design("cm", level_split=4, seed=2, gates=300000, depth=48, dffs=20000,
+                      inputs=256, outputs=128, geometric_p=0.3, invert_prob=0.5)
+    seen = {}
+    for W in (12, 10, 8, 6):
+        s, ticks = CM.profile_batched(comp, W, 2, 18)
+        block = None
+        for (m, b, i, _o, _l), v in zip(s.parts.tolist(), np.median(ticks[2:], 0).tolist()):
+            seen.setdefault((m, i), ([], []))[int((m, b) == block)].append(v)
+            block = (m, b)
+    ratio = [np.median(first) / np.median(later) for first, later in seen.values()
+             if first and later]
+    print(f"{len(ratio)} partitions, first in the block / elsewhere: {np.median(ratio):.3f}",
+          flush=True)
+    assert len(ratio) >= 30
+    assert abs(np.median(ratio) - 1) < 0.1
