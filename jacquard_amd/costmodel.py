@@ -165,50 +165,24 @@ def profile_batched(compiled, blocks, groups, sample_cycles, costs=None, seed=0)
     return s, ticks.reshape(sample_cycles, s.num_parts).astype(np.float64)
 
 
-def leads_block(script):
-    """bool per partition (blocks_data order): the first of its block in its
-    major stage.  Its ticks hold the first-layer gather, which the batched
-    kernel runs beside the preceding partition for all others."""
-    p = script.parts[:, :2].astype(np.int64)
-    lead = np.ones(len(p), bool)
-    lead[1:] = (p[1:] != p[:-1]).any(axis=1)
-    return lead
-
-
 def training_set(compiled, blocks_list, groups, sample_cycles, skip=2, seed=0):
     """(features float32[n, 24], ticks float64[n], per-partition median
     ticks by (major, index)) from profiled batched launches of several
     flattenings; every (cycle, partition) execution after the first `skip`
-    cycles is one sample, without the lead ticks (profiled_set)."""
-    return profiled_set(compiled, blocks_list, groups, sample_cycles, skip, seed)[:3]
-
-
-def profiled_set(compiled, blocks_list, groups, sample_cycles, skip=2, seed=0):
-    """training_set and the lead ticks that were taken off its samples.
-
-    Whether a partition leads its block is the assignment's doing, not the
-    partition's, and every block has one, so the ticks a leader has more
-    than the same partition elsewhere (the median over partitions seen in
-    both places, `lead ticks`) are taken off its samples: left in, they made
-    the large partitions, which the assignment puts first, look larger still
-    (300K gates on 12 blocks: prediction error 5.0%, without them 3.4%)."""
-    runs, seen = [], {}
+    cycles is one sample."""
+    xs, ys = [], []
+    med = {}
     for k, W in enumerate(blocks_list):
         s, ticks = profile_batched(compiled, W, groups, sample_cycles + skip, seed=seed + k)
-        t, lead = ticks[skip:], leads_block(s)
-        runs.append((s, t, lead))
-        for (mj, _b, idx, _o, _l), v, ld in zip(s.parts.tolist(), np.median(t, 0).tolist(),
-                                                lead.tolist()):
-            seen.setdefault((mj, idx), ([], []))[int(ld)].append(v)
-    both = [np.median(a) - np.median(b) for b, a in seen.values() if a and b]
-    extra = max(0.0, float(np.median(both))) if both else 0.0
-    xs, ys = [], []
-    for s, t, lead in runs:
         f = s.part_features()
+        t = ticks[skip:]
         xs.append(np.repeat(f[None], t.shape[0], 0).reshape(-1, f.shape[1]))
-        ys.append((t - extra * lead[None, :]).reshape(-1))
-    med = {k: float(np.median(b + [v - extra for v in a])) for k, (b, a) in seen.items()}
-    return np.concatenate(xs).astype(np.float32), np.concatenate(ys), med, extra
+        ys.append(t.reshape(-1))
+        m = np.median(t, 0)
+        for (mj, _b, idx, _o, _l), v in zip(s.parts.tolist(), m.tolist()):
+            med.setdefault((mj, idx), []).append(v)
+    med = {k: float(np.median(v)) for k, v in med.items()}
+    return np.concatenate(xs).astype(np.float32), np.concatenate(ys), med
 
 
 def batched_us_per_cycle(script, groups, cycles=48, seed=1, launches=5):
@@ -342,7 +316,7 @@ def learned_merge(compiled, model, blocks, groups=None, sample_cycles=16, epochs
     s1 = trial.flatten_shared(blocks)
     if groups and (ok.any() or okc.any()) and getattr(model, "train_x", None) is not None:
         _s, ticks = profile_batched(trial, blocks, groups, sample_cycles + 2, seed=7)
-        t = ticks[2:] - model.lead_ticks * leads_block(s1)[None, :]
+        t = ticks[2:]
         f1 = s1.part_features()
         X = np.concatenate([model.train_x, np.repeat(f1[None], t.shape[0], 0).reshape(-1, f1.shape[1])])
         y = np.concatenate([model.train_y, t.reshape(-1)])
@@ -383,13 +357,12 @@ def learn_costs(compiled, blocks, groups, sample_cycles=24, epochs=150, log=None
     import time
     widths = sorted({blocks, max(4, blocks - 8), max(4, blocks - 16)}, reverse=True)
     t = time.time()
-    X, y, med, lead_ticks = profiled_set(compiled, widths, groups, sample_cycles)
+    X, y, med = training_set(compiled, widths, groups, sample_cycles)
     t_prof = time.time() - t
     t = time.time()
     model = MLP(seed=1)
     hist = model.fit(X, y, epochs=epochs, lr=0.05, batch=4096)
     model.train_x, model.train_y = X, y  # kept for refits on new samples
-    model.lead_ticks = lead_ticks
     t_fit = time.time() - t
     s0 = compiled.flatten_shared(blocks)
     f0 = s0.part_features()

@@ -211,3 +211,71 @@ def test_a_partition_takes_as_long_first_in_its_block_as_elsewhere():
           flush=True)
     assert len(ratio) >= 30
     assert abs(np.median(ratio) - 1) < 0.1
+
+
+class _Profiled:
+    """Stands for a script with one partition per row of `parts`."""
+
+    def __init__(self, parts):
+        self.parts = np.array([(m, b, i, 0, 0) for m, b, i in parts], np.uint64)
+        self.num_parts = len(parts)
+
+    def part_features(self):
+        return np.arange(self.num_parts * I, dtype=np.float32).reshape(-1, I)
+
+
+def test_training_set_is_the_measured_ticks(monkeypatch):
+    """Every sample is the ticks that were measured, whichever partition came
+    first in its block, and the medians are theirs."""
+    from jacquard_amd import costmodel as CM
+    s = {2: _Profiled([(0, 0, 0), (0, 0, 1), (0, 1, 2), (1, 0, 0)]),
+         1: _Profiled([(0, 0, 2), (0, 0, 0), (0, 0, 1), (1, 0, 0)])}
+    rng = np.random.default_rng(5)
+    ticks = {W: rng.integers(100, 900, (6, 4)).astype(np.float64) for W in s}
+    ticks[2][:, [0, 2, 3]] += 2000  # the first of each block takes longer
+    ticks[1][:, [0, 3]] += 2000
+    monkeypatch.setattr(CM, "profile_batched", lambda comp, W, *a, **kw: (s[W], ticks[W]))
+    X, y, med = CM.training_set(None, [2, 1], 1, 4, skip=2)
+    assert X.shape == (32, I)
+    assert np.array_equal(y, np.concatenate([ticks[W][2:].reshape(-1) for W in (2, 1)]))
+    for key, a, b in (((0, 0), 0, 1), ((0, 1), 1, 2), ((0, 2), 2, 0), ((1, 0), 3, 3)):
+        assert med[key] == np.median([np.median(ticks[2][2:, a]), np.median(ticks[1][2:, b])])
+
+
+def test_learned_merge_takes_a_model_that_the_caller_fitted(monkeypatch):
+    """A model with its training set kept (train_x, train_y) and nothing else
+    is refitted on the trial design's measured ticks."""
+    from jacquard_amd import costmodel as CM
+
+    class Design:
+        def __init__(self, n):
+            self.n = n
+
+        def flatten_shared(self, blocks):
+            return _Profiled([(0, k % blocks, k) for k in range(self.n)])
+
+        def parts_per_stage(self):
+            return [self.n]
+
+        def endpoint_counts(self):
+            return [[2] * self.n]
+
+        def merged(self, pairs):
+            return Design(self.n - len(pairs)), np.ones(len(pairs), bool)
+
+    class Model:
+        train_x, train_y = np.zeros((3, I), np.float32), np.ones(3)
+
+        def predict(self, f):
+            return np.arange(10.0, 10.0 + len(f))
+
+        def fit(self, x, y, **kw):
+            self.fitted = y
+
+    measured = np.full((6, 2), 4000.0)
+    monkeypatch.setattr(CM, "profile_batched",
+                        lambda comp, W, *a, **kw: (comp.flatten_shared(W), measured))
+    model = Model()
+    design, costs, info = CM.learned_merge(Design(4), model, 2, groups=1, sample_cycles=4)
+    assert design.n == 2 and info["merged"] == 2 and info["refit_samples"] == 8
+    assert np.array_equal(model.fitted, [1.0] * 3 + [4000.0] * 8)
