@@ -185,11 +185,9 @@ def training_set(compiled, blocks_list, groups, sample_cycles, skip=2, seed=0):
     return np.concatenate(xs).astype(np.float32), np.concatenate(ys), med
 
 
-def batched_us_per_cycle(script, groups, cycles=48, seed=1, launches=5):
+def batched_us_per_cycle(script, groups, cycles=48, seed=1):
     """Kernel time per group cycle of the batched launch of `script` with
-    `groups` full groups of lanes: the median of `launches` after one that
-    is not timed (a first launch reads its script from HBM, which a long job
-    does not notice, and single launches differ by 1%)."""
+    `groups` full groups of lanes."""
     torch = _torch()
     from .batched import BatchedRun
     n = 32 * groups
@@ -197,19 +195,14 @@ def batched_us_per_cycle(script, groups, cycles=48, seed=1, launches=5):
     run = BatchedRun(script, rng.integers(1, 2**31, n), rng.uniform(0.02, 0.5, n),
                      np.full(n, cycles), obs_lits=[], groups=groups)
     run.prepare()
+    torch.cuda.synchronize()
+    e0 = torch.cuda.Event(enable_timing=True)
+    e1 = torch.cuda.Event(enable_timing=True)
+    e0.record()
     run.launch()
-    us = []
-    for _ in range(launches):
-        run.reset()
-        torch.cuda.synchronize()
-        e0 = torch.cuda.Event(enable_timing=True)
-        e1 = torch.cuda.Event(enable_timing=True)
-        e0.record()
-        run.launch()
-        e1.record()
-        torch.cuda.synchronize()
-        us.append(e0.elapsed_time(e1) * 1e3 / cycles)
-    return float(np.median(us))
+    e1.record()
+    torch.cuda.synchronize()
+    return e0.elapsed_time(e1) * 1e3 / cycles
 
 
 def compare_assignments(compiled, blocks, groups, variants, repeats=3, cycles=48,

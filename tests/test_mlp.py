@@ -279,3 +279,40 @@ def test_learned_merge_takes_a_model_that_the_caller_fitted(monkeypatch):
     design, costs, info = CM.learned_merge(Design(4), model, 2, groups=1, sample_cycles=4)
     assert design.n == 2 and info["merged"] == 2 and info["refit_samples"] == 8
     assert np.array_equal(model.fitted, [1.0] * 3 + [4000.0] * 8)
+
+
+def test_a_trial_is_one_launch(monkeypatch):
+    """batched_us_per_cycle times the one launch it makes: its run-to-run
+    spread, which a gain has to exceed, is that of single launches."""
+    from types import SimpleNamespace
+    from jacquard_amd import batched, costmodel as CM
+    calls = []
+
+    class Run:
+        def __init__(self, script, seeds, probs, cycles, obs_lits, groups):
+            self.n = len(seeds)
+
+        def prepare(self):
+            calls.append("prepare")
+
+        def reset(self):
+            calls.append("reset")
+
+        def launch(self):
+            calls.append("launch")
+
+    class Event:
+        def __init__(self, enable_timing):
+            pass
+
+        def record(self):
+            calls.append("event")
+
+        def elapsed_time(self, end):
+            return 1.6
+
+    cuda = SimpleNamespace(synchronize=lambda: None, Event=Event)
+    monkeypatch.setattr(batched, "BatchedRun", Run)
+    monkeypatch.setattr(CM, "_torch", lambda: SimpleNamespace(cuda=cuda))
+    assert CM.batched_us_per_cycle(None, 2, cycles=16) == pytest.approx(100.0)
+    assert calls == ["prepare", "event", "launch", "event"]
