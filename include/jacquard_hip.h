@@ -250,7 +250,10 @@ usize jq_wait_limit(usize polls);
  * builders find in the script take 68 bytes per state word plus 128 per
  * block.  mode 0: grid barriers everywhere.  mode < 0 only queries.
  * Returns the previous mode.  Results are identical in both modes; set it
- * only while no scan launch is being issued.
+ * only while no scan launch is being issued.  Setup/hold records come in the
+ * order of the cycles and, within one, of its major stages in both (those of
+ * one stage in any order), so an event buffer that overflows has kept the
+ * earliest.
  *
  * In either mode a launch of 8 cycles or more, and a co-simulation launch of
  * 8 edges or more, composes the first-stage permutations of its partitions

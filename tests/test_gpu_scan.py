@@ -677,3 +677,109 @@ def test_one_block_keeps_its_state_in_lds(kw, cycles):
                 out = sim.run_scan(s, st.copy(), cycles)
             assert np.array_equal(out["states"], ref), (xprop, mode)
             assert np.array_equal(out["sram"][:s.sram_storage_size], sram), (xprop, mode)
+
+
+def _stage_of_word(script):
+    """{state word: major stage that writes it}."""
+    bd = np.asarray(script.blocks_data, np.uint32)
+    return {w: int(m) for m, _b, _i, off, _l in script.parts.tolist()
+            for w in range(int(bd[int(off) + 3]), int(bd[int(off) + 3]) + int(bd[int(off) + 2]))}
+
+
+@pytest.mark.parametrize("xprop", [False, True])
+@pytest.mark.parametrize("blocks,capacity", [(1, 100), (24, 7), (24, 1024), (68, 1 << 20)])
+def test_violations_come_in_the_order_of_the_stages(xprop, blocks, capacity):
+    """In both sync modes the records lie in the buffer cycle by cycle and
+    stage by stage, as a barrier after every stage brings them, and one that
+    overflows has kept the earliest: every violation of a (cycle, stage)
+    before that of its last record is there."""
+    from jacquard_amd.script import Compiled
+    nl, _ = design("xts", level_split=6, seed=9, gates=40000, depth=48,
+                   dffs=3000, inputs=64, outputs=32, geometric_p=0.3, srams=2,
+                   delay=(20, 200))
+    s = Compiled(nl, level_split=6, max_part_nodes=400).flatten(blocks, xprop=xprop)
+    s.inject_timing()
+    s.enable_timing_arrivals()
+    cons = s.build_timing_constraint_buffer(1000, 50, 20)
+    cycles = 60
+    stage = _stage_of_word(s)
+
+    def when(events):
+        return [(int(e["cycle"]), stage[int(e["data"][0])]) for e in events]
+
+    st = stimulus.build_states(s, cycles, seed=16, p=0.3)
+    ev_ref, n_ref = oracle.run(s, st.copy(), cycles, sram=np.zeros(s.sram_storage_size, np.uint32),
+                               sram_x=np.full(s.sram_storage_size, 0xFFFFFFFF, np.uint32)
+                               if xprop else None,
+                               constraints=cons, arrival_state_offset=s.arrival_state_offset,
+                               event_capacity=1 << 20)
+    ref = when(ev_ref)
+    full = {bytes(e) for e in sim.canonical_events(ev_ref)}
+    assert n_ref == len(ref) > 1024 and len(set(ref)) > 100
+    for mode in (1, 0):
+        with _sync_mode(mode):
+            out = sim.run_scan(s, st.copy(), cycles, constraints=cons, event_capacity=capacity)
+        assert out["event_count"] == n_ref and out["overflow"] == (n_ref > capacity), mode
+        kept = when(out["events"])
+        assert len(kept) == min(n_ref, capacity)
+        assert kept == sorted(kept), mode
+        assert sum(k < kept[-1] for k in kept) == sum(k < kept[-1] for k in ref), mode
+        assert all(bytes(e) in full for e in sim.canonical_events(out["events"])), mode
+
+
+class _UnevenBlocks:
+    """Block 0 runs ten partitions of 16 words a cycle, block 1 a single one;
+    all of them read primary inputs only, so nothing but the launch's own
+    rules holds block 1 back, and every word violates its hold limit in every
+    cycle."""
+
+    num_blocks, num_major_stages, sram_storage_size, xprop_enabled = 2, 1, 0, False
+    inputs, per, slow = 256, 16, 10
+    reg_io_state_size = arrival_state_offset = inputs + per * (slow + 1)
+
+    def __init__(self):
+        from handscripts import HDR, M, tree_probe_script
+        rng = np.random.default_rng(3)
+        zeros = np.zeros(256, np.uint32)
+        parts = []
+        for k in range(self.slow + 1):
+            p = tree_probe_script(zeros, zeros, np.full(256, M, np.uint32),
+                                  rng.integers(0, 300, 256), num_ios=self.per)[:-HDR]
+            p[1] = k >= self.slow - 1  # the last of its block
+            p[3] = self.inputs + self.per * k
+            p[-1023::4] = M  # clock enables forced
+            parts.append(p)
+        n = parts[0].size
+        self.blocks_start = np.array([0, n * self.slow, n * (self.slow + 1)], np.uint64)
+        self.blocks_data = np.concatenate(parts + [np.zeros(2048, np.uint32)])
+
+    def effective_state_size(self):
+        return 2 * self.reg_io_state_size
+
+
+@pytest.mark.parametrize("mode", [1, 0])
+@pytest.mark.parametrize("symbol", [False, True])
+def test_a_block_that_runs_ahead_records_no_violation_early(mode, symbol):
+    """An event buffer of a few cycles' violations keeps those of the first
+    cycles, of every block, as grid barriers do."""
+    s = _UnevenBlocks()
+    cycles, ss = 40, s.effective_state_size()
+    rio, each = s.reg_io_state_size, s.per * (s.slow + 1)
+    cons = np.zeros(1 + rio, np.uint32)
+    cons[0] = 60000
+    cons[1 + s.inputs:] = 0xFFFF
+    st = np.zeros((cycles + 1, ss), np.uint32)
+    st[:, :s.inputs] = np.random.default_rng(4).integers(0, 1 << 32, (cycles + 1, s.inputs))
+    st = st.reshape(-1)
+    ref = st.copy()
+    _, n_ref = oracle.run(s, ref, cycles, constraints=cons, event_capacity=1 << 14,
+                          arrival_state_offset=rio)
+    assert n_ref == each * cycles
+    capacity = 1024 if symbol else 5 * each
+    with _sync_mode(mode):
+        out = sim.run_scan(s, st.copy(), cycles, constraints=cons, event_capacity=capacity,
+                           reference_symbols=symbol, validate=False)
+    assert np.array_equal(out["states"], ref)
+    assert out["event_count"] == n_ref and out["overflow"] == 1
+    kept = [int(e["cycle"]) for e in out["events"]]
+    assert kept == [k // each for k in range(capacity)]
