@@ -316,3 +316,104 @@ def test_a_trial_is_one_launch(monkeypatch):
     monkeypatch.setattr(CM, "_torch", lambda: SimpleNamespace(cuda=cuda))
     assert CM.batched_us_per_cycle(None, 2, cycles=16) == pytest.approx(100.0)
     assert calls == ["prepare", "event", "launch", "event"]
+
+
+def _fma(a, b, c):
+    """float32 a * b + c with one rounding: the product is exact in float64,
+    and a sum rounded to odd there rounds to float32 as the exact one does."""
+    p, c = np.asarray(a, np.float64) * np.asarray(b, np.float64), np.asarray(c, np.float64)
+    s = np.asarray(p + c)
+    v = s - p
+    err = (p - (s - v)) + (c - v)
+    even = (s.view(np.int64) & 1) == 0
+    s = np.where((err != 0) & even, np.nextafter(s, np.where(err > 0, np.inf, -np.inf)), s)
+    return s.astype(np.float32)
+
+
+def _chain(acc, a, b):
+    """acc + a[0] b[0] + a[1] b[1] + .. in that order, one rounding each."""
+    for x, y in zip(a, b):
+        acc = _fma(x, y, acc)
+    return acc
+
+
+def _in_order(p, x, t, i, h1, h2, lr):
+    """Forward, gradients, step and loss in float32 with every sum in the
+    order of its index, gradients per 64 samples and then over those."""
+    cut = np.cumsum([h1 * i, h1, h2 * h1, h2, h2])
+    w1, b1, w2, b2, w3, b3 = np.split(p, cut)
+    w1, w2 = w1.reshape(h1, i), w2.reshape(h2, h1)
+    n, zero = len(x), np.float32(0)
+
+    def layer(a, w, b):
+        return _chain(np.broadcast_to(b, (n, len(b))), a.T[:, :, None], w.T[:, None, :])
+
+    a1 = np.maximum(layer(x, w1, b1), zero)
+    a2 = np.maximum(layer(a1, w2, b2), zero)
+    y = layer(a2, w3[None], b3)[:, 0]
+    e = y - t
+    dy = np.float32(2) * e / np.float32(n)
+    d2 = np.where(a2 > 0, dy[:, None] * w3, zero)
+    d1 = _chain(np.zeros((n, h1), np.float32), d2.T[:, :, None], w2[:, None, :])
+    d1 = np.where(a1 > 0, d1, zero)
+    g, loss = np.zeros(len(p), np.float32), zero
+    for s in range(0, n, 64):
+        k = slice(s, s + 64)
+
+        def outer(a, b):
+            return _chain(np.zeros((a.shape[1], b.shape[1]), np.float32), a[k, :, None],
+                          b[k, None, :]).reshape(-1)
+        one = np.ones((n, 1), np.float32)
+        g = g + np.concatenate([outer(d1, x), outer(d1, one), outer(d2, a1), outer(d2, one),
+                                outer(a2, dy[:, None]), outer(dy[:, None], one)])
+        loss = loss + outer((e * e)[:, None], one)[0]
+    return y, g, _fma(np.float32(-lr), g, p), loss / np.float32(n)
+
+
+def test_fma_rounds_once():
+    """Halfway cases and products below float32's range, against the exact
+    sum."""
+    from fractions import Fraction
+    rng = np.random.default_rng(1)
+    a = np.float32(rng.normal(size=400)) * np.float32(2.0) ** rng.integers(-80, 20, 400)
+    b = np.float32(rng.normal(size=400)) * np.float32(2.0) ** rng.integers(-80, 20, 400)
+    c = np.where(rng.random(400) < 0.5, -(a * b).astype(np.float32), np.float32(1)).astype(np.float32)
+    a, b = a.astype(np.float32), b.astype(np.float32)
+    a[0], b[0], c[0] = 1 + 2.0 ** -12, 1 + 2.0 ** -12, 1  # tie to even in two roundings
+    for x, y, z, r in zip(a.tolist(), b.tolist(), c.tolist(), _fma(a, b, c).tolist()):
+        exact = Fraction(x) * Fraction(y) + Fraction(z)
+        near = [np.nextafter(np.float32(r), np.float32(d)) for d in (-np.inf, np.inf)]
+        assert all(abs(exact - Fraction(r)) <= abs(exact - Fraction(float(q))) for q in near)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dims,n", [((24, 64, 64), 128), ((17, 33, 5), 71)])
+@pytest.mark.parametrize("scale", [1.0, 1e-20])
+def test_gpu_sums_run_in_the_order_of_their_index(dims, n, scale):
+    """Every output bit of the matrix-instruction kernels is that of loops
+    over the summed index with one rounding a product, on whole tiles and off
+    them, and with products below the normal range of float32."""
+    import torch
+    from jacquard_amd import _native as N
+    from jacquard_amd.costmodel import MLP
+    i, h1, h2 = dims
+    rng = np.random.default_rng(n)
+    x = (scale * rng.normal(size=(n, i))).astype(np.float32)
+    t = rng.normal(size=n).astype(np.float32)
+    p = mo.init(i, h1, h2, seed=9).astype(np.float32)
+    p += (0.05 * rng.normal(size=p.size)).astype(np.float32)
+    p[:h1 * i] *= np.float32(scale)
+    p[h1 * i:h1 * i + h1] *= np.float32(scale * scale)
+    y, g, step, loss = _in_order(p, x, t, i, h1, h2, 0.25)
+    m = MLP(params=p.copy(), i=i, h1=h1, h2=h2)
+    xd, td = torch.from_numpy(x).cuda(), torch.from_numpy(t).cuda()
+    yd = torch.zeros(n, dtype=torch.float32, device="cuda")
+    m.forward_raw(xd, n, yd)
+    ws = torch.zeros(int(N.hip().jq_mlp_workspace_floats(i, h1, h2, n)),
+                     dtype=torch.float32, device="cuda")
+    ld = torch.zeros(1, dtype=torch.float32, device="cuda")
+    m.train_step_raw(xd, td, n, 0.25, ws, ld)
+    assert np.array_equal(yd.cpu().numpy(), y)
+    assert np.array_equal(m.grads.cpu().numpy(), g)
+    assert np.array_equal(m.params.cpu().numpy(), step)
+    assert ld.item() == loss
