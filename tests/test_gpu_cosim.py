@@ -206,3 +206,38 @@ def test_cosim_rejects_a_short_constraint_buffer():
     with pytest.raises(ValueError):
         cosim.Cosim(s, sched, doms, constraints=cons[:-1])
 
+
+
+@pytest.mark.parametrize("blocks,edges,batch", [(300, 40, 25), (512, 9, 4)])
+def test_cosim_of_more_blocks_than_compute_units(blocks, edges, batch):
+    # two workgroups share a compute unit; batches on both sides of the 8
+    # edges from which first-stage permutations are composed
+    import torch
+    from jacquard_amd.netlist import Netlist
+    from jacquard_amd.script import Compiled
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    nl = Netlist.random(seed=5, gates=40000, depth=24, dffs=3000, inputs=64, outputs=32,
+                        geometric_p=0.3, invert_prob=0.5)
+    comp = Compiled(nl, level_split=8, max_part_nodes=400)
+    s = comp.flatten(blocks)
+    assert max(comp.parts_per_stage()) > cus and cus < blocks <= 2 * cus
+    doms = [d for _, d in cosim.clock_domains_of(s)]
+    ins, _ = nl.ports()
+    data_bits = [s.input_map[p] for (_, p, f) in ins if not f and p in s.input_map]
+    doms.append(cosim.ClockDomain(data_bits[0], [data_bits[1]], [data_bits[2]]))
+    sched = cosim.MultiClockScheduler([cosim.ClockTiming(5000, 0, 0),
+                                       cosim.ClockTiming(7500, 2500, 1)])
+    consts = [(b, 1) for b in data_bits[3:20]]
+    print(f"cosim: {blocks} blocks, {s.num_major_stages} major stages, {edges} edges", flush=True)
+    c = cosim.Cosim(s, sched, doms, constants=consts)
+    got = c.run(edges, batch=batch, trace=True)
+    ops, start = [], [0]
+    for k in range(len(sched)):
+        ops += sched.edge_ops(k, doms, None, 0, consts, [])
+        start.append(len(ops))
+    st = np.zeros(2 * s.effective_state_size(), np.uint32)
+    exp = co.run_edges(s, st, np.asarray(ops, np.uint32).reshape(-1, 2),
+                       np.asarray(start, np.uint32), 0, edges)
+    bad = np.nonzero((got != exp).any(axis=1))[0]
+    assert bad.size == 0, f"first differing edge {bad[:1]}"
+    assert np.array_equal(c.snapshots(), st)

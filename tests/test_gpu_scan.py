@@ -783,3 +783,36 @@ def test_a_block_that_runs_ahead_records_no_violation_early(mode, symbol):
     assert out["event_count"] == n_ref and out["overflow"] == 1
     kept = [int(e["cycle"]) for e in out["events"]]
     assert kept == [k // each for k in range(capacity)]
+
+
+@pytest.mark.parametrize("kind", ["torch", "handle"])
+def test_device_output_changes_on_a_stream_of_the_caller(kind):
+    """The records of a run whose snapshots reach the device on a side stream,
+    extracted on that stream while the current one keeps allocating and
+    overwriting: those of the default call, from a torch stream and from an
+    object that holds a stream's handle."""
+    from types import SimpleNamespace
+
+    import torch
+    from jacquard_amd import vcd
+    nl, comp = design("xp", level_split=8, seed=5, gates=20000, depth=40,
+                      dffs=2000, inputs=64, outputs=32, geometric_p=0.3, srams=2)
+    s = comp.flatten(16)
+    cycles, rio = 300, s.reg_io_state_size
+    st = stimulus.build_states(s, cycles, seed=17, p=0.4)
+    offs = [((k + 1) * rio, vcd.U64_MAX if k % 7 == 3 else 10 * k) for k in range(cycles)]
+    d = sim.run_scan(s, st, cycles, return_device=True)["device"]["states"]
+    cnt, rec = vcd.output_changes_device(s, d, offs)
+    assert rec.size > 0
+    side = torch.cuda.Stream()
+    stream = side if kind == "torch" else SimpleNamespace(cuda_stream=side.cuda_stream)
+    for k in range(3):
+        late = torch.zeros_like(d)
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            late.copy_(d)
+        junk = [torch.full((1 << 12,), -1, dtype=torch.int32, device="cuda") for _ in range(8)]
+        got_cnt, got_rec = vcd.output_changes_device(s, late, offs, stream=stream)
+        junk += [torch.full((1 << 12,), -1, dtype=torch.int32, device="cuda") for _ in range(8)]
+        assert np.array_equal(got_cnt, cnt) and np.array_equal(got_rec, rec), k
+        assert torch.cuda.current_stream() != side
