@@ -401,10 +401,12 @@ def output_changes_device(script, d_states, offsets_timestamps, stream=None):
                        CONST0_BIT if pos is None else pos
                        for lit, pos, _ in mapping], np.uint32)
     n = snaps.size
-    if n == 0:
-        return np.zeros(0, np.uint32), np.zeros(0, np.uint32)
+    if n == 0 or bits.size == 0:
+        return np.zeros(n, np.uint32), np.zeros(0, np.uint32)
+    # tensors of the current stream: the first snapshot emits every output, so
+    # the copy of the records waits for the last kernel that reads them
     d_off = to_device(snaps * np.uint64(ess))
-    d_bits = to_device(bits if bits.size else np.zeros(1, np.uint32))
+    d_bits = to_device(bits)
     xoff = rio if script.xprop_enabled else 0
     st = stream if stream is not None else torch.cuda.current_stream()
     if not isinstance(st, torch.cuda.Stream):

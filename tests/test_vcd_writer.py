@@ -123,3 +123,17 @@ def test_timed_body_matches_the_restatement(ps_per_unit):
     assert times == sorted(times)
     if ps_per_unit > 0:
         assert max(times) > 2**64 - 1, "some shift passes the end of the u64 range"
+
+
+def test_output_changes_without_outputs_launch_nothing():
+    """A script without output ports has no records: the counts are zero for
+    every emitted snapshot, with no tensor left for a kernel still to read."""
+    from types import SimpleNamespace
+    script = SimpleNamespace(
+        reg_io_state_size=8, xprop_enabled=False, effective_state_size=lambda: 8,
+        netlist=SimpleNamespace(arrays=lambda: {"drv": np.zeros(1, np.uint8)},
+                                ports=lambda: ([], [])))
+    offs = [(8 * k, vcd.U64_MAX if k == 2 else 10 * k) for k in range(5)]
+    counts, records = vcd.output_changes_device(script, None, offs)
+    assert counts.dtype == records.dtype == np.uint32
+    assert counts.tolist() == [0, 0, 0, 0] and records.size == 0
