@@ -257,12 +257,13 @@ usize jq_wait_limit(usize polls);
  *
  * In either mode a launch of 8 cycles or more, and a co-simulation launch of
  * 8 edges or more, composes the first-stage permutations of its partitions
- * ahead of the cycles (18 KB per partition, 64 MiB at most with the ring;
- * partitions past that use the script's own).  The ring and the permutations
- * are the one allocation a launch makes, taken with hipMallocAsync on the
- * launch's stream and released with hipFreeAsync after it.  If it fails, or
- * while the stream is being captured into a graph, the launch uses grid
- * barriers and the script's permutations. */
+ * ahead of the cycles (18 KB per partition, as many as fit 64 MiB beside the
+ * ring; partitions past that use the script's own, and a ring that is larger
+ * by itself leaves room for none).  The ring and the permutations are the
+ * one allocation a launch makes, taken with hipMallocAsync on the launch's
+ * stream and released with hipFreeAsync after it.  If it fails, the ring is
+ * asked for alone; if that fails, or while the stream is being captured into
+ * a graph, the launch uses grid barriers and the script's permutations. */
 int jq_scan_sync_mode(int mode);
 
 /* ---- Output change extraction (no counterpart in the reference) ---------

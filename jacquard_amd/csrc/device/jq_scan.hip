@@ -105,8 +105,8 @@ __device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70
 // with one thread per word the 32 LDS bit-gathers and the pext loop were
 // twice as long, and each SIMD had a single wave to issue from.  Two
 // threads also halve the registers a thread needs for prefetched words
-// (194 of the 256 that two waves per SIMD leave; one thread per word had
-// spilled).  Measured together with the earlier loads, in launches that keep
+// (188 of the 256 that two waves per SIMD leave, 203 with timing; one thread
+// per word took all 256 and 53 accumulation registers).  Measured together with the earlier loads, in launches that keep
 // grid barriers: 4M gates with X and timing, 248 -> 202 us per cycle; one
 // co-simulation edge of a one-block design, 12.1 -> 10.5 us.
 constexpr int kScanThreads = 512;
@@ -1743,10 +1743,11 @@ int launch_scan(ScanArgs &A, hipStream_t stream) {
 //
 // Every prepared launch has the composed permutations, with slots for one
 // partition per block and major stage (what a script as wide as its widest
-// stage holds) or up to eight of a narrower one's, in at most kPrepareBytes
-// altogether: a stream-ordered allocation of 64 MiB takes and returns in 60
-// us, one of 66 MiB takes 370.  Where the memory is not to be had the launch
-// does without them.
+// stage holds) or up to eight of a narrower one's, as many as fit
+// kPrepareBytes beside the ring (a ring that is larger by itself leaves them
+// no room): a stream-ordered allocation of 64 MiB takes and returns in 60 us,
+// one of 66 MiB takes 370.  Where the memory is not to be had the launch does
+// without them.
 constexpr size_t kPrepareBytes = (size_t)64 << 20;
 
 void *prepare(ScanArgs &A, u32 cycles, bool flow, bool local, hipStream_t stream) {
