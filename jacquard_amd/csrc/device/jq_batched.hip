@@ -186,6 +186,7 @@ constexpr u32 kOldRows = 64;
 
 // Source lane-words of this thread's first-layer positions t + kT * j.
 constexpr int kG = kLayerWords / kT;
+static_assert(kG < 16, "the low four bits of a vmcnt");
 __device__ __forceinline__ void load_sources(u32 (&src)[kG], const u32 *gsrc) {
 #pragma unroll
   for (int j = 0; j < kG; ++j) src[j] = gsrc[threadIdx.x + kT * j];
@@ -271,6 +272,12 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
   // section buffer k & 1 (pointer arithmetic, not an array: no scratch)
   auto secb = [lds](u32 k) { return lds + 2 * kLayerWords + (k & 1u) * kSecWords; };
   size_t pi = 0;
+  // state lane-words of the next partition's first layer, loaded during
+  // the current partition when both are in this major stage (their sources
+  // are earlier major stages and the previous snapshot, complete since the
+  // barrier before this stage)
+  u32 vnext[kG];
+  bool have_next = false;
   for (;; gsrc += kLayerWords) {
     const u32 S = uniform(h.a.x);
     if (S == 0) {  // no partition in this stage: fetch the next stage's first
@@ -289,17 +296,18 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
 
     sec_fetch(secg, secb(0));
     // ---- global read through the gather table: kG independent loads per
-    // thread of state words at entries prefetched one partition ahead.  They
-    // belong to the partition's own ticks wherever it stands in its block:
-    // requested beside the preceding partition's stages (4M gates 4 x 64
-    // 15661 us so, 15775 as here; 1M gates 8 x 32 11842 and 12179) they made
-    // the first of a block 30% longer than the same partition elsewhere (as
-    // here 0.7%), and merging partitions by costs learned from such ticks
-    // gained nothing
+    // thread of state words at entries prefetched one partition ahead (or
+    // the words themselves, when the previous partition of this stage
+    // loaded them)
     u32 old[kOldRows * 32 / kT];
     {
       u32 w[kG];
-      load_words<WIDE>(w, src, B, in, out);
+      if (have_next) {
+#pragma unroll
+        for (int j = 0; j < kG; ++j) w[j] = vnext[j];
+      } else {
+        load_words<WIDE>(w, src, B, in, out);
+      }
       u32 *layer = layerb(0);
       // the commit's old values (this partition's writeouts in the previous
       // snapshot, which nothing changes during the cycle) load now and land
@@ -319,6 +327,12 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
     const u32 next_s = uniform(h.a.x);
     if (next_s != 0) load_sources(src, is_last ? ngsrc : gsrc + kLayerWords);
 
+    // in a profiled cycle every partition gathers for itself, so its ticks are
+    // its own wherever it stands in its block: with the gather beside the
+    // preceding partition's stages the first of a block had 30% more than the
+    // same partition elsewhere (2.7% so), and merging partitions by costs
+    // learned from such ticks gained nothing
+    have_next = !is_last && next_s != 0 && !prof;
     const u32 nperm = ns * 4 + nd;  // SRAM port and duplicate words
     // ---- boomerang stages: every thread gathers its 8 level-1 operands
     // from one layer and writes its gates to the other, so no wave waits for
@@ -352,6 +366,17 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
       else
         row_fetch(secg + (size_t)kSecWords * (nperm ? S : S + 1), secb(S),
                   nperm ? nperm : num_ios);
+      // the next partition of this stage: its first-layer words, beside this
+      // one's gates and tree (its entries arrived during the operand reads,
+      // and nothing looks at them before).  The gather is bound by the CU's
+      // bytes per clock, the stages by LDS and instructions: one after the
+      // other, 4M gates 4 x 64 took 16326 us and 1M gates 8 x 32 12514, beside
+      // each other 15729 and 11835
+      if (s == 0 && have_next) {
+#pragma unroll
+        for (int j = 0; j < kG; ++j) asm volatile("" : "+v"(src[j]));
+        load_words<WIDE>(vnext, src, B, in, out);
+      }
       // levels 1..5 of the subtree rooted at position 256 + v; gate g's
       // flags are bit g of F.x / F.y / F.z, this quarter's 4-apart gates
       // bits 0, 4, .. of the shifted words
@@ -406,7 +431,13 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
           layer[0] = 0;
         }
       }
-      sec_wait();  // section s+1 is read right after this barrier
+      // section s+1 is read right after this barrier; the next partition's
+      // words, kG loads requested after it, are not waited for (WIDE skips the
+      // loads of positions without a source: it cannot count them)
+      if (!WIDE && s == 0 && have_next)
+        __builtin_amdgcn_s_waitcnt(0x0F70 | kG);
+      else
+        sec_wait();
       lds_barrier();
       if ((hook >> 8) == s) {
         const u32 from = 32u * (hook & 255u) + 8 * q4, to = 32 * v + 8 * q4;
