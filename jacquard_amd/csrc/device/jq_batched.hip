@@ -569,11 +569,20 @@ __global__ __launch_bounds__(kT) void batched_kernel(BArgs A) {
     }
   }
   // header and gather entries of the block's first partition of major
-  // stage 0; a block without one has no row of the table there (past the
-  // script's last partition the table ends)
+  // stage 0.  A block without one has no row of the table there (past the
+  // script's last partition the table ends) and reads its header in place of
+  // one: no branch around the loads, for which seven more registers spilled
   u32 src[kG];
-  BHdr h = load_bhdr(A.bd + A.bs[b]);
-  if (uniform(h.a.x) != 0) load_sources(src, A.gsrc + (size_t)A.gidx[b] * kLayerWords);
+  const u32 *first = A.bd + A.bs[b];
+  BHdr h = load_bhdr(first);
+  {
+    const bool none = uniform(h.a.x) == 0;
+    const u32 *row = A.gsrc + (size_t)A.gidx[b] * kLayerWords + t;
+    if (none) row = first;
+    const u32 step = none ? 0 : kT;
+#pragma unroll
+    for (int j = 0; j < kG; ++j) src[j] = row[step * j];
+  }
   __syncthreads();
   u32 c = c0;
   for (;; ++c) {
