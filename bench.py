@@ -1165,11 +1165,12 @@ def batched_hbm(b, profile=None):
     if os.path.exists(profile):
         with open(profile) as f:
             prof = json.load(f)
-        # the profile applies to this script, or to one within 2% of its
-        # size (the tuned split and the learned merge can move a few
-        # partitions between runs)
+        # the profile applies to this script, or to one within 4% of its
+        # size (the learned cut and merge change it by that much and its
+        # traffic by half: 6.06 MB per lane-cycle for the 4M-gate netlist's
+        # script of 190 MB, 6.19 for one of 197 MB)
         pb = prof.get("script_bytes")
-        if pb is None or abs(pb - int(bs.blocks_data.nbytes)) <= 0.02 * pb:
+        if pb is None or abs(pb - int(bs.blocks_data.nbytes)) <= 0.04 * pb:
             out["traffic_gbps"] = prof["hbm_bytes_per_lane_cycle"] * rate / 1e9
             # HBM bytes per launch at this run's lane-cycles per launch
             out["traffic"] = prof["hbm_bytes_per_lane_cycle"] * b["lane_cycles"] / max(
