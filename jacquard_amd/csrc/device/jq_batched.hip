@@ -370,8 +370,9 @@ __device__ __forceinline__ void run_block_lanes(const BArgs &A, const u32 *__res
       // one's gates and tree (its entries arrived during the operand reads,
       // and nothing looks at them before).  The gather is bound by the CU's
       // bytes per clock, the stages by LDS and instructions: one after the
-      // other, 4M gates 4 x 64 took 16326 us and 1M gates 8 x 32 12514, beside
-      // each other 15729 and 11835
+      // other, 1M gates 8 x 32 took 12337 us and 4M gates 4 x 64, where 2% of
+      // the partitions have one before them, 15911; beside each other 11848
+      // and 15653
       if (s == 0 && have_next) {
 #pragma unroll
         for (int j = 0; j < kG; ++j) asm volatile("" : "+v"(src[j]));
